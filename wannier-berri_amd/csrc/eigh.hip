@@ -1,14 +1,15 @@
 // Batched Hermitian eigensolver of libwbmi: cyclic two-sided Jacobi.
 //
-// One 64-lane workgroup per k-point; the matrix A and the accumulated
-// rotations V stay in LDS for the whole solve.  Each Jacobi step rotates
-// nw/2 disjoint (p, q) pairs of the round-robin (circle) ordering at once:
-// all column updates (A G and V G), a barrier, all row updates (G^+ A).
-// The complex rotation is G = diag(1, e^{-i phi}) R diag(1, e^{i phi}) with
-// a_pq = |a_pq| e^{i phi} and R the real symmetric Jacobi rotation
-// (Golub & Van Loan, Matrix Computations, sec. 8.5.2).  Sweeps stop when a
-// whole sweep applies no rotation.  Eigenvalues are returned ascending with
-// eigenvectors as columns, as np.linalg.eigh does (data_K/data_K.py:213).
+// One workgroup per k-point; the matrix A and the accumulated rotations V stay
+// on the chip for the whole solve (LDS; V in registers above nw = 64).  Each
+// Jacobi step rotates nw/2 disjoint (p, q) pairs of the round-robin (circle)
+// ordering at once.  The complex rotation is
+// G = diag(1, e^{-i phi}) R diag(1, e^{i phi}) with a_pq = |a_pq| e^{i phi} and
+// R the real symmetric Jacobi rotation (Golub & Van Loan, Matrix Computations,
+// sec. 8.5.2).  Sweeps stop when a whole sweep applies no rotation.  Eigenvalues
+// are returned ascending with eigenvectors as columns, as np.linalg.eigh does
+// (data_K/data_K.py:213).  k_eigh_jacobi (any type, run-time size) serves
+// refine = 0; refined solves start from the FP32 kernels below it.
 #include <cfloat>
 
 #include "mfma_c64.h"
@@ -193,63 +194,126 @@ __global__ void __launch_bounds__(64) k_eigh_jacobi(int nw, const cplx<Tin>* __r
     }
 }
 
-// ---------------------------------------------------------------------------
-// FP32 Jacobi for padded sizes n = NT in {16, 32, 64}: the rotations of
-// k_eigh_jacobi, in the same order, with the size known at compile time.  A
-// round's parameters are stored once per pair as {c, s cos phi, s sin phi,
-// p | q << 16}, so an update item is one 16-byte parameter read plus its
-// element loads and stores (four of each in the column phase, two in the row
-// phase), with no per-item index arithmetic beyond two adds.  Lane t owns row
-// (column phase) or column (row phase) t % NT of the pairs t / NT,
-// t / NT + 64 / NT, ...
-// ---------------------------------------------------------------------------
-template <int NT>
-__host__ __device__ constexpr size_t jacobi_c_lds() {
-    return 2 * sizeof(cplx<float>) * NT * (NT + 1) + sizeof(float4) * (NT / 2) + 16;
+// Rotation of one FP32 pivot a_pq with diagonal app, aqq: c, s cos(phi), s sin(phi); false (and
+// the identity) where |a_pq| is below rounding.  FAST: hardware reciprocal and reciprocal square
+// root (1 ulp; c^2 + s^2 = 1 to rounding as with correctly rounded division, in far fewer
+// instructions).
+template <bool FAST>
+__device__ inline bool jacobi_rotation(cplx<float> apq, float app, float aqq, float& c, float& sc, float& ss) {
+    typedef float T;
+    const T g = sqrt(fmaf(apq.re, apq.re, apq.im * apq.im));
+    c = 1;
+    sc = 0;
+    ss = 0;
+    const T scale = fabs(app) > fabs(aqq) ? fabs(app) : fabs(aqq);
+    if (!(g > (T)0.5 * Eps<T>::v * scale && g > (T)1e-36)) return false;
+    if constexpr (FAST) {
+        const T rg = __builtin_amdgcn_rcpf(g);
+        const T tau = (aqq - app) * (T)0.5 * rg;
+        const T ta = __builtin_amdgcn_rcpf(fabs(tau) + sqrt((T)1 + tau * tau));
+        const T t = tau >= 0 ? ta : -ta;
+        c = __builtin_amdgcn_rsqf((T)1 + t * t);
+        const T s = t * c;
+        sc = s * apq.re * rg;
+        ss = s * apq.im * rg;
+    } else {
+        const T tau = (aqq - app) / (2 * g);
+        const T t = (tau >= 0 ? (T)1 : (T)-1) / (fabs(tau) + sqrt((T)1 + tau * tau));
+        c = (T)1 / sqrt((T)1 + t * t);
+        const T s = t * c;
+        sc = s * apq.re / g;
+        ss = s * apq.im / g;
+    }
+    return true;
 }
 
-// U0 (optional, NT <= 32): approximate eigenvectors (columns), e.g. those of
+// The two updates, each product pair as a multiplication and an explicit fma: complex64 vectors
+// are stored in the last bit these give, so it is not left to the compiler's contraction.
+// Columns p, q of one row: x_p <- c x_p - s e^{-i phi} x_q, x_q <- s e^{i phi} x_p + c x_q.
+// IMRE: the imaginary part of s e^{i phi} x_p starts from the product with x_p's imaginary part.
+template <bool IMRE>
+__device__ inline void rotate_cols(cplx<float>& xp, cplx<float>& xq, float c, float sc, float ss) {
+    const cplx<float> p = xp, q = xq;
+    xp.re = fmaf(c, p.re, -fmaf(q.re, sc, q.im * ss));
+    xp.im = fmaf(c, p.im, -fmaf(q.im, sc, -(q.re * ss)));
+    xq.re = fmaf(c, q.re, fmaf(p.re, sc, -(p.im * ss)));
+    xq.im = fmaf(c, q.im, IMRE ? fmaf(ss, p.re, sc * p.im) : fmaf(p.im, sc, p.re * ss));
+}
+// Rows p, q of one column: x_p <- c x_p - s e^{i phi} x_q, x_q <- s e^{-i phi} x_p + c x_q
+__device__ inline void rotate_rows(cplx<float>& xp, cplx<float>& xq, float c, float sc, float ss) {
+    const cplx<float> p = xp, q = xq;
+    xp.re = fmaf(c, p.re, -fmaf(sc, q.re, -(ss * q.im)));
+    xp.im = fmaf(c, p.im, -fmaf(ss, q.re, sc * q.im));
+    xq.re = fmaf(c, q.re, fmaf(p.re, sc, p.im * ss));
+    xq.im = fmaf(c, q.im, fmaf(p.im, sc, -(p.re * ss)));
+}
+
+// ---------------------------------------------------------------------------
+// FP32 Jacobi for padded sizes n = N <= 64: the rotations of k_eigh_jacobi, in the same order,
+// with the size known at compile time and A and V in LDS.  A round's N/2 pairs cut A into
+// (N/2)^2 blocks of rows {p_i, q_i} x columns {p_j, q_j}: a thread loads a block, rotates its
+// columns by pair j and its rows by pair i and stores it, so that every element of A is read
+// and written once a round (a column phase and a row phase, with a barrier between them, moved
+// them twice); V's column pairs are dealt out the same way in the same phase.  Every element
+// still sees the column rotation first, so the bits are those of the two phases.
+// Bound: VALU issue (about 390 instructions a round and wave at N = 32, 64 LDS operations) and,
+// for few k-points, the latency of a round.
+// One wave per k for N <= 32, four above (LDS holds four such workgroups a CU at N = 48).
+// The parameters of N = 16, 32 and 64 use the hardware reciprocals.
+// Measured against k_eigh_jacobi (sizes at run time, two phases): 9.1 -> 2.6 ms for 3898 k-points
+// at nw = 48, 1.05 -> 0.62 ms for 6112 at nw = 24, 165 -> 67 us for 1728 at nw = 12.
+// ---------------------------------------------------------------------------
+template <int N>
+__host__ __device__ constexpr int jacobi_b_threads() {
+    return N <= 32 ? 64 : 256;
+}
+template <int N>
+__host__ __device__ constexpr size_t jacobi_b_lds() {
+    return sizeof(float4) * (N / 2) + 2 * sizeof(cplx<float>) * N * (N + 1) + sizeof(int) * (N + 2);
+}
+
+// U0 (optional, N = 16 and 32): approximate eigenvectors (columns), e.g. those of
 // the same k-point index in the neighbouring K-block.  The sweeps then run on
 // A = U0^+ H U0 (both products on the FP64 matrix cores, stored in FP32) with
 // the rotations accumulated onto V = U0: a nearly diagonal start needs about
 // three active sweeps instead of six or seven.  Any unitary U0 gives the same
 // eigen-decomposition; a poor one only costs sweeps.
-// (no minimum waves per SIMD: with 4 the kernel keeps 116 VGPRs and no AGPRs but runs 15 %
-// slower than at 2 waves per SIMD with 64 AGPRs, its LDS traffic being the limit)
-template <int NT, typename Tin, typename TO>
-__global__ void __launch_bounds__(64) k_eigh_jacobi_c(int nw, const cplx<Tin>* __restrict__ H, int64_t Hstride,
-                                                      double* __restrict__ Eout, cplx<TO>* Uout,
-                                                      int max_sweeps, const cplx<TO>* U0) {
+template <int N, typename Tin, typename TO>
+__global__ void __launch_bounds__(jacobi_b_threads<N>()) k_eigh_jacobi_b(int nw, const cplx<Tin>* __restrict__ H,
+                                                                        int64_t Hstride, double* __restrict__ Eout,
+                                                                        cplx<TO>* Uout, int max_sweeps,
+                                                                        const cplx<TO>* U0) {
     typedef float T;
-    constexpr int n = NT, ld = NT + 1, np = NT / 2;
-    constexpr int LPR = 64 / NT;          // pair stride of a lane
-    constexpr int IPL = np / LPR;         // update items per lane and phase
-    constexpr int B = IPL < 8 ? IPL : 8;  // items per load batch
-    static_assert(NT % 2 == 0 && 64 % NT == 0 && IPL % B == 0, "NT must be 16, 32 or 64");
-    extern __shared__ char smem[];
-    cplx<T>* A = (cplx<T>*)smem;
+    constexpr int NTH = jacobi_b_threads<N>();
+    constexpr int n = N, ld = N + 1, np = N / 2;
+    constexpr int NB = np * np, NV = np * N;                          // A blocks and V items of a round
+    constexpr int IB = (NB + NTH - 1) / NTH, IV = (NV + NTH - 1) / NTH;  // per thread
+    constexpr bool FAST = N == 16 || N == 32 || N == 64;
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    float4* prm = (float4*)smem;  // per pair: c, s cos(phi), s sin(phi), p | q << 16
+    cplx<T>* A = (cplx<T>*)(prm + np);
     cplx<T>* V = A + n * ld;
-    float4* prm = (float4*)(V + n * ld);  // 16-byte aligned: 16 n (n + 1) bytes precede it
-    int* flag = (int*)(prm + np);
+    int* rank = (int*)(V + n * ld);
+    int* flags = rank + n;  // round flag, double-buffered by round parity (four-wave workgroups)
     const int tid = threadIdx.x;
     const int64_t k = blockIdx.x;
     const cplx<Tin>* Hk = H + k * Hstride;
 
     bool warm = false;
-    if constexpr (NT <= 32) warm = U0 != nullptr;
+    if constexpr (N == 16 || N == 32) warm = U0 != nullptr;
     if (!warm) {
-        for (int i = tid; i < n; i += 64)
-            for (int j = 0; j < n; ++j) {
-                cplx<T> a = mk((T)0, (T)0);
-                if (i < nw && j < nw) {
-                    cplx<Tin> x = Hk[i * nw + j], y = Hk[j * nw + i];
-                    a = mk((T)(0.5 * (x.re + y.re)), (T)(0.5 * (x.im - y.im)));
-                }
-                A[i * ld + j] = a;
-                V[i * ld + j] = mk((T)(i == j ? 1 : 0), (T)0);
+        for (int t = tid; t < n * n; t += NTH) {
+            const int i = t / n, j = t % n;
+            cplx<T> a = mk((T)0, (T)0);
+            if (i < nw && j < nw) {
+                cplx<Tin> x = Hk[i * nw + j], y = Hk[j * nw + i];
+                a = mk((T)(0.5 * (x.re + y.re)), (T)(0.5 * (x.im - y.im)));
             }
+            A[i * ld + j] = a;
+            V[i * ld + j] = mk((T)(i == j ? 1 : 0), (T)0);
+        }
         __syncthreads();
-    } else if constexpr (NT <= 32) {
+    } else if constexpr (N == 16 || N == 32) {
         // V = U0 (identity on the padding index of odd nw)
         const cplx<TO>* U0k = U0 + k * nw * nw;
         for (int t = tid; t < n * n; t += 64) {
@@ -300,160 +364,171 @@ __global__ void __launch_bounds__(64) k_eigh_jacobi_c(int nw, const cplx<Tin>* _
         __syncthreads();
     }
 
-    const int lr = tid % NT;
-    const int pr0 = tid / NT;
-    const T eps = Eps<T>::v;
+    // the thread's blocks: row pair i, column pair j; its V items: row, pair
+    int bij[IB], vij[IV];
+#pragma unroll
+    for (int u = 0; u < IB; ++u) {
+        const int b = tid + NTH * u;
+        bij[u] = (b / np) | (b % np) << 16;
+    }
+#pragma unroll
+    for (int u = 0; u < IV; ++u) {
+        const int b = tid + NTH * u;
+        vij[u] = (b / n) | (b % n) * ld << 16;  // pair, offset of the row
+    }
     for (int sweep = 0; sweep < max_sweeps; ++sweep) {
-        if (tid == 0) *flag = 0;
-        __syncthreads();
+        bool swept = false;
         for (int r = 0; r < n - 1; ++r) {
             bool rot = false;
             if (tid < np) {
                 int p, q;
                 rr_pair(n, r, tid, p, q);
-                cplx<T> apq = A[p * ld + q];
-                T g = sqrt(apq.re * apq.re + apq.im * apq.im);
-                T app = A[p * ld + p].re, aqq = A[q * ld + q].re;
-                T c = 1, sc = 0, ss = 0;
-                T scale = fabs(app) > fabs(aqq) ? fabs(app) : fabs(aqq);
-                if (g > (T)0.5 * eps * scale && g > (T)1e-36) {
-                    // hardware reciprocal and reciprocal square root (1 ulp): c^2 + s^2 = 1 to
-                    // rounding as with correctly rounded division, in far fewer instructions
-                    const T rg = __builtin_amdgcn_rcpf(g);
-                    const T tau = (aqq - app) * (T)0.5 * rg;
-                    const T ta = __builtin_amdgcn_rcpf(fabs(tau) + sqrt((T)1 + tau * tau));
-                    const T t = tau >= 0 ? ta : -ta;
-                    c = __builtin_amdgcn_rsqf((T)1 + t * t);
-                    const T s = t * c;
-                    sc = s * apq.re * rg;
-                    ss = s * apq.im * rg;
-                    rot = true;
-                    *flag = 1;
-                }
+                T c, sc, ss;
+                rot = jacobi_rotation<FAST>(A[p * ld + q], A[p * ld + p].re, A[q * ld + q].re, c, sc, ss);
                 prm[tid] = make_float4(c, sc, ss, __int_as_float(p | (q << 16)));
             }
-            // the workgroup is one wavefront: __any is uniform over it
-            if (!__any(rot)) continue;
-            __syncthreads();
-            // columns of A and V:  col_p <- c col_p - s e^{-i phi} col_q ; col_q <- s e^{i phi} col_p + c col_q
+            bool any;
+            if constexpr (NTH == 64) {
+                any = __any(rot);  // the workgroup is one wavefront: uniform over it
+                __syncthreads();
+            } else {
+                // the pairs belong to wave 0; the flag's other buffer is read by no one any more
+                if (tid < 64) {
+                    const bool w = __any(rot);
+                    if (tid == 0) flags[r & 1] = w;
+                }
+                __syncthreads();
+                any = flags[r & 1] != 0;
+            }
+            if (!any) continue;
+            swept = true;
+            constexpr int B = 4;  // items whose loads are issued together
 #pragma unroll
-            for (int b0 = 0; b0 < IPL; b0 += B) {
-                float4 P[B];
-                int op[B], oq[B];
-                cplx<T> ap[B], aq[B], vp[B], vq[B];
+            for (int u0 = 0; u0 < IB; u0 += B) {
+                int o[B][4];
+                cplx<T> x[B][4];
+                float4 pi[B], pj[B];
 #pragma unroll
-                for (int u = 0; u < B; ++u) {
-                    P[u] = prm[pr0 + LPR * (b0 + u)];
-                    const int pq = __float_as_int(P[u].w);
-                    op[u] = lr * ld + (pq & 0xffff);
-                    oq[u] = lr * ld + (pq >> 16);
-                    ap[u] = A[op[u]];
-                    aq[u] = A[oq[u]];
-                    vp[u] = V[op[u]];
-                    vq[u] = V[oq[u]];
+                for (int v = 0; v < B; ++v) {
+                    const int u = u0 + v;
+                    if (u >= IB || (NTH * (u + 1) > NB && tid + NTH * u >= NB)) continue;
+                    pi[v] = prm[bij[u] & 0xffff];
+                    pj[v] = prm[bij[u] >> 16];
+                    const int ri = __float_as_int(pi[v].w), cj = __float_as_int(pj[v].w);
+                    const int rp = (ri & 0xffff) * ld, rq = (ri >> 16) * ld, cp = cj & 0xffff, cq = cj >> 16;
+                    o[v][0] = rp + cp;
+                    o[v][1] = rp + cq;
+                    o[v][2] = rq + cp;
+                    o[v][3] = rq + cq;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) x[v][e] = A[o[v][e]];
                 }
 #pragma unroll
-                for (int u = 0; u < B; ++u) {
-                    const T c = P[u].x;
-                    const cplx<T> se = mk(P[u].y, P[u].z);
-                    A[op[u]] = c * ap[u] - mulc(aq[u], se);
-                    A[oq[u]] = se * ap[u] + c * aq[u];
-                    V[op[u]] = c * vp[u] - mulc(vq[u], se);
-                    V[oq[u]] = se * vp[u] + c * vq[u];
+                for (int v = 0; v < B; ++v) {
+                    const int u = u0 + v;
+                    if (u >= IB || (NTH * (u + 1) > NB && tid + NTH * u >= NB)) continue;
+                    rotate_cols<FAST>(x[v][0], x[v][1], pj[v].x, pj[v].y, pj[v].z);
+                    rotate_cols<FAST>(x[v][2], x[v][3], pj[v].x, pj[v].y, pj[v].z);
+                    rotate_rows(x[v][0], x[v][2], pi[v].x, pi[v].y, pi[v].z);
+                    rotate_rows(x[v][1], x[v][3], pi[v].x, pi[v].y, pi[v].z);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) A[o[v][e]] = x[v][e];
                 }
             }
-            __syncthreads();
-            // rows of A:  row_p <- c row_p - s e^{i phi} row_q ; row_q <- s e^{-i phi} row_p + c row_q
 #pragma unroll
-            for (int b0 = 0; b0 < IPL; b0 += B) {
-                float4 P[B];
-                int op[B], oq[B];
-                cplx<T> ap[B], aq[B];
+            for (int u0 = 0; u0 < IV; u0 += 2 * B) {
+                int op[2 * B], oq[2 * B];
+                cplx<T> xp[2 * B], xq[2 * B];
+                float4 P[2 * B];
 #pragma unroll
-                for (int u = 0; u < B; ++u) {
-                    P[u] = prm[pr0 + LPR * (b0 + u)];
-                    const int pq = __float_as_int(P[u].w);
-                    op[u] = (pq & 0xffff) * ld + lr;
-                    oq[u] = (pq >> 16) * ld + lr;
-                    ap[u] = A[op[u]];
-                    aq[u] = A[oq[u]];
+                for (int v = 0; v < 2 * B; ++v) {
+                    const int u = u0 + v;
+                    if (u >= IV || (NTH * (u + 1) > NV && tid + NTH * u >= NV)) continue;
+                    P[v] = prm[vij[u] & 0xffff];
+                    const int pq = __float_as_int(P[v].w);
+                    op[v] = (vij[u] >> 16) + (pq & 0xffff);
+                    oq[v] = (vij[u] >> 16) + (pq >> 16);
+                    xp[v] = V[op[v]];
+                    xq[v] = V[oq[v]];
                 }
 #pragma unroll
-                for (int u = 0; u < B; ++u) {
-                    const T c = P[u].x;
-                    const cplx<T> se = mk(P[u].y, P[u].z);
-                    A[op[u]] = c * ap[u] - se * aq[u];
-                    A[oq[u]] = mulc(ap[u], se) + c * aq[u];
+                for (int v = 0; v < 2 * B; ++v) {
+                    const int u = u0 + v;
+                    if (u >= IV || (NTH * (u + 1) > NV && tid + NTH * u >= NV)) continue;
+                    rotate_cols<true>(xp[v], xq[v], P[v].x, P[v].y, P[v].z);
+                    V[op[v]] = xp[v];
+                    V[oq[v]] = xq[v];
                 }
             }
             __syncthreads();
         }
-        if (*flag == 0) break;
-        __syncthreads();
+        if (!swept) break;
     }
+    __syncthreads();
     // ascending order: rank of each eigenvalue (ties broken by index)
-    for (int i = tid; i < nw; i += 64) {
-        T ei = A[i * ld + i].re;
-        int rank = 0;
+    for (int i = tid; i < nw; i += NTH) {
+        const T ei = A[i * ld + i].re;
+        int rk = 0;
         for (int j = 0; j < nw; ++j) {
-            T ej = A[j * ld + j].re;
-            rank += (ej < ei) || (ej == ei && j < i);
+            const T ej = A[j * ld + j].re;
+            rk += (ej < ei) || (ej == ei && j < i);
         }
-        Eout[k * nw + rank] = (double)ei;
-        for (int m = 0; m < nw; ++m) {
-            const cplx<T> v = V[m * ld + i];
-            Uout[(k * nw + m) * nw + rank] = mk((TO)v.re, (TO)v.im);
-        }
+        rank[i] = rk;
+        Eout[k * nw + rk] = (double)ei;
+    }
+    __syncthreads();
+    for (int t = tid; t < nw * nw; t += NTH) {
+        const int m = t / nw, i = t % nw;
+        const cplx<T> v = V[m * ld + i];
+        Uout[(k * nw + m) * nw + rank[i]] = mk((TO)v.re, (TO)v.im);
     }
 }
 
 // ---------------------------------------------------------------------------
-// 64 < n <= 128: FP32 Jacobi with A in LDS (132 KB at n = 128) and the
-// eigenvectors in row chunks.  The rotations act on V from the right, so the
-// rows of V are independent; every workgroup of the grid row blockIdx.y runs
-// the same (deterministic) Jacobi on A and accumulates rows [v0, v0 + vr) of
-// V.  Uniform control flow: the round flag is written by wave 0 and read by
-// all waves after a barrier, double-buffered by round parity.
+// 64 < n <= 128: FP32 Jacobi with A in LDS (132 KB at n = 128) and V in registers, one 16-wave
+// workgroup per k.  A is updated in blocks of two rows by two columns as in k_eigh_jacobi_b.
+// V fills no LDS: lane l of every wave stands for pair position l - (64 - n/2) of the circle
+// ordering and holds the elements of that pair's two columns in the wave's rows (rows wave,
+// wave + 16, ...).  From one round to the next the first column of pair i + 1 becomes that of
+// pair i and the second of pair i - 1 that of pair i (rr_pair), so the columns move by one lane
+// (DPP wave shifts; the pairs sit in the top lanes, whose last one takes over its own second
+// column), and after the n - 1 rounds of a sweep every column is back in place.
+// Bound: VALU issue of the one workgroup that fits a CU (A 3.5k, V 2.5k cycles a round at
+// n = 128); keeping V in row chunks of LDS took five workgroups per k, each repeating all of A
+// (150 k-points at nw = 128: 29.1 -> 3.2 ms).
 // ---------------------------------------------------------------------------
-#define JROWS_THREADS 256
+#define JREG_THREADS 1024
+#define JREG_WAVES (JREG_THREADS / 64)
 
-struct ItemWalkN {
-    int pr, i, dp, di;
-    __device__ ItemWalkN(int rows, int tid, int nth) : pr(tid / rows), i(tid % rows), dp(nth / rows), di(nth % rows) {}
-    __device__ inline void next(int rows) {
-        pr += dp;
-        i += di;
-        if (i >= rows) {
-            i -= rows;
-            ++pr;
-        }
-    }
-};
+__host__ __device__ inline size_t jreg_lds(int n) {
+    return sizeof(float4) * (n / 2) + sizeof(cplx<float>) * n * (n + 1) + sizeof(int) * (n + 2);
+}
 
-__host__ __device__ inline size_t jrows_lds(int n, int vr) {
-    const size_t ld = n + 1;
-    return sizeof(cplx<float>) * (n + vr) * ld + sizeof(float) * 3 * (n / 2) + sizeof(int) * (n + 4) + 16;
+// lane l takes lane l + 1's value (the last lane: `last`) / lane l - 1's
+__device__ inline float lane_from_next(float x, float last) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(last), __float_as_int(x), 0x130, 0xf, 0xf, false));
+}
+__device__ inline float lane_from_prev(float x) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(x), __float_as_int(x), 0x138, 0xf, 0xf, false));
 }
 
 template <typename Tin, typename TO>
-__global__ void __launch_bounds__(JROWS_THREADS) k_eigh_jacobi_rows(int nw, const cplx<Tin>* __restrict__ H,
-                                                                   int64_t Hstride, double* __restrict__ Eout,
-                                                                   cplx<TO>* __restrict__ Uout, int max_sweeps,
-                                                                   int vr) {
+__global__ void __launch_bounds__(JREG_THREADS) k_eigh_jacobi_reg(int nw, const cplx<Tin>* __restrict__ H,
+                                                                  int64_t Hstride, double* __restrict__ Eout,
+                                                                  cplx<TO>* __restrict__ Uout, int max_sweeps) {
     typedef float T;
-    extern __shared__ char smem[];
-    const int n = nw + (nw & 1), ld = n + 1, np = n / 2;
-    cplx<T>* A = (cplx<T>*)smem;
-    cplx<T>* V = A + n * ld;  // rows v0 .. v0 + nv - 1 of V
-    T* prm = (T*)(V + vr * ld);
-    int* rank = (int*)(prm + 3 * np);
-    int* flags = rank + n;  // [0] sweep, [1 + r % 2] round
-    const int tid = threadIdx.x;
+    constexpr int RV = 128 / JREG_WAVES;  // rows of V per wave
+    constexpr int IB = 64 * 64 / JREG_THREADS;
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    const int n = nw + (nw & 1), ld = n + 1, np = n / 2, nb = np * np;
+    float4* prm = (float4*)smem;
+    cplx<T>* A = (cplx<T>*)(prm + np);
+    int* rank = (int*)(A + n * ld);
+    int* flags = rank + n;  // round flag, double-buffered by round parity
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int64_t k = blockIdx.x;
-    const int v0 = blockIdx.y * vr;
-    const int nv = n - v0 < vr ? n - v0 : vr;
     const cplx<Tin>* Hk = H + k * Hstride;
-    for (int t = tid; t < n * n; t += JROWS_THREADS) {
+    for (int t = tid; t < n * n; t += JREG_THREADS) {
         const int i = t / n, j = t % n;
         cplx<T> a = mk((T)0, (T)0);
         if (i < nw && j < nw) {
@@ -462,109 +537,92 @@ __global__ void __launch_bounds__(JROWS_THREADS) k_eigh_jacobi_rows(int nw, cons
         }
         A[i * ld + j] = a;
     }
-    for (int t = tid; t < nv * n; t += JROWS_THREADS) {
-        const int r = t / n, j = t % n;
-        V[r * ld + j] = mk((T)(v0 + r == j ? 1 : 0), (T)0);
+    const int first = 64 - np, pos = lane - first;  // pos < 0: no pair
+    int p0 = 0, q0 = 0;
+    if (pos >= 0) rr_pair(n, 0, pos, p0, q0);
+    cplx<T> vp[RV], vq[RV];
+#pragma unroll
+    for (int v = 0; v < RV; ++v) {
+        const int row = wave + JREG_WAVES * v;
+        vp[v] = mk((T)(pos >= 0 && row == p0 ? 1 : 0), (T)0);
+        vq[v] = mk((T)(pos >= 0 && row == q0 ? 1 : 0), (T)0);
+    }
+    int bi[IB], bj[IB];
+#pragma unroll
+    for (int u = 0; u < IB; ++u) {
+        const int b = tid + JREG_THREADS * u;
+        bi[u] = b < nb ? b / np : -1;
+        bj[u] = b % np;
     }
     __syncthreads();
-    const T eps = Eps<T>::v;
     for (int sweep = 0; sweep < max_sweeps; ++sweep) {
-        if (tid == 0) flags[0] = 0;
-        __syncthreads();
+        bool swept = false;
         for (int r = 0; r < n - 1; ++r) {
-            bool rot = false;
-            if (tid < np) {
-                int p, q;
-                rr_pair(n, r, tid, p, q);
-                const cplx<T> apq = A[p * ld + q];
-                const T g = sqrt(apq.re * apq.re + apq.im * apq.im);
-                const T app = A[p * ld + p].re, aqq = A[q * ld + q].re;
-                T c = 1, sc = 0, ss = 0;
-                const T scale = fabs(app) > fabs(aqq) ? fabs(app) : fabs(aqq);
-                if (g > (T)0.5 * eps * scale && g > (T)1e-36) {
-                    const T tau = (aqq - app) / (2 * g);
-                    const T t = (tau >= 0 ? (T)1 : (T)-1) / (fabs(tau) + sqrt((T)1 + tau * tau));
-                    c = (T)1 / sqrt((T)1 + t * t);
-                    const T sn = t * c;
-                    sc = sn * apq.re / g;
-                    ss = sn * apq.im / g;
-                    rot = true;
-                }
-                prm[3 * tid] = c;
-                prm[3 * tid + 1] = sc;
-                prm[3 * tid + 2] = ss;
-            }
             if (tid < 64) {
-                const bool any = __any(rot);
-                if (tid == 0) {
-                    flags[1 + (r & 1)] = any;
-                    if (any) flags[0] = 1;
+                bool rot = false;
+                if (tid < np) {
+                    int p, q;
+                    rr_pair(n, r, tid, p, q);
+                    T c, sc, ss;
+                    rot = jacobi_rotation<false>(A[p * ld + q], A[p * ld + p].re, A[q * ld + q].re, c, sc, ss);
+                    prm[tid] = make_float4(c, sc, ss, __int_as_float(p | (q << 16)));
                 }
+                const bool w = __any(rot);
+                if (tid == 0) flags[r & 1] = w;
             }
             __syncthreads();
-            if (!flags[1 + (r & 1)]) continue;
-            // columns of A (rows i < n) and of the V chunk (rows < nv)
-            for (int part = 0; part < 2; ++part) {
-                cplx<T>* M = part == 0 ? A : V;
-                const int rows = part == 0 ? n : nv;
-                for (ItemWalkN w(rows, tid, JROWS_THREADS); w.pr < np;) {
-                    int ii[JB], pp[JB], qq[JB];
-                    bool ok[JB];
-                    T cc[JB];
-                    cplx<T> se[JB], ap[JB], aq[JB];
+            const bool any = flags[r & 1] != 0;
+            if (any) {
+                swept = true;
 #pragma unroll
-                    for (int u = 0; u < JB; ++u) {
-                        ok[u] = w.pr < np;
-                        const int pr = ok[u] ? w.pr : 0;
-                        rr_pair(n, r, pr, pp[u], qq[u]);
-                        ii[u] = w.i;
-                        w.next(rows);
-                        cc[u] = prm[3 * pr];
-                        se[u] = mk(prm[3 * pr + 1], prm[3 * pr + 2]);
-                        ap[u] = M[ii[u] * ld + pp[u]];
-                        aq[u] = M[ii[u] * ld + qq[u]];
+                for (int u0 = 0; u0 < IB; u0 += 2) {
+                    int o[2][4];
+                    cplx<T> x[2][4];
+                    float4 pi[2], pj[2];
+#pragma unroll
+                    for (int v = 0; v < 2; ++v) {
+                        if (bi[u0 + v] < 0) continue;
+                        pi[v] = prm[bi[u0 + v]];
+                        pj[v] = prm[bj[u0 + v]];
+                        const int ri = __float_as_int(pi[v].w), cj = __float_as_int(pj[v].w);
+                        const int rp = (ri & 0xffff) * ld, rq = (ri >> 16) * ld, cp = cj & 0xffff, cq = cj >> 16;
+                        o[v][0] = rp + cp;
+                        o[v][1] = rp + cq;
+                        o[v][2] = rq + cp;
+                        o[v][3] = rq + cq;
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) x[v][e] = A[o[v][e]];
                     }
 #pragma unroll
-                    for (int u = 0; u < JB; ++u) {
-                        if (!ok[u]) continue;
-                        M[ii[u] * ld + pp[u]] = cc[u] * ap[u] - mulc(aq[u], se[u]);
-                        M[ii[u] * ld + qq[u]] = se[u] * ap[u] + cc[u] * aq[u];
+                    for (int v = 0; v < 2; ++v) {
+                        if (bi[u0 + v] < 0) continue;
+                        rotate_cols<false>(x[v][0], x[v][1], pj[v].x, pj[v].y, pj[v].z);
+                        rotate_cols<false>(x[v][2], x[v][3], pj[v].x, pj[v].y, pj[v].z);
+                        rotate_rows(x[v][0], x[v][2], pi[v].x, pi[v].y, pi[v].z);
+                        rotate_rows(x[v][1], x[v][3], pi[v].x, pi[v].y, pi[v].z);
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) A[o[v][e]] = x[v][e];
                     }
                 }
-            }
-            __syncthreads();
-            // rows of A
-            for (ItemWalkN w(n, tid, JROWS_THREADS); w.pr < np;) {
-                int jj[JB], pp[JB], qq[JB];
-                bool ok[JB];
-                T cc[JB];
-                cplx<T> se[JB], ap[JB], aq[JB];
+                const float4 P = prm[pos >= 0 ? pos : 0];
 #pragma unroll
-                for (int u = 0; u < JB; ++u) {
-                    ok[u] = w.pr < np;
-                    const int pr = ok[u] ? w.pr : 0;
-                    rr_pair(n, r, pr, pp[u], qq[u]);
-                    jj[u] = w.i;
-                    w.next(n);
-                    cc[u] = prm[3 * pr];
-                    se[u] = mk(prm[3 * pr + 1], prm[3 * pr + 2]);
-                    ap[u] = A[pp[u] * ld + jj[u]];
-                    aq[u] = A[qq[u] * ld + jj[u]];
-                }
-#pragma unroll
-                for (int u = 0; u < JB; ++u) {
-                    if (!ok[u]) continue;
-                    A[pp[u] * ld + jj[u]] = cc[u] * ap[u] - se[u] * aq[u];
-                    A[qq[u] * ld + jj[u]] = mulc(ap[u], se[u]) + cc[u] * aq[u];
-                }
+                for (int v = 0; v < RV; ++v) rotate_cols<false>(vp[v], vq[v], P.x, P.y, P.z);
             }
-            __syncthreads();
+            // columns to their pair positions of the next round
+#pragma unroll
+            for (int v = 0; v < RV; ++v) {
+                const cplx<T> tn = mk(lane_from_next(vp[v].re, vq[v].re), lane_from_next(vp[v].im, vq[v].im));
+                const cplx<T> bn = mk(lane_from_prev(vq[v].re), lane_from_prev(vq[v].im));
+                vq[v] = pos == 0 ? tn : bn;
+                vp[v] = pos == 0 ? vp[v] : tn;
+            }
+            if (any) __syncthreads();
         }
-        if (flags[0] == 0) break;
-        __syncthreads();
+        if (!swept) break;
     }
-    // ascending order (ties by index); every chunk computes the same ranks
-    for (int i = tid; i < nw; i += JROWS_THREADS) {
+    __syncthreads();
+    // ascending order (ties by index)
+    for (int i = tid; i < nw; i += JREG_THREADS) {
         const T ei = A[i * ld + i].re;
         int rk = 0;
         for (int j = 0; j < nw; ++j) {
@@ -572,14 +630,21 @@ __global__ void __launch_bounds__(JROWS_THREADS) k_eigh_jacobi_rows(int nw, cons
             rk += (ej < ei) || (ej == ei && j < i);
         }
         rank[i] = rk;
-        if (blockIdx.y == 0) Eout[k * nw + rk] = (double)ei;
+        Eout[k * nw + rk] = (double)ei;
+    }
+    __syncthreads();  // A is read no more: V goes through it, its columns in order
+    if (pos >= 0) {
+#pragma unroll
+        for (int v = 0; v < RV; ++v) {
+            const int row = wave + JREG_WAVES * v;
+            if (row < nw && p0 < nw) A[row * ld + rank[p0]] = vp[v];
+            if (row < nw && q0 < nw) A[row * ld + rank[q0]] = vq[v];
+        }
     }
     __syncthreads();
-    for (int t = tid; t < nv * nw; t += JROWS_THREADS) {
-        const int r = t / nw, i = t % nw;
-        if (v0 + r >= nw) continue;
-        const cplx<T> v = V[r * ld + i];
-        Uout[(k * nw + v0 + r) * nw + rank[i]] = mk((TO)v.re, (TO)v.im);
+    for (int t = tid; t < nw * nw; t += JREG_THREADS) {
+        const cplx<T> v = A[(t / nw) * ld + t % nw];
+        Uout[k * nw * nw + t] = mk((TO)v.re, (TO)v.im);
     }
 }
 
@@ -1085,44 +1150,42 @@ extern "C" size_t wbmi_eigh_work_bytes(int nk, int nw, int prec, int refine) {
     return nk > 0 && nw > 0 ? eigh_work_bytes(nk, nw, refine) : 0;
 }
 
+#define JACOBI_SWEEPS 40
+
+template <int N, typename TU>
+static int launch_jacobi_b(wbmi_ctx* ctx, int nk, int nw, const cplx<double>* H64, int64_t Hstride, double* E,
+                           cplx<TU>* U, const cplx<TU>* U0) {
+    const size_t lds = jacobi_b_lds<N>();
+    if (lds > 64 * 1024)
+        WBMI_HIP_CHECK(ctx, hipFuncSetAttribute((const void*)k_eigh_jacobi_b<N, double, TU>,
+                                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    hipLaunchKernelGGL((k_eigh_jacobi_b<N, double, TU>), dim3(nk), dim3(jacobi_b_threads<N>()), lds, ctx->stream, nw,
+                       H64, Hstride, E, U, JACOBI_SWEEPS, U0);
+    WBMI_LAUNCH_CHECK(ctx);
+    return WBMI_OK;
+}
+
+// the launcher of padded size n = 2 HALF, searched from HALF down
+template <int HALF, typename TU>
+static int launch_jacobi_n(wbmi_ctx* ctx, int nk, int nw, const cplx<double>* H64, int64_t Hstride, double* E,
+                           cplx<TU>* U, const cplx<TU>* U0) {
+    if ((nw + 1) / 2 == HALF) return launch_jacobi_b<2 * HALF, TU>(ctx, nk, nw, H64, Hstride, E, U, U0);
+    if constexpr (HALF > 1)
+        return launch_jacobi_n<HALF - 1, TU>(ctx, nk, nw, H64, Hstride, E, U, U0);
+    else
+        return wbmi_fail(ctx, WBMI_ERR_ARG, "wbmi_eigh: nw = %d", nw);
+}
+
 // FP32 Jacobi of the FP64 Hamiltonian (eigenvectors stored as TU)
 template <typename TU>
 static int jacobi_f32_of_f64(wbmi_ctx* ctx, int nk, int nw, const cplx<double>* H64, int64_t Hstride, double* E,
                              cplx<TU>* U, const cplx<TU>* U0 = nullptr) {
-    const int n = nw + (nw & 1);
-    const int sweeps = 40;
-    if (n == 16 || n == 32 || n == 64) {
-        const void* fn = n == 16 ? (const void*)k_eigh_jacobi_c<16, double, TU>
-                       : n == 32 ? (const void*)k_eigh_jacobi_c<32, double, TU>
-                                 : (const void*)k_eigh_jacobi_c<64, double, TU>;
-        const size_t lds = n == 16 ? jacobi_c_lds<16>() : n == 32 ? jacobi_c_lds<32>() : jacobi_c_lds<64>();
-        WBMI_HIP_CHECK(ctx, hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-        if (n == 16)
-            hipLaunchKernelGGL((k_eigh_jacobi_c<16, double, TU>), dim3(nk), dim3(64), lds, ctx->stream, nw, H64,
-                               Hstride, E, U, sweeps, U0);
-        else if (n == 32)
-            hipLaunchKernelGGL((k_eigh_jacobi_c<32, double, TU>), dim3(nk), dim3(64), lds, ctx->stream, nw, H64,
-                               Hstride, E, U, sweeps, U0);
-        else
-            hipLaunchKernelGGL((k_eigh_jacobi_c<64, double, TU>), dim3(nk), dim3(64), lds, ctx->stream, nw, H64,
-                               Hstride, E, U, sweeps, (const cplx<TU>*)nullptr);
-    } else if (n <= 64) {
-        const size_t lds = 2 * sizeof(cplx<float>) * n * (n + 1) + 3 * sizeof(float) * (n / 2) + 16;
-        WBMI_HIP_CHECK(ctx, hipFuncSetAttribute((const void*)k_eigh_jacobi<float, double, TU>,
-                                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-        hipLaunchKernelGGL((k_eigh_jacobi<float, double, TU>), dim3(nk), dim3(64), lds, ctx->stream, nw, H64, Hstride,
-                           E, U, sweeps);
-    } else {
-        // rows of V per workgroup: what the LDS leaves after A
-        int vr = 1;
-        while (vr < n && jrows_lds(n, vr + 1) <= 160 * 1024) ++vr;
-        const int nchunk = (n + vr - 1) / vr;
-        const size_t lds = jrows_lds(n, vr);
-        WBMI_HIP_CHECK(ctx, hipFuncSetAttribute((const void*)k_eigh_jacobi_rows<double, TU>,
-                                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-        hipLaunchKernelGGL((k_eigh_jacobi_rows<double, TU>), dim3(nk, nchunk), dim3(JROWS_THREADS), lds, ctx->stream,
-                           nw, H64, Hstride, E, U, sweeps, vr);
-    }
+    if (nw <= 64) return launch_jacobi_n<32, TU>(ctx, nk, nw, H64, Hstride, E, U, U0);
+    const size_t lds = jreg_lds(nw + (nw & 1));
+    WBMI_HIP_CHECK(ctx, hipFuncSetAttribute((const void*)k_eigh_jacobi_reg<double, TU>,
+                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    hipLaunchKernelGGL((k_eigh_jacobi_reg<double, TU>), dim3(nk), dim3(JREG_THREADS), lds, ctx->stream, nw, H64,
+                       Hstride, E, U, JACOBI_SWEEPS);
     WBMI_LAUNCH_CHECK(ctx);
     return WBMI_OK;
 }
