@@ -18,13 +18,13 @@
 // cumulative cuts [0, c) of non-additive formulas (static.py:109-117) are
 // two-set partitions evaluated the same way.
 //
-// DerOmega.  With G^{bd} = V^b D'^d, H^{ad} = D'^a V^d and K^{bd} = A^b D'^d,
+// DerOmega.  With G^{bd} = V^b D'^d and K^{bd} = A^b D'^d,
 //   dD.ln = X1^{bd} = -M o [W^{bd} + G^{bd} + G^{db} - D'^b V''^d - D'^d V''^b]
-//   dD.nl = X2^{ad} = -M o [W^{ad} + V''^a D'^d + V''^d D'^a - H^{ad} - H^{da}]
+//   dD.nl = X2^{ad}, X2^{ad}_nl = -conj(X1^{ad}_ln)   (V, W Hermitian, D' anti-Hermitian)
 //   dA.ln = Y1^{bd} = A'^{bd} - D'^d A''^b + K^{bd}
-// (formula/elementary.py:63-70, formula/formula.py:108-118).  X1 and X2 are
-// symmetric in (b, d), so the elementwise terms are folded half-and-half into
-// each product: Q1 = G + (W - S)/2, Q2 = -H + (W + R)/2, Y1 = K + A' - D'A''.
+// (formula/elementary.py:63-70, formula/formula.py:108-118).  X1 is symmetric
+// in (b, d), so the elementwise terms are folded half-and-half into each
+// product: Q1 = G + (W - S)/2, Y1 = K + A' - D'A''.
 // The traces use only diagonal elements of D'^a X1, X2 A^b and D'^a Y1, so
 // every product element is consumed where it is computed: a wave task forms
 // one 16 x 32 block of one of the products on the FP64 matrix cores, adds the
@@ -334,28 +334,6 @@ __host__ __device__ constexpr bool uses_A() {
            F == WBMI_FORMULA_OMEGASPIN || F == WBMI_FORMULA_OMEGAOMEGA || F == WBMI_FORMULA_OMEGAHPLUS;
 }
 
-// The two curl components c whose index pair (alpha_c, beta_c) contains x.
-struct Pair {
-    int c, partner;
-    double sig;
-};
-// x in the second slot for sigma=+1: (sigma=+1: beta_c == x, a = alpha_c; sigma=-1: alpha_c == x, a = beta_c)
-__device__ inline Pair pair_second(int x, int which) {
-    for (int c = 0; c < 3; ++c) {
-        if (which == 0 && c_beta[c] == x) return Pair{c, c_alpha[c], 1.0};
-        if (which == 1 && c_alpha[c] == x) return Pair{c, c_beta[c], -1.0};
-    }
-    return Pair{0, 0, 0.0};
-}
-// x in the first slot for sigma=+1: (sigma=+1: alpha_c == x, b = beta_c; sigma=-1: beta_c == x, b = alpha_c)
-__device__ inline Pair pair_first(int x, int which) {
-    for (int c = 0; c < 3; ++c) {
-        if (which == 0 && c_alpha[c] == x) return Pair{c, c_beta[c], 1.0};
-        if (which == 1 && c_beta[c] == x) return Pair{c, c_alpha[c], -1.0};
-    }
-    return Pair{0, 0, 0.0};
-}
-
 // build M = dEinv o Off for the current labels (data_K.py:290-298)
 __device__ __attribute__((always_inline)) void build_M(const Smem& S, int nw) {
     const int ld = nw + 1;
@@ -383,9 +361,12 @@ __device__ inline double wave_sum(double v, int mask) {
 // the workgroup's per-band rows acc[band][comp] (LDS FP64 atomic adds, .re) after a
 // shuffle reduction over the summed index.  The band of an element is its column y (kind 1 forms its
 // product transposed for this).  Kinds (task indices b, d; for kinds 5, 6 b = c):
-//   0  Q1^{bd} = V^b D'^d + (W - D'^b V''^d - D'^d V''^b)/2, y in the partition, x off-side:
-//      DerOmega T1; DerMorb s2 (x 2 E_x), s7 (conj B^a_xy), s1 (raw V^b D'^d)
-//   1  Q2^{bd} = -D'^b V^d + (W + V''^b D'^d + V''^d D'^b)/2, x in, y off-side: DerOmega T3
+//   0  Q1^{bd} = V^b D'^d + (W - D'^b V''^d - D'^d V''^b)/2, y in the partition, x off-side, so that
+//      X1^{bd} = dD.ln = -M o (Q1^{bd} + Q1^{db}).  V and W Hermitian and D' anti-Hermitian give
+//      dD.nl = X2^{ad}_yx = -conj(X1^{ad}_xy), so every term that holds dD, from the left or from
+//      the right, is Re q^a_yx X1^{bd}_xy with one weight per partner a:
+//        q^a = -i w D'^a_yx - dw conj(A^a_xy) - 2 conj(B^a_xy)
+//      (DerOmega T1 and T3; DerMorb s2 in w, s7); DerMorb s1 reads the raw V^b D'^d
 //   2  Y1^{bd} = A^b D'^d + A' - D'^d A''^b, x off-side: DerOmega T2;
 //      x same-side (DerMorb): s5 terms of A' + A^b D'^d
 //   3  YB^{bd} = B^b D'^d + B' - D'^d B''^b, x off-side: DerMorb s6
@@ -397,34 +378,34 @@ __device__ inline double wave_sum(double v, int mask) {
 // 2 sign E_n (DerMorb's Eav o dOmega term; only cut partitions are summed, so a
 // same-side element may be credited to either of its bands).
 struct TaskCtx {
-    bool dm, in, ex;
+    bool in, ex;
     double sign;
 };
 
-template <int KIND>
+// The component c of a term with index pair (alpha_c, beta_c) = (x, y) (sig +1) or (y, x) (-1), x != y
+__device__ inline int third_index(int x, int y) { return 3 - x - y; }
+__device__ inline double pair_sign(int x, int y) { return y == (x == 2 ? 0 : x + 1) ? 1.0 : -1.0; }
+
+// per-lane sums of a task: 0 - 2 one per partner a = 0, 1, 2; kind 0 of DerMorb: [3] = s1; kind 4:
+// [3] - [5] the Omega block's components; kinds 5, 6: one per e; kind 7: one
+template <int KIND, bool DM>
 __host__ __device__ constexpr int task_nt() {
-    return KIND == 0 ? 5 : KIND == 1 ? 4 : KIND == 2 ? 2 : KIND == 3 ? 2 : KIND == 4 ? 5 : KIND == 7 ? 1 : 3;
+    return KIND == 0 ? (DM ? 4 : 3) : KIND == 4 ? 6 : KIND == 7 ? 1 : 3;
 }
 
-// M1 (kind 0 only): the task also carries the kind-1 task (d, b).  With V
-// Hermitian and D' anti-Hermitian, (D'^d V^b)_yx = -conj((V^b D'^d)_xy), so
-// kind 1's transposed product is -conj of kind 0's at the same element, and
-// its elementwise channel W^{db}_yx = conj(W^{bd}_xy): one product and one
-// load serve both consumers.
-template <int KIND, bool M1, typename T, bool LM, bool ST, bool SA, int NW, typename TS>
+template <int KIND, bool DM, typename T, bool LM, bool ST, bool SA, int NW, typename TS>
 __device__ __attribute__((always_inline)) void formula_task(const Smem& S, const KCtx<T, LM, ST, SA, NW, TS>& K, const TaskCtx& tc_,
                                                            cplx<double>* acc, int b, int d, int rh, int cb) {
+    constexpr bool dm = DM;
     const int nw = K.n_(), lane = threadIdx.x & 63;
     const int r0 = rh * 16, c0 = cb * 32;  // a 16 x 32 half block
-    const bool dm = tc_.dm, in = tc_.in, ex = tc_.ex;
+    const bool in = tc_.in, ex = tc_.ex;
     const double sign = tc_.sign;
     const int al = c_alpha[b], be = c_beta[b];  // kinds 5, 6: b = c
     MfmaHalf P;
     P.zero();
     if constexpr (KIND == 0)
         mfma_half(P, nw, nw, nw, r0, c0, [&](int r, int m) { return K.V(b, r, m); }, [&](int m, int c) { return K.Dp(d, m, c); });
-    else if constexpr (KIND == 1)  // transposed: P_xy = (D'^b V^d)_yx, so the band n = y is a column as for the others
-        mfma_half(P, nw, nw, nw, r0, c0, [&](int r, int m) { return K.V(d, m, r); }, [&](int m, int c) { return K.Dp(b, c, m); });
     else if constexpr (KIND == 2)
         mfma_half(P, nw, nw, nw, r0, c0, [&](int r, int m) { return K.A(b, r, m); }, [&](int m, int c) { return K.Dp(d, m, c); });
     else if constexpr (KIND == 3)
@@ -438,114 +419,19 @@ __device__ __attribute__((always_inline)) void formula_task(const Smem& S, const
     else
         mfma_half(P, nw, nw, nw, r0, c0, [&](int r, int m) { return K.Vin(b, r, m); }, [&](int m, int c) { return K.Ain(d, m, c); });
 
-    // targets: partner component tp, accumulator column tcol, factor tw
-    constexpr int NT = task_nt<KIND>();
-    int tp[NT], tcol[NT];
-    double tw[NT];
-#pragma unroll
-    for (int w = 0; w < NT; ++w) {
-        tp[w] = 0;
-        tcol[w] = 0;
-        tw[w] = 0.0;
-    }
-    if constexpr (KIND == 0 || KIND == 1) {
-        // the two index pairs of X1 / X2: targets coincide for b == d (one lane adds twice)
-        const int nt = b == d ? 2 : 4;
-        const double f = b == d ? 2.0 : 1.0;
-#pragma unroll
-        for (int w = 0; w < 4; ++w) {
-            const Pair p = KIND == 1 ? pair_first(w < 2 ? b : d, w % 2) : pair_second(w < 2 ? b : d, w % 2);
-            tp[w] = p.partner;
-            tcol[w] = p.c * 3 + (w < 2 ? d : b);
-            tw[w] = w < nt ? f * p.sig : 0.0;
-        }
-        if constexpr (KIND == 0) {
-            // s1: the c with beta_c = d, partner alpha_c, column (c, b)
-            for (int c = 0; c < 3; ++c)
-                if (c_beta[c] == d) {
-                    tp[4] = c_alpha[c];
-                    tcol[4] = c * 3 + b;
-                    tw[4] = 2.0;
-                }
-        }
-    } else if constexpr (KIND == 2 || KIND == 3) {
-#pragma unroll
-        for (int w = 0; w < 2; ++w) {
-            const Pair p = pair_second(b, w);
-            tp[w] = p.partner;
-            tcol[w] = p.c * 3 + d;
-            tw[w] = p.sig;
-        }
-    } else if constexpr (KIND == 4) {
-#pragma unroll
-        for (int w = 0; w < 2; ++w) {
-            const Pair p = pair_second(b, w);
-            tp[w] = p.partner;
-            tcol[w] = p.c * 3 + d;
-            tw[w] = p.sig;
-        }
-        // Omega block: D'^d A^b enters s^c with -1 for (al_c, be_c) = (d, b), +1 for (b, d)
-        for (int c = 0; c < 3; ++c) {
-            const double coef = (c_alpha[c] == d && c_beta[c] == b) ? -1.0 : (c_alpha[c] == b && c_beta[c] == d) ? 1.0 : 0.0;
-            if (coef != 0.0)
-                for (int e = 0; e < 3; ++e) {
-                    tp[2 + e] = e;
-                    tcol[2 + e] = c * 3 + e;
-                    tw[2 + e] = 2.0 * sign * coef;
-                }
-        }
-    } else if constexpr (KIND == 5 || KIND == 6) {
-#pragma unroll
-        for (int e = 0; e < 3; ++e) {
-            tp[e] = e;
-            tcol[e] = b * 3 + e;
-            tw[e] = 2.0 * sign;
-        }
-    } else {
-        for (int c = 0; c < 3; ++c)
-            if (c_beta[c] == d) {
-                tp[0] = c_alpha[c];
-                tcol[0] = c * 3 + b;
-                tw[0] = 2.0;
-            }
-    }
-    // targets of the carried kind-1 task (b1, d1) = (d, b)
-    constexpr int NT1 = M1 ? 4 : 1;
-    const int b1 = d, d1 = b;
-    int tp1[NT1], tcol1[NT1];
-    double tw1[NT1];
-#pragma unroll
-    for (int w = 0; w < NT1; ++w) {
-        tp1[w] = 0;
-        tcol1[w] = 0;
-        tw1[w] = 0.0;
-    }
-    if constexpr (M1) {
-        const int nt = b1 == d1 ? 2 : 4;
-        const double f = b1 == d1 ? 2.0 : 1.0;
-#pragma unroll
-        for (int w = 0; w < 4; ++w) {
-            const Pair p = pair_first(w < 2 ? b1 : d1, w % 2);
-            tp1[w] = p.partner;
-            tcol1[w] = p.c * 3 + (w < 2 ? d1 : b1);
-            tw1[w] = w < nt ? f * p.sig : 0.0;
-        }
-    }
-
     // part[u][w]: u = the lane's band slot, its column bj (the band n is the column y of every element)
-    constexpr int NU = 2;
-    double part[NU][NT], part1[NU][NT1];
+    constexpr int NU = 2, NT = task_nt<KIND, DM>();
+    double part[NU][NT];
 #pragma unroll
-    for (int u = 0; u < NU; ++u) {
+    for (int u = 0; u < NU; ++u)
 #pragma unroll
         for (int w = 0; w < NT; ++w) part[u][w] = 0.0;
-#pragma unroll
-        for (int w = 0; w < NT1; ++w) part1[u][w] = 0.0;
-    }
+    // s1: the c with beta_c = d, partner alpha_c
+    const int s1c = d == 2 ? 0 : d + 1;  // beta_c = c + 2
     {
         // the elementwise channel (W, A', B') of this row half: all loads issued before use
         cplx<double> gz[2][4];
-        if constexpr (KIND <= 3) {
+        if constexpr (KIND == 0 || KIND == 2 || KIND == 3) {
 #pragma unroll
             for (int bj = 0; bj < 2; ++bj)
 #pragma unroll
@@ -555,8 +441,6 @@ __device__ __attribute__((always_inline)) void formula_task(const Smem& S, const
                     const int xx = ok ? x : 0, yy = ok ? y : 0;
                     if constexpr (KIND == 0)
                         gz[bj][v] = K.W(b, d, xx, yy);  // (l, n)
-                    else if constexpr (KIND == 1)
-                        gz[bj][v] = conj(K.W(b, d, xx, yy));  // (n, l) of the Hermitian W, read along rows
                     else if constexpr (KIND == 2)
                         gz[bj][v] = ex ? K.Ad(b, d, xx, yy) : mk(0.0, 0.0);
                     else
@@ -564,106 +448,88 @@ __device__ __attribute__((always_inline)) void formula_task(const Smem& S, const
                 }
         }
 #pragma unroll
-        for (int bj = 0; bj < 2; ++bj)
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            const int x = r0 + mfma_hrow(v), y = c0 + mfma_col(bj);
-            if (x >= nw || y >= nw) continue;
-            const int i = bj, j = bj;  // part slot
-            const cplx<double> pv = P.get(bj, v);
-            const int n = y, l = x;
-            if (!S.act[n]) continue;
-            const bool same = K.lab[l] == K.lab[n];
+        for (int bj = 0; bj < 2; ++bj) {
+            const int n = c0 + mfma_col(bj);
+            if (n >= nw || !S.act[n]) continue;
             const bool single = S.ge[n] - S.gs[n] == 1;  // group {n}: the within-group sums have one term
             const double dw = dm ? 2.0 * sign * K.E[n] : 2.0;
-            if constexpr (KIND == 0) {
-                if (same) continue;
-                // (W^{bd} - D'^b V''^d - D'^d V''^b)_ln / 2, with D'_xy = -m_xy V_xy and m_nl = -m_ln
-                const double mln = K.m(l, n);
-                cplx<double> z = gz[bj][v];
-                if (single)
-                    z += mln * (K.V(b, l, n) * K.V(d, n, n) + K.V(d, l, n) * K.V(b, n, n));
-                else
-                    for (int q = S.gs[n]; q < S.ge[n]; ++q)
-                        z -= K.Dp(b, l, q) * K.V(d, q, n) + K.Dp(d, l, q) * K.V(b, q, n);
-                const cplx<double> Pm = (-mln) * (pv + 0.5 * z);
-                const double wD = (in ? dw : 0.0) + (dm && in ? 2.0 * K.E[l] : 0.0);
 #pragma unroll
-                for (int w = 0; w < 4; ++w) {
-                    const cplx<double> Dnl = mln * K.V(tp[w], n, l);
-                    double t = wD * (Dnl * Pm).im;  // Re(-i D' X1) (T1, s2)
-                    if (dm && ex) t -= 2.0 * (conj(K.B(tp[w], l, n)) * Pm).re;  // s7
-                    part[j][w] += t;
-                }
-                if (dm && in) part[j][4] += ((mln * K.V(tp[4], n, l)) * pv).im;  // s1: Re(-i D'^al V^d D'^be)
-                if constexpr (M1) {
-                    // kind 1 (b1, d1): (W^{b1 d1} + V''^b1 D'^d1 + V''^d1 D'^b1)_nl / 2, with P1 = -conj(pv)
-                    const double mnl = -mln;
-                    cplx<double> z1 = conj(gz[bj][v]);
-                    if (single)
-                        z1 -= mnl * (K.V(b1, n, n) * K.V(d1, n, l) + K.V(d1, n, n) * K.V(b1, n, l));
-                    else
-                        for (int q = S.gs[n]; q < S.ge[n]; ++q)
-                            z1 += K.V(b1, n, q) * K.Dp(d1, q, l) + K.V(d1, n, q) * K.Dp(b1, q, l);
-                    const cplx<double> Pm1 = (-mnl) * (0.5 * z1 + conj(pv));
-#pragma unroll
-                    for (int w = 0; w < 4; ++w) part1[i][w] -= dw * (Pm1 * K.A(tp1[w], l, n)).re;
-                }
-            } else if constexpr (KIND == 1) {
-                if (same) continue;
-                // (W^{bd} + V''^b D'^d + V''^d D'^b)_nl / 2
-                const double mnl = K.m(n, l);
-                cplx<double> z = gz[bj][v];
-                if (single)
-                    z -= mnl * (K.V(b, n, n) * K.V(d, n, l) + K.V(d, n, n) * K.V(b, n, l));
-                else
-                    for (int q = S.gs[n]; q < S.ge[n]; ++q)
-                        z += K.V(b, n, q) * K.Dp(d, q, l) + K.V(d, n, q) * K.Dp(b, q, l);
-                const cplx<double> Pm = (-mnl) * (0.5 * z - pv);
-#pragma unroll
-                for (int w = 0; w < 4; ++w) part[i][w] -= dw * (Pm * K.A(tp[w], l, n)).re;
-            } else if constexpr (KIND == 2) {
-                if (!same) {
-                    // A'^{bd} - D'^d A''^b
+            for (int v = 0; v < 4; ++v) {
+                const int l = r0 + mfma_hrow(v);
+                if (l >= nw) continue;
+                const cplx<double> pv = P.get(bj, v);
+                const bool same = K.lab[l] == K.lab[n];
+                if constexpr (KIND == 0) {
+                    if (same) continue;
+                    // (W^{bd} - D'^b V''^d - D'^d V''^b)_ln / 2, with D'_xy = -m_xy V_xy and m_nl = -m_ln
                     const double mln = K.m(l, n);
                     cplx<double> z = gz[bj][v];
                     if (single)
-                        z += mln * (K.V(d, l, n) * K.A(b, n, n));
+                        z += mln * (K.V(d, n, n).re * K.V(b, l, n) + K.V(b, n, n).re * K.V(d, l, n));
                     else
-                        for (int q = S.gs[n]; q < S.ge[n]; ++q) z -= K.Dp(d, l, q) * K.A(b, q, n);
-                    const cplx<double> Y1 = pv + z;
+                        for (int q = S.gs[n]; q < S.ge[n]; ++q)
+                            z -= K.Dp(b, l, q) * K.V(d, q, n) + K.Dp(d, l, q) * K.V(b, q, n);
+                    const cplx<double> Pm = (-mln) * (pv + 0.5 * z);
+                    const double wD = in ? (dm ? dw + 2.0 * K.E[l] : dw) : 0.0;
 #pragma unroll
-                    for (int w = 0; w < 2; ++w) part[j][w] -= dw * ((mln * K.V(tp[w], n, l)) * Y1).re;
-                } else if (dm) {
-                    // s5: Re(-2i sig A^a_nl E_l (A' + A^b D'^d)_ln)
-                    const cplx<double> dA = pv + K.Ad(b, d, l, n);
+                    for (int a = 0; a < 3; ++a) {
+                        // -i wD D'_nl, D'_nl = m_ln conj(V_ln)
+                        const cplx<double> va = K.V(a, l, n);
+                        cplx<double> q = (wD * mln) * mk(-va.im, -va.re);
+                        if (ex) {
+                            q -= dw * conj(K.A(a, l, n));
+                            if (dm) q -= 2.0 * conj(K.B(a, l, n));
+                        }
+                        part[bj][a] += q.re * Pm.re - q.im * Pm.im;
+                    }
+                    if constexpr (DM)
+                        if (in) part[bj][3] += ((mln * conj(K.V(c_alpha[s1c], l, n))) * pv).im;  // Re(-i D'^al V^d D'^be)
+                } else if constexpr (KIND == 2) {
+                    if (!same) {
+                        // A'^{bd} - D'^d A''^b
+                        const double mln = K.m(l, n);
+                        cplx<double> z = gz[bj][v];
+                        if (single)
+                            z += mln * (K.V(d, l, n) * K.A(b, n, n));
+                        else
+                            for (int q = S.gs[n]; q < S.ge[n]; ++q) z -= K.Dp(d, l, q) * K.A(b, q, n);
+                        const cplx<double> Y1 = (-dw * mln) * (pv + z);
 #pragma unroll
-                    for (int w = 0; w < 2; ++w) part[j][w] += 2.0 * K.E[l] * (K.A(tp[w], n, l) * dA).im;
+                        for (int a = 0; a < 3; ++a) {
+                            const cplx<double> va = K.V(a, l, n);
+                            part[bj][a] += va.re * Y1.re + va.im * Y1.im;  // Re conj(V_ln) Y1
+                        }
+                    } else if (dm) {
+                        // s5: Re(-2i sig A^a_nl E_l (A' + A^b D'^d)_ln)
+                        const cplx<double> dA = pv + K.Ad(b, d, l, n);
+#pragma unroll
+                        for (int a = 0; a < 3; ++a) part[bj][a] += 2.0 * K.E[l] * (K.A(a, n, l) * dA).im;
+                    }
+                } else if constexpr (KIND == 3) {
+                    if (same) continue;
+                    // B'^{bd} - D'^d B''^b
+                    cplx<double> z = gz[bj][v];
+                    for (int q = S.gs[n]; q < S.ge[n]; ++q) z -= K.Dp(d, l, q) * K.B(b, q, n);
+                    const cplx<double> YB = pv + z;
+#pragma unroll
+                    for (int a = 0; a < 3; ++a) part[bj][a] -= 2.0 * (K.Dp(a, n, l) * YB).re;  // s6
+                } else if constexpr (KIND == 4) {
+                    if (!same) continue;
+                    // s5: -Re(-2i sig A^a_nl E_l (D'^d A^b)_ln) ; Omega block: 2 sign coef Re(DA_ln V^e_nl)
+#pragma unroll
+                    for (int a = 0; a < 3; ++a) part[bj][a] -= 2.0 * K.E[l] * (K.A(a, n, l) * pv).im;
+#pragma unroll
+                    for (int e = 0; e < 3; ++e) part[bj][3 + e] += (pv * K.V(e, n, l)).re;
+                } else if constexpr (KIND == 5 || KIND == 6) {
+                    if (!same) continue;
+                    // Omega block term -i P_ln: 2 sign Re(-i P_ln V^e_nl)
+#pragma unroll
+                    for (int w = 0; w < 3; ++w) part[bj][w] += (pv * K.V(w, n, l)).im;
+                } else {
+                    if (!same) continue;
+                    // s4: Re(-2i A^al_np (V''^d A''^be)_pn)
+                    part[bj][0] += (K.A(c_alpha[s1c], n, l) * pv).im;
                 }
-            } else if constexpr (KIND == 3) {
-                if (same) continue;
-                // B'^{bd} - D'^d B''^b
-                cplx<double> z = gz[bj][v];
-                for (int q = S.gs[n]; q < S.ge[n]; ++q) z -= K.Dp(d, l, q) * K.B(b, q, n);
-                const cplx<double> YB = pv + z;
-#pragma unroll
-                for (int w = 0; w < 2; ++w) part[j][w] -= 2.0 * (K.Dp(tp[w], n, l) * YB).re;  // s6
-            } else if constexpr (KIND == 4) {
-                if (!same) continue;
-                // s5: -Re(-2i sig A^a_nl E_l (D'^d A^b)_ln) ; Omega block: 2 sign coef Re(DA_ln V^e_nl)
-#pragma unroll
-                for (int w = 0; w < 2; ++w) part[j][w] -= 2.0 * K.E[l] * (K.A(tp[w], n, l) * pv).im;
-#pragma unroll
-                for (int w = 2; w < 5; ++w) part[j][w] += (pv * K.V(tp[w], n, l)).re;
-            } else if constexpr (KIND == 5 || KIND == 6) {
-                if (!same) continue;
-                // Omega block term -i P_ln: 2 sign Re(-i P_ln V^e_nl)
-#pragma unroll
-                for (int w = 0; w < 3; ++w) part[j][w] += (pv * K.V(tp[w], n, l)).im;
-            } else {
-                if (!same) continue;
-                // s4: Re(-2i A^al_np (V''^d A''^be)_pn)
-                part[j][0] += (K.A(tp[0], n, l) * pv).im;
             }
         }
     }
@@ -673,17 +539,34 @@ __device__ __attribute__((always_inline)) void formula_task(const Smem& S, const
 #pragma unroll
     for (int u = 0; u < NU; ++u) {
         const int n = c0 + mfma_col(u);
+        double sum[NT];
 #pragma unroll
-        for (int w = 0; w < NT; ++w) {
-            const double sum = wave_sum(part[u][w], mask);
-            if (writer && tw[w] != 0.0 && n < nw) atomicAdd(&acc[n * 9 + tcol[w]].re, tw[w] * sum);
-        }
-        if constexpr (M1) {
+        for (int w = 0; w < NT; ++w) sum[w] = wave_sum(part[u][w], mask);
+        if (!writer || n >= nw) continue;
+        cplx<double>* row = acc + n * 9;
+        if constexpr (KIND <= 4) {
 #pragma unroll
-            for (int w = 0; w < NT1; ++w) {
-                const double sum = wave_sum(part1[u][w], mask);
-                if (writer && tw1[w] != 0.0 && n < nw) atomicAdd(&acc[n * 9 + tcol1[w]].re, tw1[w] * sum);
+            for (int a = 0; a < 3; ++a) {
+                // the component whose index pair holds b and the partner a: column (c, d); X1 is
+                // symmetric in its indices, so kind 0 also feeds (c', b) of the pair of d and a
+                if (a != b) atomicAdd(&row[third_index(a, b) * 3 + d].re, pair_sign(a, b) * sum[a]);
+                if constexpr (KIND == 0)
+                    if (a != d) atomicAdd(&row[third_index(a, d) * 3 + b].re, pair_sign(a, d) * sum[a]);
             }
+        }
+        if constexpr (KIND == 0 && DM) {
+            if (in) atomicAdd(&row[s1c * 3 + b].re, 2.0 * sum[3]);
+        } else if constexpr (KIND == 4) {
+            // Omega block: D'^d A^b enters s^c with -1 for (al_c, be_c) = (d, b), +1 for (b, d)
+            if (b != d && sign != 0.0)
+#pragma unroll
+                for (int e = 0; e < 3; ++e)
+                    atomicAdd(&row[third_index(b, d) * 3 + e].re, -2.0 * sign * pair_sign(d, b) * sum[3 + e]);
+        } else if constexpr (KIND == 5 || KIND == 6) {
+#pragma unroll
+            for (int e = 0; e < 3; ++e) atomicAdd(&row[b * 3 + e].re, 2.0 * sign * sum[e]);
+        } else if constexpr (KIND == 7) {
+            atomicAdd(&row[s1c * 3 + b].re, 2.0 * sum[0]);
         }
     }
 }
@@ -745,23 +628,19 @@ __device__ __attribute__((always_inline)) void eval_deromega(const Smem& S, cons
     if (tid == 0) S.misc[3] = 0;  // task counter
     __syncthreads();
     // wave tasks (kind, b, d, row block, column block), round-robin over the waves
-    const TaskCtx tcx{dm, in, ex, (double)sign};
+    const TaskCtx tcx{in, ex, (double)sign};
     int cnt[8];
-    cnt[0] = (in || (dm && ex)) ? 9 : 0;
-    cnt[1] = ex ? 9 : 0;
+    cnt[0] = in || ex ? 9 : 0;
+    cnt[1] = 0;
     cnt[2] = ex ? 9 : 0;
     cnt[3] = dm && ex ? 9 : 0;
     cnt[4] = dm && ex ? 9 : 0;
     cnt[5] = dm && in && sign != 0 ? 3 : 0;
     cnt[6] = dm && ex && sign != 0 ? 3 : 0;
     cnt[7] = dm && ex ? 9 : 0;
-    if (dm && sign == 0) cnt[1] = 0;  // T3 feeds only the dOmega term
-    // kind-1 tasks ride on the kind-0 tasks of the transposed index pair when both run
-    const bool merge01 = cnt[0] > 0 && cnt[1] > 0;
-    if (merge01) cnt[1] = 0;
     // a task is one 16-row x 32-column half block of one product; the waves take the next
-    // task from an LDS counter, kinds in the order above (the heaviest, kind 0 with its
-    // carried kind-1 task, first), so the waves finish together whatever the mix of kinds
+    // task from an LDS counter, kinds in the order above (the heaviest, kind 0, first), so the
+    // waves finish together whatever the mix of kinds
     const int nblk = (nw + 31) / 32, nrh = (nw + 15) / 16, nb2 = nrh * nblk;
     int ntask = 0;
 #pragma unroll
@@ -785,22 +664,16 @@ __device__ __attribute__((always_inline)) void eval_deromega(const Smem& S, cons
         const int idx = rem / nb2, rh = (rem % nb2) / nblk, cb = rem % nblk;
         const int b = kind == 5 || kind == 6 ? idx : idx / 3, d = kind == 5 || kind == 6 ? 0 : idx % 3;
         switch (kind) {
-            case 0:
-                if (merge01)
-                    formula_task<0, true>(S, K, tcx, S.acc, b, d, rh, cb);
-                else
-                    formula_task<0, false>(S, K, tcx, S.acc, b, d, rh, cb);
-                break;
-            case 1: formula_task<1, false>(S, K, tcx, S.acc, b, d, rh, cb); break;
-            case 2: formula_task<2, false>(S, K, tcx, S.acc, b, d, rh, cb); break;
+            case 0: formula_task<0, DM>(S, K, tcx, S.acc, b, d, rh, cb); break;
+            case 2: formula_task<2, DM>(S, K, tcx, S.acc, b, d, rh, cb); break;
             default:
                 if constexpr (DM) {
                     switch (kind) {
-                        case 3: formula_task<3, false>(S, K, tcx, S.acc, b, d, rh, cb); break;
-                        case 4: formula_task<4, false>(S, K, tcx, S.acc, b, d, rh, cb); break;
-                        case 5: formula_task<5, false>(S, K, tcx, S.acc, b, d, rh, cb); break;
-                        case 6: formula_task<6, false>(S, K, tcx, S.acc, b, d, rh, cb); break;
-                        default: formula_task<7, false>(S, K, tcx, S.acc, b, d, rh, cb); break;
+                        case 3: formula_task<3, DM>(S, K, tcx, S.acc, b, d, rh, cb); break;
+                        case 4: formula_task<4, DM>(S, K, tcx, S.acc, b, d, rh, cb); break;
+                        case 5: formula_task<5, DM>(S, K, tcx, S.acc, b, d, rh, cb); break;
+                        case 6: formula_task<6, DM>(S, K, tcx, S.acc, b, d, rh, cb); break;
+                        default: formula_task<7, DM>(S, K, tcx, S.acc, b, d, rh, cb); break;
                     }
                 }
                 break;
