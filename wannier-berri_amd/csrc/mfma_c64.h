@@ -85,17 +85,18 @@ struct MfmaHalf {
 
 __device__ inline int mfma_hrow(int v) { return (int)(threadIdx.x & 63) / 16 + 4 * v; }
 
+// C += X Y over klo <= k < khi (X and Y are called only with those k and r, c < nr, nc)
 template <class FX, class FY>
-__device__ __attribute__((always_inline)) void mfma_half(MfmaHalf& C, int nr, int nc, int nk, int r0, int c0, FX X, FY Y) {
+__device__ __attribute__((always_inline)) void mfma_half(MfmaHalf& C, int nr, int nc, int klo, int khi, int r0, int c0, FX X, FY Y) {
     const int li = threadIdx.x & 15, lk = (threadIdx.x & 63) >> 4;
     const bool rok = r0 + li < nr;
     bool cok[2];
 #pragma unroll
     for (int b = 0; b < 2; ++b) cok[b] = c0 + 16 * b + li < nc;
 #pragma unroll 2
-    for (int k0 = 0; k0 < nk; k0 += 4) {
+    for (int k0 = klo & ~3; k0 < khi; k0 += 4) {
         const int k = k0 + lk;
-        const bool kok = k < nk;
+        const bool kok = k >= klo && k < khi;
         const cplx<double> a = (kok && rok) ? X(r0 + li, k) : mk(0.0, 0.0);
         cplx<double> b[2];
 #pragma unroll

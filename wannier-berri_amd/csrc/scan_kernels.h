@@ -39,21 +39,17 @@
 // be stored in FP32 or FP64.
 #pragma once
 
+#include <algorithm>
 #include <cmath>
 #include <type_traits>
 
 #include "mfma_c64.h"
 #include "wbmi_common.h"
 
-#define SC_THREADS 512            // workgroup size (and launch bound) of the scan kernels
-#ifndef SC_TASK_THREADS
-#define SC_TASK_THREADS 768       // DerOmega / DerMorb: 12 waves (3 per SIMD), one workgroup per CU
-#endif
+#define SC_THREADS 512  // workgroup size of the scan kernels (DerOmega / DerMorb: task_threads)
 #define SC_NWMAX 128
-#ifndef SC_STAGE_A
-#define SC_STAGE_A 1  // A staged in LDS next to V (1) or read from the channels (0)
-#endif
-#define SC_M_NW 64    // dEinv o Off lives in LDS up to this nw, else it is formed on the fly
+#define SC_LDS (160 * 1024)
+#define SC_M_NW 64    // dEinv o Off lives in LDS up to this nw (DerOmega / DerMorb: wherever it fits)
 #define SC_LDS_NW 32  // V and A live in LDS up to this nw
 
 static __constant__ int c_alpha[3] = {1, 2, 0};  // utility.py:45-46
@@ -79,7 +75,7 @@ struct ScanArgs {
 struct Smem {
     char* V;            // [3][nw][ld] staged V (element type scan_stage)
     char* A;            // [3][nw][ld] staged A (external terms)
-    cplx<double>* acc;  // [nw][9]
+    double* acc;        // [nw][9] per-band values of the partition
     double* M;          // [nw][ld] dEinv o Off
     double* E;
     double* cut;        // [nw+1][9]
@@ -92,6 +88,7 @@ struct Smem {
     int* gin;   // group in range
     int* misc;  // [0] = ngroups, [1], [2] = sea group [lo, hi) (empty: lo == hi)
     int* ch;    // channel slot per role [WBMI_NROLES]
+    int* need;  // non-additive formulas: cut to be evaluated [nw+1]
     // tetrahedron method only (empty regions otherwise)
     double* tC;    // [nw][8] corner energies
     double* tEmn;  // [nw] min over centre and corners
@@ -111,7 +108,7 @@ struct SmemOffsets {
 };
 
 // vsz: bytes of one staged V / A element
-__host__ __device__ inline SmemOffsets smem_offsets(int nw, bool stage_v, bool stage_a, bool tetra, size_t vsz) {
+__host__ __device__ inline SmemOffsets smem_offsets(int nw, bool lm, bool stage_v, bool stage_a, bool tetra, size_t vsz) {
     const size_t ld = nw + 1;
     SmemOffsets o;
     size_t off = 0;
@@ -120,9 +117,9 @@ __host__ __device__ inline SmemOffsets smem_offsets(int nw, bool stage_v, bool s
     o.A = off;
     off = al16(off + (stage_a ? vsz * 3 * nw * ld : 0));
     o.acc = off;
-    off = al16(off + sizeof(cplx<double>) * nw * 9);
+    off = al16(off + sizeof(double) * nw * 9);
     o.M = off;
-    off = al16(off + (nw <= SC_M_NW ? sizeof(double) * nw * ld : 0));
+    off = al16(off + (lm ? sizeof(double) * nw * ld : 0));
     o.E = off;
     off = al16(off + sizeof(double) * nw);
     o.cut = off;
@@ -130,7 +127,7 @@ __host__ __device__ inline SmemOffsets smem_offsets(int nw, bool stage_v, bool s
     o.gw = off;
     off = al16(off + sizeof(double) * nw);
     o.ints = off;
-    off = al16(off + sizeof(int) * (6 * nw + 1 + 4 + WBMI_NROLES));
+    off = al16(off + sizeof(int) * (7 * nw + 2 + 4 + WBMI_NROLES));
     o.tet = off;
     off = al16(off + (tetra ? sizeof(double) * (8 * nw + 2 * nw + (nw + 1) * 9) : 0));
     o.tints = off;
@@ -139,15 +136,15 @@ __host__ __device__ inline SmemOffsets smem_offsets(int nw, bool stage_v, bool s
     return o;
 }
 
-__device__ __attribute__((always_inline)) inline Smem make_smem(char* base, int nw, bool stage_v, bool stage_a,
-                                                                bool tetra, size_t vsz) {
-    const SmemOffsets o = smem_offsets(nw, stage_v, stage_a, tetra, vsz);
+__device__ __attribute__((always_inline)) inline Smem make_smem(char* base, int nw, bool lm, bool stage_v,
+                                                                bool stage_a, bool tetra, size_t vsz) {
+    const SmemOffsets o = smem_offsets(nw, lm, stage_v, stage_a, tetra, vsz);
     Smem s;
     // LDS addresses even where a region is empty (never read then): no null tests on LDS pointers
     s.V = base + o.V;
     s.A = base + o.A;
-    s.acc = (cplx<double>*)(base + o.acc);
-    s.M = (double*)(base + o.M);  // empty region (never read) when nw > SC_M_NW
+    s.acc = (double*)(base + o.acc);
+    s.M = (double*)(base + o.M);  // empty region (never read) without LM
     s.E = (double*)(base + o.E);
     s.cut = (double*)(base + o.cut);
     s.gw = (double*)(base + o.gw);
@@ -160,6 +157,7 @@ __device__ __attribute__((always_inline)) inline Smem make_smem(char* base, int 
     s.gin = q + 5 * nw + 1;
     s.misc = q + 6 * nw + 1;
     s.ch = q + 6 * nw + 5;
+    s.need = q + 6 * nw + 5 + WBMI_NROLES;
     double* t = (double*)(base + o.tet);
     s.tC = t;
     s.tEmn = t + 8 * nw;
@@ -334,13 +332,15 @@ __host__ __device__ constexpr bool uses_A() {
            F == WBMI_FORMULA_OMEGASPIN || F == WBMI_FORMULA_OMEGAOMEGA || F == WBMI_FORMULA_OMEGAHPLUS;
 }
 
-// build M = dEinv o Off for the current labels (data_K.py:290-298)
+// build M = dEinv o Off for the current labels (data_K.py:290-298), or dEinv itself (the cut
+// partitions: one matrix for all of them, their sums run over the off-side bands alone)
+template <bool MASKED>
 __device__ __attribute__((always_inline)) void build_M(const Smem& S, int nw) {
     const int ld = nw + 1;
     for (int t = threadIdx.x; t < nw * nw; t += (int)blockDim.x) {
         int x = t / nw, y = t % nw;
         double m = 0.0;
-        if (S.lab[x] != S.lab[y]) {
+        if (!MASKED || S.lab[x] != S.lab[y]) {
             double de = S.E[x] - S.E[y];
             if (fabs(de) >= 1e-7) m = 1.0 / de;
         }
@@ -379,7 +379,10 @@ __device__ inline double wave_sum(double v, int mask) {
 // same-side element may be credited to either of its bands).
 struct TaskCtx {
     bool in, ex;
+    bool s5;      // DerMorb's s5 and T4 are summed: (2 E_l + 2 sign E_n) Im(A^a_nl dA_ln), dA Hermitian, is
+                  // odd under l <-> n for sign = +1, so its trace vanishes there
     double sign;
+    int cut;      // two-set partition [0, cut); < 0: the groups of the labels
 };
 
 // The component c of a term with index pair (alpha_c, beta_c) = (x, y) (sig +1) or (y, x) (-1), x != y
@@ -395,29 +398,90 @@ __host__ __device__ constexpr int task_nt() {
 
 template <int KIND, bool DM, typename T, bool LM, bool ST, bool SA, int NW, typename TS>
 __device__ __attribute__((always_inline)) void formula_task(const Smem& S, const KCtx<T, LM, ST, SA, NW, TS>& K, const TaskCtx& tc_,
-                                                           cplx<double>* acc, int b, int d, int rh, int cb) {
+                                                           double* acc, int b, int d, int rh, int cb) {
     constexpr bool dm = DM;
     const int nw = K.n_(), lane = threadIdx.x & 63;
     const int r0 = rh * 16, c0 = cb * 32;  // a 16 x 32 half block
     const bool in = tc_.in, ex = tc_.ex;
     const double sign = tc_.sign;
+    const int cut = tc_.cut;
     const int al = c_alpha[b], be = c_beta[b];  // kinds 5, 6: b = c
+    // blocks without an element in use, and the range [k0, k1) of the summed index with D' != 0
+    // (kinds 6, 7: with both factors in the partition)
+    int k0 = 0, k1 = nw;
+    bool act[2], multi = false;  // multi: a column whose group has several bands
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+        const int n = c0 + mfma_col(u);
+        act[u] = n < nw && S.act[n];
+        multi |= act[u] && S.ge[n] - S.gs[n] > 1;
+    }
+    if (!__any(act[0] || act[1])) return;
+    if (cut >= 0) {
+        if constexpr (KIND == 0 || KIND == 3) {
+            if (r0 + 16 <= cut) return;
+        } else if constexpr (KIND == 2) {
+            if (r0 + 16 <= cut && !(dm && tc_.s5)) return;
+        } else {
+            if (r0 >= cut) return;
+        }
+        if constexpr (KIND == 6 || KIND == 7)
+            k1 = cut;
+        else
+            k0 = cut;
+    }
     MfmaHalf P;
     P.zero();
     if constexpr (KIND == 0)
-        mfma_half(P, nw, nw, nw, r0, c0, [&](int r, int m) { return K.V(b, r, m); }, [&](int m, int c) { return K.Dp(d, m, c); });
+        mfma_half(P, nw, nw, k0, k1, r0, c0, [&](int r, int m) { return K.V(b, r, m); }, [&](int m, int c) { return K.Dp(d, m, c); });
     else if constexpr (KIND == 2)
-        mfma_half(P, nw, nw, nw, r0, c0, [&](int r, int m) { return K.A(b, r, m); }, [&](int m, int c) { return K.Dp(d, m, c); });
+        mfma_half(P, nw, nw, k0, k1, r0, c0, [&](int r, int m) { return K.A(b, r, m); }, [&](int m, int c) { return K.Dp(d, m, c); });
     else if constexpr (KIND == 3)
-        mfma_half(P, nw, nw, nw, r0, c0, [&](int r, int m) { return K.B(b, r, m); }, [&](int m, int c) { return K.Dp(d, m, c); });
+        mfma_half(P, nw, nw, k0, k1, r0, c0, [&](int r, int m) { return K.B(b, r, m); }, [&](int m, int c) { return K.Dp(d, m, c); });
     else if constexpr (KIND == 4)
-        mfma_half(P, nw, nw, nw, r0, c0, [&](int r, int m) { return K.Dp(d, r, m); }, [&](int m, int c) { return K.A(b, m, c); });
+        mfma_half(P, nw, nw, k0, k1, r0, c0, [&](int r, int m) { return K.Dp(d, r, m); }, [&](int m, int c) { return K.A(b, m, c); });
     else if constexpr (KIND == 5)
-        mfma_half(P, nw, nw, nw, r0, c0, [&](int r, int m) { return K.Dp(al, r, m); }, [&](int m, int c) { return K.Dp(be, m, c); });
+        mfma_half(P, nw, nw, k0, k1, r0, c0, [&](int r, int m) { return K.Dp(al, r, m); }, [&](int m, int c) { return K.Dp(be, m, c); });
     else if constexpr (KIND == 6)
-        mfma_half(P, nw, nw, nw, r0, c0, [&](int r, int m) { return K.Ain(al, r, m); }, [&](int m, int c) { return K.Ain(be, m, c); });
+        mfma_half(P, nw, nw, k0, k1, r0, c0, [&](int r, int m) { return K.Ain(al, r, m); }, [&](int m, int c) { return K.Ain(be, m, c); });
     else
-        mfma_half(P, nw, nw, nw, r0, c0, [&](int r, int m) { return K.Vin(b, r, m); }, [&](int m, int c) { return K.Ain(d, m, c); });
+        mfma_half(P, nw, nw, k0, k1, r0, c0, [&](int r, int m) { return K.Vin(b, r, m); }, [&](int m, int c) { return K.Ain(d, m, c); });
+    // kinds 0, 2, 3, the within-group part -D'^d X''^b (X = V, A, B): one term for a group of one
+    // band (the epilogue's), else a second product over the bands of the columns' groups.  Kind 0 of
+    // DerMorb keeps it apart, as s1 reads the first product alone
+    constexpr bool within = KIND == 0 || KIND == 2 || KIND == 3;
+    bool big = false;
+    MfmaHalf P2;
+    MfmaHalf& Pw = (KIND == 0 && DM) ? P2 : P;
+    if constexpr (within) {
+        big = __any(multi);
+        if constexpr (KIND == 0 && DM) P2.zero();
+        if (big) {
+            int g0 = 0, g1 = cut;
+            if (cut < 0) {
+                g0 = nw;
+                g1 = 0;
+#pragma unroll
+                for (int u = 0; u < 2; ++u)
+                    if (act[u]) {
+                        g0 = min(g0, S.gs[c0 + mfma_col(u)]);
+                        g1 = max(g1, S.ge[c0 + mfma_col(u)]);
+                    }
+                for (int o = 8; o >= 1; o >>= 1) {
+                    g0 = min(g0, __shfl_xor(g0, o));
+                    g1 = max(g1, __shfl_xor(g1, o));
+                }
+            }
+            mfma_half(
+                Pw, nw, nw, g0, g1, r0, c0, [&](int r, int m) { return r < cut ? mk(0.0, 0.0) : -K.Dp(d, r, m); },
+                [&](int m, int c) {
+                    if (K.lab[m] != K.lab[c]) return mk(0.0, 0.0);
+                    if constexpr (KIND == 0) return K.V(b, m, c);
+                    else if constexpr (KIND == 2) return K.A(b, m, c);
+                    else return K.B(b, m, c);
+                });
+        }
+    }
 
     // part[u][w]: u = the lane's band slot, its column bj (the band n is the column y of every element)
     constexpr int NU = 2, NT = task_nt<KIND, DM>();
@@ -450,8 +514,7 @@ __device__ __attribute__((always_inline)) void formula_task(const Smem& S, const
 #pragma unroll
         for (int bj = 0; bj < 2; ++bj) {
             const int n = c0 + mfma_col(bj);
-            if (n >= nw || !S.act[n]) continue;
-            const bool single = S.ge[n] - S.gs[n] == 1;  // group {n}: the within-group sums have one term
+            if (!act[bj]) continue;
             const double dw = dm ? 2.0 * sign * K.E[n] : 2.0;
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
@@ -461,15 +524,12 @@ __device__ __attribute__((always_inline)) void formula_task(const Smem& S, const
                 const bool same = K.lab[l] == K.lab[n];
                 if constexpr (KIND == 0) {
                     if (same) continue;
-                    // (W^{bd} - D'^b V''^d - D'^d V''^b)_ln / 2, with D'_xy = -m_xy V_xy and m_nl = -m_ln
+                    // W^{bd}_ln / 2 - (D'^d V''^b)_ln, with D'_xy = -m_xy V_xy and m_nl = -m_ln
                     const double mln = K.m(l, n);
-                    cplx<double> z = gz[bj][v];
-                    if (single)
-                        z += mln * (K.V(d, n, n).re * K.V(b, l, n) + K.V(b, n, n).re * K.V(d, l, n));
-                    else
-                        for (int q = S.gs[n]; q < S.ge[n]; ++q)
-                            z -= K.Dp(b, l, q) * K.V(d, q, n) + K.Dp(d, l, q) * K.V(b, q, n);
-                    const cplx<double> Pm = (-mln) * (pv + 0.5 * z);
+                    cplx<double> z = 0.5 * gz[bj][v];
+                    if (!big) z += (mln * K.V(b, n, n).re) * K.V(d, l, n);
+                    if constexpr (DM) z += P2.get(bj, v);
+                    const cplx<double> Pm = (-mln) * (pv + z);
                     const double wD = in ? (dm ? dw + 2.0 * K.E[l] : dw) : 0.0;
 #pragma unroll
                     for (int a = 0; a < 3; ++a) {
@@ -489,35 +549,33 @@ __device__ __attribute__((always_inline)) void formula_task(const Smem& S, const
                         // A'^{bd} - D'^d A''^b
                         const double mln = K.m(l, n);
                         cplx<double> z = gz[bj][v];
-                        if (single)
-                            z += mln * (K.V(d, l, n) * K.A(b, n, n));
-                        else
-                            for (int q = S.gs[n]; q < S.ge[n]; ++q) z -= K.Dp(d, l, q) * K.A(b, q, n);
+                        if (!big) z += mln * (K.V(d, l, n) * K.A(b, n, n));
                         const cplx<double> Y1 = (-dw * mln) * (pv + z);
 #pragma unroll
                         for (int a = 0; a < 3; ++a) {
                             const cplx<double> va = K.V(a, l, n);
                             part[bj][a] += va.re * Y1.re + va.im * Y1.im;  // Re conj(V_ln) Y1
                         }
-                    } else if (dm) {
-                        // s5: Re(-2i sig A^a_nl E_l (A' + A^b D'^d)_ln)
+                    } else if (dm && tc_.s5) {
+                        // s5 and T4: Re(-i sig (2 E_l + 2 sign E_n) A^a_nl (A' + A^b D'^d)_ln)
                         const cplx<double> dA = pv + K.Ad(b, d, l, n);
 #pragma unroll
-                        for (int a = 0; a < 3; ++a) part[bj][a] += 2.0 * K.E[l] * (K.A(a, n, l) * dA).im;
+                        for (int a = 0; a < 3; ++a) part[bj][a] += (dw + 2.0 * K.E[l]) * (K.A(a, n, l) * dA).im;
                     }
                 } else if constexpr (KIND == 3) {
                     if (same) continue;
                     // B'^{bd} - D'^d B''^b
                     cplx<double> z = gz[bj][v];
-                    for (int q = S.gs[n]; q < S.ge[n]; ++q) z -= K.Dp(d, l, q) * K.B(b, q, n);
+                    if (!big) z -= K.Dp(d, l, n) * K.B(b, n, n);
                     const cplx<double> YB = pv + z;
 #pragma unroll
                     for (int a = 0; a < 3; ++a) part[bj][a] -= 2.0 * (K.Dp(a, n, l) * YB).re;  // s6
                 } else if constexpr (KIND == 4) {
                     if (!same) continue;
-                    // s5: -Re(-2i sig A^a_nl E_l (D'^d A^b)_ln) ; Omega block: 2 sign coef Re(DA_ln V^e_nl)
+                    // s5 and T4 with -D'^d A^b in place of dA; Omega block: 2 sign coef Re(DA_ln V^e_nl)
+                    if (tc_.s5)
 #pragma unroll
-                    for (int a = 0; a < 3; ++a) part[bj][a] -= 2.0 * K.E[l] * (K.A(a, n, l) * pv).im;
+                        for (int a = 0; a < 3; ++a) part[bj][a] -= (dw + 2.0 * K.E[l]) * (K.A(a, n, l) * pv).im;
 #pragma unroll
                     for (int e = 0; e < 3; ++e) part[bj][3 + e] += (pv * K.V(e, n, l)).re;
                 } else if constexpr (KIND == 5 || KIND == 6) {
@@ -543,98 +601,87 @@ __device__ __attribute__((always_inline)) void formula_task(const Smem& S, const
 #pragma unroll
         for (int w = 0; w < NT; ++w) sum[w] = wave_sum(part[u][w], mask);
         if (!writer || n >= nw) continue;
-        cplx<double>* row = acc + n * 9;
+        double* row = acc + n * 9;
         if constexpr (KIND <= 4) {
 #pragma unroll
             for (int a = 0; a < 3; ++a) {
                 // the component whose index pair holds b and the partner a: column (c, d); X1 is
                 // symmetric in its indices, so kind 0 also feeds (c', b) of the pair of d and a
-                if (a != b) atomicAdd(&row[third_index(a, b) * 3 + d].re, pair_sign(a, b) * sum[a]);
+                if (a != b) atomicAdd(&row[third_index(a, b) * 3 + d], pair_sign(a, b) * sum[a]);
                 if constexpr (KIND == 0)
-                    if (a != d) atomicAdd(&row[third_index(a, d) * 3 + b].re, pair_sign(a, d) * sum[a]);
+                    if (a != d) atomicAdd(&row[third_index(a, d) * 3 + b], pair_sign(a, d) * sum[a]);
             }
         }
         if constexpr (KIND == 0 && DM) {
-            if (in) atomicAdd(&row[s1c * 3 + b].re, 2.0 * sum[3]);
+            if (in) atomicAdd(&row[s1c * 3 + b], 2.0 * sum[3]);
         } else if constexpr (KIND == 4) {
             // Omega block: D'^d A^b enters s^c with -1 for (al_c, be_c) = (d, b), +1 for (b, d)
             if (b != d && sign != 0.0)
 #pragma unroll
                 for (int e = 0; e < 3; ++e)
-                    atomicAdd(&row[third_index(b, d) * 3 + e].re, -2.0 * sign * pair_sign(d, b) * sum[3 + e]);
+                    atomicAdd(&row[third_index(b, d) * 3 + e], -2.0 * sign * pair_sign(d, b) * sum[3 + e]);
         } else if constexpr (KIND == 5 || KIND == 6) {
 #pragma unroll
-            for (int e = 0; e < 3; ++e) atomicAdd(&row[b * 3 + e].re, 2.0 * sign * sum[e]);
+            for (int e = 0; e < 3; ++e) atomicAdd(&row[b * 3 + e], 2.0 * sign * sum[e]);
         } else if constexpr (KIND == 7) {
-            atomicAdd(&row[s1c * 3 + b].re, 2.0 * sum[0]);
+            atomicAdd(&row[s1c * 3 + b], 2.0 * sum[0]);
         }
     }
 }
 
 // DerOmega (formula/covariant.py:212-259) or, dm = true, DerMorb
-// (formula/covariant.py:463-552) per-band values into S.acc[n][c*3+d].
+// (formula/covariant.py:463-552) per-band values into S.acc[n][c*3+d], for the partition of the
+// labels (cut < 0) or [0, cut) (the labels set likewise).
 // DerMorb = DerMorb_H + sign [Eav o dOmega + (Omega V + V Omega)/2] on cut
 // partitions; its trace terms (s1 ... s7, the Omega block) are listed at
-// formula_task.
-// DM is compile-time so that the DerOmega kernel carries only the kinds it runs (0 - 2): its
+// formula_task.  DerOmega's term T4, -i sig Tr A^a dA.nn^{bd}, is a real trace of two Hermitian
+// matrices times -i: it has no real part and is left out.
+// DM is compile-time so that the DerOmega kernel carries only the kinds it runs (0 and 2): its
 // register allocation and code size are not those of the DerMorb kinds.
+// The workgroups blockIdx.y = 0, 1, .. of one k share its tasks: each adds up its own (the first also
+// the per-band terms), and the sums over groups are linear in them.
 template <bool DM, typename T, bool LM, bool ST, bool SA, int NW, typename TS>
 __device__ __attribute__((always_inline)) void eval_deromega(const Smem& S, const KCtx<T, LM, ST, SA, NW, TS>& K, bool in, bool ex,
-                                                            int sign) {
+                                                            int sign, int cut) {
     constexpr bool dm = DM;
     const int nw = K.n_(), tid = threadIdx.x;
+    const bool lead = blockIdx.y == 0;
+    const int l0 = cut >= 0 ? cut : 0;  // D' != 0 from here on
     // per-band terms, lanes running over (n, c, d)
     for (int t = tid; t < nw * 9; t += (int)blockDim.x) {
         const int n = t % nw, c = (t / nw) / 3, d = (t / nw) % 3;
         double v = 0.0;
-        if (S.act[n] && ex) {
-            cplx<double> s = mk(0.0, 0.0);
-            const int g0 = S.gs[n], g1 = S.ge[n];
-            for (int sg = 0; sg < 2; ++sg) {
-                const int a = sg == 0 ? c_alpha[c] : c_beta[c];
-                const int b = sg == 0 ? c_beta[c] : c_alpha[c];
-                const double sig = sg == 0 ? 1.0 : -1.0;
-                // T4: -i sigma sum_{n' in G} A^a_nn' dA.nn^{bd}_n'n
-                for (int m = g0; m < g1; ++m) {
-                    cplx<double> y2 = K.Ad(b, d, m, n);
-#pragma unroll 4
-                    for (int l = 0; l < nw; ++l) y2 += K.A(b, m, l) * K.Dp(d, l, n) - K.Dp(d, m, l) * K.A(b, l, n);
-                    s += times_i(-(sig * (K.A(a, n, m) * y2)));
-                }
-            }
+        if (S.act[n] && ex && lead) {
             // T5: 0.5 dO.nn = 0.5 [O'^{cd}_nn - (D'^d O^c)_nn + (O^c D'^d)_nn].  O is Hermitian
             // and D' anti-Hermitian, so (D'^d O^c)_nn = -conj((O^c D'^d)_nn) and only the real part,
             // Re O'_nn + 2 Re sum_l conj(O_ln) D'_ln, is used: column n of O, which consecutive
             // threads (consecutive n) read from consecutive addresses
             double t5 = K.Od(c, d, n, n).re;
 #pragma unroll 8
-            for (int l = 0; l < nw; ++l) t5 += 2.0 * (conj(K.O(c, l, n)) * K.Dp(d, l, n)).re;
-            s.re += 0.5 * t5;
-            v = (dm ? 2.0 * sign * S.E[n] : 2.0) * s.re;
+            for (int l = l0; l < nw; ++l) t5 += 2.0 * (conj(K.O(c, l, n)) * K.Dp(d, l, n)).re;
+            v = (dm ? 2.0 * sign * S.E[n] : 2.0) * (0.5 * t5);
             if (dm) {
                 // s3: dH.nn = C'^{cd}_nn - (D'^d C^c)_nn + (C^c D'^d)_nn
                 cplx<double> s3 = K.Cd(c, d, n, n);
+                for (int l = l0; l < nw; ++l) s3 += K.C(c, n, l) * K.Dp(d, l, n) - K.Dp(d, n, l) * K.C(c, l, n);
                 // Omega block, elementwise part: 2 sign Re sum_{l in G} (O^c_nl / 2) V^d_ln
                 cplx<double> ov = mk(0.0, 0.0);
-                for (int l = 0; l < nw; ++l) {
-                    s3 += K.C(c, n, l) * K.Dp(d, l, n) - K.Dp(d, n, l) * K.C(c, l, n);
-                    if (K.lab[l] == K.lab[n]) ov += K.O(c, n, l) * K.V(d, l, n);
-                }
+                for (int l = S.gs[n]; l < S.ge[n]; ++l) ov += K.O(c, n, l) * K.V(d, l, n);
                 v += s3.re + sign * ov.re;
             }
         }
-        S.acc[n * 9 + c * 3 + d] = mk(v, 0.0);
+        S.acc[n * 9 + c * 3 + d] = v;
     }
     if (tid == 0) S.misc[3] = 0;  // task counter
     __syncthreads();
     // wave tasks (kind, b, d, row block, column block), round-robin over the waves
-    const TaskCtx tcx{in, ex, (double)sign};
+    const TaskCtx tcx{in, ex, dm && ex && sign != 1, (double)sign, cut};
     int cnt[8];
     cnt[0] = in || ex ? 9 : 0;
     cnt[1] = 0;
     cnt[2] = ex ? 9 : 0;
     cnt[3] = dm && ex ? 9 : 0;
-    cnt[4] = dm && ex ? 9 : 0;
+    cnt[4] = dm && ex && (tcx.s5 || sign != 0) ? 9 : 0;
     cnt[5] = dm && in && sign != 0 ? 3 : 0;
     cnt[6] = dm && ex && sign != 0 ? 3 : 0;
     cnt[7] = dm && ex ? 9 : 0;
@@ -649,7 +696,7 @@ __device__ __attribute__((always_inline)) void eval_deromega(const Smem& S, cons
     for (;;) {
         int t = 0;
         if (lane == 0) t = atomicAdd(&S.misc[3], 1);
-        t = __builtin_amdgcn_readfirstlane(t);
+        t = __builtin_amdgcn_readfirstlane(t) * (int)gridDim.y + (int)blockIdx.y;
         if (t >= ntask) break;
         int kind = -1, rem = 0, base = 0;
 #pragma unroll
@@ -681,18 +728,20 @@ __device__ __attribute__((always_inline)) void eval_deromega(const Smem& S, cons
     }
 }
 
-// Per-band values for the current partition into S.acc[n][comp] (.re).
+// Per-band values for the current partition (the labels'; cut >= 0: they are those of [0, cut), and M
+// holds the unmasked dEinv) into S.acc[n][comp].
 template <int F, typename T, bool LM, bool ST, bool SA, int NW, typename TS>
-__device__ __attribute__((always_inline)) void eval_partition(const Smem& S, const KCtx<T, LM, ST, SA, NW, TS>& K, const wbmi_scan_params& p) {
+__device__ __attribute__((always_inline)) void eval_partition(const Smem& S, const KCtx<T, LM, ST, SA, NW, TS>& K, const wbmi_scan_params& p, int cut = -1) {
     const int nw = K.n_();
     const int tid = threadIdx.x;
     const bool in = p.internal_terms, ex = p.external_terms;
-    if constexpr (LM) build_M(S, nw);
-    for (int t = tid; t < nw * 9; t += (int)blockDim.x) S.acc[t] = mk(0.0, 0.0);
+    if constexpr (LM)
+        if (cut < 0) build_M<true>(S, nw);
+    for (int t = tid; t < nw * 9; t += (int)blockDim.x) S.acc[t] = 0.0;
     __syncthreads();
     if (F == WBMI_FORMULA_IDENTITY) {
         for (int n = tid; n < nw; n += (int)blockDim.x)
-            if (S.act[n]) S.acc[n * 9] = mk(1.0, 0.0);
+            if (S.act[n]) S.acc[n * 9] = 1.0;
     } else if (F == WBMI_FORMULA_OMEGA) {
         if constexpr (ST) {
             // V and A in LDS: four adjacent lanes share (n, c) and split the sum over l,
@@ -710,13 +759,13 @@ __device__ __attribute__((always_inline)) void eval_partition(const Smem& S, con
                 }
                 v += __shfl_xor(v, 1);
                 v += __shfl_xor(v, 2);
-                if (act && qq == 0) S.acc[n * 9 + c] = mk(2.0 * v, 0.0);
+                if (act && qq == 0) S.acc[n * 9 + c] = 2.0 * v;
             }
         } else {
             for (int t = tid; t < nw * 3; t += (int)blockDim.x) {
                 int n = t / 3, c = t % 3;
                 if (!S.act[n]) continue;
-                S.acc[n * 9 + c] = mk(2.0 * omega_s(K, c, n, n, in, ex).re, 0.0);
+                S.acc[n * 9 + c] = 2.0 * omega_s(K, c, n, n, in, ex).re;
             }
         }
     } else if (F == WBMI_FORMULA_MORB_HPM) {
@@ -725,7 +774,7 @@ __device__ __attribute__((always_inline)) void eval_partition(const Smem& S, con
             if (!S.act[n]) continue;
             double v = 2.0 * morbh_s(K, c, n, n, in, ex).re;
             if (p.sign != 0) v += p.sign * S.E[n] * 2.0 * omega_s(K, c, n, n, in, ex).re;
-            S.acc[n * 9 + c] = mk(v, 0.0);
+            S.acc[n * 9 + c] = v;
         }
     } else if (F == WBMI_FORMULA_VELOMEGA) {
         // Re sum_{n' in G} V^a_nn' Omega^b_n'n, Omega = s + s^+ (formula/formula.py:141-148)
@@ -737,7 +786,7 @@ __device__ __attribute__((always_inline)) void eval_partition(const Smem& S, con
                 cplx<double> om = omega_s(K, b, m, n, in, ex) + conj(omega_s(K, b, n, m, in, ex));
                 v += K.V(a, n, m) * om;
             }
-            S.acc[t] = mk(v.re, 0.0);
+            S.acc[t] = v.re;
         }
     } else if (F == WBMI_FORMULA_VELHPLUS) {
         // Re sum_{n' in G} V^a_nn' Hpm^b_n'n with the group block of Morb_Hpm,
@@ -754,7 +803,7 @@ __device__ __attribute__((always_inline)) void eval_partition(const Smem& S, con
                          (omega_s(K, b, m, n, in, ex) + conj(omega_s(K, b, n, m, in, ex)));
                 v += K.V(a, n, m) * h;
             }
-            S.acc[t] = mk(v.re, 0.0);
+            S.acc[t] = v.re;
         }
     } else if (F == WBMI_FORMULA_DERSPIN) {
         // generalised derivative of the spin (formula/formula.py:95-107 with A = Xbar('SS'),
@@ -767,13 +816,13 @@ __device__ __attribute__((always_inline)) void eval_partition(const Smem& S, con
                 v -= K.Dp(d, n, l) * K.S(b, l, n);
                 v += K.S(b, n, l) * K.Dp(d, l, n);
             }
-            S.acc[t] = mk(v.re, 0.0);
+            S.acc[t] = v.re;
         }
     } else if (F == WBMI_FORMULA_SPIN) {
         // Re S^s_nn: the group trace of Xbar('SS') (formula/covariant.py:331-335)
         for (int t = tid; t < nw * 3; t += (int)blockDim.x) {
             const int n = t / 3, sp = t % 3;
-            if (S.act[n]) S.acc[n * 9 + sp] = mk(K.S(sp, n, n).re, 0.0);
+            if (S.act[n]) S.acc[n * 9 + sp] = K.S(sp, n, n).re;
         }
     } else if (F == WBMI_FORMULA_VELSPIN) {
         // Re sum_{n' in G} V^a_nn' S^b_n'n (formula/formula.py:121-148, covariant.py:811-814)
@@ -782,7 +831,7 @@ __device__ __attribute__((always_inline)) void eval_partition(const Smem& S, con
             if (!S.act[n]) continue;
             cplx<double> v = mk(0.0, 0.0);
             for (int m = S.gs[n]; m < S.ge[n]; ++m) v += K.V(a, n, m) * K.S(b, m, n);
-            S.acc[t] = mk(v.re, 0.0);
+            S.acc[t] = v.re;
         }
     } else if (F == WBMI_FORMULA_INVMASS) {
         // inverse effective mass, the generalised derivative of the velocity (formula/elementary.py:28-33,
@@ -796,7 +845,7 @@ __device__ __attribute__((always_inline)) void eval_partition(const Smem& S, con
                 v -= K.Dp(d, n, l) * K.V(b, l, n);
                 v += K.V(b, n, l) * K.Dp(d, l, n);
             }
-            S.acc[t] = mk(v.re, 0.0);
+            S.acc[t] = v.re;
         }
     } else if (F == WBMI_FORMULA_VELVEL) {
         // Re sum_{n' in G} V^a_nn' V^b_n'n (FormulaProduct of two velocities, formula/covariant.py:817-820)
@@ -805,7 +854,7 @@ __device__ __attribute__((always_inline)) void eval_partition(const Smem& S, con
             if (!S.act[n]) continue;
             cplx<double> v = mk(0.0, 0.0);
             for (int m = S.gs[n]; m < S.ge[n]; ++m) v += K.V(a, n, m) * K.V(b, m, n);
-            S.acc[t] = mk(v.re, 0.0);
+            S.acc[t] = v.re;
         }
     } else if (F == WBMI_FORMULA_VELVELVEL) {
         // [a][b][c] = Re sum_{m, l in G} V^a_nm V^b_ml V^c_ln (formula/formula.py:121-148), a = comp_slice
@@ -816,7 +865,7 @@ __device__ __attribute__((always_inline)) void eval_partition(const Smem& S, con
             cplx<double> v = mk(0.0, 0.0);
             for (int m = S.gs[n]; m < S.ge[n]; ++m)
                 for (int l = S.gs[n]; l < S.ge[n]; ++l) v += K.V(a, n, m) * K.V(b, m, l) * K.V(c, l, n);
-            S.acc[t] = mk(v.re, 0.0);
+            S.acc[t] = v.re;
         }
     } else if (F == WBMI_FORMULA_MASSVEL) {
         // [a][b][c] = Re sum_{m in G} M^{ab}_nm V^c_mn, a = comp_slice
@@ -826,7 +875,7 @@ __device__ __attribute__((always_inline)) void eval_partition(const Smem& S, con
             if (!S.act[n]) continue;
             cplx<double> v = mk(0.0, 0.0);
             for (int m = S.gs[n]; m < S.ge[n]; ++m) v += mass_xy(K, a, b, n, m) * K.V(c, m, n);
-            S.acc[t] = mk(v.re, 0.0);
+            S.acc[t] = v.re;
         }
     } else if (F == WBMI_FORMULA_HALL_SURF) {
         // VelMassVel X[a][b][c][d] = Re sum_{m, l in G} V^a_nm M^{bc}_ml V^d_ln, contracted
@@ -839,7 +888,7 @@ __device__ __attribute__((always_inline)) void eval_partition(const Smem& S, con
                     for (int l = S.gs[n]; l < S.ge[n]; ++l) x += K.V(a, n, m) * mass_xy(K, b, c, m, l) * K.V(d, l, n);
                 return x;
             });
-            S.acc[t] = mk(v.re, 0.0);
+            S.acc[t] = v.re;
         }
     } else if (F == WBMI_FORMULA_HALL_SEA) {
         // MassMass X[a][b][c][d] = Re sum_{m in G} M^{ab}_nm M^{cd}_mn, its axes moved as
@@ -852,7 +901,7 @@ __device__ __attribute__((always_inline)) void eval_partition(const Smem& S, con
                 for (int m = S.gs[n]; m < S.ge[n]; ++m) x += mass_xy(K, q, r, n, m) * mass_xy(K, s4, p0, m, n);
                 return x;
             });
-            S.acc[t] = mk(v.re, 0.0);
+            S.acc[t] = v.re;
         }
     } else if (F == WBMI_FORMULA_OMEGASPIN || F == WBMI_FORMULA_OMEGAOMEGA || F == WBMI_FORMULA_OMEGAHPLUS) {
         // Re sum_{n' in G} Omega^a_nn' Y^b_n'n, Omega = s + s^+, Y = S (OmegaS), Omega (OmegaOmega)
@@ -876,18 +925,18 @@ __device__ __attribute__((always_inline)) void eval_partition(const Smem& S, con
                 }
                 v += om * y;
             }
-            S.acc[t] = mk(v.re, 0.0);
+            S.acc[t] = v.re;
         }
     } else if (F == WBMI_FORMULA_BANDVALUES) {
         // the caller's per-band shares of the group traces, 9 of them from row comp_slice * 9
         for (int t = tid; t < nw * 9; t += (int)blockDim.x) {
             const int n = t / 9, c = t % 9;
-            if (S.act[n]) S.acc[t] = mk(K.bv[n * K.nbv + p.comp_slice * 9 + c], 0.0);
+            if (S.act[n]) S.acc[t] = K.bv[n * K.nbv + p.comp_slice * 9 + c];
         }
     } else if (F == WBMI_FORMULA_DEROMEGA) {
-        eval_deromega<false>(S, K, in, ex, 0);
+        eval_deromega<false>(S, K, in, ex, 0, cut);
     } else if (F == WBMI_FORMULA_DERMORB) {
-        eval_deromega<true>(S, K, in, ex, p.sign);
+        eval_deromega<true>(S, K, in, ex, p.sign, cut);
     }
     __syncthreads();
 }
@@ -1057,38 +1106,25 @@ __device__ inline int fermi_bin(const wbmi_scan_params& p, double E) {
 // MODE: 0 = Fermi-level bins, 1 = tetrahedron weights, 2 = per-band table (hist is then
 // out[nk][nw][ncomp]: each band gets its group's trace / group size, or, for the identity
 // formula, the group's mean energy)
-// element type of the staged V and A: complex128 for DerOmega / DerMorb (one workgroup per CU
-// holds them anyway; converted once at staging instead of at every access), the channels'
-// storage type for Omega (two complex64 workgroups per CU)
-template <typename T, int F>
-struct scan_stage {
-    typedef typename std::conditional<F == WBMI_FORMULA_DEROMEGA || F == WBMI_FORMULA_DERMORB, double, T>::type type;
-};
 
-// workgroup size of k_static_scan<T, F, .., MODE> (its launch bound).  The tetrahedron
-// variants (MODE 1) of DerOmega / DerMorb keep 8-wave workgroups: with their weight code
-// inlined, the 168-register bound of 12-wave workgroups spills several hundred registers
-template <typename T, int F, int MODE>
-__host__ __device__ constexpr int scan_threads() {
-    constexpr bool tasks = F == WBMI_FORMULA_DEROMEGA || F == WBMI_FORMULA_DERMORB;
-    if (!tasks || MODE == 1) return SC_THREADS;
-    return SC_TASK_THREADS;
-}
-
-#ifndef SC_TASK_MINW
-#define SC_TASK_MINW 1  // minimum waves per SIMD asked of the DerOmega / DerMorb Fermi-bin kernels
-#endif
-template <typename T, int F, int MODE>
-__host__ __device__ constexpr int scan_min_waves() {
-    constexpr bool tasks = F == WBMI_FORMULA_DEROMEGA || F == WBMI_FORMULA_DERMORB;
-    return tasks && MODE != 1 ? SC_TASK_MINW : 1;
-}
+// Workgroup sizes of the DerOmega / DerMorb kernels.  The epilogues and the LDS and L2 latencies, not
+// the products, bound them, so what counts is waves in flight from workgroups in different phases: four
+// waves per SIMD at 128 registers, in as many workgroups as the LDS of a CU holds (staged V, A in their
+// storage type).  DerOmega at 4096 k-points, nw = 32: complex64 (two workgroups of 8 waves) 0.78 ms
+// against 0.94 for one of 12 waves; complex128 fits one workgroup, 12 waves of 168 registers 0.95 ms
+// against 1.01 for 16 of 128.  nw = 18, 1331 k-points: 0.20 ms in 4-wave workgroups, 0.25 in 12-wave ones.
+// Within-group sums of large groups (the Fermi sea, the cuts of DerMorb) are a second product of the
+// task instead of a loop per element, ranges of the summed index without a term are left out, and the
+// sea is one more group of the main partition: DerMorb of 294 k-points at nw = 64, internal terms,
+// every cut: 39.7 -> 7.6 ms; with external terms at nw = 18 and a narrow window 2.02 -> 0.92 ms per
+// 1287 k-points; DerOmega of 150 k-points at nw = 128 10.4 -> 2.1 ms.
+// The tetrahedron variants (MODE 1) keep 8 waves: their weight code is inlined.
+__host__ __device__ constexpr int scan_min_waves(bool tasks, int nth) { return !tasks ? 1 : nth == 768 ? 3 : 4; }
 
 // NW > 0: the kernel for nw = NW only, every size and row stride a compile-time constant
-template <typename T, int F, bool LM, bool ST, int MODE, int NW>
-__global__ void __launch_bounds__((scan_threads<T, F, MODE>()), (scan_min_waves<T, F, MODE>())) k_static_scan(ScanArgs args, const double* __restrict__ Eall,
-                                                            const cplx<T>* __restrict__ Xall,
-                                                            double* __restrict__ hist) {
+template <typename T, int F, bool LM, bool ST, int MODE, int NW, int NTH>
+__global__ void __launch_bounds__(NTH, (scan_min_waves((F == WBMI_FORMULA_DEROMEGA || F == WBMI_FORMULA_DERMORB) && MODE != 1, NTH)))
+k_static_scan(ScanArgs args, const double* __restrict__ Eall, const cplx<T>* __restrict__ Xall, double* __restrict__ hist) {
     extern __shared__ __attribute__((aligned(16))) char smem_raw[];
     const wbmi_scan_params& p = args.p;
     const int nw = NW > 0 ? NW : args.nw, ld = nw + 1;
@@ -1097,13 +1133,13 @@ __global__ void __launch_bounds__((scan_threads<T, F, MODE>()), (scan_min_waves<
     if (MODE != 2) hist += k * args.hist_stride;
     constexpr bool tasks = F == WBMI_FORMULA_DEROMEGA || F == WBMI_FORMULA_DERMORB;
     static_assert(tasks || F == WBMI_FORMULA_OMEGA || !ST, "V and A are staged for DerOmega, DerMorb and Omega");
-    using TS = typename scan_stage<T, F>::type;
-    constexpr bool SA = ST && SC_STAGE_A;
+    using TS = T;
+    constexpr bool SA = ST;
     constexpr bool stage_v = ST;
     const bool stage_a = SA && p.external_terms;
     constexpr bool tetra = MODE == 1;  // compile-time: the Fermi-bin kernels carry no tetrahedron code
     constexpr bool tab = MODE == 2;
-    const Smem S = make_smem(smem_raw, nw, stage_v, stage_a, tetra, sizeof(cplx<TS>));
+    const Smem S = make_smem(smem_raw, nw, LM, stage_v, stage_a, tetra, sizeof(cplx<TS>));
     for (int n = tid; n < nw; n += (int)blockDim.x) S.E[n] = Eall[k * nw + n];
     for (int r = tid; r < WBMI_NROLES; r += (int)blockDim.x) S.ch[r] = p.ch[r];
     if (tetra)
@@ -1127,40 +1163,34 @@ __global__ void __launch_bounds__((scan_threads<T, F, MODE>()), (scan_min_waves<
     }
     const cplx<T>* Xk = Xall + k * (int64_t)args.nch * nw * nw;
     if (stage_v) {
-        // staged only for nw <= SC_LDS_NW: 3 nw^2 <= 3072 elements per array, NS per thread of
-        // the workgroup.  Each copy loop is branch-free (indices clamped into range; a thread past
-        // the end rewrites the last element with its own value), so it is one basic block and the
-        // scheduler issues all of a thread's loads before its first LDS store
-        constexpr int NTH = scan_threads<T, F, MODE>();
-        constexpr int NS = (3 * SC_LDS_NW * SC_LDS_NW + NTH - 1) / NTH;
+        // SB elements per thread and pass, indices clamped into range (a thread past the end
+        // rewrites the last element with its own value): no branches, so the scheduler issues all
+        // of a pass's loads before its first LDS store
+        constexpr int SB = NW > 0 ? (3 * NW * NW + NTH - 1) / NTH : 4;
         const int nw2 = nw * nw, n3 = 3 * nw2;
-        int so[NS], lo[NS];  // source element (channel-relative) and LDS element of each slot
+        const cplx<T>* src[2][3];
 #pragma unroll
-        for (int u = 0; u < NS; ++u) {
-            const int t = min(tid + NTH * u, n3 - 1);
-            const int a = t >= 2 * nw2 ? 2 : t >= nw2 ? 1 : 0, xy = t - a * nw2;
-            const int x = xy / nw, y = xy - x * nw;
-            so[u] = a * 4096 + xy;  // a in the bits above xy (nw^2 <= 1024)
-            lo[u] = (a * nw + x) * ld + y;
+        for (int a = 0; a < 3; ++a) {
+            src[0][a] = Xk + (int64_t)S.ch[WBMI_ROLE_V + a] * nw2;
+            src[1][a] = Xk + (int64_t)(stage_a ? S.ch[WBMI_ROLE_A + a] : 0) * nw2;
         }
-        const cplx<T>* srcv[3] = {Xk + (int64_t)S.ch[WBMI_ROLE_V] * nw2, Xk + (int64_t)S.ch[WBMI_ROLE_V + 1] * nw2,
-                                  Xk + (int64_t)S.ch[WBMI_ROLE_V + 2] * nw2};
-        cplx<TS>* dv = (cplx<TS>*)S.V;
 #pragma unroll
-        for (int u = 0; u < NS; ++u) {
-            const int a = so[u] >> 12, xy = so[u] & 4095;
-            const cplx<T> v = (a == 0 ? srcv[0] : a == 1 ? srcv[1] : srcv[2])[xy];
-            dv[lo[u]] = mk((TS)v.re, (TS)v.im);
-        }
-        if (stage_a) {
-            const cplx<T>* srca[3] = {Xk + (int64_t)S.ch[WBMI_ROLE_A] * nw2, Xk + (int64_t)S.ch[WBMI_ROLE_A + 1] * nw2,
-                                      Xk + (int64_t)S.ch[WBMI_ROLE_A + 2] * nw2};
-            cplx<TS>* da = (cplx<TS>*)S.A;
+        for (int q = 0; q < 2; ++q) {
+            if (q == 1 && !stage_a) break;
+            cplx<T>* dst = (cplx<T>*)(q == 0 ? S.V : S.A);
+            for (int t0 = 0; t0 < n3; t0 += SB * NTH) {
+                cplx<T> v[SB];
+                int lo[SB];
 #pragma unroll
-            for (int u = 0; u < NS; ++u) {
-                const int a = so[u] >> 12, xy = so[u] & 4095;
-                const cplx<T> v = (a == 0 ? srca[0] : a == 1 ? srca[1] : srca[2])[xy];
-                da[lo[u]] = mk((TS)v.re, (TS)v.im);
+                for (int u = 0; u < SB; ++u) {
+                    const int t = min(t0 + tid + NTH * u, n3 - 1);
+                    const int a = t >= 2 * nw2 ? 2 : t >= nw2 ? 1 : 0, xy = t - a * nw2;
+                    const int x = xy / nw;
+                    lo[u] = (a * nw + x) * ld + xy - x * nw;
+                    v[u] = (a == 0 ? src[q][0] : a == 1 ? src[q][1] : src[q][2])[xy];
+                }
+#pragma unroll
+                for (int u = 0; u < SB; ++u) dst[lo[u]] = v[u];
             }
         }
     }
@@ -1310,6 +1340,16 @@ __global__ void __launch_bounds__((scan_threads<T, F, MODE>()), (scan_min_waves<
                 S.act[n] = S.gin[g];
             }
         __syncthreads();
+        // the Fermi-sea group [sea_lo, sea_hi) (hole-like tetra: the bands above) as one more group:
+        // it holds whole groups, none of them in range, and a group's values do not depend on how
+        // the bands outside it are grouped
+        for (int n = sea_lo + tid; n < sea_hi; n += (int)blockDim.x) {
+            S.lab[n] = ng;
+            S.gs[n] = sea_lo;
+            S.ge[n] = sea_hi;
+            S.act[n] = 1;
+        }
+        __syncthreads();
         eval_partition<F>(S, K, p);
         for (int t = tid; t < ng * ncomp; t += (int)blockDim.x) {
             const int g = t / ncomp, c = t % ncomp;
@@ -1319,7 +1359,7 @@ __global__ void __launch_bounds__((scan_threads<T, F, MODE>()), (scan_min_waves<
                     v = S.gw[g];  // Eavln: mean energy of the group
                 } else {
                     v = 0.0;
-                    for (int n = S.gb[g]; n < S.gb[g + 1]; ++n) v += S.acc[n * 9 + c].re;
+                    for (int n = S.gb[g]; n < S.gb[g + 1]; ++n) v += S.acc[n * 9 + c];
                     v /= (S.gb[g + 1] - S.gb[g]);
                 }
                 for (int n = S.gb[g]; n < S.gb[g + 1]; ++n) hist[(k * nw + n) * ncomp + c] = v;
@@ -1328,44 +1368,39 @@ __global__ void __launch_bounds__((scan_threads<T, F, MODE>()), (scan_min_waves<
             if (tetra) {
                 if (!S.gin[g]) continue;
                 double s = 0.0;
-                for (int n = S.gb[g]; n < S.gb[g + 1]; ++n) s += S.acc[n * 9 + c].re;
+                for (int n = S.gb[g]; n < S.gb[g + 1]; ++n) s += S.acc[n * 9 + c];
                 S.tv[g * 9 + c] = s * group_selected(p, S.gb[g], S.gb[g + 1]);
                 continue;
             }
             const int bin = S.gin[g] ? fermi_bin(p, S.gw[g]) : -1;
             if (bin < 0) continue;
             double s = 0.0;
-            for (int n = S.gb[g]; n < S.gb[g + 1]; ++n) s += S.acc[n * 9 + c].re;
+            for (int n = S.gb[g]; n < S.gb[g + 1]; ++n) s += S.acc[n * 9 + c];
             unsafeAtomicAdd(hist + (int64_t)bin * ncomp + c, args.weight * s * group_selected(p, S.gb[g], S.gb[g + 1]));
         }
         __syncthreads();
         if (sea_hi > sea_lo) {
-            // Fermi-sea group [sea_lo, sea_hi) (weight -inf; hole-like tetra: the bands above),
-            // added at every level; every other band is its "out" (with Emin / Emax on both
-            // sides of it: each side its own block)
-            for (int n = tid; n < nw; n += (int)blockDim.x) {
-                int inn = n >= sea_lo && n < sea_hi;
-                S.lab[n] = inn ? 0 : 1;
-                S.gs[n] = inn ? sea_lo : (n < sea_lo ? 0 : sea_hi);
-                S.ge[n] = inn ? sea_hi : (n < sea_lo ? sea_lo : nw);
-                S.act[n] = inn;
-            }
-            __syncthreads();
-            eval_partition<F>(S, K, p);
-            for (int c = tid; c < ncomp; c += (int)blockDim.x) {
-                double s = 0.0;
-                for (int n = sea_lo; n < sea_hi; ++n) s += S.acc[n * 9 + c].re;
-                unsafeAtomicAdd(hist + c, args.weight * s);  // bin 0: every level
+            // the sea's sum at every level (bin 0); one wave per component
+            for (int c = tid >> 6; c < ncomp; c += (int)blockDim.x >> 6) {
+                double v = 0.0;
+                for (int n = sea_lo + (tid & 63); n < sea_hi; n += 64) v += S.acc[n * 9 + c];
+                v = wave_sum(v, 63);
+                if ((tid & 63) == 0) unsafeAtomicAdd(hist + c, args.weight * v);
             }
             __syncthreads();
         }
     } else {
-        // non-additive: traces of the cumulative cuts [0, c) (static.py:109-117)
+        // non-additive: traces of the cumulative cuts [0, c) (static.py:109-117) at the borders of
+        // the groups in range and of the sea
+        for (int n = tid; n <= nw; n += (int)blockDim.x) S.need[n] = 0;
+        if constexpr (LM) build_M<false>(S, nw);
+        __syncthreads();
+        for (int g = tid; g < ng; g += (int)blockDim.x)
+            if (S.gin[g]) S.need[S.gb[g]] = S.need[S.gb[g + 1]] = 1;
+        if (tid == 0 && sea_hi > sea_lo) S.need[sea_lo] = S.need[sea_hi] = 1;
+        __syncthreads();
         for (int cidx = 1; cidx <= nw; ++cidx) {
-            bool need = sea_hi > sea_lo && (cidx == sea_hi || cidx == sea_lo);
-            for (int g = 0; g < ng; ++g)
-                if (S.gin[g] && (S.gb[g] == cidx || S.gb[g + 1] == cidx)) need = true;
-            if (!need) continue;
+            if (!S.need[cidx]) continue;
             for (int n = tid; n < nw; n += (int)blockDim.x) {
                 int inn = n < cidx;
                 S.lab[n] = inn ? 0 : 1;
@@ -1374,13 +1409,13 @@ __global__ void __launch_bounds__((scan_threads<T, F, MODE>()), (scan_min_waves<
                 S.act[n] = inn;
             }
             __syncthreads();
-            eval_partition<F>(S, K, p);
-            if (tid == 0)
-                for (int c = 0; c < ncomp; ++c) {
-                    double s = 0.0;
-                    for (int n = 0; n < cidx; ++n) s += S.acc[n * 9 + c].re;
-                    S.cut[cidx * 9 + c] = s;
-                }
+            eval_partition<F>(S, K, p, cidx);
+            for (int c = tid >> 6; c < ncomp; c += (int)blockDim.x >> 6) {
+                double v = 0.0;
+                for (int n = tid & 63; n < cidx; n += 64) v += S.acc[n * 9 + c];
+                v = wave_sum(v, 63);
+                if ((tid & 63) == 0) S.cut[cidx * 9 + c] = v;
+            }
             __syncthreads();
         }
         for (int c = tid; c < ncomp; c += (int)blockDim.x) S.cut[c] = 0.0;
@@ -1408,37 +1443,55 @@ __global__ void __launch_bounds__((scan_threads<T, F, MODE>()), (scan_min_waves<
     }
 }
 
-template <typename T, int F, bool LM, bool ST, int MODE, int NW = 0>
+template <typename T, int F, bool LM, bool ST, int MODE, int NW = 0, int NTH = SC_THREADS>
 static int launch_scan_t(wbmi_ctx* ctx, int nk, const ScanArgs& a, const double* E, const void* X, double* hist) {
-    const bool stage_a = ST && SC_STAGE_A && a.p.external_terms;
-    // DerOmega / DerMorb: 12 waves (3 per SIMD at <= 168 VGPRs), one workgroup per CU (at nw = 32
-    // LDS holds V and A, 118 KB as complex128)
-    const int threads = scan_threads<T, F, MODE>();
-    size_t lds = smem_offsets(a.nw, ST, stage_a, MODE == 1, sizeof(cplx<typename scan_stage<T, F>::type>)).total;
-    if (lds > 160 * 1024) return wbmi_fail(ctx, WBMI_ERR_ARG, "wbmi_static_scan: %zu bytes of LDS needed", lds);
-    WBMI_HIP_CHECK(ctx, hipFuncSetAttribute((const void*)k_static_scan<T, F, LM, ST, MODE, NW>,
+    const bool stage_a = ST && a.p.external_terms;
+    const size_t lds = smem_offsets(a.nw, LM, ST, stage_a, MODE == 1, sizeof(cplx<T>)).total;
+    if (lds > SC_LDS) return wbmi_fail(ctx, WBMI_ERR_ARG, "wbmi_static_scan: %zu bytes of LDS needed", lds);
+    // DerOmega / DerMorb of few k-points: several workgroups share a k-point's tasks, so that there are
+    // about four per CU (above nw = 32, where a k-point's tasks fill them; two below).  Fermi bins only: the
+    // other modes use a k-point's sums before they are complete.
+    constexpr bool tasks = F == WBMI_FORMULA_DEROMEGA || F == WBMI_FORMULA_DERMORB;
+    const int want = a.nw > 32 ? 1024 : 512;
+    const int parts = tasks && MODE == 0 && nk < want ? std::min(8, want / nk) : 1;
+    WBMI_HIP_CHECK(ctx, hipFuncSetAttribute((const void*)k_static_scan<T, F, LM, ST, MODE, NW, NTH>,
                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    hipLaunchKernelGGL((k_static_scan<T, F, LM, ST, MODE, NW>), dim3(nk), dim3(threads), lds,
-                       ctx->stream, a, E,
+    hipLaunchKernelGGL((k_static_scan<T, F, LM, ST, MODE, NW, NTH>), dim3(nk, parts), dim3(NTH), lds, ctx->stream, a, E,
                        (const cplx<T>*)X, hist);
     WBMI_LAUNCH_CHECK(ctx);
     return WBMI_OK;
 }
 
-// dEinv o Off in LDS up to SC_M_NW (the layout of smem_offsets), formed on the fly above;
-// V and A in LDS up to SC_LDS_NW for the formulas with wave tasks
+// dEinv o Off in LDS up to SC_M_NW (DerOmega / DerMorb: wherever it fits: an element formed on the fly
+// costs a division), else formed on the fly; V and A in LDS up to SC_LDS_NW for the formulas with
+// wave tasks and Omega.  Sizes: see scan_min_waves
 template <typename T, int F, int MODE>
 static int launch_scan(wbmi_ctx* ctx, int nk, const ScanArgs& a, const double* E, const void* X, double* hist) {
-    constexpr bool staged = F == WBMI_FORMULA_DEROMEGA || F == WBMI_FORMULA_DERMORB || F == WBMI_FORMULA_OMEGA;
-    if constexpr (staged) {
-        // nw = 32 (a single 32-column block, the spin blocks of the spinor models) has its own
-        // Fermi-bin kernels with the size fixed at compile time
-        if constexpr (MODE == 0)
-            if (a.stage_va && a.nw == 32) return launch_scan_t<T, F, true, true, MODE, 32>(ctx, nk, a, E, X, hist);
-        if (a.stage_va) return launch_scan_t<T, F, true, true, MODE>(ctx, nk, a, E, X, hist);
+    constexpr bool tasks = F == WBMI_FORMULA_DEROMEGA || F == WBMI_FORMULA_DERMORB;
+    if constexpr (tasks && MODE != 1) {
+        if (a.stage_va) {
+            if constexpr (MODE == 0 && F == WBMI_FORMULA_DEROMEGA)
+                // nw = 32 (a single 32-column block, the spin blocks of the spinor models) has its own
+                // Fermi-bin kernels with the size fixed at compile time
+                if (a.nw == 32) return launch_scan_t<T, F, true, true, MODE, 32, sizeof(T) == 4 ? 512 : 768>(ctx, nk, a, E, X, hist);
+            const size_t lds = smem_offsets(a.nw, true, true, a.p.external_terms, false, sizeof(cplx<T>)).total;
+            if (lds <= SC_LDS / 4) return launch_scan_t<T, F, true, true, MODE, 0, 256>(ctx, nk, a, E, X, hist);
+            if (lds <= SC_LDS / 2) return launch_scan_t<T, F, true, true, MODE, 0, 512>(ctx, nk, a, E, X, hist);
+            return launch_scan_t<T, F, true, true, MODE, 0, 768>(ctx, nk, a, E, X, hist);
+        }
+        const size_t lds = smem_offsets(a.nw, true, false, false, false, sizeof(cplx<T>)).total;
+        if (lds <= SC_LDS / 2) return launch_scan_t<T, F, true, false, MODE, 0, 512>(ctx, nk, a, E, X, hist);
+        return launch_scan_t<T, F, true, false, MODE, 0, 1024>(ctx, nk, a, E, X, hist);
+    } else {
+        constexpr bool staged = tasks || F == WBMI_FORMULA_OMEGA;
+        if constexpr (staged) {
+            if constexpr (MODE == 0)
+                if (a.stage_va && a.nw == 32) return launch_scan_t<T, F, true, true, MODE, 32>(ctx, nk, a, E, X, hist);
+            if (a.stage_va) return launch_scan_t<T, F, true, true, MODE>(ctx, nk, a, E, X, hist);
+        }
+        if (a.nw <= SC_M_NW) return launch_scan_t<T, F, true, false, MODE>(ctx, nk, a, E, X, hist);
+        return launch_scan_t<T, F, false, false, MODE>(ctx, nk, a, E, X, hist);
     }
-    if (a.nw <= SC_M_NW) return launch_scan_t<T, F, true, false, MODE>(ctx, nk, a, E, X, hist);
-    return launch_scan_t<T, F, false, false, MODE>(ctx, nk, a, E, X, hist);
 }
 
 template <typename T, int MODE>
