@@ -353,7 +353,7 @@ int wbmi_optical_conductivity_ws(wbmi_ctx* ctx, int nk, int nw, int nch, const d
  * Complex64 channels (prec = WBMI_F32) are rotated with FP64 arithmetic;
  * only the stored result is rounded.  Flag arrays may be NULL (all 0).
  * nw <= 128; work_dev / work_bytes: device workspace of at least
- * wbmi_rotate_work_bytes(...) bytes (nonzero only for nw > 64).            */
+ * wbmi_rotate_work_bytes(...) bytes (0 for every size now).                */
 int wbmi_rotate(wbmi_ctx* ctx, int nk, int nw, int nch, const void* U_dev,
                 void* X_dev, const int32_t* herm_host, const int32_t* skip_host, int prec,
                 void* work_dev, size_t work_bytes);

@@ -80,3 +80,28 @@ def test_scan_sea_and_split(ctx, nw, ef, precision):
         print(f"test_scan_sea_and_split nw={nw} {precision} {name}: {err:.2e}", flush=True)
         # the close pair's denominators are cut out of the sums (one group); the rest is of order one
         assert err < (1e-9 if precision == "fp64" else 2e-5), name
+
+
+@pytest.mark.parametrize("nw", [1, 2, 15, 16, 17, 31, 32, 33, 48, 49, 64, 65, 80, 81, 97, 112, 113, 128])
+def test_rotate_sizes(ctx, nw):
+    """One size at each edge of the rotation's 16-row blocks, flagged (Hermitian part), plain and
+    skipped channels: sums of nw^2 products in FP64 (complex64: rounded once more on storing)."""
+    import torch
+    from wannierberri_amd import _lib
+    rng = np.random.default_rng(nw)
+    nk, nch = 3, 6
+    U = np.linalg.qr(rng.standard_normal((nk, nw, nw)) + 1j * rng.standard_normal((nk, nw, nw)))[0]
+    X = rng.standard_normal((nk, nch, nw, nw)) + 1j * rng.standard_normal((nk, nch, nw, nw))
+    herm = np.array([0, 1, 1, 0, 0, 1], dtype=np.int32)
+    skip = np.array([0, 0, 1, 0, 1, 0], dtype=np.int32)
+    for prec, cd, nd, eps in ((_lib.WBMI_F64, torch.complex128, complex, EPS), (_lib.WBMI_F32, torch.complex64, np.complex64, 6e-8)):
+        Us, Xs = U.astype(nd), X.astype(nd)
+        Xd, Ud = torch.from_numpy(Xs).cuda(), torch.from_numpy(Us).cuda()
+        ctx.rotate(Ud, Xd, herm, skip, prec)
+        got = Xd.cpu().numpy()
+        Uw, Xw = Us.astype(complex), Xs.astype(complex)
+        Xw = np.where(herm[None, :, None, None] == 1, 0.5 * (Xw + Xw.conj().swapaxes(2, 3)), Xw)
+        ref = Uw.conj().swapaxes(1, 2)[:, None] @ Xw @ Uw[:, None]
+        ref = np.where(skip[None, :, None, None] == 1, Xs, ref)
+        bound = 4 * EPS * nw * np.abs(X).max() * np.sqrt(nw) + (eps * np.abs(ref).max() if eps > EPS else 0)
+        assert np.abs(got - ref).max() < bound
