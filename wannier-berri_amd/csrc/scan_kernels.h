@@ -380,7 +380,8 @@ __device__ inline double wave_sum(double v, int mask) {
 struct TaskCtx {
     bool in, ex;
     bool s5;      // DerMorb's s5 and T4 are summed: (2 E_l + 2 sign E_n) Im(A^a_nl dA_ln), dA Hermitian, is
-                  // odd under l <-> n for sign = +1, so its trace vanishes there
+                  // odd under l <-> n for sign = +1, so its trace vanishes there (complex64 channels, whose
+                  // A is Hermitian to storage rounding only, keep it)
     double sign;
     int cut;      // two-set partition [0, cut); < 0: the groups of the labels
 };
@@ -389,11 +390,19 @@ struct TaskCtx {
 __device__ inline int third_index(int x, int y) { return 3 - x - y; }
 __device__ inline double pair_sign(int x, int y) { return y == (x == 2 ? 0 : x + 1) ? 1.0 : -1.0; }
 
+// DerOmega's T4 has no real trace for Hermitian A; complex64 channels, whose A is Hermitian to storage
+// rounding only, keep it: groups of up to SC_T4_LOOP bands by a loop per band, larger ones as tasks
+#define SC_T4_LOOP 4
+template <bool DM, typename T>
+__host__ __device__ constexpr bool keep_t4() {
+    return !DM && sizeof(T) == 4;
+}
+
 // per-lane sums of a task: 0 - 2 one per partner a = 0, 1, 2; kind 0 of DerMorb: [3] = s1; kind 4:
 // [3] - [5] the Omega block's components; kinds 5, 6: one per e; kind 7: one
 template <int KIND, bool DM>
 __host__ __device__ constexpr int task_nt() {
-    return KIND == 0 ? (DM ? 4 : 3) : KIND == 4 ? 6 : KIND == 7 ? 1 : 3;
+    return KIND == 0 ? (DM ? 4 : 3) : KIND == 4 ? (DM ? 6 : 3) : KIND == 7 ? 1 : 3;
 }
 
 template <int KIND, bool DM, typename T, bool LM, bool ST, bool SA, int NW, typename TS>
@@ -556,11 +565,12 @@ __device__ __attribute__((always_inline)) void formula_task(const Smem& S, const
                             const cplx<double> va = K.V(a, l, n);
                             part[bj][a] += va.re * Y1.re + va.im * Y1.im;  // Re conj(V_ln) Y1
                         }
-                    } else if (dm && tc_.s5) {
+                    } else if (dm ? tc_.s5 : keep_t4<DM, T>() && S.ge[n] - S.gs[n] > SC_T4_LOOP) {
                         // s5 and T4: Re(-i sig (2 E_l + 2 sign E_n) A^a_nl (A' + A^b D'^d)_ln)
                         const cplx<double> dA = pv + K.Ad(b, d, l, n);
+                        const double w5 = dm ? dw + 2.0 * K.E[l] : dw;
 #pragma unroll
-                        for (int a = 0; a < 3; ++a) part[bj][a] += (dw + 2.0 * K.E[l]) * (K.A(a, n, l) * dA).im;
+                        for (int a = 0; a < 3; ++a) part[bj][a] += w5 * (K.A(a, n, l) * dA).im;
                     }
                 } else if constexpr (KIND == 3) {
                     if (same) continue;
@@ -573,11 +583,14 @@ __device__ __attribute__((always_inline)) void formula_task(const Smem& S, const
                 } else if constexpr (KIND == 4) {
                     if (!same) continue;
                     // s5 and T4 with -D'^d A^b in place of dA; Omega block: 2 sign coef Re(DA_ln V^e_nl)
-                    if (tc_.s5)
+                    if (dm ? tc_.s5 : S.ge[n] - S.gs[n] > SC_T4_LOOP) {
+                        const double w5 = dm ? dw + 2.0 * K.E[l] : dw;
 #pragma unroll
-                        for (int a = 0; a < 3; ++a) part[bj][a] -= (dw + 2.0 * K.E[l]) * (K.A(a, n, l) * pv).im;
+                        for (int a = 0; a < 3; ++a) part[bj][a] -= w5 * (K.A(a, n, l) * pv).im;
+                    }
+                    if constexpr (DM)
 #pragma unroll
-                    for (int e = 0; e < 3; ++e) part[bj][3 + e] += (pv * K.V(e, n, l)).re;
+                        for (int e = 0; e < 3; ++e) part[bj][3 + e] += (pv * K.V(e, n, l)).re;
                 } else if constexpr (KIND == 5 || KIND == 6) {
                     if (!same) continue;
                     // Omega block term -i P_ln: 2 sign Re(-i P_ln V^e_nl)
@@ -614,7 +627,7 @@ __device__ __attribute__((always_inline)) void formula_task(const Smem& S, const
         }
         if constexpr (KIND == 0 && DM) {
             if (in) atomicAdd(&row[s1c * 3 + b], 2.0 * sum[3]);
-        } else if constexpr (KIND == 4) {
+        } else if constexpr (KIND == 4 && DM) {
             // Omega block: D'^d A^b enters s^c with -1 for (al_c, be_c) = (d, b), +1 for (b, d)
             if (b != d && sign != 0.0)
 #pragma unroll
@@ -635,7 +648,7 @@ __device__ __attribute__((always_inline)) void formula_task(const Smem& S, const
 // DerMorb = DerMorb_H + sign [Eav o dOmega + (Omega V + V Omega)/2] on cut
 // partitions; its trace terms (s1 ... s7, the Omega block) are listed at
 // formula_task.  DerOmega's term T4, -i sig Tr A^a dA.nn^{bd}, is a real trace of two Hermitian
-// matrices times -i: it has no real part and is left out.
+// matrices times -i: it has no real part and is left out (complex64 channels: keep_t4).
 // DM is compile-time so that the DerOmega kernel carries only the kinds it runs (0 and 2): its
 // register allocation and code size are not those of the DerMorb kinds.
 // The workgroups blockIdx.y = 0, 1, .. of one k share its tasks: each adds up its own (the first also
@@ -672,16 +685,36 @@ __device__ __attribute__((always_inline)) void eval_deromega(const Smem& S, cons
         }
         S.acc[n * 9 + c * 3 + d] = v;
     }
+    int t4 = 0;  // tasks for T4: some group is too large for the loop
+    if constexpr (keep_t4<DM, T>()) {
+        for (int n = tid; n < nw; n += (int)blockDim.x) t4 |= S.act[n] && S.ge[n] - S.gs[n] > SC_T4_LOOP;
+        t4 = __syncthreads_or(t4);
+        for (int t = tid; t < nw * 9 && ex && lead; t += (int)blockDim.x) {
+            const int n = t % nw, b = (t / nw) / 3, d = (t / nw) % 3, g0 = S.gs[n], g1 = S.ge[n];
+            if (!S.act[n] || g1 - g0 > SC_T4_LOOP) continue;
+            double v[3] = {0.0, 0.0, 0.0};
+            for (int m = g0; m < g1; ++m) {
+                cplx<double> y = K.Ad(b, d, m, n);  // dA.nn^{bd}_mn
+#pragma unroll 4
+                for (int l = 0; l < nw; ++l) y += K.A(b, m, l) * K.Dp(d, l, n) - K.Dp(d, m, l) * K.A(b, l, n);
+#pragma unroll
+                for (int a = 0; a < 3; ++a) v[a] += (K.A(a, n, m) * y).im;
+            }
+#pragma unroll
+            for (int a = 0; a < 3; ++a)
+                if (a != b) atomicAdd(&S.acc[n * 9 + third_index(a, b) * 3 + d], 2.0 * pair_sign(a, b) * v[a]);
+        }
+    }
     if (tid == 0) S.misc[3] = 0;  // task counter
     __syncthreads();
     // wave tasks (kind, b, d, row block, column block), round-robin over the waves
-    const TaskCtx tcx{in, ex, dm && ex && sign != 1, (double)sign, cut};
+    const TaskCtx tcx{in, ex, dm && ex && (sign != 1 || sizeof(T) == 4), (double)sign, cut};
     int cnt[8];
     cnt[0] = in || ex ? 9 : 0;
     cnt[1] = 0;
     cnt[2] = ex ? 9 : 0;
     cnt[3] = dm && ex ? 9 : 0;
-    cnt[4] = dm && ex && (tcx.s5 || sign != 0) ? 9 : 0;
+    cnt[4] = ex && (dm ? tcx.s5 || sign != 0 : t4 != 0) ? 9 : 0;
     cnt[5] = dm && in && sign != 0 ? 3 : 0;
     cnt[6] = dm && ex && sign != 0 ? 3 : 0;
     cnt[7] = dm && ex ? 9 : 0;
@@ -713,11 +746,13 @@ __device__ __attribute__((always_inline)) void eval_deromega(const Smem& S, cons
         switch (kind) {
             case 0: formula_task<0, DM>(S, K, tcx, S.acc, b, d, rh, cb); break;
             case 2: formula_task<2, DM>(S, K, tcx, S.acc, b, d, rh, cb); break;
+            case 4:
+                if constexpr (DM || keep_t4<DM, T>()) formula_task<4, DM>(S, K, tcx, S.acc, b, d, rh, cb);
+                break;
             default:
                 if constexpr (DM) {
                     switch (kind) {
                         case 3: formula_task<3, DM>(S, K, tcx, S.acc, b, d, rh, cb); break;
-                        case 4: formula_task<4, DM>(S, K, tcx, S.acc, b, d, rh, cb); break;
                         case 5: formula_task<5, DM>(S, K, tcx, S.acc, b, d, rh, cb); break;
                         case 6: formula_task<6, DM>(S, K, tcx, S.acc, b, d, rh, cb); break;
                         default: formula_task<7, DM>(S, K, tcx, S.acc, b, d, rh, cb); break;
