@@ -239,7 +239,7 @@ def bench_klists(args):
     for st, (n, ms, _) in sorted(stats.items(), key=lambda x: -x[1][1]):
         log(f"    {st:12s} calls/step={n // args.steps:5d} ms/step={ms / args.steps:9.2f} avg={ms / n:.3f} ms")
     n, ms, units = stats["r2k_klist"]
-    flops = sum(8.0 * nk * nelem * nR for nk, nelem, nR in units)
+    flops = sum(4.0 * nk * nelem * nR for nk, nelem, nR in units)   # real phases of the pairs (R, -R)
     ach = flops / (ms / 1e3) / 1e12
     cb = None
     if not args.no_cpu:

@@ -218,11 +218,18 @@ int wbmi_r2k_yx(wbmi_ctx* ctx, const wbmi_r2k_plan* plan, const void* w1_dev, co
  *   XR_dev    : complex128 [nR, nelem];  out_dev : [nk, nelem] (prec)       */
 int wbmi_r2k_klist(wbmi_ctx* ctx, int nR, const int32_t* iRvec_dev, int64_t nelem,
                    const void* XR_dev, int nk, const double* klist_dev, void* out_dev, int prec);
-/* The same transform with an explicit workgroup tile (0 .. WBMI_KLIST_NTILES-1; 0 is what
- * wbmi_r2k_klist uses): no counterpart in the reference, for the per-nw autotuner
- * (wannierberri_amd/autotune.py) that times the tiles on the caller's shapes.
- * wbmi_r2k_klist_tile_shape gives a tile's k-points x elements per workgroup.         */
-#define WBMI_KLIST_NTILES 5
+/* The same transform with an explicit workgroup tile (0 .. WBMI_KLIST_NTILES-1;
+ * wbmi_r2k_klist chooses one from nk and nelem): no counterpart in the reference, for the
+ * per-nw autotuner (wannierberri_amd/autotune.py) that times the tiles on the caller's
+ * shapes.  wbmi_r2k_klist_tile_shape gives a tile's k-points x elements per workgroup.
+ * wbmi_r2k_klist_pairs: the same transform with half the products, given the R-vectors as
+ * pairs: pairs_dev int32 [npair, 2], every index 0 .. nR-1 in exactly one of them, (i, j)
+ * with R_j = -R_i, or (i, -1) for an R-vector alone; null: every R-vector alone.
+ * tile -1: chosen as by wbmi_r2k_klist.                                               */
+#define WBMI_KLIST_NTILES 7
+int wbmi_r2k_klist_pairs(wbmi_ctx* ctx, int nR, int npair, const int32_t* pairs_dev, const int32_t* iRvec_dev,
+                         int64_t nelem, const void* XR_dev, int nk, const double* klist_dev, void* out_dev,
+                         int prec, int tile);
 int wbmi_r2k_klist_tile(wbmi_ctx* ctx, int nR, const int32_t* iRvec_dev, int64_t nelem,
                         const void* XR_dev, int nk, const double* klist_dev, void* out_dev, int prec,
                         int tile);

@@ -105,3 +105,37 @@ def test_rotate_sizes(ctx, nw):
         ref = np.where(skip[None, :, None, None] == 1, Xs, ref)
         bound = 4 * EPS * nw * np.abs(X).max() * np.sqrt(nw) + (eps * np.abs(ref).max() if eps > EPS else 0)
         assert np.abs(got - ref).max() < bound
+
+
+@pytest.mark.parametrize("nk,nw,extra", [(1, 1, 0), (7, 3, 0), (17, 5, 1), (33, 4, 2), (130, 7, 1)])
+def test_klist_pairs(ctx, nk, nw, extra):
+    """R -> k with the R-vectors in pairs against the single-vector form and the plain sum: lists with
+    R-vectors that lack their -R, a repeated vector, and numbers of pairs off the chunk size."""
+    import torch
+    from wannierberri_amd import _lib
+    from wannierberri_amd.data_k import r_pairs
+    rng = np.random.default_rng(nk)
+    r = np.arange(-2, 3)
+    iR = np.array([[x, y, z] for x in r for y in r for z in r[:3 + extra % 2]], dtype=np.int32)
+    iR = np.concatenate([rng.permutation(iR), [[7, 0, -1]], iR[:extra]]).astype(np.int32)
+    pairs = r_pairs(iR)
+    flat = pairs.ravel()
+    assert sorted(flat[flat >= 0]) == list(range(len(iR)))
+    for i, j in pairs:
+        assert j < 0 or (iR[i] == -iR[j]).all()
+    nelem = 3 * nw * nw
+    X = rng.standard_normal((len(iR), nelem)) + 1j * rng.standard_normal((len(iR), nelem))
+    k = rng.random((nk, 3))
+    ref = np.exp(2j * np.pi * (k @ iR.T)) @ X
+    d = lambda x: torch.from_numpy(np.ascontiguousarray(x)).cuda()  # noqa: E731
+    Xd, kd, iRd = d(X), d(k), d(iR)
+    # phases are off by the rounding of k.R (|R| <= 8) times 2 pi
+    bound = 2 * np.pi * 16 * EPS * np.abs(X).sum(axis=0).max()
+    for prec, cd in ((_lib.WBMI_F64, torch.complex128), (_lib.WBMI_F32, torch.complex64)):
+        out = torch.empty((nk, 3, nw, nw), dtype=cd, device="cuda")
+        for tile in [None] + list(range(7)):
+            for p in (None, d(pairs)):
+                out.zero_()
+                ctx.r2k_klist(iRd, Xd, kd, out, prec, tile=tile, pairs=p)
+                err = np.abs(out.cpu().numpy().reshape(nk, nelem) - ref).max()
+                assert err < bound + (1.2e-7 * np.abs(ref).max() if prec == _lib.WBMI_F32 else 0), (tile, p is None)

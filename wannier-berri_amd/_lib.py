@@ -57,7 +57,7 @@ SYMBOLS = [
     "wbmi_static_scan_tetra", "wbmi_finalize_tetra", "wbmi_jdos", "wbmi_spin_hall", "wbmi_spin_hall_work_bytes",
     "wbmi_tabulate", "wbmi_tabulate_diag", "wbmi_shift_current", "wbmi_injection_current",
     "wbmi_static_scan_k", "wbmi_finalize_k", "wbmi_static_scan_tetra_k", "wbmi_finalize_tetra_k",
-    "wbmi_tabulate_invmass", "wbmi_eigh_noalloc", "wbmi_eigh_noalloc_max_bytes", "wbmi_r2k_klist_tile",
+    "wbmi_tabulate_invmass", "wbmi_eigh_noalloc", "wbmi_eigh_noalloc_max_bytes", "wbmi_r2k_klist_tile", "wbmi_r2k_klist_pairs",
     "wbmi_r2k_klist_tile_shape", "wbmi_tabulate_spin_berry", "wbmi_spin_berry_bands", "wbmi_der3e_bands",
     "wbmi_optical_conductivity_work_bytes", "wbmi_optical_conductivity_ws", "wbmi_r2k_w1_bytes", "wbmi_r2k_zpass",
     "wbmi_r2k_yx",
@@ -121,6 +121,7 @@ _PROTOS = {
     "wbmi_r2k_yx": (_i, [_vp, _vp, _vp, _vp, _vp, _vp, _i]),
     "wbmi_r2k_klist": (_i, [_vp, _i, _vp, _i64, _vp, _i, _vp, _vp, _i]),
     "wbmi_r2k_klist_tile": (_i, [_vp, _i, _vp, _i64, _vp, _i, _vp, _vp, _i, _i]),
+    "wbmi_r2k_klist_pairs": (_i, [_vp, _i, _i, _vp, _vp, _i64, _vp, _i, _vp, _vp, _i, _i]),
     "wbmi_r2k_klist_tile_shape": (_i, [_i, ctypes.POINTER(_i), ctypes.POINTER(_i)]),
     "wbmi_eigh": (_i, [_vp, _i, _i, _vp, _i64, _vp, _vp, _i, _i, _vp, _vp, ctypes.c_size_t]),
     "wbmi_eigh_noalloc": (_i, [_vp, _i, _i, _vp, _i64, _vp, _vp, _i, _i, _vp]),
@@ -261,16 +262,18 @@ class Context:
     def r2k_plan(self, iRvec, NKFFT, nelem):
         return R2KPlan(self, iRvec, NKFFT, nelem)
 
-    def r2k_klist(self, iRvec_dev, XR, klist_dev, out, prec, tile=None):
+    def r2k_klist(self, iRvec_dev, XR, klist_dev, out, prec, tile=None, pairs=None):
         """Phase-GEMM R -> k; `tile` defaults to the tuned tile for out's nw and `prec`
-        (self.tuning[("klist_tile", nw, prec)], set by wannierberri_amd.autotune), else tile 0."""
+        (self.tuning[("klist_tile", nw, prec)], set by wannierberri_amd.autotune), else one chosen
+        by the library.  `pairs`: the R-vectors as pairs (R, -R) (wbmi_r2k_klist_pairs), half the products."""
         nR = iRvec_dev.shape[0]
         nelem = XR[0].numel()
         if tile is None:
-            tile = self.tuning.get(("klist_tile", int(out.shape[-1]), int(prec)), 0)
-        self.check(self._timed("r2k_klist", (klist_dev.shape[0], nelem, nR), lib().wbmi_r2k_klist_tile, self.h, nR,
-                               _ptr(iRvec_dev), nelem, _ptr(XR), klist_dev.shape[0], _ptr(klist_dev), _ptr(out),
-                               prec, int(tile)), "wbmi_r2k_klist")
+            tile = self.tuning.get(("klist_tile", int(out.shape[-1]), int(prec)), -1)
+        npair = 0 if pairs is None else pairs.shape[0]
+        self.check(self._timed("r2k_klist", (klist_dev.shape[0], nelem, nR), lib().wbmi_r2k_klist_pairs, self.h, nR,
+                               npair, _ptr(pairs), _ptr(iRvec_dev), nelem, _ptr(XR), klist_dev.shape[0],
+                               _ptr(klist_dev), _ptr(out), prec, int(tile)), "wbmi_r2k_klist")
 
     def _workspace(self, nbytes):
         """Device workspace of at least nbytes (kept and grown on demand; None for 0)."""

@@ -50,12 +50,12 @@ def tune_klist(system, channels, nk=4096, prec=_lib.WBMI_F64, ctx=None, reps=3, 
     saved, ctx.timer = ctx.timer, None
     try:
         for tile in range(len(tile_shapes())):
-            ctx.r2k_klist(dev.iRvec_dev, stack, kl, out, prec, tile=tile)   # warm-up
+            ctx.r2k_klist(dev.iRvec_dev, stack, kl, out, prec, tile=tile, pairs=dev.pairs_dev)   # warm-up
             e0 = torch.cuda.Event(enable_timing=True)
             e1 = torch.cuda.Event(enable_timing=True)
             e0.record(ctx.stream)
             for _ in range(reps):
-                ctx.r2k_klist(dev.iRvec_dev, stack, kl, out, prec, tile=tile)
+                ctx.r2k_klist(dev.iRvec_dev, stack, kl, out, prec, tile=tile, pairs=dev.pairs_dev)
             e1.record(ctx.stream)
             e1.synchronize()
             times[tile] = e0.elapsed_time(e1) / reps

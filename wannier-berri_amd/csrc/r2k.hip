@@ -659,44 +659,71 @@ int wbmi_r2k_yx(wbmi_ctx* ctx, const wbmi_r2k_plan* p, const void* w1_dev, const
 // ---------------------------------------------------------------------------
 // arbitrary k-list: out[k][e] = sum_R exp(2 pi i k.R) X[R][e]
 //
-// A complex GEMM (M = nk, N = nelem, K = nR) on the FP64 matrix cores.  A
-// workgroup owns 64 k x 128 elements (8 waves of 32 x 32, mfma_c64.h); the
-// phase factors of its 64 k-points are formed in LDS, KLM_RC R-vectors at a
-// time, and the X operand is read straight from HBM (each 16-element row
-// segment is 256 contiguous bytes).  blockIdx.x runs over k-tiles, so the
-// workgroups resident on one XCD at a time share their X columns
-// (nR x 128 x 16 B) through that XCD's L2.
+// With cos and sin of k.R and a list of pairs (R, -R),
+//   e^{i phi} X_R + e^{-i phi} X_-R = cos(phi) (X_R + X_-R) + sin(phi) i (X_R - X_-R):
+// a product of real phases [nk, 2 npair] with complex matrices formed from the two operands as they are
+// loaded, half the multiplications of the complex product over single R-vectors (which a list of pairs
+// without partners gives).  On the FP64 matrix cores: a wave owns 16 KT k-points x 16 ET elements, real
+// and imaginary parts as two column tiles; the phases of a workgroup's k-points are formed in LDS, KLM_RC
+// pairs at a time; the X operands come straight from memory (256 contiguous bytes per 16 elements), those
+// of the next step loaded before the products of this one.  blockIdx.x runs over k-tiles, so the
+// workgroups resident on one XCD at a time share their X columns through that XCD's L2.
+// Bound: the matrix cores.  6112 k-points, 729 R, 5760 elements: 4.86 ms for the complex product
+// (42 TFLOP/s of 8 nk nR nelem) -> 1.91 ms (54 TFLOP/s of the 4 nk nR nelem it executes).
 // ---------------------------------------------------------------------------
 
 #define KLM_RC 32
 
-// Workgroup tiles (waves along k x waves along the elements), chosen per nw by the tuning
-// table of the context (wbmi_tune_set, WBMI_KNOB_KLIST_TILE); index 0 is the default.
-static const int klm_tiles[WBMI_KLIST_NTILES][2] = {{2, 4}, {4, 2}, {1, 8}, {2, 2}, {1, 4}};
+// Workgroup tiles: 16-row blocks of k-points and 16-column blocks of elements per wave, waves along k,
+// waves along the elements; chosen per nw by the tuning table of the context (wannierberri_amd/autotune.py)
+// or by klm_rule.  The first five keep their shapes (64 x 128, 128 x 64, 32 x 256, 64 x 64, 32 x 128).
+struct KlmTile {
+    int kt, et, wk, we;
+};
+static const KlmTile klm_tiles[WBMI_KLIST_NTILES] = {{4, 2, 1, 4}, {4, 2, 2, 2}, {2, 2, 1, 8}, {4, 2, 1, 2},
+                                                     {2, 2, 1, 4}, {2, 1, 1, 4}, {1, 1, 1, 4}};
 
-template <typename Tout, int WK, int WE>
-__global__ void __launch_bounds__(64 * WK * WE) k_r2k_klist(int nR, const int32_t* __restrict__ iR, int64_t nelem,
-                                                           const cplx<double>* __restrict__ X, int nk,
-                                                           const double* __restrict__ kl,
-                                                           cplx<Tout>* __restrict__ out) {
-    constexpr int TK = 32 * WK, TE = 32 * WE, NT = 64 * WK * WE;
-    __shared__ cplx<double> ph[TK][KLM_RC + 1];
-    const int wave = threadIdx.x >> 6;
+// The 32 x 32 wave tile where there are at least two of them for every SIMD (6112 k-points x 5760 elements:
+// 1.91 ms; 64 x 32, with half the waves on a SIMD, 2.00; 32 x 16 2.22), then 32 x 16, else the smallest
+// (a path batch of 50 k-points x 3240 elements: 32 us, against 39 and 52 with the larger ones).
+static int klm_rule(int nk, int64_t nelem) {
+    for (int t : {4, 5}) {
+        const KlmTile& q = klm_tiles[t];
+        if (nk > 8 * q.kt && ceil_div(nk, 16 * q.kt) * ceil_div(nelem, 16 * q.et) >= 2048) return t;
+    }
+    return 6;
+}
+
+template <typename Tout, bool PAIRS, int KT, int ET, int WK, int WE>
+__global__ void __launch_bounds__(64 * WK * WE, KT * ET > 4 ? 2 : 4)
+k_r2k_klist(int npair, const int2* __restrict__ pairs, const int32_t* __restrict__ iR, int64_t nelem,
+            const cplx<double>* __restrict__ X, int nk, const double* __restrict__ kl, cplx<Tout>* __restrict__ out) {
+    constexpr int TK = 16 * KT * WK, TE = 16 * ET * WE, NT = 64 * WK * WE, NS = KLM_RC / 4;
+    __shared__ cplx<double> ph[TK][KLM_RC + 1];  // cos, sin
+    __shared__ int2 pl[KLM_RC];
+    const int wave = threadIdx.x >> 6, li = threadIdx.x & 15, g = (threadIdx.x & 63) >> 4;
     const int k0 = blockIdx.x * TK;
-    const int64_t e0 = (int64_t)blockIdx.y * TE;
-    const int kw = k0 + 32 * (wave / WE);          // first k of this wave's tile
-    const int64_t ew = e0 + 32 * (wave % WE);      // first element of this wave's tile
-    const int nrow = nk - kw < 32 ? nk - kw : 32;
-    const int ncol = nelem - ew < 32 ? (int)(nelem - ew) : 32;
-    MfmaBlock C;
-    C.zero();
-    for (int r0 = 0; r0 < nR; r0 += KLM_RC) {
+    const int krow = 16 * KT * (wave / WE);  // first row of this wave's tile
+    const int64_t ew = (int64_t)blockIdx.y * TE + 16 * ET * (wave % WE) + li;
+    int64_t e[ET];
+#pragma unroll
+    for (int t = 0; t < ET; ++t) e[t] = ew + 16 * t < nelem ? ew + 16 * t : nelem - 1;
+    wbmi_v4d re[KT][ET], im[KT][ET];
+#pragma unroll
+    for (int q = 0; q < KT; ++q)
+#pragma unroll
+        for (int t = 0; t < ET; ++t) {
+            re[q][t] = wbmi_v4d{0.0, 0.0, 0.0, 0.0};
+            im[q][t] = re[q][t];
+        }
+    for (int r0 = 0; r0 < npair; r0 += KLM_RC) {
         __syncthreads();
         for (int t = threadIdx.x; t < TK * KLM_RC; t += NT) {
             const int q = t / KLM_RC, rr = t % KLM_RC;
-            const int k = k0 + q, r = r0 + rr;
+            const int k = k0 + q, p = r0 + rr;
             cplx<double> v = mk(0.0, 0.0);
-            if (k < nk && r < nR) {
+            if (k < nk && p < npair) {
+                const int r = PAIRS ? pairs[p].x : p;
                 double f = kl[3 * k] * iR[3 * r] + kl[3 * k + 1] * iR[3 * r + 1] + kl[3 * k + 2] * iR[3 * r + 2];
                 f -= floor(f);
                 double sn, cs;
@@ -705,79 +732,128 @@ __global__ void __launch_bounds__(64 * WK * WE) k_r2k_klist(int nR, const int32_
             }
             ph[q][rr] = v;
         }
+        for (int t = threadIdx.x; t < KLM_RC; t += NT) {
+            const int p = r0 + t;  // past the end: any row, with zero phases
+            pl[t] = p >= npair ? make_int2(0, -1) : PAIRS ? pairs[p] : make_int2(p, -1);
+        }
         __syncthreads();
-        if (nrow > 0 && ncol > 0) {
-            const int rc = nR - r0 < KLM_RC ? nR - r0 : KLM_RC;
-            const int prow = 32 * (wave / WE);
-            const cplx<double>* Xr = X + (int64_t)r0 * nelem + ew;
-            mfma_block(
-                C, nrow, ncol, rc, 0, 0, [&](int r, int k) { return ph[prow + r][k]; },
-                [&](int k, int c) { return Xr[(int64_t)k * nelem + c]; });
+        const int ns = (min(KLM_RC, npair - r0) + 3) / 4;
+        cplx<double> xp[2][ET], xm[2][ET];
+        double w[2];
+        auto load = [&](int s, int buf) {
+            const int2 p = pl[4 * s + g];
+            w[buf] = p.y < 0 ? 0.0 : 1.0;
+#pragma unroll
+            for (int t = 0; t < ET; ++t) {
+                xp[buf][t] = X[(int64_t)p.x * nelem + e[t]];
+                if constexpr (PAIRS) xm[buf][t] = X[(int64_t)(p.y < 0 ? p.x : p.y) * nelem + e[t]];
+            }
+        };
+        load(0, 0);
+#pragma unroll
+        for (int s = 0; s < NS; ++s) {
+            if (s >= ns) break;
+            const int buf = s & 1;
+            if (s + 1 < NS) load(s + 1 < ns ? s + 1 : s, buf ^ 1);
+            cplx<double> a[KT];
+#pragma unroll
+            for (int q = 0; q < KT; ++q) a[q] = ph[krow + 16 * q + li][4 * s + g];
+#pragma unroll
+            for (int t = 0; t < ET; ++t) {
+                cplx<double> c = xp[buf][t], d = mk(-c.im, c.re);  // X_R + X_-R, i (X_R - X_-R)
+                if constexpr (PAIRS) {
+                    d = mk(fma(w[buf], xm[buf][t].im, d.re), fma(-w[buf], xm[buf][t].re, d.im));
+                    c = mk(fma(w[buf], xm[buf][t].re, c.re), fma(w[buf], xm[buf][t].im, c.im));
+                }
+#pragma unroll
+                for (int q = 0; q < KT; ++q) {
+                    re[q][t] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[q].re, c.re, re[q][t], 0, 0, 0);
+                    im[q][t] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[q].re, c.im, im[q][t], 0, 0, 0);
+                }
+#pragma unroll
+                for (int q = 0; q < KT; ++q) {
+                    re[q][t] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[q].im, d.re, re[q][t], 0, 0, 0);
+                    im[q][t] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[q].im, d.im, im[q][t], 0, 0, 0);
+                }
+            }
         }
     }
-    if (nrow <= 0 || ncol <= 0) return;
 #pragma unroll
-    for (int bi = 0; bi < 2; ++bi)
+    for (int q = 0; q < KT; ++q)
 #pragma unroll
-        for (int bj = 0; bj < 2; ++bj)
+        for (int t = 0; t < ET; ++t)
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
-                const int r = mfma_row(bi, v), c = mfma_col(bj);
-                if (r < nrow && c < ncol) {
-                    const cplx<double> z = C.get(bi, bj, v);
-                    out[(int64_t)(kw + r) * nelem + ew + c] = mk((Tout)z.re, (Tout)z.im);
-                }
+                const int k = k0 + krow + 16 * q + g + 4 * v;
+                if (k < nk && ew + 16 * t < nelem)
+                    out[(int64_t)k * nelem + ew + 16 * t] = mk((Tout)re[q][t][v], (Tout)im[q][t][v]);
             }
 }
 
-template <typename Tout, int WK, int WE>
-static int launch_klist(wbmi_ctx* ctx, int nR, const int32_t* iR, int64_t nelem, const void* XR, int nk,
-                        const double* kl, void* out) {
-    constexpr int TK = 32 * WK, TE = 32 * WE;
+template <typename Tout, int KT, int ET, int WK, int WE>
+static int launch_klist(wbmi_ctx* ctx, int nR, int npair, const int32_t* pairs, const int32_t* iR, int64_t nelem,
+                        const void* XR, int nk, const double* kl, void* out) {
+    constexpr int TK = 16 * KT * WK, TE = 16 * ET * WE;
     if (ceil_div(nelem, TE) > 65535)
         return wbmi_fail(ctx, WBMI_ERR_ARG, "wbmi_r2k_klist: more than %d elements per k-point", 65535 * TE);
     dim3 g((unsigned)ceil_div(nk, TK), (unsigned)ceil_div(nelem, TE));
-    hipLaunchKernelGGL((k_r2k_klist<Tout, WK, WE>), g, dim3(64 * WK * WE), 0, ctx->stream, nR, iR, nelem,
-                       (const cplx<double>*)XR, nk, kl, (cplx<Tout>*)out);
+    if (pairs)
+        hipLaunchKernelGGL((k_r2k_klist<Tout, true, KT, ET, WK, WE>), g, dim3(64 * WK * WE), 0, ctx->stream, npair,
+                           (const int2*)pairs, iR, nelem, (const cplx<double>*)XR, nk, kl, (cplx<Tout>*)out);
+    else
+        hipLaunchKernelGGL((k_r2k_klist<Tout, false, KT, ET, WK, WE>), g, dim3(64 * WK * WE), 0, ctx->stream, nR,
+                           (const int2*)nullptr, iR, nelem, (const cplx<double>*)XR, nk, kl, (cplx<Tout>*)out);
     WBMI_LAUNCH_CHECK(ctx);
     return WBMI_OK;
 }
 
 template <typename Tout>
-static int launch_klist_tile(wbmi_ctx* ctx, int tile, int nR, const int32_t* iR, int64_t nelem, const void* XR,
-                             int nk, const double* kl, void* out) {
+static int launch_klist_tile(wbmi_ctx* ctx, int tile, int nR, int npair, const int32_t* pairs, const int32_t* iR,
+                             int64_t nelem, const void* XR, int nk, const double* kl, void* out) {
     switch (tile) {
-        case 1: return launch_klist<Tout, 4, 2>(ctx, nR, iR, nelem, XR, nk, kl, out);
-        case 2: return launch_klist<Tout, 1, 8>(ctx, nR, iR, nelem, XR, nk, kl, out);
-        case 3: return launch_klist<Tout, 2, 2>(ctx, nR, iR, nelem, XR, nk, kl, out);
-        case 4: return launch_klist<Tout, 1, 4>(ctx, nR, iR, nelem, XR, nk, kl, out);
-        default: return launch_klist<Tout, 2, 4>(ctx, nR, iR, nelem, XR, nk, kl, out);
+        case 1: return launch_klist<Tout, 4, 2, 2, 2>(ctx, nR, npair, pairs, iR, nelem, XR, nk, kl, out);
+        case 2: return launch_klist<Tout, 2, 2, 1, 8>(ctx, nR, npair, pairs, iR, nelem, XR, nk, kl, out);
+        case 3: return launch_klist<Tout, 4, 2, 1, 2>(ctx, nR, npair, pairs, iR, nelem, XR, nk, kl, out);
+        case 4: return launch_klist<Tout, 2, 2, 1, 4>(ctx, nR, npair, pairs, iR, nelem, XR, nk, kl, out);
+        case 5: return launch_klist<Tout, 2, 1, 1, 4>(ctx, nR, npair, pairs, iR, nelem, XR, nk, kl, out);
+        case 6: return launch_klist<Tout, 1, 1, 1, 4>(ctx, nR, npair, pairs, iR, nelem, XR, nk, kl, out);
+        default: return launch_klist<Tout, 4, 2, 1, 4>(ctx, nR, npair, pairs, iR, nelem, XR, nk, kl, out);
     }
+}
+
+extern "C" int wbmi_r2k_klist_pairs(wbmi_ctx* ctx, int nR, int npair, const int32_t* pairs_dev,
+                                    const int32_t* iRvec_dev, int64_t nelem, const void* XR_dev, int nk,
+                                    const double* klist_dev, void* out_dev, int prec, int tile) {
+    if (!ctx) return WBMI_ERR_ARG;
+    if (nR <= 0 || nelem <= 0 || nk <= 0 || !iRvec_dev || !XR_dev || !klist_dev || !out_dev ||
+        (pairs_dev && (npair <= 0 || npair > nR)))
+        return wbmi_fail(ctx, WBMI_ERR_ARG, "wbmi_r2k_klist: bad arguments");
+    if (tile < -1 || tile >= WBMI_KLIST_NTILES)
+        return wbmi_fail(ctx, WBMI_ERR_ARG, "wbmi_r2k_klist_tile: tile must be 0..%d", WBMI_KLIST_NTILES - 1);
+    if (tile < 0) tile = klm_rule(nk, nelem);
+    if (prec == WBMI_F64)
+        return launch_klist_tile<double>(ctx, tile, nR, npair, pairs_dev, iRvec_dev, nelem, XR_dev, nk, klist_dev, out_dev);
+    if (prec == WBMI_F32)
+        return launch_klist_tile<float>(ctx, tile, nR, npair, pairs_dev, iRvec_dev, nelem, XR_dev, nk, klist_dev, out_dev);
+    return wbmi_fail(ctx, WBMI_ERR_ARG, "wbmi_r2k_klist: bad precision");
 }
 
 extern "C" int wbmi_r2k_klist_tile(wbmi_ctx* ctx, int nR, const int32_t* iRvec_dev, int64_t nelem,
                                    const void* XR_dev, int nk, const double* klist_dev, void* out_dev, int prec,
                                    int tile) {
-    if (!ctx) return WBMI_ERR_ARG;
-    if (nR <= 0 || nelem <= 0 || nk <= 0 || !iRvec_dev || !XR_dev || !klist_dev || !out_dev)
-        return wbmi_fail(ctx, WBMI_ERR_ARG, "wbmi_r2k_klist: bad arguments");
-    if (tile < 0 || tile >= WBMI_KLIST_NTILES)
+    if (ctx && tile < 0)
         return wbmi_fail(ctx, WBMI_ERR_ARG, "wbmi_r2k_klist_tile: tile must be 0..%d", WBMI_KLIST_NTILES - 1);
-    if (prec == WBMI_F64)
-        return launch_klist_tile<double>(ctx, tile, nR, iRvec_dev, nelem, XR_dev, nk, klist_dev, out_dev);
-    if (prec == WBMI_F32)
-        return launch_klist_tile<float>(ctx, tile, nR, iRvec_dev, nelem, XR_dev, nk, klist_dev, out_dev);
-    return wbmi_fail(ctx, WBMI_ERR_ARG, "wbmi_r2k_klist: bad precision");
+    return wbmi_r2k_klist_pairs(ctx, nR, 0, nullptr, iRvec_dev, nelem, XR_dev, nk, klist_dev, out_dev, prec, tile);
 }
 
 extern "C" int wbmi_r2k_klist(wbmi_ctx* ctx, int nR, const int32_t* iRvec_dev, int64_t nelem, const void* XR_dev,
                               int nk, const double* klist_dev, void* out_dev, int prec) {
-    return wbmi_r2k_klist_tile(ctx, nR, iRvec_dev, nelem, XR_dev, nk, klist_dev, out_dev, prec, 0);
+    return wbmi_r2k_klist_pairs(ctx, nR, 0, nullptr, iRvec_dev, nelem, XR_dev, nk, klist_dev, out_dev, prec, -1);
 }
 
 extern "C" int wbmi_r2k_klist_tile_shape(int tile, int* k_rows, int* elements) {
     if (tile < 0 || tile >= WBMI_KLIST_NTILES || !k_rows || !elements) return WBMI_ERR_ARG;
-    *k_rows = 32 * klm_tiles[tile][0];
-    *elements = 32 * klm_tiles[tile][1];
+    *k_rows = 16 * klm_tiles[tile].kt * klm_tiles[tile].wk;
+    *elements = 16 * klm_tiles[tile].et * klm_tiles[tile].we;
     return WBMI_OK;
 }

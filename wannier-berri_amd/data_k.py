@@ -76,6 +76,23 @@ def channel_terms(name, der, base_offset):
     return [[[1, b0 + a, d, -1], [0, 0, -1, -1]] for a in range(3) for d in range(3)]
 
 
+def r_pairs(iRvec):
+    """The R-vectors as pairs, int32 [npair, 2]: (i, j) with R_j = -R_i, (i, -1) for one without a
+    partner (R = 0, a missing -R, repeated vectors beyond the first match)."""
+    partner = {}
+    for j, R in enumerate(iRvec.tolist()):
+        partner.setdefault(tuple(R), []).append(j)
+    pairs, used = [], set()
+    for i, R in enumerate(iRvec.tolist()):
+        if i in used:
+            continue
+        used.add(i)
+        j = next((j for j in partner.get((-R[0], -R[1], -R[2]), ()) if j not in used), -1)
+        used.add(j)
+        pairs.append((i, j))
+    return np.array(pairs, dtype=np.int32)
+
+
 class DeviceSystem:
     """Device copies of a System_R's R-space data (cached per system and device)."""
 
@@ -103,6 +120,7 @@ class DeviceSystem:
         self.cR = torch.from_numpy(np.ascontiguousarray(system.cRvec_shifted)).to(dev)
         self.iRvec = np.ascontiguousarray(system.rvec.iRvec, dtype=np.int32)
         self.iRvec_dev = torch.from_numpy(self.iRvec).to(dev)
+        self.pairs_dev = torch.from_numpy(r_pairs(self.iRvec)).to(dev)
         self._stacks = {}
         self._plans = {}
         self._zcache = collections.OrderedDict()   # z-pass outputs, least recently used first
@@ -308,7 +326,7 @@ class Data_K:
             del work
         else:
             kl = self.k_list_dev if self.k_list_dev is not None else torch.from_numpy(self.k_list).to(self.ctx.device)
-            self.ctx.r2k_klist(self.dev.iRvec_dev, stack, kl, X, prec)
+            self.ctx.r2k_klist(self.dev.iRvec_dev, stack, kl, X, prec, pairs=self.dev.pairs_dev)
         return X
 
     def _channel_keys(self):
