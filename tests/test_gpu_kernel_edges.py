@@ -139,3 +139,32 @@ def test_klist_pairs(ctx, nk, nw, extra):
                 ctx.r2k_klist(iRd, Xd, kd, out, prec, tile=tile, pairs=p)
                 err = np.abs(out.cpu().numpy().reshape(nk, nelem) - ref).max()
                 assert err < bound + (1.2e-7 * np.abs(ref).max() if prec == _lib.WBMI_F32 else 0), (tile, p is None)
+
+
+@pytest.mark.parametrize("nw,nef,nom,kbt,smr", [(2, 1, 1, 0.0, "Lorentzian"), (5, 8, 16, 0.05, "Gaussian"), (6, 15, 17, 0.0, "Lorentzian"),
+                                                (9, 7, 129, 0.05, "Lorentzian"), (20, 3, 128, 0.05, "Lorentzian"),
+                                                (34, 2, 3, 0.05, "Lorentzian")])
+def test_optical_tiles(ctx, nw, nef, nom, kbt, smr):
+    """Optical conductivity at the edges of its output tiles (128 frequencies, 64 columns of (Fermi level,
+    component)), of the pair batches and of the LDS form, with a pair of bands in one group, vs the oracle."""
+    import wannierberri_amd as wb
+    from oracle import wb_oracle as O
+    from wannierberri_amd import models
+    s = models.synthetic(num_wann=nw, Rmax=1, seed=70 + nw)
+    ham = s.get_R_mat("Ham").copy()
+    if nw > 4:
+        ham[:, -2:, :] = 0.
+        ham[:, :, -2:] = 0.
+        ham[s.rvec.iR0, -2, -2], ham[s.rvec.iR0, -1, -1] = 0.3, 0.3 + 5e-5
+        s.set_R_mat("Ham", ham, reset=True)
+    Ef, om = np.linspace(-0.5, 0.5, nef), np.linspace(0.0, 4.0, nom)
+    k = np.random.default_rng(nw).random((5, 3))
+    kw = dict(kBT=kbt, smr_fixed_width=0.1, smr_type=smr)
+    got = wb.run_klists(s, [k], {"opt": wb.calculators.dynamic.OpticalConductivity(Efermi=Ef, omega=om, **kw)})
+    o = O.OracleSystem(s.real_lattice, s.rvec.iRvec, s.wannier_centers_cart, {m: s.get_R_mat(m) for m in ("Ham", "AA")})
+    ref = O.OpticalConductivity(Ef, om, **kw)(O.OracleDataK(o, k_list=k)).data
+    scale = np.abs(ref).max()
+    if scale == 0:
+        assert np.abs(got.results["opt"].data).max() == 0
+    else:
+        assert np.abs(got.results["opt"].data - ref).max() < 1e-10 * scale

@@ -8,18 +8,14 @@
 // range, M^{ab} = sum_{i in m, j in n} i A^a_ij A^b_ji, and
 //   out[EF][w][a][b] += (f(E_n) - f(E_m)) (E_n - E_m) / (E_n - E_m - w - i eta) M^{ab}
 // (Gaussian smearing: the imaginary part is pi G(E_n - E_m - w)).
-//
-// Workgroup = (a tile of 256 (EF, w) outputs, one per thread with nine complex
-// accumulators) x (a chunk of k-points).  For each k the workgroup forms A in
-// LDS and walks the group pairs 256 at a time: every thread forms one pair's
-// M into an LDS slot, then every thread adds all slots into its outputs.  The
-// tile is added to `out` once, with FP64 atomics, at the end.
+#include <algorithm>
 #include <cmath>
 
+#include "mfma_c64.h"
 #include "wbmi_common.h"
 
 #define OC_THREADS 256
-#define OC_KCHUNK 16
+#define OC_KCHUNK 16  // k-points per workgroup of the 27-component pair kernel
 #define OC_NWMAX 128  // band groups of one k (LDS arrays of this size)
 #define OC_LDS_NW 32  // the per-k matrices (A, Y) live in LDS up to this nw, else in the workspace
 
@@ -83,36 +79,55 @@ __global__ void __launch_bounds__(256) k_build_y(int nw, int nch, wbmi_optcond_p
     }
 }
 
+// Kubo optical conductivity.  For one k, out[EF][w][ab] += sum_p F[w][p] G[p][EF ab] over its pairs p of
+// band groups, F = 1 / (x - i eta), x = E_n - E_m - w, G = (f_n - f_m)(E_n - E_m) M^{ab}: a complex matrix
+// product, on the FP64 matrix cores.  A workgroup owns OC_W frequencies x OC_C columns (EF, ab) of the output
+// (one 16-column block per wave) and accumulates them over a chunk of k-points; the pairs that some Fermi level of its
+// columns tells apart are taken OC_P at a time, their F and G formed in LDS (F once for all columns, G once
+// for all frequencies).  The tile is added to `out` once, with FP64 atomics, at the end.
+// Bound: the matrix cores (8 nw^2 nEF 9 nomega flop per k and pair kept).  One thread per output, every pair's F
+// and occupations formed by every thread, in 189 workgroups: 2.05 ms for 1000 k-points, nw = 18, 7 x 101
+// outputs; now 0.41 ms.
 // GA: A read from the workspace (nw > OC_LDS_NW, filled by k_build_y) instead of LDS.
+#define OC_P 16
+#define OC_W 128
+#define OC_C 64
+#define OC_NE (OC_C / 9 + 2)  // Fermi levels that OC_C columns touch
+
 template <typename T, bool GA>
-__global__ void __launch_bounds__(OC_THREADS) k_optcond(int nk, OcArgs a, const double* __restrict__ Eall,
-                                                        const cplx<T>* __restrict__ Xall,
-                                                        const cplx<double>* __restrict__ Aws, double* __restrict__ out) {
+__global__ void __launch_bounds__(OC_THREADS, 2) k_optcond(int nk, int kchunk, OcArgs a, const double* __restrict__ Eall,
+                                                           const cplx<T>* __restrict__ Xall,
+                                                           const cplx<double>* __restrict__ Aws, double* __restrict__ out) {
     extern __shared__ __attribute__((aligned(16))) char smem[];
     const wbmi_optcond_params& p = a.p;
     const int nw = a.nw, nw2 = nw * nw, tid = threadIdx.x;
-    cplx<double>* sA = (cplx<double>*)smem;       // [3][nw][nw] (LDS form only)
-    cplx<double>* sM = sA + (GA ? 0 : 3 * nw2);  // [OC_THREADS][9]
-    double* sEm = (double*)(sM + OC_THREADS * 9);
-    double* sEn = sEm + OC_THREADS;
-    double* sE = sEn + OC_THREADS;
-    double* sGm = sE + OC_NWMAX;
-    int* sOk = (int*)(sGm + OC_NWMAX);
-    int* sGb = sOk + OC_THREADS;
-    int& sNg = sGb[OC_NWMAX + 1];
-    const int o = blockIdx.x * OC_THREADS + tid;  // output index EF * nomega + w
-    const bool has_out = o < p.nEF * p.nomega;
-    const double mu = has_out ? p.Efermi[o / p.nomega] : 0.0;
-    const double w = has_out ? p.omega[o % p.nomega] : 0.0;
+    const int lane = tid & 63, wave = tid >> 6, li = lane & 15, g = lane >> 4;
+    cplx<double>* sF = (cplx<double>*)smem;           // [OC_P][OC_W + 1]
+    cplx<double>* sG = sF + OC_P * (OC_W + 1);        // [OC_P][OC_C + 1]
+    cplx<double>* sM = sG + OC_P * (OC_C + 1);        // [OC_P][9]
+    cplx<double>* sA = sM + OC_P * 9;                 // [3][nw][nw] (LDS form only)
+    double* sE = (double*)(sA + (GA ? 0 : 3 * nw2));  // [OC_NWMAX]
+    double* sGm = sE + OC_NWMAX;                      // [OC_NWMAX]
+    double* sOcc = sGm + OC_NWMAX;                    // [OC_NWMAX][OC_NE] occupations of the groups
+    int* sGb = (int*)(sOcc + OC_NWMAX * OC_NE);       // [OC_NWMAX + 1]
+    int* sP = sGb + OC_NWMAX + 2;                     // [OC_THREADS] pairs kept, gm | gn << 16
+    int* sN = sP + OC_THREADS;                        // [0] number of groups, [1] .. [4] pairs kept per wave
+    const int ntw = (p.nomega + OC_W - 1) / OC_W;
+    const int w0 = ((int)blockIdx.x % ntw) * OC_W, c0 = ((int)blockIdx.x / ntw) * OC_C;
+    const int ncol = min(OC_C, p.nEF * 9 - c0), nom = min(OC_W, p.nomega - w0);
+    const int e0 = c0 / 9, ne = (c0 + ncol - 1) / 9 - e0 + 1;  // Fermi levels of the columns
     const double occ_lo = p.EFmin - 30.0 * p.kBT, occ_hi = p.EFmax + 30.0 * p.kBT;
-    cplx<double> acc[9];
+    wbmi_v4d re[OC_W / 16], im[OC_W / 16];
 #pragma unroll
-    for (int ab = 0; ab < 9; ++ab) acc[ab] = mk(0.0, 0.0);
-    const int k1 = min(nk, (int)(blockIdx.y + 1) * OC_KCHUNK);
-    for (int k = blockIdx.y * OC_KCHUNK; k < k1; ++k) {
+    for (int r = 0; r < OC_W / 16; ++r) {
+        re[r] = wbmi_v4d{0.0, 0.0, 0.0, 0.0};
+        im[r] = re[r];
+    }
+    const int k1 = min(nk, (int)(blockIdx.y + 1) * kchunk);
+    for (int k = blockIdx.y * kchunk; k < k1; ++k) {
         for (int i = tid; i < nw; i += OC_THREADS) sE[i] = Eall[(int64_t)k * nw + i];
         __syncthreads();
-        if (tid == 0) sNg = band_groups(sE, nw, p.degen_thresh, p.degen_Kramers, sGb, sGm);
+        if (tid == 0) sN[0] = band_groups(sE, nw, p.degen_thresh, p.degen_Kramers, sGb, sGm);
         // A^a_ij = i D_H^a_ij (+ Abar^a_ij), D_H = -V dEinv (0 where |E_i - E_j| < 1e-7)
         const cplx<double>* Ak = GA ? Aws + (int64_t)k * 3 * nw2 : sA;
         if (!GA) {
@@ -132,59 +147,106 @@ __global__ void __launch_bounds__(OC_THREADS) k_optcond(int nk, OcArgs a, const 
             }
         }
         __syncthreads();
-        const int ng = sNg, ncand = ng * ng;
-        for (int c0 = 0; c0 < ncand; c0 += OC_THREADS) {
-            const int cnd = c0 + tid;
-            int ok = 0;
+        const int ng = sN[0], ncand = ng * ng;
+        for (int t = tid; t < ng * ne; t += OC_THREADS)
+            sOcc[(t / ne) * OC_NE + t % ne] = fermi_dirac(sGm[t / ne], p.Efermi[e0 + t % ne], p.kBT);
+        __syncthreads();
+        for (int d0 = 0; d0 < ncand; d0 += OC_THREADS) {
+            // the pairs of this stretch whose occupations differ at some level of the columns
+            const int cnd = d0 + tid;
+            bool ok = false;
+            int gm = 0, gn = 0;
             if (cnd < ncand) {
-                const int gm = cnd / ng, gn = cnd % ng;
+                gm = cnd / ng;
+                gn = cnd % ng;
                 const double Em = sGm[gm], En = sGm[gn];
-                ok = !((Em < occ_lo && En < occ_lo) || (Em > occ_hi && En > occ_hi));
-                if (ok) {
-                    sEm[tid] = Em;
-                    sEn[tid] = En;
-                    for (int ab = 0; ab < 9; ++ab) {
-                        const int ca = ab / 3, cb = ab % 3;
-                        cplx<double> s = mk(0.0, 0.0);
-                        for (int i = sGb[gm]; i < sGb[gm + 1]; ++i)
-                            for (int j = sGb[gn]; j < sGb[gn + 1]; ++j)
+                if (!((Em < occ_lo && En < occ_lo) || (Em > occ_hi && En > occ_hi)))
+                    for (int e = 0; e < ne; ++e) ok |= sOcc[gn * OC_NE + e] != sOcc[gm * OC_NE + e];
+            }
+            const uint64_t mask = __ballot(ok);
+            if (lane == 0) sN[1 + wave] = __popcll(mask);
+            __syncthreads();
+            int at = 0, np = 0;
+            for (int w = 0; w < OC_THREADS / 64; ++w) {
+                if (w < wave) at += sN[1 + w];
+                np += sN[1 + w];
+            }
+            if (ok) sP[at + __popcll(mask & ((1ull << lane) - 1))] = gm | gn << 16;
+            __syncthreads();
+            for (int p0 = 0; p0 < np; p0 += OC_P) {
+                // M^{ab} = i sum_{i in m, j in n} A^a_ij A^b_ji of the batch (none past the end)
+                if (tid < OC_P * 9) {
+                    const int q = tid / 9, ca = (tid % 9) / 3, cb = tid % 3;
+                    cplx<double> s = mk(0.0, 0.0);
+                    if (p0 + q < np) {
+                        const int m = sP[p0 + q] & 0xffff, n = sP[p0 + q] >> 16;
+                        for (int i = sGb[m]; i < sGb[m + 1]; ++i)
+                            for (int j = sGb[n]; j < sGb[n + 1]; ++j)
                                 s += Ak[(ca * nw + i) * nw + j] * Ak[(cb * nw + j) * nw + i];
-                        sM[tid * 9 + ab] = times_i(s);
+                        const double de = sGm[n] - sGm[m];
+                        s = mk(-de * s.im, de * s.re);
                     }
+                    sM[tid] = s;
                 }
-            }
-            sOk[tid] = ok;
-            __syncthreads();
-            const int ns = ncand - c0 < OC_THREADS ? ncand - c0 : OC_THREADS;
-            if (has_out) {
-                for (int s = 0; s < ns; ++s) {
-                    if (!sOk[s]) continue;
-                    const double Em = sEm[s], En = sEn[s];
-                    const double fE = fermi_dirac(En, mu, p.kBT) - fermi_dirac(Em, mu, p.kBT);
-                    if (fE == 0.0) continue;
-                    // (E_n - E_m) / (x - i eta), x = E_n - E_m - w
-                    const double x = En - Em - w;
-                    const double den = 1.0 / (x * x + p.eta * p.eta);
-                    double fr = x * den, fi = p.eta * den;
-                    if (p.smr_gaussian) {
-                        const double y = x / p.eta;
-                        fi = fabs(x) < p.eta * sqrt(200.0) ? M_PI / (sqrt(M_PI) * p.eta) * exp(-y * y) : 0.0;
+                for (int t = tid; t < OC_P * nom; t += OC_THREADS) {
+                    const int q = t / nom, w = t % nom;
+                    cplx<double> f = mk(0.0, 0.0);
+                    if (p0 + q < np) {
+                        const int m = sP[p0 + q] & 0xffff, n = sP[p0 + q] >> 16;
+                        // 1 / (x - i eta)
+                        const double x = sGm[n] - sGm[m] - p.omega[w0 + w];
+                        const double den = 1.0 / (x * x + p.eta * p.eta);
+                        f = mk(x * den, p.eta * den);
+                        if (p.smr_gaussian) {
+                            const double y = x / p.eta;
+                            f.im = fabs(x) < p.eta * sqrt(200.0) ? M_PI / (sqrt(M_PI) * p.eta) * exp(-y * y) : 0.0;
+                        }
                     }
-                    const double sc = (En - Em) * fE;
-                    const cplx<double> f = mk(sc * fr, sc * fi);
+                    sF[q * (OC_W + 1) + w] = f;
+                }
+                __syncthreads();
+                for (int t = tid; t < OC_P * OC_C; t += OC_THREADS) {
+                    const int q = t / OC_C, c = t % OC_C;
+                    cplx<double> v = mk(0.0, 0.0);
+                    if (p0 + q < np && c < ncol) {
+                        const int m = sP[p0 + q] & 0xffff, n = sP[p0 + q] >> 16, e = (c0 + c) / 9 - e0;
+                        v = (sOcc[n * OC_NE + e] - sOcc[m * OC_NE + e]) * sM[q * 9 + (c0 + c) % 9];
+                    }
+                    sG[q * (OC_C + 1) + c] = v;
+                }
+                __syncthreads();
+                if (16 * wave < ncol) {
 #pragma unroll
-                    for (int ab = 0; ab < 9; ++ab) acc[ab] += f * sM[s * 9 + ab];
+                    for (int s = 0; s < OC_P / 4; ++s) {
+                        const cplx<double> b = sG[(4 * s + g) * (OC_C + 1) + 16 * wave + li];
+#pragma unroll
+                        for (int r = 0; r < OC_W / 16; ++r) {
+                            if (16 * r >= nom) continue;
+                            const cplx<double> f = sF[(4 * s + g) * (OC_W + 1) + 16 * r + li];
+                            re[r] = __builtin_amdgcn_mfma_f64_16x16x4f64(f.re, b.re, re[r], 0, 0, 0);
+                            im[r] = __builtin_amdgcn_mfma_f64_16x16x4f64(f.re, b.im, im[r], 0, 0, 0);
+                            re[r] = __builtin_amdgcn_mfma_f64_16x16x4f64(-f.im, b.im, re[r], 0, 0, 0);
+                            im[r] = __builtin_amdgcn_mfma_f64_16x16x4f64(f.im, b.re, im[r], 0, 0, 0);
+                        }
+                    }
                 }
+                __syncthreads();
             }
-            __syncthreads();
         }
     }
-    if (has_out) {
+    const int c = 16 * wave + li;
+    if (c < ncol) {
+        const int e = (c0 + c) / 9, ab = (c0 + c) % 9;
 #pragma unroll
-        for (int ab = 0; ab < 9; ++ab) {
-            unsafeAtomicAdd(out + ((int64_t)o * 9 + ab) * 2, acc[ab].re);
-            unsafeAtomicAdd(out + ((int64_t)o * 9 + ab) * 2 + 1, acc[ab].im);
-        }
+        for (int r = 0; r < OC_W / 16; ++r)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const int w = 16 * r + g + 4 * v;
+                if (w >= nom) continue;
+                double* o = out + (((int64_t)e * p.nomega + w0 + w) * 9 + ab) * 2;
+                unsafeAtomicAdd(o, re[r][v]);
+                unsafeAtomicAdd(o + 1, im[r][v]);
+            }
     }
 }
 
@@ -197,22 +259,24 @@ static int launch_optcond(wbmi_ctx* ctx, int nk, const OcArgs& a, const double* 
                           double* out) {
     const int nw = a.nw;
     const bool ga = nw > OC_LDS_NW;
-    const int64_t nout = (int64_t)a.p.nEF * a.p.nomega;
-    dim3 g((unsigned)ceil_div(nout, OC_THREADS), (unsigned)ceil_div(nk, OC_KCHUNK));
-    const size_t lds = sizeof(cplx<double>) * ((ga ? 0 : 3 * (size_t)nw * nw) + OC_THREADS * 9) +
-                       sizeof(double) * (2 * OC_THREADS + 2 * OC_NWMAX) + sizeof(int) * (OC_THREADS + OC_NWMAX + 2);
+    const int64_t tiles = ceil_div(a.p.nomega, OC_W) * ceil_div((int64_t)a.p.nEF * 9, OC_C);
+    // k-points per workgroup: about three workgroups per CU, each adding its tile to `out` once
+    const int kchunk = (int)std::max<int64_t>({1, ceil_div((int64_t)nk * tiles, 768), ceil_div(nk, 65535)});
+    dim3 g((unsigned)tiles, (unsigned)ceil_div(nk, kchunk));
+    const size_t lds = sizeof(cplx<double>) * (OC_P * (OC_W + 1 + OC_C + 1 + 9) + (ga ? 0 : 3 * (size_t)nw * nw)) +
+                       sizeof(double) * OC_NWMAX * (2 + OC_NE) + sizeof(int) * (OC_NWMAX + 2 + OC_THREADS + 8);
     if (ga) {
         hipLaunchKernelGGL((k_build_y<T, 1>), dim3(nk), dim3(256), 0, ctx->stream, nw, a.nch, a.p, E,
                            (const cplx<T>*)X, (cplx<double>*)work);
         WBMI_LAUNCH_CHECK(ctx);
         WBMI_HIP_CHECK(ctx, hipFuncSetAttribute((const void*)k_optcond<T, true>,
                                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-        hipLaunchKernelGGL((k_optcond<T, true>), g, dim3(OC_THREADS), lds, ctx->stream, nk, a, E, (const cplx<T>*)X,
+        hipLaunchKernelGGL((k_optcond<T, true>), g, dim3(OC_THREADS), lds, ctx->stream, nk, kchunk, a, E, (const cplx<T>*)X,
                            (const cplx<double>*)work, out);
     } else {
         WBMI_HIP_CHECK(ctx, hipFuncSetAttribute((const void*)k_optcond<T, false>,
                                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-        hipLaunchKernelGGL((k_optcond<T, false>), g, dim3(OC_THREADS), lds, ctx->stream, nk, a, E,
+        hipLaunchKernelGGL((k_optcond<T, false>), g, dim3(OC_THREADS), lds, ctx->stream, nk, kchunk, a, E,
                            (const cplx<T>*)X, (const cplx<double>*)nullptr, out);
     }
     WBMI_LAUNCH_CHECK(ctx);
