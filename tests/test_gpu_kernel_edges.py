@@ -82,6 +82,35 @@ def test_scan_sea_and_split(ctx, nw, ef, precision):
         assert err < (1e-9 if precision == "fp64" else 2e-5), name
 
 
+@pytest.mark.parametrize("nw,ef,precision,terms", [
+    (2, 40.0, "fp64", "in"), (15, 40.0, "fp64", "in"), (16, 1.0, "fp32", "in"), (17, 40.0, "fp64", "in"),
+    (17, 40.0, "fp32", "in"), (33, 40.0, "fp32", "in"), (49, 2.0, "fp64", "in"), (100, 1.0, "fp64", "in"),
+    (16, 40.0, "fp64", "ex"), (17, 40.0, "fp64", "ex"), (16, 40.0, "fp64", "both"), (17, 1.0, "fp32", "both"),
+    (33, 40.0, "fp64", "both")])
+def test_scan_all_cuts(nw, ef, precision, terms):
+    """The non-additive formulas (Morb, DerMorb) at the edges of the 16-band blocks, with every border in
+    the levels' range or few of them: internal terms, external terms and both, against the oracle."""
+    import wannierberri_amd as wb
+    from oracle import wb_oracle as O
+    from wannierberri_amd import models
+    s = models.synthetic(num_wann=nw, Rmax=1, seed=70 + nw, with_BBCC=True)
+    Ef = np.linspace(-ef, ef, 9)
+    k = np.random.default_rng(nw).random((2, 3))
+    st = wb.calculators.static
+    kw = dict(kwargs_formula={"internal_terms": terms != "ex", "external_terms": terms != "in"})
+    got = wb.run_klists(s, [k], {"morb": st.Morb(Efermi=Ef, **kw), "gme": st.GME_orb_FermiSea(Efermi=Ef, **kw)},
+                        parameters_K={"precision": precision})
+    o = O.OracleSystem(s.real_lattice, s.rvec.iRvec, s.wannier_centers_cart,
+                       {m: s.get_R_mat(m) for m in ("Ham", "AA", "BB", "CC")})
+    d = O.OracleDataK(o, k_list=k)
+    for name, calc in (("morb", O.Morb(Ef, **kw)), ("gme", O.GME_orb_FermiSea(Ef, **kw))):
+        ref = calc(d).data
+        err = np.abs(got.results[name].data - ref).max() / np.abs(ref).max()
+        print(f"test_scan_all_cuts nw={nw} {precision} {terms} {name}: {err:.2e}", flush=True)
+        # sums of 1 / dE^3 over gaps above 1e-4 (the group threshold), typically 1e-2: 1e-16 * 1e6 and a margin
+        assert err < (1e-9 if precision == "fp64" else 2e-5), name
+
+
 @pytest.mark.parametrize("nw", [1, 2, 15, 16, 17, 31, 32, 33, 48, 49, 64, 65, 80, 81, 97, 112, 113, 128])
 def test_rotate_sizes(ctx, nw):
     """One size at each edge of the rotation's 16-row blocks, flagged (Hermitian part), plain and

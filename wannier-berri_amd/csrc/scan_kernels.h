@@ -51,6 +51,11 @@
 #define SC_LDS (160 * 1024)
 #define SC_M_NW 64    // dEinv o Off lives in LDS up to this nw (DerOmega / DerMorb: wherever it fits)
 #define SC_LDS_NW 32  // V and A live in LDS up to this nw
+// DerMorb with internal terms only: kernels of their own, for V and W Hermitian to the rounding of FP64
+// sums, and for complex64 channels at nw <= 32, which the rotation forms in FP32 arithmetic
+#define SC_DERMORB_IN (WBMI_FORMULA_OMEGAHPLUS + 1000)
+#define SC_DERMORB_IN32 (SC_DERMORB_IN + 1)
+#define SC_IS_DERMORB_IN(F) ((F) == SC_DERMORB_IN || (F) == SC_DERMORB_IN32)
 
 static __constant__ int c_alpha[3] = {1, 2, 0};  // utility.py:45-46
 static __constant__ int c_beta[3] = {2, 0, 1};
@@ -763,6 +768,269 @@ __device__ __attribute__((always_inline)) void eval_deromega(const Smem& S, cons
     }
 }
 
+// ---------------------------------------------------------------------------
+// every cut of a non-additive formula at once
+// ---------------------------------------------------------------------------
+//
+// Morb_Hpm and DerMorb are scanned as T(c), the trace over the bands [0, c) with the rest outside, at
+// every border c of a group in range: up to nw partitions per k-point.  Evaluated one by one they cost
+// O(nw^4) (DerMorb) and O(nw^3) (Morb_Hpm) per k.  Each term of T(c) is a sum over bands of which some
+// are below c and some are not, so it belongs to the cuts between its highest band inside and its lowest
+// band outside, and
+//     T(c) = sum_{n < c <= l} g(n, l) + sum_{x < c} r(x)
+// with g(n, l) what remains when the other bands of the term are summed over q <= n or m >= l.  These
+// sums are triangular matrix products, formed once for all cuts.  T(c) is added up from its own terms
+// only, never as a difference of running sums: bands that no evaluated cut separates may be degenerate
+// to 1e-7, and their terms exceed the rest by as much as the inverse cube of that.
+
+// T(c) += sum over n < c <= l of a 16 x 16 tile's values (rows n of block nb, columns l of block lb >= nb;
+// the lane's elements (n, l) = (lane / 16 + 4 v, lane % 16), zero where n >= l), component comp.
+// The sums over n < c are a product with a triangle of ones (the values already have the operand layout).
+__device__ __attribute__((always_inline)) inline void cut_tile_add(const Smem& S, int nw, int nb, int lb, const double (&val)[4],
+                                                                  int comp) {
+    const int lane = threadIdx.x & 63, g = lane >> 4, j = lane & 15;
+    wbmi_v4d L = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int v = 0; v < 4; ++v) L = __builtin_amdgcn_mfma_f64_16x16x4f64(4 * v + g < j ? 1.0 : 0.0, val[v], L, 0, 0, 0);
+    // L: (c, l), sum over n < c; rows summed over l, each lane keeping row g + 4 (lane % 4)
+    double x[4];
+#pragma unroll
+    for (int v = 0; v < 4; ++v) x[v] = nb < lb || g + 4 * v <= j ? L[v] : 0.0;
+    const double r0 = (lane & 1 ? x[1] : x[0]) + __shfl_xor(lane & 1 ? x[0] : x[1], 1);
+    const double r1 = (lane & 1 ? x[3] : x[2]) + __shfl_xor(lane & 1 ? x[2] : x[3], 1);
+    double r = (lane & 2 ? r1 : r0) + __shfl_xor(lane & 2 ? r0 : r1, 2);
+    r = wave_sum(r, 0xc);
+    const int c = 16 * nb + g + 4 * (lane & 3);
+    if ((lane & 0xc) == 0 && c < nw) atomicAdd(&S.cut[c * 9 + comp], r);
+    if (nb == lb) return;
+    // cuts above the rows: the columns l >= c
+    double cs = wave_sum((val[0] + val[1]) + (val[2] + val[3]), 0x30);
+    for (int o = 1; o < 16; o <<= 1) {
+        const double t = __shfl_down(cs, o, 16);
+        if (j + o < 16) cs += t;
+    }
+    const int l0 = 16 * lb, cend = min(l0 + 16, nw);
+    const double all = __shfl(cs, 0);
+    for (int c0 = 16 * nb + 16; c0 < cend; c0 += 64) {
+        const int cc = c0 + lane;
+        const double t = __shfl(cs, cc > l0 ? (cc - l0) & 15 : 0);
+        if (cc < cend) atomicAdd(&S.cut[cc * 9 + comp], cc <= l0 ? all : t);
+    }
+}
+
+// Some evaluated cut separates block nb's rows from block lb's columns (one answer per wave)
+__device__ inline bool cut_tile_needed(const Smem& S, int nw, int nb, int lb) {
+    bool any = false;
+    for (int c = 16 * nb + 1 + (int)(threadIdx.x & 63); c < min(16 * lb + 16, nw); c += 64) any |= S.need[c] != 0;
+    return __any(any);
+}
+
+// Tile pair t of the nb (nb + 1) / 2 pairs rb <= cb, by their distance (the nearest sum over most bands)
+__device__ inline void cut_tile_pair(int t, int nblk, int& rb, int& cb) {
+    int d = 0;
+    while (t >= nblk - d) {
+        t -= nblk - d;
+        ++d;
+    }
+    rb = t;
+    cb = t + d;
+}
+
+// DerMorb with internal terms only (formula/covariant.py:463-552), every needed cut into S.cut.  With
+// P = D' without its mask (anti-Hermitian), Q^a_nl = i (1 / (E_l - E_n)) (2 sign E_n + 2 E_l) P^a_nl and
+// n < c <= l, the per-cut terms (formula_task: kinds 0, s1 and 5) are, summed over n and l,
+//     Re Q^a_nl F^{bd}_ln  to the pair of a and b, column d, and (X1 symmetric) to that of a and d, column b
+//     2 Im P^a_nl H^{bd}_ln  to the pair of a and d, column b
+//     F = Y + U + W / 2, H = Y - sign U,  Y_ln = sum_{m >= c} V^b_lm P^d_mn,  U_ln = -sum_{q < c} P^d_lq V^b_qn.
+// A term of Y with m > l stays with the pair (n, l); one with m < l belongs to the pair (n, m), where
+// Q V (for F) or, because swapping l and m conjugates it, P V again (for H) collects it; m = l counts half
+// in both.  U the same with q and n.  So a task, one pair of 16-band blocks and one b, is the products
+//     [P; Q] (n, m) V^b (m, l) over m >= l,   V^b (n, q) [P, Q] (q, l) over q <= n
+// for three d and three a at once: a V and three P elements per 24 MFMAs, which leaves the matrix cores
+// as the bound.  294 k-points at nw = 64, every cut (complex64): 7.5 ms one by one, 0.45 ms together.
+// HERM: V and W are Hermitian to the rounding of the sums.  Otherwise (complex64 from the rotation in FP32
+// arithmetic, whose two triangles differ by their rounding) every term reads the triangle that
+// formula_task reads, 36 MFMAs: P V with both triangles of V, V P with both of P.
+template <bool HERM, typename T, bool LM, bool ST, bool SA, int NW, typename TS>
+__device__ __attribute__((always_inline)) void eval_dermorb_in(const Smem& S, const KCtx<T, LM, ST, SA, NW, TS>& K, double sign) {
+    constexpr int NS = HERM ? 1 : 2;
+    const int nw = K.n_(), lane = threadIdx.x & 63, lk = lane >> 4, li = lane & 15;
+    const int nblk = (nw + 15) / 16, ntask = 3 * (nblk * (nblk + 1) / 2);
+    struct Acc {
+        wbmi_v4d re[3], im[3];
+        __device__ inline void zero() {
+#pragma unroll
+            for (int r = 0; r < 3; ++r) re[r] = im[r] = wbmi_v4d{0.0, 0.0, 0.0, 0.0};
+        }
+        __device__ inline void add(int r, cplx<double> x, cplx<double> y) {
+            re[r] = __builtin_amdgcn_mfma_f64_16x16x4f64(x.re, y.re, re[r], 0, 0, 0);
+            im[r] = __builtin_amdgcn_mfma_f64_16x16x4f64(x.re, y.im, im[r], 0, 0, 0);
+            re[r] = __builtin_amdgcn_mfma_f64_16x16x4f64(-x.im, y.im, re[r], 0, 0, 0);
+            im[r] = __builtin_amdgcn_mfma_f64_16x16x4f64(x.im, y.re, im[r], 0, 0, 0);
+        }
+        __device__ inline cplx<double> get(int r, int v) const { return mk(re[r][v], im[r][v]); }
+    };
+    for (;;) {
+        int t = 0;
+        if (lane == 0) t = atomicAdd(&S.misc[3], 1);
+        t = __builtin_amdgcn_readfirstlane(t) * (int)gridDim.y + (int)blockIdx.y;
+        if (t >= ntask) break;
+        const int b = t % 3;
+        int nb, lb;
+        cut_tile_pair(t / 3, nblk, nb, lb);
+        if (!cut_tile_needed(S, nw, nb, lb)) continue;
+        int ax[3];  // the indices b, b + 1, b + 2: everything below is relative to b
+#pragma unroll
+        for (int r = 0; r < 3; ++r) ax[r] = (b + r) % 3;
+        // the pairs' values: components (c, d) relative to b, c = 1, 2 in [0, 6), (0, 0) in [6]
+        double o[7][4];
+#pragma unroll
+        for (int q = 0; q < 7; ++q)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) o[q][v] = 0.0;
+        Acc G[NS], Z;  // P V or V P of both kinds of V or P; Q V or V Q
+        // FIRST: the sums over m >= l, with f = W / 2 - (P V) = conj(F), h = -(P V) = conj(H); else those
+        // over q <= n, with f = (V P), h = -sign (V P)
+        auto add_pairs = [&](auto first) {
+            constexpr bool FIRST = decltype(first)::value;
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                // an opaque row: the operands are loaded anew for each v and call, not kept in registers
+                int nn = 16 * nb + lk + 4 * v;
+                asm volatile("" : "+v"(nn));
+                const int ll = 16 * lb + li;
+                const bool ok = nn < ll && ll < nw;
+                const int x = min(nn, nw - 1), y = min(ll, nw - 1);
+                const double m = K.m(x, y), kap = -m * (2.0 * sign * S.E[x] + 2.0 * S.E[y]);
+                cplx<double> P[3], Pu[3];
+#pragma unroll
+                for (int r = 0; r < 3; ++r) {
+                    Pu[r] = FIRST && !HERM ? mk(0.0, 0.0) : (-m) * K.V(ax[r], x, y);
+                    P[r] = HERM && !FIRST ? Pu[r] : HERM ? (-m) * K.V(ax[r], x, y) : (-m) * conj(K.V(ax[r], y, x));
+                }
+#pragma unroll
+                for (int d = 0; d < 3; ++d) {
+                    cplx<double> f = G[0].get(d, v);
+                    if constexpr (FIRST) f = (HERM ? 0.5 * K.W(b, ax[d], x, y) : 0.5 * conj(K.W(b, ax[d], y, x))) - f;
+#pragma unroll
+                    for (int a = 0; a < 3; ++a) {
+                        const double s = -kap * (P[a] * conj(f)).im - (Z.get(a, v) * conj(P[d])).re;
+                        if (a != 0) {
+                            const double e = pair_sign(a, 0) * s;
+                            o[(third_index(a, 0) - 1) * 3 + d][v] += ok ? e : 0.0;
+                        }
+                        if (a != d) {
+                            const bool pos = pair_sign(a, d) > 0.0;
+                            const cplx<double> h = G[pos ? 0 : NS - 1].get(d, v);
+                            const double hw = FIRST ? -2.0 : -2.0 * sign;
+                            const double e = pair_sign(a, d) * (s + hw * ((!FIRST && pos ? Pu[a] : P[a]) * conj(h)).im);
+                            const int c = third_index(a, d);
+                            o[c == 0 ? 6 : (c - 1) * 3][v] += ok ? e : 0.0;
+                        }
+                    }
+                }
+            }
+        };
+        // rows and columns past the end repeat the last one; their results are not read
+        const int n = min(16 * nb + li, nw - 1), l = min(16 * lb + li, nw - 1);
+        const double En = S.E[n], El = S.E[l];
+        Z.zero();
+#pragma unroll
+        for (int q = 0; q < NS; ++q) G[q].zero();
+        for (int k0 = 16 * lb; k0 < nw; k0 += 4) {
+            const int m = min(k0 + lk, nw - 1);
+            const double w = k0 + lk >= nw || m < l ? 0.0 : m == l ? 0.5 : 1.0;
+            const cplx<double> vl = w * K.V(b, m, l), vu = HERM ? vl : w * conj(K.V(b, l, m));
+            const double mm = K.m(n, m), kap = -mm * (2.0 * sign * En + 2.0 * S.E[m]);
+#pragma unroll
+            for (int r = 0; r < 3; ++r) {
+                const cplx<double> P = (-mm) * conj(K.V(ax[r], m, n));
+                G[0].add(r, P, vu);
+                if constexpr (!HERM) G[1].add(r, P, vl);
+                Z.add(r, mk(-kap * P.im, kap * P.re), vl);
+            }
+        }
+        add_pairs(std::true_type{});
+        Z.zero();
+#pragma unroll
+        for (int q = 0; q < NS; ++q) G[q].zero();
+        for (int k0 = 0; k0 < min(16 * nb + 16, nw); k0 += 4) {
+            const int q = min(k0 + lk, nw - 1);
+            const double w = k0 + lk >= nw || q > n ? 0.0 : q == n ? 0.5 : 1.0;
+            const cplx<double> vl = w * K.V(b, n, q), vu = HERM ? vl : w * conj(K.V(b, q, n));
+            const double mm = K.m(q, l), kap = mm * (2.0 * sign * S.E[q] + 2.0 * El);  // Q enters with -
+#pragma unroll
+            for (int r = 0; r < 3; ++r) {
+                const cplx<double> Pu = (-mm) * K.V(ax[r], q, l), P = HERM ? Pu : (-mm) * conj(K.V(ax[r], l, q));
+                G[0].add(r, vu, P);
+                if constexpr (!HERM) G[1].add(r, vl, Pu);
+                Z.add(r, vl, mk(-kap * P.im, kap * P.re));
+            }
+        }
+        add_pairs(std::false_type{});
+#pragma unroll
+        for (int q = 0; q < 7; ++q) cut_tile_add(S, nw, nb, lb, o[q], q == 6 ? b * 4 : ax[1 + q / 3] * 3 + ax[q % 3]);
+    }
+}
+
+// Morb_Hpm (formula/covariant.py:390-414), every needed cut into S.cut: the sums over l outside are
+// pair values, those over m inside are r(max(n, m)).  One wave per pair of 16-band blocks.
+// 294 k-points at nw = 64, every cut: 1.72 ms with a loop over l per cut and band, 0.028 ms.
+template <typename T, bool LM, bool ST, bool SA, int NW, typename TS>
+__device__ __attribute__((always_inline)) void eval_morb_cuts(const Smem& S, const KCtx<T, LM, ST, SA, NW, TS>& K, bool in, bool ex,
+                                                             double sign) {
+    const int nw = K.n_(), tid = threadIdx.x, lane = tid & 63, lk = lane >> 4, li = lane & 15;
+    const int nblk = (nw + 15) / 16;
+    for (int t = tid >> 6; t < nblk * (nblk + 1) / 2; t += (int)blockDim.x >> 6) {
+        int nb, lb;
+        cut_tile_pair(t, nblk, nb, lb);
+        double o[3][4], r[3] = {0.0, 0.0, 0.0};
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const int nn = 16 * nb + lk + 4 * v, ll = 16 * lb + li;
+            const bool ok = nn < ll && ll < nw, okd = nn == ll && ll < nw;
+            const int x = min(nn, nw - 1), y = min(ll, nw - 1);
+            const double Ex = sign * S.E[x], Ey = S.E[y];
+            cplx<double> D[3], Dt[3], A[3], At[3], B[3];
+#pragma unroll
+            for (int a = 0; a < 3; ++a) {
+                D[a] = K.Dp(a, x, y);
+                Dt[a] = in ? K.Dp(a, y, x) : mk(0.0, 0.0);
+                A[a] = ex ? K.A(a, x, y) : mk(0.0, 0.0);
+                At[a] = ex ? K.A(a, y, x) : mk(0.0, 0.0);
+                B[a] = ex ? K.B(a, y, x) : mk(0.0, 0.0);
+            }
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+                const int al = c == 2 ? 0 : c + 1, be = c == 0 ? 2 : c - 1;
+                double g = 0.0, w = 0.0;
+                if (in) g += 2.0 * (Ey + Ex) * (D[al] * Dt[be]).im;
+                if (ex) {
+                    g += 2.0 * (D[be] * B[al] - D[al] * B[be]).re + 2.0 * Ex * (D[be] * At[al] - D[al] * At[be]).re;
+                    w = 2.0 * (Ey + Ex) * (A[al] * At[be]).im;
+                    if (ok) w += 2.0 * (S.E[x] + sign * Ey) * (At[al] * A[be]).im;
+                    if (okd) w += K.C(c, x, x).re + Ex * K.O(c, x, x).re;
+                }
+                o[c][v] = ok ? g : 0.0;
+                r[c] += ok || okd ? w : 0.0;
+            }
+        }
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            cut_tile_add(S, nw, nb, lb, o[c], c);
+            const double rs = wave_sum(r[c], 0x30);
+            if (lane < 16 && 16 * lb + lane < nw) atomicAdd(&S.acc[(16 * lb + lane) * 9 + c], rs);
+        }
+    }
+    __syncthreads();
+    for (int t = tid; t < nw * 3 && ex; t += (int)blockDim.x) {
+        const int c = t / 3 + 1, q = t % 3;
+        double v = S.cut[c * 9 + q];
+        for (int x = 0; x < c; ++x) v += S.acc[x * 9 + q];
+        S.cut[c * 9 + q] = v;
+    }
+}
+
 // Per-band values for the current partition (the labels'; cut >= 0: they are those of [0, cut), and M
 // holds the unmasked dEinv) into S.acc[n][comp].
 template <int F, typename T, bool LM, bool ST, bool SA, int NW, typename TS>
@@ -1158,7 +1426,7 @@ __host__ __device__ constexpr int scan_min_waves(bool tasks, int nth) { return !
 
 // NW > 0: the kernel for nw = NW only, every size and row stride a compile-time constant
 template <typename T, int F, bool LM, bool ST, int MODE, int NW, int NTH>
-__global__ void __launch_bounds__(NTH, (scan_min_waves((F == WBMI_FORMULA_DEROMEGA || F == WBMI_FORMULA_DERMORB) && MODE != 1, NTH)))
+__global__ void __launch_bounds__(NTH, SC_IS_DERMORB_IN(F) ? 2 : (scan_min_waves((F == WBMI_FORMULA_DEROMEGA || F == WBMI_FORMULA_DERMORB) && MODE != 1, NTH)))
 k_static_scan(ScanArgs args, const double* __restrict__ Eall, const cplx<T>* __restrict__ Xall, double* __restrict__ hist) {
     extern __shared__ __attribute__((aligned(16))) char smem_raw[];
     const wbmi_scan_params& p = args.p;
@@ -1427,31 +1695,45 @@ k_static_scan(ScanArgs args, const double* __restrict__ Eall, const cplx<T>* __r
     } else {
         // non-additive: traces of the cumulative cuts [0, c) (static.py:109-117) at the borders of
         // the groups in range and of the sea
+        constexpr bool all_cuts = SC_IS_DERMORB_IN(F) || F == WBMI_FORMULA_MORB_HPM;
         for (int n = tid; n <= nw; n += (int)blockDim.x) S.need[n] = 0;
+        if constexpr (all_cuts) {
+            for (int t = tid; t < nw * 9; t += (int)blockDim.x) S.acc[t] = S.cut[t + 9] = 0.0;
+            for (int n = tid; n < nw; n += (int)blockDim.x) S.lab[n] = n;  // D' unmasked
+            if (tid == 0) S.misc[3] = 0;                                  // task counter
+        }
         if constexpr (LM) build_M<false>(S, nw);
         __syncthreads();
         for (int g = tid; g < ng; g += (int)blockDim.x)
             if (S.gin[g]) S.need[S.gb[g]] = S.need[S.gb[g + 1]] = 1;
         if (tid == 0 && sea_hi > sea_lo) S.need[sea_lo] = S.need[sea_hi] = 1;
         __syncthreads();
-        for (int cidx = 1; cidx <= nw; ++cidx) {
-            if (!S.need[cidx]) continue;
-            for (int n = tid; n < nw; n += (int)blockDim.x) {
-                int inn = n < cidx;
-                S.lab[n] = inn ? 0 : 1;
-                S.gs[n] = inn ? 0 : cidx;
-                S.ge[n] = inn ? cidx : nw;
-                S.act[n] = inn;
-            }
+        if constexpr (SC_IS_DERMORB_IN(F)) {
+            if (p.internal_terms) eval_dermorb_in<F == SC_DERMORB_IN>(S, K, (double)p.sign);
             __syncthreads();
-            eval_partition<F>(S, K, p, cidx);
-            for (int c = tid >> 6; c < ncomp; c += (int)blockDim.x >> 6) {
-                double v = 0.0;
-                for (int n = tid & 63; n < cidx; n += 64) v += S.acc[n * 9 + c];
-                v = wave_sum(v, 63);
-                if ((tid & 63) == 0) S.cut[cidx * 9 + c] = v;
-            }
+        } else if constexpr (all_cuts) {
+            eval_morb_cuts(S, K, p.internal_terms, p.external_terms, (double)p.sign);
             __syncthreads();
+        } else {
+            for (int cidx = 1; cidx <= nw; ++cidx) {
+                if (!S.need[cidx]) continue;
+                for (int n = tid; n < nw; n += (int)blockDim.x) {
+                    int inn = n < cidx;
+                    S.lab[n] = inn ? 0 : 1;
+                    S.gs[n] = inn ? 0 : cidx;
+                    S.ge[n] = inn ? cidx : nw;
+                    S.act[n] = inn;
+                }
+                __syncthreads();
+                eval_partition<F>(S, K, p, cidx);
+                for (int c = tid >> 6; c < ncomp; c += (int)blockDim.x >> 6) {
+                    double v = 0.0;
+                    for (int n = tid & 63; n < cidx; n += 64) v += S.acc[n * 9 + c];
+                    v = wave_sum(v, 63);
+                    if ((tid & 63) == 0) S.cut[cidx * 9 + c] = v;
+                }
+                __syncthreads();
+            }
         }
         for (int c = tid; c < ncomp; c += (int)blockDim.x) S.cut[c] = 0.0;
         __syncthreads();
@@ -1488,7 +1770,7 @@ static int launch_scan_t(wbmi_ctx* ctx, int nk, const ScanArgs& a, const double*
     // other modes use a k-point's sums before they are complete.
     constexpr bool tasks = F == WBMI_FORMULA_DEROMEGA || F == WBMI_FORMULA_DERMORB;
     const int want = a.nw > 32 ? 1024 : 512;
-    const int parts = tasks && MODE == 0 && nk < want ? std::min(8, want / nk) : 1;
+    const int parts = (tasks || SC_IS_DERMORB_IN(F)) && MODE == 0 && nk < want ? std::min(8, want / nk) : 1;
     WBMI_HIP_CHECK(ctx, hipFuncSetAttribute((const void*)k_static_scan<T, F, LM, ST, MODE, NW, NTH>,
                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     hipLaunchKernelGGL((k_static_scan<T, F, LM, ST, MODE, NW, NTH>), dim3(nk, parts), dim3(NTH), lds, ctx->stream, a, E,
@@ -1503,7 +1785,15 @@ static int launch_scan_t(wbmi_ctx* ctx, int nk, const ScanArgs& a, const double*
 template <typename T, int F, int MODE>
 static int launch_scan(wbmi_ctx* ctx, int nk, const ScanArgs& a, const double* E, const void* X, double* hist) {
     constexpr bool tasks = F == WBMI_FORMULA_DEROMEGA || F == WBMI_FORMULA_DERMORB;
-    if constexpr (tasks && MODE != 1) {
+    // the kernels of all cuts: Morb_Hpm reads each dEinv once; DerMorb's is bound by its 256 registers,
+    // two waves per SIMD
+    if constexpr (F == WBMI_FORMULA_MORB_HPM && MODE != 2) {
+        return launch_scan_t<T, F, false, false, MODE, 0, 256>(ctx, nk, a, E, X, hist);
+    } else if constexpr (SC_IS_DERMORB_IN(F)) {
+        if (smem_offsets(a.nw, true, false, false, MODE == 1, sizeof(cplx<T>)).total <= SC_LDS / 2)
+            return launch_scan_t<T, F, true, false, MODE, 0, 256>(ctx, nk, a, E, X, hist);
+        return launch_scan_t<T, F, MODE == 0, false, MODE, 0, 512>(ctx, nk, a, E, X, hist);
+    } else if constexpr (tasks && MODE != 1) {
         if (a.stage_va) {
             if constexpr (MODE == 0 && F == WBMI_FORMULA_DEROMEGA)
                 // nw = 32 (a single 32-column block, the spin blocks of the spinor models) has its own
@@ -1538,7 +1828,14 @@ static int dispatch_scan(wbmi_ctx* ctx, int nk, const ScanArgs& a, const double*
         case WBMI_FORMULA_VELOMEGA: return launch_scan<T, WBMI_FORMULA_VELOMEGA, MODE>(ctx, nk, a, E, X, hist);
         case WBMI_FORMULA_MORB_HPM: return launch_scan<T, WBMI_FORMULA_MORB_HPM, MODE>(ctx, nk, a, E, X, hist);
         case WBMI_FORMULA_VELHPLUS: return launch_scan<T, WBMI_FORMULA_VELHPLUS, MODE>(ctx, nk, a, E, X, hist);
-        case WBMI_FORMULA_DERMORB: return launch_scan<T, WBMI_FORMULA_DERMORB, MODE>(ctx, nk, a, E, X, hist);
+        case WBMI_FORMULA_DERMORB:
+            if constexpr (MODE != 2)
+                if (!a.p.external_terms) {
+                    if constexpr (sizeof(T) == 4)
+                        if (a.nw <= 32) return launch_scan<T, SC_DERMORB_IN32, MODE>(ctx, nk, a, E, X, hist);
+                    return launch_scan<T, SC_DERMORB_IN, MODE>(ctx, nk, a, E, X, hist);
+                }
+            return launch_scan<T, WBMI_FORMULA_DERMORB, MODE>(ctx, nk, a, E, X, hist);
         case WBMI_FORMULA_DERSPIN: return launch_scan<T, WBMI_FORMULA_DERSPIN, MODE>(ctx, nk, a, E, X, hist);
         case WBMI_FORMULA_VELSPIN: return launch_scan<T, WBMI_FORMULA_VELSPIN, MODE>(ctx, nk, a, E, X, hist);
         case WBMI_FORMULA_SPIN: return launch_scan<T, WBMI_FORMULA_SPIN, MODE>(ctx, nk, a, E, X, hist);
