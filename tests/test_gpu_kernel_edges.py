@@ -47,6 +47,30 @@ def test_eigh_sizes(ctx, nw):
         assert np.abs(U.conj().swapaxes(1, 2) @ U - np.eye(nw)).max() < 8 * eps * nw
 
 
+@pytest.mark.parametrize("nw", [5, 16, 17, 32, 44, 45, 48, 49, 64, 65])
+@pytest.mark.parametrize("gap", [1.0, 1e-9])
+def test_eigh_refine_blocks(ctx, nw, gap):
+    """The refinement at the edges of its 16 x 16 blocks, without and with a pair of eigenvalues so close
+    that the correction steps leave it mixed (the Jacobi pass over clusters)."""
+    import torch
+    from wannierberri_amd import _lib
+    rng = np.random.default_rng(nw)
+    nk = 3
+    E = np.cumsum(0.5 + rng.random((nk, nw)), axis=1)
+    E[:, nw // 2] = E[:, nw // 2 - 1] + gap * (0.5 if gap == 1.0 else 1.0)
+    V = np.linalg.qr(rng.standard_normal((nk, nw, nw)) + 1j * rng.standard_normal((nk, nw, nw)))[0]
+    H = (V * E[:, None, :]) @ V.conj().swapaxes(1, 2)
+    H = 0.5 * (H + H.conj().swapaxes(1, 2))
+    norm = np.abs(E).max()
+    Ed = torch.empty((nk, nw), dtype=torch.float64, device="cuda")
+    U = torch.empty((nk, nw, nw), dtype=torch.complex128, device="cuda")
+    ctx.eigh(torch.from_numpy(H).cuda(), nw * nw, Ed, U, _lib.WBMI_F64, nw, refine=16)
+    e, u = Ed.cpu().numpy(), U.cpu().numpy()
+    assert np.abs(e - np.linalg.eigvalsh(H)).max() < 8 * EPS * nw * norm
+    assert np.abs(H @ u - u * e[:, None, :]).max() < 8 * EPS * nw * norm
+    assert np.abs(u.conj().swapaxes(1, 2) @ u - np.eye(nw)).max() < 8 * EPS * nw
+
+
 @pytest.mark.parametrize("nw,ef,precision", [(3, 0.6, "fp64"), (16, 1.0, "fp64"), (17, 1.0, "fp32"), (24, 40.0, "fp64"),
                                              (32, 1.0, "fp64"), (32, 1.0, "fp32"), (33, 1.5, "fp64")])
 def test_scan_sea_and_split(ctx, nw, ef, precision):

@@ -12,6 +12,8 @@
 // refine = 0; refined solves start from the FP32 kernels below it.
 #include <cfloat>
 
+#include <type_traits>
+
 #include "mfma_c64.h"
 #include "wbmi_common.h"
 
@@ -660,7 +662,6 @@ __global__ void __launch_bounds__(JREG_THREADS) k_eigh_jacobi_reg(int nw, const 
 // clusters below delta are re-orthogonalised only.
 // ---------------------------------------------------------------------------
 
-#define OA_THREADS 256
 // stop refining once ||E||_F is below this: complex64 vectors are limited by
 // their storage; complex128 vectors after a step with ||E|| < 1e-10 are
 // accurate to ~||E||^2 ||H|| / gap, i.e. to FP64 rounding
@@ -672,47 +673,6 @@ __global__ void __launch_bounds__(JREG_THREADS) k_eigh_jacobi_reg(int nw, const 
 // and the cluster pass that follows rotates every pair still mixed by more than
 // OA_TOL_C64 (close pairs converge more slowly).
 #define OA_LAST_C64 1e-4
-
-// C = X Y (nw x nw, complex FP64) on the matrix cores: 16 x 16 output blocks
-// dealt to the waves of the workgroup, four independent accumulators per block
-// (re re, re im, im re, im im) so that consecutive MFMAs never wait on each
-// other; out(r, c, value) for r, c < nw.  Lane layout as in mfma_c64.h.
-template <int NTHREADS, class FX, class FY, class FO>
-__device__ __attribute__((always_inline)) void oa_gemm(int nw, FX X, FY Y, FO out) {
-    const int wave = threadIdx.x >> 6, nwave = NTHREADS / 64;
-    const int li = threadIdx.x & 15, lk = (threadIdx.x & 63) >> 4;
-    const int nb = (nw + 15) / 16;
-    for (int t = wave; t < nb * nb; t += nwave) {
-        const int r0 = (t / nb) * 16, c0 = (t % nb) * 16;
-        const bool rok = r0 + li < nw, cok = c0 + li < nw;
-        wbmi_v4d rr = {0.0, 0.0, 0.0, 0.0}, ri = rr, ir = rr, ii = rr;
-#pragma unroll 2
-        for (int k0 = 0; k0 < nw; k0 += 4) {
-            const int k = k0 + lk;
-            const bool kok = k < nw;
-            const cplx<double> a = (kok && rok) ? X(r0 + li, k) : mk(0.0, 0.0);
-            const cplx<double> b = (kok && cok) ? Y(k, c0 + li) : mk(0.0, 0.0);
-            rr = __builtin_amdgcn_mfma_f64_16x16x4f64(a.re, b.re, rr, 0, 0, 0);
-            ri = __builtin_amdgcn_mfma_f64_16x16x4f64(a.re, b.im, ri, 0, 0, 0);
-            ir = __builtin_amdgcn_mfma_f64_16x16x4f64(a.im, b.re, ir, 0, 0, 0);
-            ii = __builtin_amdgcn_mfma_f64_16x16x4f64(a.im, b.im, ii, 0, 0, 0);
-        }
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            const int r = r0 + lk + 4 * v, c = c0 + li;
-            if (r < nw && c < nw) out(r, c, mk(rr[v] - ii[v], ri[v] + ir[v]));
-        }
-    }
-}
-
-// A = (H + H^+)/2 of k-point Hk into LDS
-__device__ inline void oa_load_a(int nw, int ld, const cplx<double>* __restrict__ Hk, cplx<double>* sA) {
-    for (int t = threadIdx.x; t < nw * nw; t += OA_THREADS) {
-        const int i = t / nw, j = t % nw;
-        const cplx<double> x = Hk[i * nw + j], y = Hk[j * nw + i];
-        sA[i * ld + j] = mk(0.5 * (x.re + y.re), 0.5 * (x.im - y.im));
-    }
-}
 
 // Scratch of cluster_jacobi in LDS: per pair {c, s cos phi, s sin phi} and
 // (p, q), plus a round flag pair.
@@ -734,6 +694,11 @@ __host__ __device__ inline size_t cj_lds(int n) {
 // The rotations update S (columns and rows) and the columns of X.
 // Uniform control flow: the round flag is set by the rotating threads and
 // read by every thread after a barrier (double-buffered by round parity).
+__device__ inline bool cluster_pair(cplx<double> apq, double app, double aqq, double theta, double floor_abs) {
+    const double g = sqrt(apq.re * apq.re + apq.im * apq.im);
+    return g > floor_abs && g > theta * fabs(aqq - app);
+}
+
 template <int NTH, class FS, class FX>
 __device__ void cluster_jacobi(int n, FS S, FX X, char* scratch, double theta, double floor_abs, int max_sweeps) {
     const int ne = n + (n & 1), np = ne / 2;
@@ -755,7 +720,7 @@ __device__ void cluster_jacobi(int n, FS S, FX X, char* scratch, double theta, d
                     const cplx<double> apq = S(p, q);
                     const double g = sqrt(apq.re * apq.re + apq.im * apq.im);
                     const double app = S(p, p).re, aqq = S(q, q).re;
-                    if (g > floor_abs && g > theta * fabs(aqq - app)) {
+                    if (cluster_pair(apq, app, aqq, theta, floor_abs)) {
                         const double tau = (aqq - app) / (2.0 * g);
                         const double t = (tau >= 0 ? 1.0 : -1.0) / (fabs(tau) + sqrt(1.0 + tau * tau));
                         c = 1.0 / sqrt(1.0 + t * t);
@@ -816,59 +781,159 @@ __device__ void cluster_jacobi(int n, FS S, FX X, char* scratch, double theta, d
 // re-orthogonalised there; the following steps separate it, converging
 // quadratically once the mixing angle is small (six to eight steps for a
 // relative gap of 4e-6 at nw = 18..40).
-// (at least 5 waves per SIMD: 72 VGPRs and no AGPRs, 7 waves per SIMD)
-template <typename TU>
-__global__ void __launch_bounds__(OA_THREADS, 5) k_eigh_refine(int nw, const cplx<double>* __restrict__ H64,
-                                                            int64_t Hstride, double* __restrict__ Eout,
-                                                            cplx<TU>* __restrict__ U, int iters, double tol) {
+//
+// One wave per 16 x 16 block of the matrices, NB x NB waves per k-point (nw <= 64): a wave keeps its block
+// of S, R and X + X E in registers from the product to the elementwise step that uses it, S and X^+ X
+// share their operand, and X, T = A X / E and (NB <= 3) A are the matrices in LDS; at NB = 4 A comes from
+// L2.  The chain of dependent products and barriers bounds it, not the matrix cores, so what counts is
+// k-points in flight and steps left out: the cluster pass runs only where a pair needs it.
+// With four waves per k-point for every size, S and R through LDS and the cluster pass always, against now:
+// nw = 32, 4096 k-points: complex128 657 -> 406 us (0.18 ms of matrix instructions), complex64 382 -> 192;
+// nw = 12, 1728: 42.5 -> 26.2; nw = 2, 625: 32.9 -> 15.2; through global memory before, nw = 48, 3898
+// k-points, complex64: 1509 -> 725; nw = 64, 294: 314 -> 182.
+// SPLIT: re re, im im, re im and im re summed apart, the order of every complex64 result up to nw = 44 (above,
+// and for complex128, together: half the accumulators).  A last-bit difference in the FP64 vectors moves a
+// complex64 element by its rounding now and then, which close bands magnify.
+template <typename TU, int NB, bool SPLIT>
+__global__ void __launch_bounds__(64 * NB * NB, NB == 3 ? 5 : NB == 4 ? 4 : 3)
+k_eigh_refine(int nw, const cplx<double>* __restrict__ H64, int64_t Hstride, double* __restrict__ Eout,
+              cplx<TU>* __restrict__ U, int iters, double tol) {
+    constexpr int NTH = 64 * NB * NB;
+    constexpr bool ALDS = NB <= 3;
     extern __shared__ __attribute__((aligned(16))) char smem[];
     const int ld = nw + 1;
-    cplx<double>* sX = (cplx<double>*)smem;   // X (approximate eigenvectors)
-    cplx<double>* sA = sX + nw * ld;          // A (for the whole solve)
-    cplx<double>* sT = sA + nw * ld;          // A X, then R, then X + X E
-    cplx<double>* sS = sT + nw * ld;          // S, then E
-    double* lam = (double*)(sS + nw * ld);
-    double* red = lam + nw;                   // [0] ||S-D||^2, [1] ||R||^2, [2] max|lam|, [3] ||E||^2
-    char* cjs = (char*)(red + 4);             // cluster_jacobi scratch
+    cplx<double>* sX = (cplx<double>*)smem;                 // X (approximate eigenvectors)
+    cplx<double>* sT = sX + nw * ld;                        // A X, then E
+    cplx<double>* sA = sT + nw * ld;                        // A (for the whole solve)
+    double* lam = (double*)(ALDS ? sA + nw * ld : sA);
+    double* den = lam + nw;                                 // squared norms of the columns
+    double* red2 = den + nw;                                // two sets, steps in turn:
+    // [0] ||S-D||^2, [1] ||R||^2, [2] max|lam|, [3] ||E||^2
+    char* cjs = (char*)(red2 + 8);                          // cluster_jacobi scratch
     int* rank = (int*)(cjs + cj_lds(nw));
-    const int tid = threadIdx.x;
+    const int tid = threadIdx.x, li = tid & 15, lk = (tid & 63) >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), r0 = 16 * (wave / NB), c0 = 16 * (wave % NB);
     const int64_t k = blockIdx.x;
     const cplx<double>* Hk = H64 + k * Hstride;
     cplx<TU>* Uk = U + k * nw * nw;
-    for (int t = tid; t < nw * nw; t += OA_THREADS) {
-        const cplx<TU> u = Uk[t];
-        sX[(t / nw) * ld + t % nw] = mk((double)u.re, (double)u.im);
-    }
-    oa_load_a(nw, ld, Hk, sA);
+    const int c = c0 + li;                                       // the lane's elements: (r0 + lk + 4 v, c)
+    const int ra = min(r0 + li, nw - 1), cc = min(c, nw - 1);    // operand row and column
+    auto row = [&](int v) { return r0 + lk + 4 * v; };
+    auto inside = [&](int v) { return c < nw && row(v) < nw; };
+    auto herm = [&](int i, int j) {  // (H + H^+)/2
+        const cplx<double> x = Hk[i * nw + j], y = Hk[j * nw + i];
+        return mk(0.5 * (x.re + y.re), 0.5 * (x.im - y.im));
+    };
+    struct Tile {
+        wbmi_v4d re, im;
+        __device__ inline cplx<double> get(int v) const { return mk(re[v], im[v]); }
+    };
+    const wbmi_v4d z4 = {0.0, 0.0, 0.0, 0.0};
+    struct Sum {
+        wbmi_v4d re, im, ii, ir;  // ii, ir: SPLIT only
+        __device__ inline void add(cplx<double> a, cplx<double> b) {
+            re = __builtin_amdgcn_mfma_f64_16x16x4f64(a.re, b.re, re, 0, 0, 0);
+            im = __builtin_amdgcn_mfma_f64_16x16x4f64(a.re, b.im, im, 0, 0, 0);
+            if constexpr (SPLIT) {
+                ir = __builtin_amdgcn_mfma_f64_16x16x4f64(a.im, b.re, ir, 0, 0, 0);
+                ii = __builtin_amdgcn_mfma_f64_16x16x4f64(a.im, b.im, ii, 0, 0, 0);
+            } else {
+                re = __builtin_amdgcn_mfma_f64_16x16x4f64(-a.im, b.im, re, 0, 0, 0);
+                im = __builtin_amdgcn_mfma_f64_16x16x4f64(a.im, b.re, im, 0, 0, 0);
+            }
+        }
+        __device__ inline Tile tile() const {
+            if constexpr (SPLIT) return Tile{re - ii, im + ir};
+            else return Tile{re, im};
+        }
+    };
+    // the wave's block of P Q, and of P Q and P Q2 together; operand columns / rows from nw on count zero
+    auto product = [&](auto P, auto Q) {
+        Sum t{z4, z4, z4, z4};
+#pragma unroll 2
+        for (int k0 = 0; k0 < nw; k0 += 4) {
+            const int m = min(k0 + lk, nw - 1);
+            const cplx<double> a = P(m);
+            cplx<double> b = Q(m);
+            if (k0 + lk >= nw) b = mk(0.0, 0.0);
+            t.add(a, b);
+        }
+        return t.tile();
+    };
+    auto products = [&](auto P, auto Q, auto Q2, Tile& r, Tile& r2) {
+        Sum t{z4, z4, z4, z4}, t2 = t;
+#pragma unroll 2
+        for (int k0 = 0; k0 < nw; k0 += 4) {
+            const int m = min(k0 + lk, nw - 1);
+            cplx<double> a = P(m);
+            const cplx<double> b = Q(m), b2 = Q2(m);
+            if (k0 + lk >= nw) a = mk(0.0, 0.0);
+            t.add(a, b);
+            t2.add(a, b2);
+        }
+        r = t.tile();
+        r2 = t2.tile();
+    };
+    auto Arow = [&](int m) {
+        if constexpr (ALDS) return sA[ra * ld + m];
+        else return herm(ra, m);
+    };
+    auto Xrow = [&](int m) { return sX[ra * ld + m]; };
+    auto Xadj = [&](int m) { return conj(sX[m * ld + ra]); };
+    auto Xcol = [&](int m) { return sX[m * ld + cc]; };
+    auto Tcol = [&](int m) { return sT[m * ld + cc]; };
+    auto store = [&](cplx<double>* M, const Tile& t) {
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+            if (inside(v)) M[row(v) * ld + c] = t.get(v);
+    };
+    auto add_X_times_T = [&] {  // X <- X + X sT
+        Tile t = product(Xrow, Tcol);
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+            if (inside(v)) {
+                const cplx<double> x = sX[row(v) * ld + c];
+                t.re[v] += x.re;
+                t.im[v] += x.im;
+            }
+        __syncthreads();
+        store(sX, t);
+    };
+#pragma unroll
+    for (int v = 0; v < 4; ++v)
+        if (inside(v)) {
+            const cplx<TU> u = Uk[row(v) * nw + c];
+            sX[row(v) * ld + c] = mk((double)u.re, (double)u.im);
+            if constexpr (ALDS) sA[row(v) * ld + c] = herm(row(v), c);
+        }
+    for (int i = tid; i < nw; i += NTH) den[i] = 0.0;
+    double scale = 0.0;
     for (int it = 0; it < iters; ++it) {
+        double* red = red2 + 4 * (it & 1);
         if (tid < 4) red[tid] = 0.0;
         __syncthreads();
-        // T = A X
-        oa_gemm<OA_THREADS>(nw, [&](int r, int m) { return sA[r * ld + m]; }, [&](int m, int c) { return sX[m * ld + c]; },
-                    [&](int r, int c, cplx<double> v) { sT[r * ld + c] = v; });
+        store(sT, product(Arow, Xcol));
         __syncthreads();
-        // S = X^+ T ; then R = I - X^+ X into sT
-        oa_gemm<OA_THREADS>(nw, [&](int r, int m) { return conj(sX[m * ld + r]); },
-                    [&](int m, int c) { return sT[m * ld + c]; },
-                    [&](int r, int c, cplx<double> v) { sS[r * ld + c] = v; });
-        __syncthreads();
-        oa_gemm<OA_THREADS>(nw, [&](int r, int m) { return conj(sX[m * ld + r]); },
-                    [&](int m, int c) { return sX[m * ld + c]; },
-                    [&](int r, int c, cplx<double> v) { sT[r * ld + c] = mk((r == c ? 1.0 : 0.0) - v.re, -v.im); });
-        __syncthreads();
-        for (int i = tid; i < nw; i += OA_THREADS) lam[i] = sS[i * ld + i].re / (1.0 - sT[i * ld + i].re);
-        __syncthreads();
-        // Frobenius norms and max|lam|
+        Tile S, R;
+        products(Xadj, Tcol, Xcol, S, R);
+        // R = I - X^+ X, the eigenvalues, Frobenius norms and max|lam|
         double s2 = 0.0, r2 = 0.0, lm = 0.0;
-        for (int t = tid; t < nw * nw; t += OA_THREADS) {
-            const int i = t / nw, j = t % nw;
-            cplx<double> sv = sS[i * ld + j];
-            if (i == j) sv.re -= lam[i];
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            if (!inside(v)) continue;
+            const bool diag = row(v) == c;
+            R.re[v] = (diag ? 1.0 : 0.0) - R.re[v];
+            R.im[v] = -R.im[v];
+            cplx<double> sv = S.get(v);
+            if (diag) {
+                const double l = sv.re / (1.0 - R.re[v]);
+                lam[c] = l;
+                lm = fabs(l);
+                sv.re -= l;
+            }
             s2 += sv.re * sv.re + sv.im * sv.im;
-            const cplx<double> rv = sT[i * ld + j];
-            r2 += rv.re * rv.re + rv.im * rv.im;
+            r2 += R.re[v] * R.re[v] + R.im[v] * R.im[v];
         }
-        for (int i = tid; i < nw; i += OA_THREADS) lm = fmax(lm, fabs(lam[i]));
         for (int off = 32; off > 0; off >>= 1) {
             s2 += __shfl_down(s2, off);
             r2 += __shfl_down(r2, off);
@@ -880,95 +945,110 @@ __global__ void __launch_bounds__(OA_THREADS, 5) k_eigh_refine(int nw, const cpl
             atomicMax((unsigned long long*)&red[2], (unsigned long long)__double_as_longlong(lm));
         }
         __syncthreads();
-        const double delta = 2.0 * (sqrt(red[0]) + red[2] * sqrt(red[1]));
-        // E into sS, ||E||^2 into red[3]
+        scale = red[2];
+        const double delta = 2.0 * (sqrt(red[0]) + scale * sqrt(red[1]));
+        // E into sT (A X is no longer read), ||E||^2 into red[3]
         double e2 = 0.0;
-        for (int t = tid; t < nw * nw; t += OA_THREADS) {
-            const int i = t / nw, j = t % nw;
-            const double dl = lam[j] - lam[i];
-            const cplx<double> r = sT[i * ld + j];
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            if (!inside(v)) continue;
+            const double lc = lam[c], dl = lc - lam[row(v)];
             cplx<double> e;
-            if (fabs(dl) > delta) {
-                const cplx<double> sv = sS[i * ld + j];
-                e = (1.0 / dl) * mk(sv.re + lam[j] * r.re, sv.im + lam[j] * r.im);
-            } else {
-                e = 0.5 * r;
-            }
-            sS[i * ld + j] = e;
+            if (fabs(dl) > delta)
+                e = (1.0 / dl) * mk(S.re[v] + lc * R.re[v], S.im[v] + lc * R.im[v]);
+            else
+                e = mk(0.5 * R.re[v], 0.5 * R.im[v]);
+            sT[row(v) * ld + c] = e;
             e2 += e.re * e.re + e.im * e.im;
         }
         for (int off = 32; off > 0; off >>= 1) e2 += __shfl_down(e2, off);
         if ((tid & 63) == 0) atomicAdd(&red[3], e2);
         __syncthreads();
-        // every thread reads red[3] here; it is cleared only after the next barrier
+        // (this set is cleared two steps on, after barriers that follow every thread's reading)
         const bool converged = red[3] < tol * tol || (sizeof(TU) == 4 && red[3] < OA_LAST_C64 * OA_LAST_C64);
-        // X + X E into sT (R is no longer read), which becomes X
-        oa_gemm<OA_THREADS>(nw, [&](int r, int m) { return sX[r * ld + m]; }, [&](int m, int c) { return sS[m * ld + c]; },
-                    [&](int r, int c, cplx<double> v) { sT[r * ld + c] = sX[r * ld + c] + v; });
-        __syncthreads();
-        cplx<double>* t = sX;
-        sX = sT;
-        sT = t;
+        add_X_times_T();
         if (converged) break;
     }
+    __syncthreads();
     if (sizeof(TU) == 8) {
         // complex128 output: one Newton-Schulz step X <- X (I + R/2), R = I - X^+ X, so that the
         // basis is orthonormal to rounding also where a close pair leaves the vectors themselves
         // accurate only to ~eps |H| / gap (the correction steps do not preserve orthogonality)
-        oa_gemm<OA_THREADS>(nw, [&](int r, int m) { return conj(sX[m * ld + r]); },
-                    [&](int m, int c) { return sX[m * ld + c]; },
-                    [&](int r, int c, cplx<double> v) { sS[r * ld + c] = mk(0.5 * ((r == c ? 1.0 : 0.0) - v.re), -0.5 * v.im); });
-        __syncthreads();
-        oa_gemm<OA_THREADS>(nw, [&](int r, int m) { return sX[r * ld + m]; }, [&](int m, int c) { return sS[m * ld + c]; },
-                    [&](int r, int c, cplx<double> v) { sT[r * ld + c] = sX[r * ld + c] + v; });
-        __syncthreads();
-        cplx<double>* t = sX;
-        sX = sT;
-        sT = t;
-    }
-    // S = X^+ A X of the refined columns; pairs left mixed are rotated apart
-    const double scale = red[2];  // max |lam| of the last step
-    oa_gemm<OA_THREADS>(nw, [&](int r, int m) { return sA[r * ld + m]; }, [&](int m, int c) { return sX[m * ld + c]; },
-                [&](int r, int c, cplx<double> v) { sT[r * ld + c] = v; });
-    __syncthreads();
-    oa_gemm<OA_THREADS>(nw, [&](int r, int m) { return conj(sX[m * ld + r]); },
-                [&](int m, int c) { return sT[m * ld + c]; },
-                [&](int r, int c, cplx<double> v) { sS[r * ld + c] = v; });
-    __syncthreads();
-    cluster_jacobi<OA_THREADS>(
-        nw, [&](int i, int j) -> cplx<double>& { return sS[i * ld + j]; },
-        [&](int i, int j) -> cplx<double>& { return sX[i * ld + j]; }, cjs, tol, 64.0 * DBL_EPSILON * scale, 10);
-    // eigenvalues: Rayleigh quotients x_c^+ A x_c / x_c^+ x_c = S_cc / x_c^+ x_c
-    for (int c = tid; c < nw; c += OA_THREADS) {
-        double den = 0.0;
-        for (int m = 0; m < nw; ++m) {
-            const cplx<double> x = sX[m * ld + c];
-            den += x.re * x.re + x.im * x.im;
+        Tile t = product(Xadj, Xcol);
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            t.re[v] = 0.5 * ((row(v) == c ? 1.0 : 0.0) - t.re[v]);
+            t.im[v] = -0.5 * t.im[v];
         }
-        lam[c] = sS[c * ld + c].re / den;
+        store(sT, t);
+        __syncthreads();
+        add_X_times_T();
+        __syncthreads();
     }
+    // S = X^+ A X of the refined columns; pairs left mixed are rotated apart (scale: max |lam| of the last step)
+    store(sT, product(Arow, Xcol));
+    __syncthreads();
+    const Tile S = product(Xadj, Tcol);
+    double x2 = 0.0;
+#pragma unroll
+    for (int v = 0; v < 4; ++v)
+        if (inside(v)) {
+            const cplx<double> x = sX[row(v) * ld + c];
+            x2 += x.re * x.re + x.im * x.im;
+            if (row(v) == c) lam[c] = S.re[v];
+        }
+    x2 += __shfl_xor(x2, 16);
+    x2 += __shfl_xor(x2, 32);
+    if (lk == 0 && c < nw) atomicAdd(&den[c], x2);
+    __syncthreads();
+    const double theta = tol, floor_abs = 64.0 * DBL_EPSILON * scale;
+    int mixed = 0;
+#pragma unroll
+    for (int v = 0; v < 4; ++v)
+        if (inside(v) && row(v) != c) mixed |= cluster_pair(S.get(v), lam[row(v)], lam[c], theta, floor_abs);
+    if (__syncthreads_or(mixed)) {
+        store(sT, S);
+        __syncthreads();
+        cluster_jacobi<NTH>(
+            nw, [&](int i, int j) -> cplx<double>& { return sT[i * ld + j]; },
+            [&](int i, int j) -> cplx<double>& { return sX[i * ld + j]; }, cjs, theta, floor_abs, 10);
+        for (int i = tid; i < nw; i += NTH) {
+            double d = 0.0;
+            for (int m = 0; m < nw; ++m) {
+                const cplx<double> x = sX[m * ld + i];
+                d += x.re * x.re + x.im * x.im;
+            }
+            den[i] = d;
+            lam[i] = sT[i * ld + i].re;
+        }
+        __syncthreads();
+    }
+    // eigenvalues: Rayleigh quotients x_c^+ A x_c / x_c^+ x_c = S_cc / x_c^+ x_c
+    for (int i = tid; i < nw; i += NTH) lam[i] /= den[i];
     __syncthreads();
     // ascending order (ties by index)
-    for (int i = tid; i < nw; i += OA_THREADS) {
+    for (int i = tid; i < nw; i += NTH) {
+        const double l = lam[i];
         int rk = 0;
-        for (int j = 0; j < nw; ++j) rk += (lam[j] < lam[i]) || (lam[j] == lam[i] && j < i);
+        for (int j = 0; j < nw; ++j) rk += (lam[j] < l) || (lam[j] == l && j < i);
         rank[i] = rk;
+        Eout[k * nw + rk] = l;
     }
     __syncthreads();
-    for (int t = tid; t < nw * nw; t += OA_THREADS) {
-        const int r = t / nw, c = t % nw;
-        const cplx<double> x = sX[r * ld + c];
-        Uk[r * nw + rank[c]] = mk((TU)x.re, (TU)x.im);
-    }
-    for (int i = tid; i < nw; i += OA_THREADS) Eout[k * nw + rank[i]] = lam[i];
+#pragma unroll
+    for (int v = 0; v < 4; ++v)
+        if (inside(v)) {
+            const cplx<double> x = sX[row(v) * ld + c];
+            Uk[row(v) * nw + rank[c]] = mk((TU)x.re, (TU)x.im);
+        }
 }
 
 // ---------------------------------------------------------------------------
-// Refinement for 44 < nw <= 128: the same steps with the four nw x nw matrices
+// Refinement for 64 < nw <= 128: the same steps with the four nw x nw matrices
 // (X, T, S/E, R) in a per-k workspace of global memory and every product as
 // 32 x 32 wave tasks on the FP64 matrix cores (operands read through L2).
 // ---------------------------------------------------------------------------
-#define OAG_THREADS 512
+#define OAG_THREADS 1024  // one wave per 32 x 32 block; nw = 128, 150 k-points: 1.60 ms in 8 waves, 1.25 in 16
 #define OAG_NWMAX 128
 
 // C = P Q (n x n) as wave tasks; out(r, c, value) for r, c < n
@@ -1098,9 +1178,17 @@ __global__ void __launch_bounds__(OAG_THREADS) k_eigh_refine_g(int n, const cplx
     wg_gemm(n, [&](int r, int m) { return conj(X[m * n + r]); }, [&](int m, int c) { return T[m * n + c]; },
             [&](int r, int c, cplx<double> v) { S[r * n + c] = v; });
     __syncthreads();
-    cluster_jacobi<OAG_THREADS>(
-        n, [&](int i, int j) -> cplx<double>& { return S[i * n + j]; },
-        [&](int i, int j) -> cplx<double>& { return X[i * n + j]; }, cjs, tol, 64.0 * DBL_EPSILON * scale, 10);
+    for (int i = tid; i < n; i += OAG_THREADS) lam[i] = S[i * n + i].re;
+    __syncthreads();
+    int mixed = 0;
+    for (int t = tid; t < n2; t += OAG_THREADS) {
+        const int i = t / n, j = t % n;
+        if (i != j) mixed |= cluster_pair(S[t], lam[i], lam[j], tol, 64.0 * DBL_EPSILON * scale);
+    }
+    if (__syncthreads_or(mixed))
+        cluster_jacobi<OAG_THREADS>(
+            n, [&](int i, int j) -> cplx<double>& { return S[i * n + j]; },
+            [&](int i, int j) -> cplx<double>& { return X[i * n + j]; }, cjs, tol, 64.0 * DBL_EPSILON * scale, 10);
     // Rayleigh quotients x_c^+ A x_c / x_c^+ x_c = S_cc / x_c^+ x_c
     for (int c = tid; c < n; c += OAG_THREADS) {
         double den = 0.0;
@@ -1190,6 +1278,24 @@ static int jacobi_f32_of_f64(wbmi_ctx* ctx, int nk, int nw, const cplx<double>* 
     return WBMI_OK;
 }
 
+template <typename TU, int NB>
+static int launch_refine(wbmi_ctx* ctx, int nk, int nw, const cplx<double>* H64, int64_t Hstride, double* E,
+                         cplx<TU>* U, int steps, double tol) {
+    const size_t lds = (NB <= 3 ? 3 : 2) * sizeof(cplx<double>) * nw * (nw + 1) + sizeof(double) * (2 * nw + 8) +
+                       cj_lds(nw) + sizeof(int) * nw + 16;
+    auto launch = [&](auto split) -> int {
+        auto kernel = k_eigh_refine<TU, NB, decltype(split)::value>;
+        WBMI_HIP_CHECK(ctx, hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+        hipLaunchKernelGGL(kernel, dim3(nk), dim3(64 * NB * NB), lds, ctx->stream, nw, H64, Hstride, E, U, steps, tol);
+        WBMI_LAUNCH_CHECK(ctx);
+        return WBMI_OK;
+    };
+    if constexpr (sizeof(TU) == 4 && NB <= 3)
+        if (NB < 3 || nw <= 44) return launch(std::true_type{});
+    if constexpr (sizeof(TU) == 8 || NB >= 3) return launch(std::false_type{});
+    return WBMI_OK;
+}
+
 // FP32 Jacobi of the FP64 Hamiltonian, then FP64 Ogita-Aishima steps; eigenvectors stored as TU
 template <typename TU>
 static int eigh_refined(wbmi_ctx* ctx, int nk, int nw, const cplx<double>* H64, int64_t Hstride, double* E,
@@ -1197,23 +1303,19 @@ static int eigh_refined(wbmi_ctx* ctx, int nk, int nw, const cplx<double>* H64, 
     const double tol = sizeof(TU) == 4 ? OA_TOL_C64 : OA_TOL_C128;
     int rc = jacobi_f32_of_f64<TU>(ctx, nk, nw, H64, Hstride, E, U, U0);
     if (rc) return rc;
-    if (nw > 44) {
-        if (!work || work_bytes < eigh_work_bytes(nk, nw, steps))
-            return wbmi_fail(ctx, WBMI_ERR_ARG, "wbmi_eigh: refinement at nw = %d needs %zu bytes of workspace", nw,
-                             eigh_work_bytes(nk, nw, steps));
+    if (nw > 44 && (!work || work_bytes < eigh_work_bytes(nk, nw, steps)))
+        return wbmi_fail(ctx, WBMI_ERR_ARG, "wbmi_eigh: refinement at nw = %d needs %zu bytes of workspace", nw,
+                         eigh_work_bytes(nk, nw, steps));
+    if (nw > 64) {
         hipLaunchKernelGGL((k_eigh_refine_g<TU>), dim3(nk), dim3(OAG_THREADS), 0, ctx->stream, nw, H64, Hstride, E, U,
                            steps, tol, (cplx<double>*)work);
         WBMI_LAUNCH_CHECK(ctx);
         return WBMI_OK;
     }
-    const size_t lds2 =
-        4 * sizeof(cplx<double>) * nw * (nw + 1) + sizeof(double) * (nw + 4) + cj_lds(nw) + sizeof(int) * nw + 16;
-    WBMI_HIP_CHECK(ctx, hipFuncSetAttribute((const void*)k_eigh_refine<TU>,
-                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds2));
-    hipLaunchKernelGGL((k_eigh_refine<TU>), dim3(nk), dim3(OA_THREADS), lds2, ctx->stream, nw, H64, Hstride, E, U,
-                       steps, tol);
-    WBMI_LAUNCH_CHECK(ctx);
-    return WBMI_OK;
+    return nw <= 16   ? launch_refine<TU, 1>(ctx, nk, nw, H64, Hstride, E, U, steps, tol)
+           : nw <= 32 ? launch_refine<TU, 2>(ctx, nk, nw, H64, Hstride, E, U, steps, tol)
+           : nw <= 48 ? launch_refine<TU, 3>(ctx, nk, nw, H64, Hstride, E, U, steps, tol)
+                      : launch_refine<TU, 4>(ctx, nk, nw, H64, Hstride, E, U, steps, tol);
 }
 
 extern "C" int wbmi_eigh(wbmi_ctx* ctx, int nk, int nw, const void* H_dev, int64_t Hstride, double* E_dev,
