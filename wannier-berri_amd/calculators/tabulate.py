@@ -9,7 +9,7 @@ import numpy as np
 
 from .. import _lib
 from .. import factors
-from ..result import KBandResult, TABresult
+from ..result import HostCopy, KBandResult, TABresult
 from .static import (Calculator, StaticCalculator, _PARITY, _external, der3e_bands, spin_current_channels,
                      spin_current_params)
 
@@ -33,6 +33,13 @@ class Tabulator(Calculator):
     def needed_channels(self, system):
         return StaticCalculator.needed_channels(self, system)
 
+    def _bands_on_host(self, data_K, out, tail):
+        """The rows `ibands` of the device table `out` times the constant factor, [nk, nband] + tail."""
+        ib = np.arange(data_K.num_wann)
+        ib = ib if self.ibands is None else ib[self.ibands]
+        factor = self.constant_factor
+        return HostCopy(out, lambda a: a[:, ib] * factor, (data_K.nk, len(ib)) + tail)
+
     def __call__(self, data_K):
         torch = data_K.torch
         data_K.ensure(self.needed_channels(data_K.system))
@@ -47,8 +54,7 @@ class Tabulator(Calculator):
         ncomp = 3 ** self.ndim
         out = torch.empty((data_K.nk, data_K.num_wann, ncomp), dtype=torch.float64, device=data_K.ctx.device)
         data_K.tabulate(p, out)
-        ib = np.arange(data_K.num_wann) if self.ibands is None else self.ibands
-        data = out.cpu().numpy()[:, ib].reshape((data_K.nk, len(ib)) + (3,) * self.ndim) * self.constant_factor
+        data = self._bands_on_host(data_K, out, (3,) * self.ndim)
         tr, inv = _PARITY[self.formula]
         return KBandResult(data, transformTR=tr, transformInv=inv)
 
@@ -96,8 +102,7 @@ class Der3E(Tabulator):
     def __call__(self, data_K):
         data_K.ensure(self.needed_channels(data_K.system))
         out = der3e_bands(data_K, self.degen_thresh, self.degen_Kramers, 0)
-        ib = np.arange(data_K.num_wann) if self.ibands is None else self.ibands
-        data = out.cpu().numpy()[:, ib].reshape((data_K.nk, len(ib), 3, 3, 3)) * self.constant_factor
+        data = self._bands_on_host(data_K, out, (3, 3, 3))
         return KBandResult(data, transformTR=-1, transformInv=-1)
 
 
@@ -123,8 +128,7 @@ class _DiagTabulator(Tabulator):
         out = torch.empty((data_K.nk, data_K.num_wann, 3), dtype=torch.float64, device=data_K.ctx.device)
         data_K.ctx.tabulate_diag(data_K.E_dev, data_K.Xk, data_K.prec, [s0, s0 + 1, s0 + 2], self.degen_thresh,
                                  self.degen_Kramers, out)
-        ib = np.arange(data_K.num_wann) if self.ibands is None else self.ibands
-        data = out.cpu().numpy()[:, ib] * self.constant_factor
+        data = self._bands_on_host(data_K, out, (3,))
         return KBandResult(data, transformTR=self.parity[0], transformInv=self.parity[1])
 
 
@@ -154,8 +158,7 @@ class InvMass(Tabulator):
         out = torch.empty((data_K.nk, data_K.num_wann, 9), dtype=torch.float64, device=data_K.ctx.device)
         data_K.ctx.tabulate_invmass(data_K.E_dev, data_K.Xk, data_K.prec, [v0 + i for i in range(3)],
                                     [w0 + i for i in range(9)], self.degen_thresh, self.degen_Kramers, out)
-        ib = np.arange(data_K.num_wann) if self.ibands is None else self.ibands
-        data = out.cpu().numpy()[:, ib].reshape((data_K.nk, len(ib), 3, 3)) * self.constant_factor
+        data = self._bands_on_host(data_K, out, (3, 3))
         return KBandResult(data, transformTR=1, transformInv=1)
 
 
@@ -182,8 +185,7 @@ class SpinBerry(Tabulator):
         p = spin_current_params(data_K, self.spin_current_type, ext, self.degen_thresh, self.degen_Kramers)
         out = torch.empty((data_K.nk, data_K.num_wann, 27), dtype=torch.float64, device=data_K.ctx.device)
         data_K.ctx.tabulate_spin_berry(data_K.E_dev, data_K.Xk, data_K.prec, p, out)
-        ib = np.arange(data_K.num_wann) if self.ibands is None else self.ibands
-        data = out.cpu().numpy()[:, ib].reshape((data_K.nk, len(ib), 3, 3, 3)) * self.constant_factor
+        data = self._bands_on_host(data_K, out, (3, 3, 3))
         return KBandResult(data, transformTR=1, transformInv=1)
 
 

@@ -41,6 +41,10 @@ BASES = ["Ham", "AA", "BB", "CC", "SS", "SA", "SHA", "SH", "SR", "SHR"]
 # two or three steps for separated spectra, up to about ten for a pair
 # closer than ~1e-5 |H|, whose first-order correction is large)
 OA_STEPS = 16
+# K-blocks with fewer channel elements than this are not transformed ahead on the side stream: the
+# transform is shorter than the 45 us of host time that the events and stream changes cost, which a
+# small block waits for (a 2-band layer, 16 blocks of 156 k-points: 2.42 against 3.40 ms)
+PREFETCH_MIN = 1 << 21
 _ALPHA = [1, 2, 0]
 _BETA = [2, 0, 1]
 
@@ -190,22 +194,23 @@ class DeviceSystem:
         ent = self._zcache.get(key)
         if ent is not None:
             self._zcache.move_to_end(key)
-            w1, ev = ent
-            cur.wait_event(ev)
-            w1.record_stream(cur)
+            w1, ev, writer = ent
+            if cur != writer:   # on the writing stream (recorded then) the order is the stream's own
+                cur.wait_event(ev)
+                w1.record_stream(cur)
             return w1
         nb = plan.w1_bytes(prec)
         if nb > self.zcache_limit:
             return None
         while self._zcache_used + nb > self.zcache_limit:
-            _, (old, _) = self._zcache.popitem(last=False)
+            _, (old, _, _) = self._zcache.popitem(last=False)
             self._zcache_used -= old.numel()
         w1 = torch.empty(nb, dtype=torch.uint8, device=self.ctx.device)
         w1.record_stream(cur)
         plan.zpass(box, dK, work, w1, prec)
         ev = torch.cuda.Event()
         ev.record(cur)
-        self._zcache[key] = (w1, ev)
+        self._zcache[key] = (w1, ev, cur)
         self._zcache_used += nb
         return w1
 
@@ -325,7 +330,12 @@ class Data_K:
                 keep.extend([work, box])
             del work
         else:
-            kl = self.k_list_dev if self.k_list_dev is not None else torch.from_numpy(self.k_list).to(self.ctx.device)
+            kl = self.k_list_dev
+            if kl is None:
+                # behind queued work through pinned memory: a pageable copy would wait for it
+                kl = torch.from_numpy(self.k_list)
+                idle = self.ctx.stream.query()
+                kl = kl.to(self.ctx.device) if idle else kl.pin_memory().to(self.ctx.device, non_blocking=True)
             self.ctx.r2k_klist(self.dev.iRvec_dev, stack, kl, X, prec, pairs=self.dev.pairs_dev)
         return X
 
@@ -354,6 +364,8 @@ class Data_K:
         if self.k_list is not None or self._slots is not None or self._pref is not None:
             return
         keys = self._channel_keys()
+        if self.nk * self.num_wann ** 2 * sum(CHANNEL_NCOMP[k] for k in keys) < PREFETCH_MIN:
+            return
         main = self.ctx.stream
         stream.wait_stream(main)
         keep = []
