@@ -85,6 +85,18 @@ def channel_terms(name, der, base_offset):
 def r_pairs(iRvec):
     """The R-vectors as pairs, int32 [npair, 2]: (i, j) with R_j = -R_i, (i, -1) for one without a
     partner (R = 0, a missing -R, repeated vectors beyond the first match)."""
+    R = np.asarray(iRvec).reshape(-1, 3).astype(np.int64)
+    span = 2 * np.abs(R).max(axis=0, initial=0) + 1
+    if len(R) and np.prod(span.astype(float)) < 2.0 ** 62:
+        weight = np.array([span[1] * span[2], span[2], 1])
+        key = R @ weight   # one number per vector, -R's is its negative
+        order = np.argsort(key, kind="stable")
+        ks = key[order]
+        if np.all(np.diff(ks) > 0):   # no repeated vector
+            at = np.minimum(np.searchsorted(ks, -key), len(ks) - 1)
+            i, j = np.arange(len(R)), np.where(ks[at] == -key, order[at], -1)
+            keep = (j < 0) | (j >= i)
+            return np.stack([i, np.where(j == i, -1, j)], axis=1)[keep].astype(np.int32)
     partner = {}
     for j, R in enumerate(iRvec.tolist()):
         partner.setdefault(tuple(R), []).append(j)
