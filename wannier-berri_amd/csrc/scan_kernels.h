@@ -49,6 +49,8 @@
 #define SC_THREADS 512  // workgroup size of the scan kernels (DerOmega / DerMorb: task_threads)
 #define SC_NWMAX 128
 #define SC_LDS (160 * 1024)
+#define SC_XCD_LOG 3
+#define SC_XCD (1 << SC_XCD_LOG)
 #define SC_M_NW 64    // dEinv o Off lives in LDS up to this nw (DerOmega / DerMorb: wherever it fits)
 #define SC_LDS_NW 32  // V and A live in LDS up to this nw
 // DerMorb with internal terms only: kernels of their own, for V and W Hermitian to the rounding of FP64
@@ -63,6 +65,7 @@ static __constant__ int c_beta[3] = {2, 0, 1};
 struct ScanArgs {
     wbmi_scan_params p;
     int nw, nch, stage_va;
+    int nk, parts;  // workgroups per k-point, set at the launch
     double weight;
     // tetrahedron method: `tetra` = number of corners, 8 (parallelepiped: corner ix*4 + iy*2 + iz
     // at k + (2i-1) dK/2, 12 tetrahedra around the centre) or 4 (tetrahedral K-block: the vertices,
@@ -204,6 +207,7 @@ struct KCtx {
     const cplx<TS>* sA;
     const double* bv;    // WBMI_FORMULA_BANDVALUES: this k's caller values [nw][nbv]
     int nbv;
+    int part, parts;  // this workgroup's share of the k-point's tasks
     __device__ inline cplx<double> get(int role, int x, int y) const {
         cplx<T> v = X[((int64_t)ch[role] * n_() + x) * n_() + y];
         return mk((double)v.re, (double)v.im);
@@ -656,14 +660,14 @@ __device__ __attribute__((always_inline)) void formula_task(const Smem& S, const
 // matrices times -i: it has no real part and is left out (complex64 channels: keep_t4).
 // DM is compile-time so that the DerOmega kernel carries only the kinds it runs (0 and 2): its
 // register allocation and code size are not those of the DerMorb kinds.
-// The workgroups blockIdx.y = 0, 1, .. of one k share its tasks: each adds up its own (the first also
+// The workgroups part = 0, 1, .. of one k share its tasks: each adds up its own (the first also
 // the per-band terms), and the sums over groups are linear in them.
 template <bool DM, typename T, bool LM, bool ST, bool SA, int NW, typename TS>
 __device__ __attribute__((always_inline)) void eval_deromega(const Smem& S, const KCtx<T, LM, ST, SA, NW, TS>& K, bool in, bool ex,
                                                             int sign, int cut) {
     constexpr bool dm = DM;
     const int nw = K.n_(), tid = threadIdx.x;
-    const bool lead = blockIdx.y == 0;
+    const bool lead = K.part == 0;
     const int l0 = cut >= 0 ? cut : 0;  // D' != 0 from here on
     // per-band terms, lanes running over (n, c, d)
     for (int t = tid; t < nw * 9; t += (int)blockDim.x) {
@@ -734,7 +738,7 @@ __device__ __attribute__((always_inline)) void eval_deromega(const Smem& S, cons
     for (;;) {
         int t = 0;
         if (lane == 0) t = atomicAdd(&S.misc[3], 1);
-        t = __builtin_amdgcn_readfirstlane(t) * (int)gridDim.y + (int)blockIdx.y;
+        t = __builtin_amdgcn_readfirstlane(t) * K.parts + K.part;
         if (t >= ntask) break;
         int kind = -1, rem = 0, base = 0;
 #pragma unroll
@@ -873,7 +877,7 @@ __device__ __attribute__((always_inline)) void eval_dermorb_in(const Smem& S, co
     for (;;) {
         int t = 0;
         if (lane == 0) t = atomicAdd(&S.misc[3], 1);
-        t = __builtin_amdgcn_readfirstlane(t) * (int)gridDim.y + (int)blockIdx.y;
+        t = __builtin_amdgcn_readfirstlane(t) * K.parts + K.part;
         if (t >= ntask) break;
         const int b = t % 3;
         int nb, lb;
@@ -1431,7 +1435,12 @@ k_static_scan(ScanArgs args, const double* __restrict__ Eall, const cplx<T>* __r
     extern __shared__ __attribute__((aligned(16))) char smem_raw[];
     const wbmi_scan_params& p = args.p;
     const int nw = NW > 0 ? NW : args.nw, ld = nw + 1;
-    const int64_t k = blockIdx.x;
+    // the workgroups of one k-point (args.parts) follow each other on one XCD (workgroups go round the
+    // XCDs in turn), so that its channels come from that XCD's L2: 294 k-points at nw = 64, complex64, DerOmega
+    // 364 -> 339 us, DerMorb 446 -> 431; at nw = 128 no difference (2.88 -> 2.85 ms)
+    const int parts = args.parts, unit = (int)blockIdx.x >> SC_XCD_LOG;
+    const int64_t k = parts > 1 ? (int64_t)(unit / parts) * SC_XCD + (blockIdx.x & (SC_XCD - 1)) : blockIdx.x;
+    if (parts > 1 && k >= args.nk) return;
     const int tid = threadIdx.x;
     if (MODE != 2) hist += k * args.hist_stride;
     constexpr bool tasks = F == WBMI_FORMULA_DEROMEGA || F == WBMI_FORMULA_DERMORB;
@@ -1623,6 +1632,8 @@ k_static_scan(ScanArgs args, const double* __restrict__ Eall, const cplx<T>* __r
     K.sA = (const cplx<TS>*)S.A;
     K.bv = (const double*)(const void*)Xall + k * (int64_t)nw * args.nch;
     K.nbv = args.nch;
+    K.parts = parts;
+    K.part = parts > 1 ? unit % parts : 0;
 
     if (additive || tab) {
         // main partition: every group at once (each group's trace with inn = the group,
@@ -1773,7 +1784,11 @@ static int launch_scan_t(wbmi_ctx* ctx, int nk, const ScanArgs& a, const double*
     const int parts = (tasks || SC_IS_DERMORB_IN(F)) && MODE == 0 && nk < want ? std::min(8, want / nk) : 1;
     WBMI_HIP_CHECK(ctx, hipFuncSetAttribute((const void*)k_static_scan<T, F, LM, ST, MODE, NW, NTH>,
                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    hipLaunchKernelGGL((k_static_scan<T, F, LM, ST, MODE, NW, NTH>), dim3(nk, parts), dim3(NTH), lds, ctx->stream, a, E,
+    ScanArgs args = a;
+    args.nk = nk;
+    args.parts = parts;
+    const int grid = parts > 1 ? (nk + SC_XCD - 1) / SC_XCD * SC_XCD * parts : nk;
+    hipLaunchKernelGGL((k_static_scan<T, F, LM, ST, MODE, NW, NTH>), dim3(grid), dim3(NTH), lds, ctx->stream, args, E,
                        (const cplx<T>*)X, hist);
     WBMI_LAUNCH_CHECK(ctx);
     return WBMI_OK;
