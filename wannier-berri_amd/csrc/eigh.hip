@@ -260,14 +260,18 @@ __device__ inline void rotate_rows(cplx<float>& xp, cplx<float>& xq, float c, fl
 // still sees the column rotation first, so the bits are those of the two phases.
 // Bound: VALU issue (about 390 instructions a round and wave at N = 32, 64 LDS operations) and,
 // for few k-points, the latency of a round.
-// One wave per k for N <= 32, four above (LDS holds four such workgroups a CU at N = 48).
+// One wave per k for N <= 32, four above (LDS holds four such workgroups a CU at N = 48); few k-points: below.
 // The parameters of N = 16, 32 and 64 use the hardware reciprocals.
 // Measured against k_eigh_jacobi (sizes at run time, two phases): 9.1 -> 2.6 ms for 3898 k-points
 // at nw = 48, 1.05 -> 0.62 ms for 6112 at nw = 24, 165 -> 67 us for 1728 at nw = 12.
 // ---------------------------------------------------------------------------
+// Waves per k: with fewer k-points than fill the GPU, four (N > 16) and sixteen (N > 32): a round's items
+// over more SIMDs, the same operations per element.  Diagonalisation and refinement of 50 k-points: nw = 18
+// 136 -> 121 us, 32 292 -> 201, 48 574 -> 451, 64 885 -> 697; where the waves no longer fit side by side
+// it costs (nw = 32, 1024 k-points 429 -> 453; nw = 48, 640 915 -> 1008).
 template <int N>
-__host__ __device__ constexpr int jacobi_b_threads() {
-    return N <= 32 ? 64 : 256;
+__host__ __device__ constexpr int jacobi_b_waves(bool few) {
+    return N <= 16 ? 1 : N <= 32 ? (few ? 4 : 1) : (few ? 16 : 4);
 }
 template <int N>
 __host__ __device__ constexpr size_t jacobi_b_lds() {
@@ -280,13 +284,12 @@ __host__ __device__ constexpr size_t jacobi_b_lds() {
 // the rotations accumulated onto V = U0: a nearly diagonal start needs about
 // three active sweeps instead of six or seven.  Any unitary U0 gives the same
 // eigen-decomposition; a poor one only costs sweeps.
-template <int N, typename Tin, typename TO>
-__global__ void __launch_bounds__(jacobi_b_threads<N>()) k_eigh_jacobi_b(int nw, const cplx<Tin>* __restrict__ H,
-                                                                        int64_t Hstride, double* __restrict__ Eout,
-                                                                        cplx<TO>* Uout, int max_sweeps,
-                                                                        const cplx<TO>* U0) {
+template <int N, int NWAVE, typename Tin, typename TO>
+__global__ void __launch_bounds__(64 * NWAVE) k_eigh_jacobi_b(int nw, const cplx<Tin>* __restrict__ H, int64_t Hstride,
+                                                             double* __restrict__ Eout, cplx<TO>* Uout, int max_sweeps,
+                                                             const cplx<TO>* U0) {
     typedef float T;
-    constexpr int NTH = jacobi_b_threads<N>();
+    constexpr int NTH = 64 * NWAVE;
     constexpr int n = N, ld = N + 1, np = N / 2;
     constexpr int NB = np * np, NV = np * N;                          // A blocks and V items of a round
     constexpr int IB = (NB + NTH - 1) / NTH, IV = (NV + NTH - 1) / NTH;  // per thread
@@ -318,7 +321,7 @@ __global__ void __launch_bounds__(jacobi_b_threads<N>()) k_eigh_jacobi_b(int nw,
     } else if constexpr (N == 16 || N == 32) {
         // V = U0 (identity on the padding index of odd nw)
         const cplx<TO>* U0k = U0 + k * nw * nw;
-        for (int t = tid; t < n * n; t += 64) {
+        for (int t = tid; t < n * n; t += NTH) {
             const int i = t / n, j = t % n;
             cplx<T> v = mk((T)(i == j ? 1 : 0), (T)0);
             if (i < nw && j < nw) {
@@ -328,41 +331,40 @@ __global__ void __launch_bounds__(jacobi_b_threads<N>()) k_eigh_jacobi_b(int nw,
             V[i * ld + j] = v;
         }
         __syncthreads();
-        // T = H U0 into A, then A = U0^+ T (one 32 x 32 block per product)
+        // T = H U0 into A, then A = U0^+ T (one 32 x 32 block per product, the first wave's)
         MfmaBlock C;
-        C.zero();
-        mfma_block(
-            C, n, n, n, 0, 0,
-            [&](int r, int m) {
-                if (r >= nw || m >= nw) return mk(0.0, 0.0);
-                const cplx<Tin> x = Hk[r * nw + m], y = Hk[m * nw + r];
-                return mk(0.5 * ((double)x.re + (double)y.re), 0.5 * ((double)x.im - (double)y.im));
-            },
-            [&](int m, int c) { return mk((double)V[m * ld + c].re, (double)V[m * ld + c].im); });
+        auto store = [&] {
 #pragma unroll
-        for (int bi = 0; bi < 2; ++bi)
+            for (int bi = 0; bi < 2; ++bi)
 #pragma unroll
-            for (int bj = 0; bj < 2; ++bj)
+                for (int bj = 0; bj < 2; ++bj)
 #pragma unroll
-                for (int v = 0; v < 4; ++v) {
-                    const int r = mfma_row(bi, v), c = mfma_col(bj);
-                    if (r < n && c < n) A[r * ld + c] = mk((T)C.re[bi][bj][v], (T)C.im[bi][bj][v]);
-                }
+                    for (int v = 0; v < 4; ++v) {
+                        const int r = mfma_row(bi, v), c = mfma_col(bj);
+                        if (r < n && c < n) A[r * ld + c] = mk((T)C.re[bi][bj][v], (T)C.im[bi][bj][v]);
+                    }
+        };
+        if (tid < 64) {
+            C.zero();
+            mfma_block(
+                C, n, n, n, 0, 0,
+                [&](int r, int m) {
+                    if (r >= nw || m >= nw) return mk(0.0, 0.0);
+                    const cplx<Tin> x = Hk[r * nw + m], y = Hk[m * nw + r];
+                    return mk(0.5 * ((double)x.re + (double)y.re), 0.5 * ((double)x.im - (double)y.im));
+                },
+                [&](int m, int c) { return mk((double)V[m * ld + c].re, (double)V[m * ld + c].im); });
+            store();
+        }
         __syncthreads();
-        C.zero();
-        mfma_block(
-            C, n, n, n, 0, 0, [&](int r, int m) { return mk((double)V[m * ld + r].re, -(double)V[m * ld + r].im); },
-            [&](int m, int c) { return mk((double)A[m * ld + c].re, (double)A[m * ld + c].im); });
-        __syncthreads();  // every read of T is done
-#pragma unroll
-        for (int bi = 0; bi < 2; ++bi)
-#pragma unroll
-            for (int bj = 0; bj < 2; ++bj)
-#pragma unroll
-                for (int v = 0; v < 4; ++v) {
-                    const int r = mfma_row(bi, v), c = mfma_col(bj);
-                    if (r < n && c < n) A[r * ld + c] = mk((T)C.re[bi][bj][v], (T)C.im[bi][bj][v]);
-                }
+        if (tid < 64) {
+            C.zero();
+            mfma_block(
+                C, n, n, n, 0, 0, [&](int r, int m) { return mk((double)V[m * ld + r].re, -(double)V[m * ld + r].im); },
+                [&](int m, int c) { return mk((double)A[m * ld + c].re, (double)A[m * ld + c].im); });
+            __builtin_amdgcn_wave_barrier();  // every read of T is done (one wave, in order)
+            store();
+        }
         __syncthreads();
     }
 
@@ -1239,18 +1241,23 @@ extern "C" size_t wbmi_eigh_work_bytes(int nk, int nw, int prec, int refine) {
 }
 
 #define JACOBI_SWEEPS 40
+#define JACOBI_FEW_1 768  // k-points up to which four waves (N <= 32), sixteen (N > 32) share one
+#define JACOBI_FEW_4 512
 
 template <int N, typename TU>
 static int launch_jacobi_b(wbmi_ctx* ctx, int nk, int nw, const cplx<double>* H64, int64_t Hstride, double* E,
                            cplx<TU>* U, const cplx<TU>* U0) {
     const size_t lds = jacobi_b_lds<N>();
-    if (lds > 64 * 1024)
-        WBMI_HIP_CHECK(ctx, hipFuncSetAttribute((const void*)k_eigh_jacobi_b<N, double, TU>,
-                                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    hipLaunchKernelGGL((k_eigh_jacobi_b<N, double, TU>), dim3(nk), dim3(jacobi_b_threads<N>()), lds, ctx->stream, nw,
-                       H64, Hstride, E, U, JACOBI_SWEEPS, U0);
-    WBMI_LAUNCH_CHECK(ctx);
-    return WBMI_OK;
+    auto launch = [&](auto few) -> int {
+        constexpr int NWAVE = jacobi_b_waves<N>(decltype(few)::value);
+        auto kernel = k_eigh_jacobi_b<N, NWAVE, double, TU>;
+        if (lds > 64 * 1024)
+            WBMI_HIP_CHECK(ctx, hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+        hipLaunchKernelGGL(kernel, dim3(nk), dim3(64 * NWAVE), lds, ctx->stream, nw, H64, Hstride, E, U, JACOBI_SWEEPS, U0);
+        WBMI_LAUNCH_CHECK(ctx);
+        return WBMI_OK;
+    };
+    return N > 16 && nk <= (N <= 32 ? JACOBI_FEW_1 : JACOBI_FEW_4) ? launch(std::true_type{}) : launch(std::false_type{});
 }
 
 // the launcher of padded size n = 2 HALF, searched from HALF down
