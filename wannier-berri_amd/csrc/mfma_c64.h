@@ -57,13 +57,19 @@ __device__ __attribute__((always_inline)) void mfma_block(MfmaBlock& C, int nr, 
             a[q] = (kok && rok[q]) ? X(r0 + 16 * q + li, k) : mk(0.0, 0.0);
             b[q] = (kok && cok[q]) ? Y(k, c0 + 16 * q + li) : mk(0.0, 0.0);
         }
+        // an accumulator's two products apart, so that neither waits for the other
 #pragma unroll
         for (int bi = 0; bi < 2; ++bi)
 #pragma unroll
             for (int bj = 0; bj < 2; ++bj) {
                 C.re[bi][bj] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[bi].re, b[bj].re, C.re[bi][bj], 0, 0, 0);
-                C.re[bi][bj] = __builtin_amdgcn_mfma_f64_16x16x4f64(-a[bi].im, b[bj].im, C.re[bi][bj], 0, 0, 0);
                 C.im[bi][bj] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[bi].re, b[bj].im, C.im[bi][bj], 0, 0, 0);
+            }
+#pragma unroll
+        for (int bi = 0; bi < 2; ++bi)
+#pragma unroll
+            for (int bj = 0; bj < 2; ++bj) {
+                C.re[bi][bj] = __builtin_amdgcn_mfma_f64_16x16x4f64(-a[bi].im, b[bj].im, C.re[bi][bj], 0, 0, 0);
                 C.im[bi][bj] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[bi].im, b[bj].re, C.im[bi][bj], 0, 0, 0);
             }
     }

@@ -46,6 +46,16 @@ __device__ inline cplx<double> rot_x(const cplx<T>* X, int nw, int r, int c) {
     return x;
 }
 
+// the two halves of rot_cmac: between them, other accumulators' products keep the matrix core busy
+__device__ inline void rot_cmac_re(wbmi_v4d& re, wbmi_v4d& im, cplx<double> a, cplx<double> b) {
+    re = __builtin_amdgcn_mfma_f64_16x16x4f64(a.re, b.re, re, 0, 0, 0);
+    im = __builtin_amdgcn_mfma_f64_16x16x4f64(a.re, b.im, im, 0, 0, 0);
+}
+__device__ inline void rot_cmac_im(wbmi_v4d& re, wbmi_v4d& im, cplx<double> a, cplx<double> b) {
+    re = __builtin_amdgcn_mfma_f64_16x16x4f64(-a.im, b.im, re, 0, 0, 0);
+    im = __builtin_amdgcn_mfma_f64_16x16x4f64(a.im, b.re, im, 0, 0, 0);
+}
+
 __device__ inline void rot_cmac(wbmi_v4d& re, wbmi_v4d& im, cplx<double> a, cplx<double> b) {
     re = __builtin_amdgcn_mfma_f64_16x16x4f64(a.re, b.re, re, 0, 0, 0);
     re = __builtin_amdgcn_mfma_f64_16x16x4f64(-a.im, b.im, re, 0, 0, 0);
@@ -175,9 +185,12 @@ __global__ void __launch_bounds__(64 * NB, NB <= 4 ? 3 : 2) k_rotate_s(int nw, i
                 for (int b = 0; b < NB; ++b) x[j][b] = rot_x<decltype(hermitian)::value>(Xc, nw, 16 * b + li, m);
             }
 #pragma unroll
-            for (int j = 0; j < J; ++j)
+            for (int j = 0; j < J; ++j) {
 #pragma unroll
-                for (int b = 0; b < NB; ++b) rot_cmac(tr[b], ti[b], x[j][b], u[j]);
+                for (int b = 0; b < NB; ++b) rot_cmac_re(tr[b], ti[b], x[j][b], u[j]);
+#pragma unroll
+                for (int b = 0; b < NB; ++b) rot_cmac_im(tr[b], ti[b], x[j][b], u[j]);
+            }
         }
     };
     if (herm)
@@ -185,19 +198,33 @@ __global__ void __launch_bounds__(64 * NB, NB <= 4 ? 3 : 2) k_rotate_s(int nw, i
     else
         first(std::false_type{});
     __syncthreads();
-    for (int bo = 0; bo < NB; ++bo) {
-        wbmi_v4d re = {0.0, 0.0, 0.0, 0.0}, im = re;
+    // two row blocks at a time (four accumulators in turn)
+    auto second = [&](int bo, auto two) {
+        constexpr int NO = decltype(two)::value ? 2 : 1;
+        wbmi_v4d re[NO], im[NO];
+#pragma unroll
+        for (int q = 0; q < NO; ++q) re[q] = im[q] = wbmi_v4d{0.0, 0.0, 0.0, 0.0};
 #pragma unroll
         for (int s = 0; s < NS; ++s) {
-            const cplx<double> u = rot_elem(Uk, nw, 4 * s + g, 16 * bo + li);
-            rot_cmac(re, im, conj(u), mk(tr[s / 4][s % 4], ti[s / 4][s % 4]));
+            cplx<double> u[NO];
+            const cplx<double> t = mk(tr[s / 4][s % 4], ti[s / 4][s % 4]);
+#pragma unroll
+            for (int q = 0; q < NO; ++q) u[q] = conj(rot_elem(Uk, nw, 4 * s + g, 16 * (bo + q) + li));
+#pragma unroll
+            for (int q = 0; q < NO; ++q) rot_cmac_re(re[q], im[q], u[q], t);
+#pragma unroll
+            for (int q = 0; q < NO; ++q) rot_cmac_im(re[q], im[q], u[q], t);
         }
 #pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            const int r = 16 * bo + g + 4 * v;
-            if (r < nw && col < nw) Xc[r * nw + col] = mk((T)re[v], (T)im[v]);
-        }
-    }
+        for (int q = 0; q < NO; ++q)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const int r = 16 * (bo + q) + g + 4 * v;
+                if (r < nw && col < nw) Xc[r * nw + col] = mk((T)re[q][v], (T)im[q][v]);
+            }
+    };
+    for (int bo = 0; bo + 1 < NB; bo += 2) second(bo, std::true_type{});
+    if constexpr (NB & 1) second(NB - 1, std::false_type{});
 }
 
 // Split-half rotation (complex64 storage, nw <= 32): Xbar = U^+ X U with both products
