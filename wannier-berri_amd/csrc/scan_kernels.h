@@ -57,7 +57,9 @@
 // sums, and for complex64 channels at nw <= 32, which the rotation forms in FP32 arithmetic
 #define SC_DERMORB_IN (WBMI_FORMULA_OMEGAHPLUS + 1000)
 #define SC_DERMORB_IN32 (SC_DERMORB_IN + 1)
+#define SC_DERMORB_EX (SC_DERMORB_IN + 2)  // with external terms, sign = +1, complex128
 #define SC_IS_DERMORB_IN(F) ((F) == SC_DERMORB_IN || (F) == SC_DERMORB_IN32)
+#define SC_IS_DERMORB_CUTS(F) (SC_IS_DERMORB_IN(F) || (F) == SC_DERMORB_EX)
 
 static __constant__ int c_alpha[3] = {1, 2, 0};  // utility.py:45-46
 static __constant__ int c_beta[3] = {2, 0, 1};
@@ -211,6 +213,20 @@ struct KCtx {
     __device__ inline cplx<double> get(int role, int x, int y) const {
         cplx<T> v = X[((int64_t)ch[role] * n_() + x) * n_() + y];
         return mk((double)v.re, (double)v.im);
+    }
+    // the same for a role that is the same in every lane: one scalar base, one 32-bit offset for all roles
+    __device__ inline cplx<double> getu(int role, int x, int y) const {
+        const cplx<T>* p = X + (int64_t)__builtin_amdgcn_readfirstlane(ch[role]) * n_() * n_();
+        const cplx<T> v = p[(unsigned)(x * n_() + y)];
+        return mk((double)v.re, (double)v.im);
+    }
+    __device__ inline cplx<double> Vu(int a, int x, int y) const {
+        if constexpr (ST) return V(a, x, y);
+        else return getu(WBMI_ROLE_V + a, x, y);
+    }
+    __device__ inline cplx<double> Au(int a, int x, int y) const {
+        if constexpr (SA) return A(a, x, y);
+        else return getu(WBMI_ROLE_A + a, x, y);
     }
     __device__ inline cplx<double> V(int a, int x, int y) const {
         if constexpr (ST) {
@@ -840,6 +856,28 @@ __device__ inline void cut_tile_pair(int t, int nblk, int& rb, int& cb) {
     cb = t + d;
 }
 
+// the sums of row v are formed here, not put off to their use with every operand kept in registers
+__device__ __attribute__((always_inline)) inline void cut_pin(double (&o)[7][4], int v) {
+#pragma unroll
+    for (int q = 0; q < 7; ++q) asm volatile("" : "+v"(o[q][v]));
+}
+
+// three complex 16 x 16 blocks in the accumulators
+struct CutAcc {
+    wbmi_v4d re[3], im[3];
+    __device__ inline void zero() {
+#pragma unroll
+        for (int r = 0; r < 3; ++r) re[r] = im[r] = wbmi_v4d{0.0, 0.0, 0.0, 0.0};
+    }
+    __device__ inline void add(int r, cplx<double> x, cplx<double> y) {
+        re[r] = __builtin_amdgcn_mfma_f64_16x16x4f64(x.re, y.re, re[r], 0, 0, 0);
+        im[r] = __builtin_amdgcn_mfma_f64_16x16x4f64(x.re, y.im, im[r], 0, 0, 0);
+        re[r] = __builtin_amdgcn_mfma_f64_16x16x4f64(-x.im, y.im, re[r], 0, 0, 0);
+        im[r] = __builtin_amdgcn_mfma_f64_16x16x4f64(x.im, y.re, im[r], 0, 0, 0);
+    }
+    __device__ inline cplx<double> get(int r, int v) const { return mk(re[r][v], im[r][v]); }
+};
+
 // DerMorb with internal terms only (formula/covariant.py:463-552), every needed cut into S.cut.  With
 // P = D' without its mask (anti-Hermitian), Q^a_nl = i (1 / (E_l - E_n)) (2 sign E_n + 2 E_l) P^a_nl and
 // n < c <= l, the per-cut terms (formula_task: kinds 0, s1 and 5) are, summed over n and l,
@@ -851,7 +889,7 @@ __device__ inline void cut_tile_pair(int t, int nblk, int& rb, int& cb) {
 // in both.  U the same with q and n.  So a task, one pair of 16-band blocks and one b, is the products
 //     [P; Q] (n, m) V^b (m, l) over m >= l,   V^b (n, q) [P, Q] (q, l) over q <= n
 // for three d and three a at once: a V and three P elements per 24 MFMAs, which leaves the matrix cores
-// as the bound.  294 k-points at nw = 64, every cut (complex64): 7.5 ms one by one, 0.45 ms together.
+// as the bound.  294 k-points at nw = 64, every cut (complex64): 7.5 ms one by one, 0.25 ms together.
 // HERM: V and W are Hermitian to the rounding of the sums.  Otherwise (complex64 from the rotation in FP32
 // arithmetic, whose two triangles differ by their rounding) every term reads the triangle that
 // formula_task reads, 36 MFMAs: P V with both triangles of V, V P with both of P.
@@ -860,20 +898,6 @@ __device__ __attribute__((always_inline)) void eval_dermorb_in(const Smem& S, co
     constexpr int NS = HERM ? 1 : 2;
     const int nw = K.n_(), lane = threadIdx.x & 63, lk = lane >> 4, li = lane & 15;
     const int nblk = (nw + 15) / 16, ntask = 3 * (nblk * (nblk + 1) / 2);
-    struct Acc {
-        wbmi_v4d re[3], im[3];
-        __device__ inline void zero() {
-#pragma unroll
-            for (int r = 0; r < 3; ++r) re[r] = im[r] = wbmi_v4d{0.0, 0.0, 0.0, 0.0};
-        }
-        __device__ inline void add(int r, cplx<double> x, cplx<double> y) {
-            re[r] = __builtin_amdgcn_mfma_f64_16x16x4f64(x.re, y.re, re[r], 0, 0, 0);
-            im[r] = __builtin_amdgcn_mfma_f64_16x16x4f64(x.re, y.im, im[r], 0, 0, 0);
-            re[r] = __builtin_amdgcn_mfma_f64_16x16x4f64(-x.im, y.im, re[r], 0, 0, 0);
-            im[r] = __builtin_amdgcn_mfma_f64_16x16x4f64(x.im, y.re, im[r], 0, 0, 0);
-        }
-        __device__ inline cplx<double> get(int r, int v) const { return mk(re[r][v], im[r][v]); }
-    };
     for (;;) {
         int t = 0;
         if (lane == 0) t = atomicAdd(&S.misc[3], 1);
@@ -892,7 +916,7 @@ __device__ __attribute__((always_inline)) void eval_dermorb_in(const Smem& S, co
         for (int q = 0; q < 7; ++q)
 #pragma unroll
             for (int v = 0; v < 4; ++v) o[q][v] = 0.0;
-        Acc G[NS], Z;  // P V or V P of both kinds of V or P; Q V or V Q
+        CutAcc G[NS], Z;  // P V or V P of both kinds of V or P; Q V or V Q
         // FIRST: the sums over m >= l, with f = W / 2 - (P V) = conj(F), h = -(P V) = conj(H); else those
         // over q <= n, with f = (V P), h = -sign (V P)
         auto add_pairs = [&](auto first) {
@@ -901,7 +925,7 @@ __device__ __attribute__((always_inline)) void eval_dermorb_in(const Smem& S, co
             for (int v = 0; v < 4; ++v) {
                 // an opaque row: the operands are loaded anew for each v and call, not kept in registers
                 int nn = 16 * nb + lk + 4 * v;
-                asm volatile("" : "+v"(nn));
+                asm volatile("" : "+v"(nn)::"memory");
                 const int ll = 16 * lb + li;
                 const bool ok = nn < ll && ll < nw;
                 const int x = min(nn, nw - 1), y = min(ll, nw - 1);
@@ -909,13 +933,13 @@ __device__ __attribute__((always_inline)) void eval_dermorb_in(const Smem& S, co
                 cplx<double> P[3], Pu[3];
 #pragma unroll
                 for (int r = 0; r < 3; ++r) {
-                    Pu[r] = FIRST && !HERM ? mk(0.0, 0.0) : (-m) * K.V(ax[r], x, y);
-                    P[r] = HERM && !FIRST ? Pu[r] : HERM ? (-m) * K.V(ax[r], x, y) : (-m) * conj(K.V(ax[r], y, x));
+                    Pu[r] = FIRST && !HERM ? mk(0.0, 0.0) : (-m) * K.Vu(ax[r], x, y);
+                    P[r] = HERM && !FIRST ? Pu[r] : HERM ? (-m) * K.Vu(ax[r], x, y) : (-m) * conj(K.Vu(ax[r], y, x));
                 }
 #pragma unroll
                 for (int d = 0; d < 3; ++d) {
                     cplx<double> f = G[0].get(d, v);
-                    if constexpr (FIRST) f = (HERM ? 0.5 * K.W(b, ax[d], x, y) : 0.5 * conj(K.W(b, ax[d], y, x))) - f;
+                    if constexpr (FIRST) f = (HERM ? 0.5 * K.getu(WBMI_ROLE_W + 3 * b + ax[d], x, y) : 0.5 * conj(K.getu(WBMI_ROLE_W + 3 * b + ax[d], y, x))) - f;
 #pragma unroll
                     for (int a = 0; a < 3; ++a) {
                         const double s = -kap * (P[a] * conj(f)).im - (Z.get(a, v) * conj(P[d])).re;
@@ -933,6 +957,7 @@ __device__ __attribute__((always_inline)) void eval_dermorb_in(const Smem& S, co
                         }
                     }
                 }
+                cut_pin(o, v);
             }
         };
         // rows and columns past the end repeat the last one; their results are not read
@@ -944,11 +969,11 @@ __device__ __attribute__((always_inline)) void eval_dermorb_in(const Smem& S, co
         for (int k0 = 16 * lb; k0 < nw; k0 += 4) {
             const int m = min(k0 + lk, nw - 1);
             const double w = k0 + lk >= nw || m < l ? 0.0 : m == l ? 0.5 : 1.0;
-            const cplx<double> vl = w * K.V(b, m, l), vu = HERM ? vl : w * conj(K.V(b, l, m));
+            const cplx<double> vl = w * K.Vu(b, m, l), vu = HERM ? vl : w * conj(K.Vu(b, l, m));
             const double mm = K.m(n, m), kap = -mm * (2.0 * sign * En + 2.0 * S.E[m]);
 #pragma unroll
             for (int r = 0; r < 3; ++r) {
-                const cplx<double> P = (-mm) * conj(K.V(ax[r], m, n));
+                const cplx<double> P = (-mm) * conj(K.Vu(ax[r], m, n));
                 G[0].add(r, P, vu);
                 if constexpr (!HERM) G[1].add(r, P, vl);
                 Z.add(r, mk(-kap * P.im, kap * P.re), vl);
@@ -961,11 +986,11 @@ __device__ __attribute__((always_inline)) void eval_dermorb_in(const Smem& S, co
         for (int k0 = 0; k0 < min(16 * nb + 16, nw); k0 += 4) {
             const int q = min(k0 + lk, nw - 1);
             const double w = k0 + lk >= nw || q > n ? 0.0 : q == n ? 0.5 : 1.0;
-            const cplx<double> vl = w * K.V(b, n, q), vu = HERM ? vl : w * conj(K.V(b, q, n));
+            const cplx<double> vl = w * K.Vu(b, n, q), vu = HERM ? vl : w * conj(K.Vu(b, q, n));
             const double mm = K.m(q, l), kap = mm * (2.0 * sign * S.E[q] + 2.0 * El);  // Q enters with -
 #pragma unroll
             for (int r = 0; r < 3; ++r) {
-                const cplx<double> Pu = (-mm) * K.V(ax[r], q, l), P = HERM ? Pu : (-mm) * conj(K.V(ax[r], l, q));
+                const cplx<double> Pu = (-mm) * K.Vu(ax[r], q, l), P = HERM ? Pu : (-mm) * conj(K.Vu(ax[r], l, q));
                 G[0].add(r, vu, P);
                 if constexpr (!HERM) G[1].add(r, vl, Pu);
                 Z.add(r, vl, mk(-kap * P.im, kap * P.re));
@@ -974,6 +999,238 @@ __device__ __attribute__((always_inline)) void eval_dermorb_in(const Smem& S, co
         add_pairs(std::false_type{});
 #pragma unroll
         for (int q = 0; q < 7; ++q) cut_tile_add(S, nw, nb, lb, o[q], q == 6 ? b * 4 : ax[1 + q / 3] * 3 + ax[q % 3]);
+    }
+}
+
+// DerMorb with external terms for sign = +1 and complex128 channels, every needed cut into S.cut (internal
+// terms too when `in`).  Next to eval_dermorb_in (A, V Hermitian; B is not):
+//   Q^a_nl also holds (2 E_n conj(A^a_ln) + 2 conj(B^a_ln)) / (E_l - E_n);
+//   formula_task's kinds 2 and 3 together are Re -2 P^a_nl (E_n FA + FB)^{bd}_ln to the pair of a and b, with A
+//     and B in the place of V and A', B' in that of W / 2;
+//   kind 4's Omega block, -2 Re (P^d A^b)_ln V^e_nl over l, n < c, belongs to the pair (n, m) of A^b_mn with
+//     (V^e P^d)_nm, and to that of P^d_nm with (V^e A^b)_nm;
+//   kinds 6 and 7 cancel, 2 Im tr V^e A^al A^be + 2 Im tr V^e A^be A^al, and the s5 terms vanish;
+//   the per-band terms with O and C are pair values and r(max(n, l)).
+// A task is a pair of 16-band blocks and one b, in two passes (V, then A and B), or the per-band terms of one c.
+// 1287 k-points at nw = 18, a narrow window: 0.94 ms one by one, 0.50 together, 0.39 with V and A in LDS
+// and the per-band terms as tasks.
+template <typename T, bool LM, bool ST, bool SA, int NW, typename TS>
+__device__ __attribute__((always_inline)) void eval_dermorb_ex(const Smem& S, const KCtx<T, LM, ST, SA, NW, TS>& K, bool in) {
+    const int nw = K.n_(), tid = threadIdx.x, lane = tid & 63, lk = lane >> 4, li = lane & 15;
+    const int nblk = (nw + 15) / 16, ntask = 6 * (nblk * (nblk + 1) / 2);
+    const double win = in ? 1.0 : 0.0;
+    for (;;) {
+        int t = 0;
+        if (lane == 0) t = atomicAdd(&S.misc[3], 1);
+        t = __builtin_amdgcn_readfirstlane(t) * K.parts + K.part;
+        if (t >= ntask) break;
+        const int npair = ntask / 6, b = t / npair;
+        int nb, lb;
+        cut_tile_pair(t % npair, nblk, nb, lb);
+        // the lane's pair (x, y) of a tile, its rows opaque (operands loaded anew, not kept in registers)
+        auto pair = [&](int v, int& x, int& y) {
+            int nn = 16 * nb + lk + 4 * v;
+            asm volatile("" : "+v"(nn)::"memory");
+            const int ll = 16 * lb + li;
+            x = min(nn, nw - 1);
+            y = min(ll, nw - 1);
+            return nn < nw && ll < nw ? ll - nn : -1;
+        };
+        if (b >= 3) {
+            const int c = b - 3;
+            double g[3][4], r[3] = {0.0, 0.0, 0.0};
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                int x, y;
+                const int dist = pair(v, x, y);
+                const double m = K.m(x, y), Ex = S.E[x];
+                const cplx<double> Oxy = K.getu(WBMI_ROLE_O + c, x, y), Oyx = K.getu(WBMI_ROLE_O + c, y, x);
+                const cplx<double> Cxy = K.getu(WBMI_ROLE_C + c, x, y), Cyx = K.getu(WBMI_ROLE_C + c, y, x);
+#pragma unroll
+                for (int d = 0; d < 3; ++d) {
+                    const cplx<double> Vxy = K.Vu(d, x, y), Vyx = K.Vu(d, y, x);
+                    const double e = 2.0 * Ex * (conj(Oyx) * Vyx).re + (Cxy * Vyx + Vxy * Cyx).re;
+                    g[d][v] = dist > 0 ? m * e : 0.0;
+                    if (dist > 0) r[d] += (Oxy * Vyx + Oyx * Vxy).re;
+                    if (dist == 0)
+                        r[d] += (Oxy * Vxy).re + Ex * K.getu(WBMI_ROLE_OD + 3 * c + d, x, x).re + K.getu(WBMI_ROLE_CD + 3 * c + d, x, x).re;
+                }
+            }
+#pragma unroll
+            for (int d = 0; d < 3; ++d) {
+                cut_tile_add(S, nw, nb, lb, g[d], c * 3 + d);
+                r[d] = wave_sum(r[d], 0x30);
+                if (lane < 16 && 16 * lb + lane < nw) atomicAdd(&S.acc[(16 * lb + lane) * 9 + c * 3 + d], r[d]);
+            }
+            continue;
+        }
+        if (!cut_tile_needed(S, nw, nb, lb)) continue;
+        int ax[3];  // the indices b, b + 1, b + 2: everything below is relative to b
+#pragma unroll
+        for (int r = 0; r < 3; ++r) ax[r] = (b + r) % 3;
+        // the pairs' values: components (c, d) relative to b, c = 1, 2 in [0, 6), (0, 0) in [6]
+        double o[7][4];
+#pragma unroll
+        for (int q = 0; q < 7; ++q)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) o[q][v] = 0.0;
+        const int n = min(16 * nb + li, nw - 1), l = min(16 * lb + li, nw - 1);
+        const double En = S.E[n], El = S.E[l];
+        // weight of the summed band k0 + lk: beyond the limit counted fully, on it half
+        auto above = [&](int k0) { return k0 + lk >= nw || k0 + lk < l ? 0.0 : k0 + lk == l ? 0.5 : 1.0; };
+        auto below = [&](int k0) { return k0 + lk >= nw || k0 + lk > n ? 0.0 : k0 + lk == n ? 0.5 : 1.0; };
+        const int kmax = min(16 * nb + 16, nw);
+        // Q^a_xy, x inside
+        auto Qof = [&](int a, int x, int y, double m, double Ex, double Ey, cplx<double> P) {
+            const double kap = -win * m * (2.0 * Ex + 2.0 * Ey);
+            const cplx<double> A = K.Au(a, y, x), B = K.getu(WBMI_ROLE_B + a, y, x);
+            return mk(-kap * P.im - m * (2.0 * Ex * A.re + 2.0 * B.re), kap * P.re + m * (2.0 * Ex * A.im + 2.0 * B.im));
+        };
+        {
+            CutAcc G, Z, D;  // P V or V P; Q V or -V Q; V A
+            auto add_pairs = [&](auto first) {
+                constexpr bool FIRST = decltype(first)::value;
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    int x, y;
+                    const bool ok = pair(v, x, y) > 0;
+                    const double m = K.m(x, y);
+                    cplx<double> P[3], Q[3];
+#pragma unroll
+                    for (int r = 0; r < 3; ++r) {
+                        P[r] = (-m) * K.Vu(ax[r], x, y);
+                        Q[r] = Qof(ax[r], x, y, m, S.E[x], S.E[y], P[r]);
+                    }
+#pragma unroll
+                    for (int d = 0; d < 3; ++d) {
+                        cplx<double> f = G.get(d, v);
+                        const cplx<double> h = f;
+                        if constexpr (FIRST) f = 0.5 * K.getu(WBMI_ROLE_W + 3 * b + ax[d], x, y) - f;
+                        const cplx<double> A = FIRST ? mk(0.0, 0.0) : K.Au(ax[d], x, y);
+#pragma unroll
+                        for (int a = 0; a < 3; ++a) {
+                            const double s = (Q[a] * conj(f)).re - (Z.get(a, v) * conj(P[d])).re;
+                            if (a != 0) {
+                                const double e = pair_sign(a, 0) * s;
+                                o[(third_index(a, 0) - 1) * 3 + d][v] += ok ? e : 0.0;
+                            }
+                            if (a != d) {
+                                double e = s - 2.0 * win * (P[a] * conj(h)).im;
+                                // the Omega block's A^d with (V P^a) and P^a with (V A^d)
+                                if constexpr (!FIRST)
+                                    e -= 2.0 * ((G.get(a, v) * conj(A)).re + (P[a] * conj(D.get(d, v))).re);
+                                e *= pair_sign(a, d);
+                                const int c = third_index(a, d);
+                                o[c == 0 ? 6 : (c - 1) * 3][v] += ok ? e : 0.0;
+                            }
+                        }
+                    }
+                    cut_pin(o, v);
+                }
+            };
+            G.zero();
+            Z.zero();
+            for (int k0 = 16 * lb; k0 < nw; k0 += 4) {
+                const int m = min(k0 + lk, nw - 1);
+                const cplx<double> vl = above(k0) * K.Vu(b, m, l);
+                const double mm = K.m(n, m), Em = S.E[m];
+#pragma unroll
+                for (int r = 0; r < 3; ++r) {
+                    const cplx<double> P = (-mm) * conj(K.Vu(ax[r], m, n));
+                    G.add(r, P, vl);
+                    Z.add(r, Qof(ax[r], n, m, mm, En, Em, P), vl);
+                }
+            }
+            add_pairs(std::true_type{});
+            G.zero();
+            Z.zero();
+            D.zero();
+            for (int k0 = 0; k0 < kmax; k0 += 4) {
+                const int q = min(k0 + lk, nw - 1);
+                const cplx<double> vl = below(k0) * K.Vu(b, n, q);
+                const double mm = K.m(q, l), Eq = S.E[q];
+#pragma unroll
+                for (int r = 0; r < 3; ++r) {
+                    const cplx<double> P = (-mm) * K.Vu(ax[r], q, l);
+                    G.add(r, vl, P);
+                    Z.add(r, vl, -Qof(ax[r], q, l, mm, Eq, El, P));
+                    D.add(r, vl, K.Au(ax[r], q, l));
+                }
+            }
+            add_pairs(std::false_type{});
+        }
+        {
+            // A and B: f = conj(E_n FA + FB), the weight -2 P
+            CutAcc G, H, Z;
+            auto add_pairs = [&](auto first) {
+                constexpr bool FIRST = decltype(first)::value;
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    int x, y;
+                    const bool ok = pair(v, x, y) > 0;
+                    const double m = K.m(x, y), Ex = S.E[x];
+                    cplx<double> P[3];
+#pragma unroll
+                    for (int r = 0; r < 3; ++r) P[r] = (-m) * K.Vu(ax[r], x, y);
+#pragma unroll
+                    for (int d = 0; d < 3; ++d) {
+                        cplx<double> f = G.get(d, v);
+                        if constexpr (FIRST)
+                            f = Ex * conj(K.getu(WBMI_ROLE_AD + 3 * b + ax[d], y, x)) + conj(K.getu(WBMI_ROLE_BD + 3 * b + ax[d], y, x)) - Ex * f - H.get(d, v);
+#pragma unroll
+                        for (int a = 1; a < 3; ++a) {
+                            cplx<double> z = Z.get(a, v);
+                            if constexpr (FIRST) z += Ex * G.get(a, v);
+                            const double s = -2.0 * (P[a] * conj(f)).re + (FIRST ? 2.0 : -2.0) * (z * conj(P[d])).re;
+                            const double e = pair_sign(a, 0) * s;
+                            o[(third_index(a, 0) - 1) * 3 + d][v] += ok ? e : 0.0;
+                        }
+                    }
+                    cut_pin(o, v);
+                }
+            };
+            // G = P A, H = P conj(B)^T, Z = P B
+            G.zero();
+            H.zero();
+            Z.zero();
+            for (int k0 = 16 * lb; k0 < nw; k0 += 4) {
+                const int m = min(k0 + lk, nw - 1);
+                const double w = above(k0), mm = K.m(n, m);
+                const cplx<double> al = w * K.Au(b, m, l), bl = w * K.getu(WBMI_ROLE_B + b, m, l), bu = w * conj(K.getu(WBMI_ROLE_B + b, l, m));
+#pragma unroll
+                for (int r = 0; r < 3; ++r) {
+                    const cplx<double> P = (-mm) * conj(K.Vu(ax[r], m, n));
+                    G.add(r, P, al);
+                    H.add(r, P, bu);
+                    if (r > 0) Z.add(r, P, bl);
+                }
+            }
+            add_pairs(std::true_type{});
+            // G = (E_n A + B^+) P, Z = (E A + B) P with the summed band's energy
+            G.zero();
+            Z.zero();
+            for (int k0 = 0; k0 < kmax; k0 += 4) {
+                const int q = min(k0 + lk, nw - 1);
+                const double w = below(k0), mm = K.m(q, l), Eq = S.E[q];
+                const cplx<double> A = K.Au(b, n, q);
+                const cplx<double> m1 = w * (En * A + conj(K.getu(WBMI_ROLE_B + b, q, n))), m2 = w * (Eq * A + K.getu(WBMI_ROLE_B + b, n, q));
+#pragma unroll
+                for (int r = 0; r < 3; ++r) {
+                    const cplx<double> P = (-mm) * K.Vu(ax[r], q, l);
+                    G.add(r, m1, P);
+                    if (r > 0) Z.add(r, m2, P);
+                }
+            }
+            add_pairs(std::false_type{});
+        }
+#pragma unroll
+        for (int q = 0; q < 7; ++q) cut_tile_add(S, nw, nb, lb, o[q], q == 6 ? b * 4 : ax[1 + q / 3] * 3 + ax[q % 3]);
+    }
+    __syncthreads();
+    for (int t = tid; t < nw * 9; t += (int)blockDim.x) {
+        double v = S.cut[t + 9];
+        for (int x = 0; x <= t / 9; ++x) v += S.acc[x * 9 + t % 9];
+        S.cut[t + 9] = v;
     }
 }
 
@@ -1430,7 +1687,7 @@ __host__ __device__ constexpr int scan_min_waves(bool tasks, int nth) { return !
 
 // NW > 0: the kernel for nw = NW only, every size and row stride a compile-time constant
 template <typename T, int F, bool LM, bool ST, int MODE, int NW, int NTH>
-__global__ void __launch_bounds__(NTH, SC_IS_DERMORB_IN(F) ? 2 : (scan_min_waves((F == WBMI_FORMULA_DEROMEGA || F == WBMI_FORMULA_DERMORB) && MODE != 1, NTH)))
+__global__ void __launch_bounds__(NTH, SC_IS_DERMORB_CUTS(F) ? 2 : (scan_min_waves((F == WBMI_FORMULA_DEROMEGA || F == WBMI_FORMULA_DERMORB) && MODE != 1, NTH)))
 k_static_scan(ScanArgs args, const double* __restrict__ Eall, const cplx<T>* __restrict__ Xall, double* __restrict__ hist) {
     extern __shared__ __attribute__((aligned(16))) char smem_raw[];
     const wbmi_scan_params& p = args.p;
@@ -1444,7 +1701,8 @@ k_static_scan(ScanArgs args, const double* __restrict__ Eall, const cplx<T>* __r
     const int tid = threadIdx.x;
     if (MODE != 2) hist += k * args.hist_stride;
     constexpr bool tasks = F == WBMI_FORMULA_DEROMEGA || F == WBMI_FORMULA_DERMORB;
-    static_assert(tasks || F == WBMI_FORMULA_OMEGA || !ST, "V and A are staged for DerOmega, DerMorb and Omega");
+    static_assert(tasks || SC_IS_DERMORB_CUTS(F) || F == WBMI_FORMULA_OMEGA || !ST,
+                  "V and A are staged for DerOmega, DerMorb and Omega");
     using TS = T;
     constexpr bool SA = ST;
     constexpr bool stage_v = ST;
@@ -1706,7 +1964,7 @@ k_static_scan(ScanArgs args, const double* __restrict__ Eall, const cplx<T>* __r
     } else {
         // non-additive: traces of the cumulative cuts [0, c) (static.py:109-117) at the borders of
         // the groups in range and of the sea
-        constexpr bool all_cuts = SC_IS_DERMORB_IN(F) || F == WBMI_FORMULA_MORB_HPM;
+        constexpr bool all_cuts = SC_IS_DERMORB_CUTS(F) || F == WBMI_FORMULA_MORB_HPM;
         for (int n = tid; n <= nw; n += (int)blockDim.x) S.need[n] = 0;
         if constexpr (all_cuts) {
             for (int t = tid; t < nw * 9; t += (int)blockDim.x) S.acc[t] = S.cut[t + 9] = 0.0;
@@ -1721,6 +1979,9 @@ k_static_scan(ScanArgs args, const double* __restrict__ Eall, const cplx<T>* __r
         __syncthreads();
         if constexpr (SC_IS_DERMORB_IN(F)) {
             if (p.internal_terms) eval_dermorb_in<F == SC_DERMORB_IN>(S, K, (double)p.sign);
+            __syncthreads();
+        } else if constexpr (F == SC_DERMORB_EX) {
+            eval_dermorb_ex(S, K, p.internal_terms);
             __syncthreads();
         } else if constexpr (all_cuts) {
             eval_morb_cuts(S, K, p.internal_terms, p.external_terms, (double)p.sign);
@@ -1780,8 +2041,8 @@ static int launch_scan_t(wbmi_ctx* ctx, int nk, const ScanArgs& a, const double*
     // about four per CU (above nw = 32, where a k-point's tasks fill them; two below).  Fermi bins only: the
     // other modes use a k-point's sums before they are complete.
     constexpr bool tasks = F == WBMI_FORMULA_DEROMEGA || F == WBMI_FORMULA_DERMORB;
-    const int want = a.nw > 32 ? 1024 : 512;
-    const int parts = (tasks || SC_IS_DERMORB_IN(F)) && MODE == 0 && nk < want ? std::min(8, want / nk) : 1;
+    const int want = SC_IS_DERMORB_CUTS(F) ? (a.nw > 32 ? 4096 : 2048) : a.nw > 32 ? 1024 : 512;
+    const int parts = (tasks || SC_IS_DERMORB_CUTS(F)) && MODE == 0 && nk < want ? std::min(8, want / nk) : 1;
     WBMI_HIP_CHECK(ctx, hipFuncSetAttribute((const void*)k_static_scan<T, F, LM, ST, MODE, NW, NTH>,
                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     ScanArgs args = a;
@@ -1804,7 +2065,11 @@ static int launch_scan(wbmi_ctx* ctx, int nk, const ScanArgs& a, const double* E
     // two waves per SIMD
     if constexpr (F == WBMI_FORMULA_MORB_HPM && MODE != 2) {
         return launch_scan_t<T, F, false, false, MODE, 0, 256>(ctx, nk, a, E, X, hist);
-    } else if constexpr (SC_IS_DERMORB_IN(F)) {
+    } else if constexpr (SC_IS_DERMORB_CUTS(F)) {
+        // (complex64 channels of the sizes that are staged go to SC_DERMORB_IN32)
+        if constexpr (sizeof(T) == 8 || F == SC_DERMORB_IN32)
+            if (a.stage_va && smem_offsets(a.nw, true, true, a.p.external_terms, MODE == 1, sizeof(cplx<T>)).total <= SC_LDS / 2)
+                return launch_scan_t<T, F, true, true, MODE, 0, 256>(ctx, nk, a, E, X, hist);
         if (smem_offsets(a.nw, true, false, false, MODE == 1, sizeof(cplx<T>)).total <= SC_LDS / 2)
             return launch_scan_t<T, F, true, false, MODE, 0, 256>(ctx, nk, a, E, X, hist);
         return launch_scan_t<T, F, MODE == 0, false, MODE, 0, 512>(ctx, nk, a, E, X, hist);
@@ -1850,6 +2115,8 @@ static int dispatch_scan(wbmi_ctx* ctx, int nk, const ScanArgs& a, const double*
                         if (a.nw <= 32) return launch_scan<T, SC_DERMORB_IN32, MODE>(ctx, nk, a, E, X, hist);
                     return launch_scan<T, SC_DERMORB_IN, MODE>(ctx, nk, a, E, X, hist);
                 }
+            if constexpr (MODE != 2 && sizeof(T) == 8)
+                if (a.p.sign == 1) return launch_scan<T, SC_DERMORB_EX, MODE>(ctx, nk, a, E, X, hist);
             return launch_scan<T, WBMI_FORMULA_DERMORB, MODE>(ctx, nk, a, E, X, hist);
         case WBMI_FORMULA_DERSPIN: return launch_scan<T, WBMI_FORMULA_DERSPIN, MODE>(ctx, nk, a, E, X, hist);
         case WBMI_FORMULA_VELSPIN: return launch_scan<T, WBMI_FORMULA_VELSPIN, MODE>(ctx, nk, a, E, X, hist);
