@@ -163,6 +163,40 @@ def test_scan_all_cuts(nw, ef, precision, terms):
         assert err < (1e-9 if precision == "fp64" else 2e-5), name
 
 
+@pytest.mark.parametrize("nw,precision,kramers", [
+    (2, "fp64", False), (7, "fp64", False), (8, "fp32", True), (9, "fp64", True), (17, "fp32", False), (24, "fp64", True),
+    (25, "fp64", False), (33, "fp32", False), (49, "fp64", True), (65, "fp64", False)])
+def test_scan_diagonal_traces(nw, precision, kramers):
+    """Omega and the velocity products with Omega and Morb_Hpm at the edges of the 8 x 8 blocks, groups of one
+    band, a pair 5e-5 apart, or every two bands a group: against the oracle."""
+    import wannierberri_amd as wb
+    from oracle import wb_oracle as O
+    from wannierberri_amd import models
+    s = models.synthetic(num_wann=nw, Rmax=1, seed=90 + nw, with_BBCC=True)
+    ham = s.get_R_mat("Ham").copy()
+    ham[:, -2:, :] = 0.
+    ham[:, :, -2:] = 0.
+    i0 = s.rvec.iR0
+    ham[i0, -2, -2], ham[i0, -1, -1] = 0.5, 0.5 + 5e-5
+    s.set_R_mat("Ham", ham, reset=True)
+    Ef = np.linspace(-40., 40., 41)
+    k = np.random.default_rng(nw).random((3, 3))
+    st = wb.calculators.static
+    kw = dict(degen_Kramers=kramers)
+    names = {"ahc": "AHC", "bcd": "BerryDipole_FermiSurf", "gme": "GME_orb_FermiSurf"}
+    got = wb.run_klists(s, [k], {n: getattr(st, c)(Efermi=Ef, **kw) for n, c in names.items()},
+                        parameters_K={"precision": precision})
+    o = O.OracleSystem(s.real_lattice, s.rvec.iRvec, s.wannier_centers_cart,
+                       {m: s.get_R_mat(m) for m in ("Ham", "AA", "BB", "CC")})
+    d = O.OracleDataK(o, k_list=k)
+    for name, c in names.items():
+        ref = getattr(O, c)(Ef, **kw)(d).data
+        err, scale = np.abs(got.results[name].data - ref).max(), np.abs(ref).max()   # (zero at nw = 2: flat bands)
+        print(f"test_scan_diagonal_traces nw={nw} {precision} {name}: {err:.2e} of {scale:.2e}", flush=True)
+        # sums of 1 / dE^2 over gaps above 1e-4 between groups, typically 1e-2: 1e-16 * 1e4 and a margin
+        assert err <= (1e-9 if precision == "fp64" else 2e-5) * scale, name
+
+
 @pytest.mark.parametrize("nw", [1, 2, 15, 16, 17, 31, 32, 33, 48, 49, 64, 65, 80, 81, 97, 112, 113, 128])
 def test_rotate_sizes(ctx, nw):
     """One size at each edge of the rotation's 16-row blocks, flagged (Hermitian part), plain and

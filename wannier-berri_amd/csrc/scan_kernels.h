@@ -46,7 +46,7 @@
 #include "mfma_c64.h"
 #include "wbmi_common.h"
 
-#define SC_THREADS 512  // workgroup size of the scan kernels (DerOmega / DerMorb: task_threads)
+#define SC_THREADS 512  // workgroup size of the scan kernels (others: launch_scan)
 #define SC_NWMAX 128
 #define SC_LDS (160 * 1024)
 #define SC_XCD_LOG 3
@@ -183,7 +183,7 @@ __device__ __attribute__((always_inline)) inline Smem make_smem(char* base, int 
 
 // Element access to the channels of one k-point.
 // LM: dEinv o Off read from LDS (nw <= SC_M_NW) or formed from E and the labels.
-// ST: V read from its LDS copy (DerOmega, DerMorb and Omega at nw <= SC_LDS_NW) or from the
+// ST: V read from its LDS copy (DerOmega and DerMorb at nw <= SC_LDS_NW) or from the
 // channels; SA: the same for A (staged together with V, and only with external terms, the only
 // case that reads it).
 // Both are compile-time so that every access is a plain LDS or global load.
@@ -271,29 +271,22 @@ struct KCtx {
 };
 
 // pre-Hermitian Omega summand s^c_xy for x, y in the same group
-// (formula/covariant.py:175-200): Omega.nn = s + s^+.  The sum over the
-// off-group bands l runs over [l0, l1); `tail` adds the within-group and O terms.
+// (formula/covariant.py:175-200): Omega.nn = s + s^+
 template <typename T, bool LM, bool ST, bool SA, int NW, typename TS>
-__device__ __attribute__((always_inline)) cplx<double> omega_s(const KCtx<T, LM, ST, SA, NW, TS>& K, int c, int x, int y, bool internal,
-                                                              bool external, int l0, int l1, bool tail) {
+__device__ __attribute__((always_inline)) cplx<double> omega_s(const KCtx<T, LM, ST, SA, NW, TS>& K, int c, int x, int y, bool internal, bool external) {
     const int al = c_alpha[c], be = c_beta[c];
     cplx<double> s = mk(0.0, 0.0);
-    for (int l = l0; l < l1; ++l) {
+    for (int l = 0; l < K.n_(); ++l) {
         if (K.lab[l] == K.lab[x]) continue;
         cplx<double> dxa = K.Dp(al, x, l);
         if (internal) s += times_i(-(dxa * K.Dp(be, l, y)));
         if (external) s += K.Dp(be, x, l) * K.A(al, l, y) - dxa * K.A(be, l, y);
     }
-    if (external && tail) {
+    if (external) {
         for (int m = K.gs[x]; m < K.ge[x]; ++m) s += times_i(-(K.A(al, x, m) * K.A(be, m, y)));
         s += 0.5 * K.O(c, x, y);
     }
     return s;
-}
-template <typename T, bool LM, bool ST, bool SA, int NW, typename TS>
-__device__ __attribute__((always_inline)) cplx<double> omega_s(const KCtx<T, LM, ST, SA, NW, TS>& K, int c, int x, int y, bool internal,
-                                                              bool external) {
-    return omega_s(K, c, x, y, internal, external, 0, K.n_(), true);
 }
 
 // pre-Hermitian Morb_H summand h^c_xy for x, y in the same group
@@ -1292,6 +1285,112 @@ __device__ __attribute__((always_inline)) void eval_morb_cuts(const Smem& S, con
     }
 }
 
+// Diagonal elements of the band-group blocks of Omega (formula/covariant.py:175-200) or, MORB, of
+// Morb_H + sign E o Omega (formula/covariant.py:390-414) for the partition of the labels, added to
+// S.acc[n][c], c = 0 .. 2; `single`: only for groups of one band.
+// A wave takes 8 bands n by 8 bands l at a time and all three components: rows (n, l) and columns (l, n) of the
+// channels are both read in runs of 8 elements, each element once, with no copy of V and A in LDS (which
+// held one workgroup a CU at nw = 32) and no element read once per component.  Bound: the channels' bytes
+// and the latency of the loads.  Against four lanes
+// per (n, c) on LDS copies up to nw = 32 and one thread per (n, c) above: Omega of 4096 k-points at nw = 32
+// 255 -> 105 us complex128, 127 -> 100 complex64; 5832 at nw = 24 172 -> 90 and 95 -> 78; 3375 at nw = 48
+// 540 -> 201 and 490 -> 193.  Velocity products (one thread per (n, a, b), each Omega or Morb_Hpm element formed
+// for every a and both orders) of 1331 k-points at nw = 18: 105 -> 28 (Omega), 186 -> 41 us (Morb_Hpm).
+template <bool MORB, typename T, bool LM, bool ST, bool SA, int NW, typename TS>
+__device__ __attribute__((always_inline)) void diag_traces(const Smem& S, const KCtx<T, LM, ST, SA, NW, TS>& K, bool in, bool ex, double sign,
+                                                          bool single) {
+    const int nw = K.n_(), lane = threadIdx.x & 63, nwave = (int)blockDim.x >> 6;
+    const int n8 = (nw + 7) / 8, split = min(max(nwave / n8, 1), n8);  // waves that share 8 rows
+    for (int t = threadIdx.x >> 6; t < n8 * split; t += nwave) {
+        const int nn = 8 * (t % n8) + (lane >> 3), n = min(nn, nw - 1);
+        const bool on = nn < nw && S.act[n] && !(single && S.ge[n] - S.gs[n] > 1);
+        if (!__any(on)) continue;
+        const int lab = S.lab[n];
+        const double En = S.E[n];
+        double v[3] = {0.0, 0.0, 0.0};
+        for (int l0 = 8 * (t / n8); l0 < nw; l0 += 8 * split) {
+            const int ll = l0 + (lane & 7), l = min(ll, nw - 1);
+            if (!on || ll >= nw) continue;
+            const bool same = S.lab[l] == lab;
+            const double m = K.m(n, l), El = S.E[l];  // zero within the group
+            // weights of the internal and the A A terms: Omega's and Morb_H's
+            const double w = MORB ? El + sign * En : 1.0;
+            cplx<double> D[3], Vt[3], At[3], Bt[3];
+#pragma unroll
+            for (int a = 0; a < 3; ++a) {
+                D[a] = K.getu(WBMI_ROLE_V + a, n, l);
+                Vt[a] = in ? K.getu(WBMI_ROLE_V + a, l, n) : mk(0.0, 0.0);
+                At[a] = ex ? K.getu(WBMI_ROLE_A + a, l, n) : mk(0.0, 0.0);
+                if constexpr (MORB) Bt[a] = ex ? K.getu(WBMI_ROLE_B + a, l, n) : mk(0.0, 0.0);
+            }
+            if (ex && same) {
+                // the A A terms, and O and C (D' is zero here)
+                cplx<double> A[3];
+#pragma unroll
+                for (int a = 0; a < 3; ++a) A[a] = K.getu(WBMI_ROLE_A + a, n, l);
+#pragma unroll
+                for (int c = 0; c < 3; ++c) {
+                    v[c] += 2.0 * w * (A[c == 2 ? 0 : c + 1] * At[c == 0 ? 2 : c - 1]).im;
+                    if (l == n) {
+                        const double o = K.getu(WBMI_ROLE_O + c, n, n).re;
+                        v[c] += MORB ? K.getu(WBMI_ROLE_C + c, n, n).re + sign * En * o : o;
+                    }
+                }
+            }
+#pragma unroll
+            for (int a = 0; a < 3; ++a) {
+                D[a] = (-m) * D[a];
+                Vt[a] = m * Vt[a];  // D'_ln = -m_ln V_ln
+                // the external terms' factor of D'_nl: A (Omega) or B + sign E_n A (Morb_Hpm)
+                if constexpr (MORB) Bt[a] += (sign * En) * At[a];
+                else Bt[a] = At[a];
+            }
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+                const int al = c == 2 ? 0 : c + 1, be = c == 0 ? 2 : c - 1;
+                double x = w * (D[al] * Vt[be]).im;
+                if (ex) x += (D[be] * Bt[al] - D[al] * Bt[be]).re;
+                v[c] += 2.0 * x;
+            }
+        }
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            const double x = wave_sum(v[c], 7);
+            if ((lane & 7) == 0 && on) atomicAdd(&S.acc[n * 9 + c], x);
+        }
+    }
+}
+
+// Products with the velocity, acc[n][a][b] = Re sum_{m in G} V^a_nm H^b_mn: groups of one band from their
+// diagonal elements H^b_nn in acc[n][b], larger ones from H(b, m, n)
+template <typename T, bool LM, bool ST, bool SA, int NW, typename TS, class FH>
+__device__ __attribute__((always_inline)) void vel_times(const Smem& S, const KCtx<T, LM, ST, SA, NW, TS>& K, FH H) {
+    const int nw = K.n_(), tid = threadIdx.x;
+    __syncthreads();
+    for (int n = tid; n < nw; n += (int)blockDim.x) {
+        if (!S.act[n] || S.ge[n] - S.gs[n] > 1) continue;
+        const double h[3] = {S.acc[n * 9], S.acc[n * 9 + 1], S.acc[n * 9 + 2]};
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+            const double v = K.getu(WBMI_ROLE_V + a, n, n).re;
+#pragma unroll
+            for (int b = 0; b < 3; ++b) S.acc[n * 9 + a * 3 + b] = v * h[b];
+        }
+    }
+    for (int t = tid; t < nw * 3; t += (int)blockDim.x) {
+        const int n = t / 3, b = t % 3;
+        if (!S.act[n] || S.ge[n] - S.gs[n] <= 1) continue;
+        double v[3] = {0.0, 0.0, 0.0};
+        for (int m = S.gs[n]; m < S.ge[n]; ++m) {
+            const cplx<double> h = H(b, m, n);
+#pragma unroll
+            for (int a = 0; a < 3; ++a) v[a] += (K.V(a, n, m) * h).re;
+        }
+#pragma unroll
+        for (int a = 0; a < 3; ++a) S.acc[n * 9 + a * 3 + b] = v[a];
+    }
+}
+
 // Per-band values for the current partition (the labels'; cut >= 0: they are those of [0, cut), and M
 // holds the unmasked dEinv) into S.acc[n][comp].
 template <int F, typename T, bool LM, bool ST, bool SA, int NW, typename TS>
@@ -1307,68 +1406,24 @@ __device__ __attribute__((always_inline)) void eval_partition(const Smem& S, con
         for (int n = tid; n < nw; n += (int)blockDim.x)
             if (S.act[n]) S.acc[n * 9] = 1.0;
     } else if (F == WBMI_FORMULA_OMEGA) {
-        if constexpr (ST) {
-            // V and A in LDS: four adjacent lanes share (n, c) and split the sum over l,
-            // reduced by two shuffles (a uniform loop, so every lane reaches them)
-            const int L4 = (nw + 3) / 4;
-            for (int t0 = 0; t0 < nw * 12; t0 += (int)blockDim.x) {
-                const int t = t0 + tid;
-                const bool ok = t < nw * 12;
-                const int n = ok ? t / 12 : 0, c = (t / 4) % 3, qq = t % 4;
-                const bool act = ok && S.act[n];
-                double v = 0.0;
-                if (act) {
-                    const int l0 = qq * L4, l1 = l0 + L4 < nw ? l0 + L4 : nw;
-                    v = omega_s(K, c, n, n, in, ex, l0, l1, qq == 0).re;
-                }
-                v += __shfl_xor(v, 1);
-                v += __shfl_xor(v, 2);
-                if (act && qq == 0) S.acc[n * 9 + c] = 2.0 * v;
-            }
-        } else {
-            for (int t = tid; t < nw * 3; t += (int)blockDim.x) {
-                int n = t / 3, c = t % 3;
-                if (!S.act[n]) continue;
-                S.acc[n * 9 + c] = 2.0 * omega_s(K, c, n, n, in, ex).re;
-            }
-        }
+        diag_traces<false>(S, K, in, ex, 0.0, false);
     } else if (F == WBMI_FORMULA_MORB_HPM) {
-        for (int t = tid; t < nw * 3; t += (int)blockDim.x) {
-            int n = t / 3, c = t % 3;
-            if (!S.act[n]) continue;
-            double v = 2.0 * morbh_s(K, c, n, n, in, ex).re;
-            if (p.sign != 0) v += p.sign * S.E[n] * 2.0 * omega_s(K, c, n, n, in, ex).re;
-            S.acc[n * 9 + c] = v;
-        }
+        diag_traces<true>(S, K, in, ex, (double)p.sign, false);
     } else if (F == WBMI_FORMULA_VELOMEGA) {
         // Re sum_{n' in G} V^a_nn' Omega^b_n'n, Omega = s + s^+ (formula/formula.py:141-148)
-        for (int t = tid; t < nw * 9; t += (int)blockDim.x) {
-            int n = t / 9, a = (t % 9) / 3, b = t % 3;
-            if (!S.act[n]) continue;
-            cplx<double> v = mk(0.0, 0.0);
-            for (int m = S.gs[n]; m < S.ge[n]; ++m) {
-                cplx<double> om = omega_s(K, b, m, n, in, ex) + conj(omega_s(K, b, n, m, in, ex));
-                v += K.V(a, n, m) * om;
-            }
-            S.acc[t] = v.re;
-        }
+        diag_traces<false>(S, K, in, ex, 0.0, true);
+        vel_times(S, K, [&](int b, int m, int n) { return omega_s(K, b, m, n, in, ex) + conj(omega_s(K, b, n, m, in, ex)); });
     } else if (F == WBMI_FORMULA_VELHPLUS) {
         // Re sum_{n' in G} V^a_nn' Hpm^b_n'n with the group block of Morb_Hpm,
         // Hpm = Morb_H.nn + sign Eav o Omega.nn (formula/covariant.py:424-449,
         // formula/formula.py:141-148; FormulaProduct is additive)
-        for (int t = tid; t < nw * 9; t += (int)blockDim.x) {
-            int n = t / 9, a = (t % 9) / 3, b = t % 3;
-            if (!S.act[n]) continue;
-            cplx<double> v = mk(0.0, 0.0);
-            for (int m = S.gs[n]; m < S.ge[n]; ++m) {
-                cplx<double> h = morbh_s(K, b, m, n, in, ex) + conj(morbh_s(K, b, n, m, in, ex));
-                if (p.sign != 0)
-                    h += (p.sign * 0.5 * (S.E[m] + S.E[n])) *
-                         (omega_s(K, b, m, n, in, ex) + conj(omega_s(K, b, n, m, in, ex)));
-                v += K.V(a, n, m) * h;
-            }
-            S.acc[t] = v.re;
-        }
+        diag_traces<true>(S, K, in, ex, (double)p.sign, true);
+        vel_times(S, K, [&](int b, int m, int n) {
+            cplx<double> h = morbh_s(K, b, m, n, in, ex) + conj(morbh_s(K, b, n, m, in, ex));
+            if (p.sign != 0)
+                h += (p.sign * 0.5 * (S.E[m] + S.E[n])) * (omega_s(K, b, m, n, in, ex) + conj(omega_s(K, b, n, m, in, ex)));
+            return h;
+        });
     } else if (F == WBMI_FORMULA_DERSPIN) {
         // generalised derivative of the spin (formula/formula.py:95-107 with A = Xbar('SS'),
         // dA = Xbar('SS', 1)): Re [S'^{bd}_nn - sum_{l off} D^d_nl S^b_ln + sum_{l off} S^b_nl D^d_ln]
@@ -1701,8 +1756,7 @@ k_static_scan(ScanArgs args, const double* __restrict__ Eall, const cplx<T>* __r
     const int tid = threadIdx.x;
     if (MODE != 2) hist += k * args.hist_stride;
     constexpr bool tasks = F == WBMI_FORMULA_DEROMEGA || F == WBMI_FORMULA_DERMORB;
-    static_assert(tasks || SC_IS_DERMORB_CUTS(F) || F == WBMI_FORMULA_OMEGA || !ST,
-                  "V and A are staged for DerOmega, DerMorb and Omega");
+    static_assert(tasks || SC_IS_DERMORB_CUTS(F) || !ST, "V and A are staged for DerOmega and DerMorb");
     using TS = T;
     constexpr bool SA = ST;
     constexpr bool stage_v = ST;
@@ -2057,7 +2111,7 @@ static int launch_scan_t(wbmi_ctx* ctx, int nk, const ScanArgs& a, const double*
 
 // dEinv o Off in LDS up to SC_M_NW (DerOmega / DerMorb: wherever it fits: an element formed on the fly
 // costs a division), else formed on the fly; V and A in LDS up to SC_LDS_NW for the formulas with
-// wave tasks and Omega.  Sizes: see scan_min_waves
+// wave tasks.  Sizes: see scan_min_waves
 template <typename T, int F, int MODE>
 static int launch_scan(wbmi_ctx* ctx, int nk, const ScanArgs& a, const double* E, const void* X, double* hist) {
     constexpr bool tasks = F == WBMI_FORMULA_DEROMEGA || F == WBMI_FORMULA_DERMORB;
@@ -2073,6 +2127,22 @@ static int launch_scan(wbmi_ctx* ctx, int nk, const ScanArgs& a, const double* E
         if (smem_offsets(a.nw, true, false, false, MODE == 1, sizeof(cplx<T>)).total <= SC_LDS / 2)
             return launch_scan_t<T, F, true, false, MODE, 0, 256>(ctx, nk, a, E, X, hist);
         return launch_scan_t<T, F, MODE == 0, false, MODE, 0, 512>(ctx, nk, a, E, X, hist);
+    } else if constexpr (F == WBMI_FORMULA_OMEGA || F == WBMI_FORMULA_VELOMEGA || F == WBMI_FORMULA_VELHPLUS ||
+                         F == WBMI_FORMULA_IDENTITY || F == WBMI_FORMULA_MORB_HPM) {
+        // as many waves as diag_traces has rows of 8 bands: a workgroup's prologue costs every wave of it (nw = 24,
+        // 5832 k-points: 90 us in 3 waves, 121 in 4, 182 in 8); dEinv in LDS only for velocity products, whose
+        // groups of several bands read it more than once.  The tetrahedron kernels keep 8 waves for their weights
+        // (1728 k-points at nw = 12, 201 levels: 159 us, 200 in 2 waves).
+        constexpr bool lm = F == WBMI_FORMULA_VELOMEGA || F == WBMI_FORMULA_VELHPLUS;
+        if constexpr (MODE != 1) {
+            if (a.nw <= 8) return launch_scan_t<T, F, lm, false, MODE, 0, 64>(ctx, nk, a, E, X, hist);
+            if (a.nw <= 16) return launch_scan_t<T, F, lm, false, MODE, 0, 128>(ctx, nk, a, E, X, hist);
+            if (a.nw <= 24) return launch_scan_t<T, F, lm, false, MODE, 0, 192>(ctx, nk, a, E, X, hist);
+            if (a.nw <= 32) return launch_scan_t<T, F, lm, false, MODE, 0, 256>(ctx, nk, a, E, X, hist);
+            if (a.nw <= 48) return launch_scan_t<T, F, lm, false, MODE, 0, 384>(ctx, nk, a, E, X, hist);
+        }
+        if (a.nw <= SC_M_NW) return launch_scan_t<T, F, lm, false, MODE, 0, 512>(ctx, nk, a, E, X, hist);
+        return launch_scan_t<T, F, false, false, MODE, 0, 512>(ctx, nk, a, E, X, hist);
     } else if constexpr (tasks && MODE != 1) {
         if (a.stage_va) {
             if constexpr (MODE == 0 && F == WBMI_FORMULA_DEROMEGA)
@@ -2088,12 +2158,8 @@ static int launch_scan(wbmi_ctx* ctx, int nk, const ScanArgs& a, const double* E
         if (lds <= SC_LDS / 2) return launch_scan_t<T, F, true, false, MODE, 0, 512>(ctx, nk, a, E, X, hist);
         return launch_scan_t<T, F, true, false, MODE, 0, 1024>(ctx, nk, a, E, X, hist);
     } else {
-        constexpr bool staged = tasks || F == WBMI_FORMULA_OMEGA;
-        if constexpr (staged) {
-            if constexpr (MODE == 0)
-                if (a.stage_va && a.nw == 32) return launch_scan_t<T, F, true, true, MODE, 32>(ctx, nk, a, E, X, hist);
+        if constexpr (tasks)
             if (a.stage_va) return launch_scan_t<T, F, true, true, MODE>(ctx, nk, a, E, X, hist);
-        }
         if (a.nw <= SC_M_NW) return launch_scan_t<T, F, true, false, MODE>(ctx, nk, a, E, X, hist);
         return launch_scan_t<T, F, false, false, MODE>(ctx, nk, a, E, X, hist);
     }
