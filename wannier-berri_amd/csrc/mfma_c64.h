@@ -91,22 +91,27 @@ struct MfmaHalf {
 
 __device__ inline int mfma_hrow(int v) { return (int)(threadIdx.x & 63) / 16 + 4 * v; }
 
-// C += X Y over klo <= k < khi (X and Y are called only with those k and r, c < nr, nc)
+// C += X Y over klo <= k < khi.  X and Y are called with those k and r, c < nr, nc only: an entry past the
+// end repeats the last one (its row or column of C is not to be read) or is multiplied by zero, so that the
+// loads need no branches and are issued together.
 template <class FX, class FY>
 __device__ __attribute__((always_inline)) void mfma_half(MfmaHalf& C, int nr, int nc, int klo, int khi, int r0, int c0, FX X, FY Y) {
     const int li = threadIdx.x & 15, lk = (threadIdx.x & 63) >> 4;
-    const bool rok = r0 + li < nr;
-    bool cok[2];
+    const int r = min(r0 + li, nr - 1);
+    int c[2];
 #pragma unroll
-    for (int b = 0; b < 2; ++b) cok[b] = c0 + 16 * b + li < nc;
+    for (int b = 0; b < 2; ++b) c[b] = min(c0 + 16 * b + li, nc - 1);
 #pragma unroll 2
     for (int k0 = klo & ~3; k0 < khi; k0 += 4) {
-        const int k = k0 + lk;
-        const bool kok = k >= klo && k < khi;
-        const cplx<double> a = (kok && rok) ? X(r0 + li, k) : mk(0.0, 0.0);
+        const bool kok = k0 + lk >= klo && k0 + lk < khi;
+        const int k = min(max(k0 + lk, klo), khi - 1);
+        const cplx<double> a = X(r, k);
         cplx<double> b[2];
 #pragma unroll
-        for (int q = 0; q < 2; ++q) b[q] = (kok && cok[q]) ? Y(k, c0 + 16 * q + li) : mk(0.0, 0.0);
+        for (int q = 0; q < 2; ++q) {
+            const cplx<double> y = Y(k, c[q]);
+            b[q] = mk(kok ? y.re : 0.0, kok ? y.im : 0.0);
+        }
 #pragma unroll
         for (int bj = 0; bj < 2; ++bj) {
             C.re[bj] = __builtin_amdgcn_mfma_f64_16x16x4f64(a.re, b[bj].re, C.re[bj], 0, 0, 0);
@@ -119,4 +124,3 @@ __device__ __attribute__((always_inline)) void mfma_half(MfmaHalf& C, int nr, in
         }
     }
 }
-

@@ -255,8 +255,8 @@ struct KCtx {
     __device__ inline cplx<double> S(int b, int x, int y) const { return get(WBMI_ROLE_S + b, x, y); }
     __device__ inline cplx<double> Sd(int b, int d, int x, int y) const { return get(WBMI_ROLE_SD + 3 * b + d, x, y); }
     // X o On: elements between bands of the same group
-    __device__ inline cplx<double> Ain(int a, int x, int y) const { return lab[x] == lab[y] ? A(a, x, y) : mk(0.0, 0.0); }
-    __device__ inline cplx<double> Vin(int a, int x, int y) const { return lab[x] == lab[y] ? V(a, x, y) : mk(0.0, 0.0); }
+    __device__ inline cplx<double> Ainu(int a, int x, int y) const { return lab[x] == lab[y] ? Au(a, x, y) : mk(0.0, 0.0); }
+    __device__ inline cplx<double> Vinu(int a, int x, int y) const { return lab[x] == lab[y] ? Vu(a, x, y) : mk(0.0, 0.0); }
     // dEinv_xy Off(x, y) (data_K.py:290-298): from LDS, or formed from E and the labels
     __device__ inline double m(int x, int y) const {
         if constexpr (LM) {
@@ -268,6 +268,7 @@ struct KCtx {
     }
     // D'^a_xy = -V^a_xy dEinv_xy Off(x, y)  (branch-free: M = 0 gives an exact zero for finite V)
     __device__ inline cplx<double> Dp(int a, int x, int y) const { return (-m(x, y)) * V(a, x, y); }
+    __device__ inline cplx<double> Dpu(int a, int x, int y) const { return (-m(x, y)) * Vu(a, x, y); }
 };
 
 // pre-Hermitian Omega summand s^c_xy for x, y in the same group
@@ -460,19 +461,19 @@ __device__ __attribute__((always_inline)) void formula_task(const Smem& S, const
     MfmaHalf P;
     P.zero();
     if constexpr (KIND == 0)
-        mfma_half(P, nw, nw, k0, k1, r0, c0, [&](int r, int m) { return K.V(b, r, m); }, [&](int m, int c) { return K.Dp(d, m, c); });
+        mfma_half(P, nw, nw, k0, k1, r0, c0, [&](int r, int m) { return K.Vu(b, r, m); }, [&](int m, int c) { return K.Dpu(d, m, c); });
     else if constexpr (KIND == 2)
-        mfma_half(P, nw, nw, k0, k1, r0, c0, [&](int r, int m) { return K.A(b, r, m); }, [&](int m, int c) { return K.Dp(d, m, c); });
+        mfma_half(P, nw, nw, k0, k1, r0, c0, [&](int r, int m) { return K.Au(b, r, m); }, [&](int m, int c) { return K.Dpu(d, m, c); });
     else if constexpr (KIND == 3)
-        mfma_half(P, nw, nw, k0, k1, r0, c0, [&](int r, int m) { return K.B(b, r, m); }, [&](int m, int c) { return K.Dp(d, m, c); });
+        mfma_half(P, nw, nw, k0, k1, r0, c0, [&](int r, int m) { return K.getu(WBMI_ROLE_B + b, r, m); }, [&](int m, int c) { return K.Dpu(d, m, c); });
     else if constexpr (KIND == 4)
-        mfma_half(P, nw, nw, k0, k1, r0, c0, [&](int r, int m) { return K.Dp(d, r, m); }, [&](int m, int c) { return K.A(b, m, c); });
+        mfma_half(P, nw, nw, k0, k1, r0, c0, [&](int r, int m) { return K.Dpu(d, r, m); }, [&](int m, int c) { return K.Au(b, m, c); });
     else if constexpr (KIND == 5)
-        mfma_half(P, nw, nw, k0, k1, r0, c0, [&](int r, int m) { return K.Dp(al, r, m); }, [&](int m, int c) { return K.Dp(be, m, c); });
+        mfma_half(P, nw, nw, k0, k1, r0, c0, [&](int r, int m) { return K.Dpu(al, r, m); }, [&](int m, int c) { return K.Dpu(be, m, c); });
     else if constexpr (KIND == 6)
-        mfma_half(P, nw, nw, k0, k1, r0, c0, [&](int r, int m) { return K.Ain(al, r, m); }, [&](int m, int c) { return K.Ain(be, m, c); });
+        mfma_half(P, nw, nw, k0, k1, r0, c0, [&](int r, int m) { return K.Ainu(al, r, m); }, [&](int m, int c) { return K.Ainu(be, m, c); });
     else
-        mfma_half(P, nw, nw, k0, k1, r0, c0, [&](int r, int m) { return K.Vin(b, r, m); }, [&](int m, int c) { return K.Ain(d, m, c); });
+        mfma_half(P, nw, nw, k0, k1, r0, c0, [&](int r, int m) { return K.Vinu(b, r, m); }, [&](int m, int c) { return K.Ainu(d, m, c); });
     // kinds 0, 2, 3, the within-group part -D'^d X''^b (X = V, A, B): one term for a group of one
     // band (the epilogue's), else a second product over the bands of the columns' groups.  Kind 0 of
     // DerMorb keeps it apart, as s1 reads the first product alone
@@ -500,12 +501,12 @@ __device__ __attribute__((always_inline)) void formula_task(const Smem& S, const
                 }
             }
             mfma_half(
-                Pw, nw, nw, g0, g1, r0, c0, [&](int r, int m) { return r < cut ? mk(0.0, 0.0) : -K.Dp(d, r, m); },
+                Pw, nw, nw, g0, g1, r0, c0, [&](int r, int m) { return r < cut ? mk(0.0, 0.0) : -K.Dpu(d, r, m); },
                 [&](int m, int c) {
                     if (K.lab[m] != K.lab[c]) return mk(0.0, 0.0);
-                    if constexpr (KIND == 0) return K.V(b, m, c);
-                    else if constexpr (KIND == 2) return K.A(b, m, c);
-                    else return K.B(b, m, c);
+                    if constexpr (KIND == 0) return K.Vu(b, m, c);
+                    else if constexpr (KIND == 2) return K.Au(b, m, c);
+                    else return K.getu(WBMI_ROLE_B + b, m, c);
                 });
         }
     }
@@ -531,11 +532,11 @@ __device__ __attribute__((always_inline)) void formula_task(const Smem& S, const
                     const bool ok = x < nw && y < nw;
                     const int xx = ok ? x : 0, yy = ok ? y : 0;
                     if constexpr (KIND == 0)
-                        gz[bj][v] = K.W(b, d, xx, yy);  // (l, n)
+                        gz[bj][v] = K.getu(WBMI_ROLE_W + 3 * (b) + d, xx, yy);  // (l, n)
                     else if constexpr (KIND == 2)
-                        gz[bj][v] = ex ? K.Ad(b, d, xx, yy) : mk(0.0, 0.0);
+                        gz[bj][v] = ex ? K.getu(WBMI_ROLE_AD + 3 * (b) + d, xx, yy) : mk(0.0, 0.0);
                     else
-                        gz[bj][v] = K.Bd(b, d, xx, yy);
+                        gz[bj][v] = K.getu(WBMI_ROLE_BD + 3 * (b) + d, xx, yy);
                 }
         }
 #pragma unroll
@@ -554,70 +555,70 @@ __device__ __attribute__((always_inline)) void formula_task(const Smem& S, const
                     // W^{bd}_ln / 2 - (D'^d V''^b)_ln, with D'_xy = -m_xy V_xy and m_nl = -m_ln
                     const double mln = K.m(l, n);
                     cplx<double> z = 0.5 * gz[bj][v];
-                    if (!big) z += (mln * K.V(b, n, n).re) * K.V(d, l, n);
+                    if (!big) z += (mln * K.Vu(b, n, n).re) * K.Vu(d, l, n);
                     if constexpr (DM) z += P2.get(bj, v);
                     const cplx<double> Pm = (-mln) * (pv + z);
                     const double wD = in ? (dm ? dw + 2.0 * K.E[l] : dw) : 0.0;
 #pragma unroll
                     for (int a = 0; a < 3; ++a) {
                         // -i wD D'_nl, D'_nl = m_ln conj(V_ln)
-                        const cplx<double> va = K.V(a, l, n);
+                        const cplx<double> va = K.Vu(a, l, n);
                         cplx<double> q = (wD * mln) * mk(-va.im, -va.re);
                         if (ex) {
-                            q -= dw * conj(K.A(a, l, n));
-                            if (dm) q -= 2.0 * conj(K.B(a, l, n));
+                            q -= dw * conj(K.Au(a, l, n));
+                            if (dm) q -= 2.0 * conj(K.getu(WBMI_ROLE_B + a, l, n));
                         }
                         part[bj][a] += q.re * Pm.re - q.im * Pm.im;
                     }
                     if constexpr (DM)
-                        if (in) part[bj][3] += ((mln * conj(K.V(c_alpha[s1c], l, n))) * pv).im;  // Re(-i D'^al V^d D'^be)
+                        if (in) part[bj][3] += ((mln * conj(K.Vu(c_alpha[s1c], l, n))) * pv).im;  // Re(-i D'^al V^d D'^be)
                 } else if constexpr (KIND == 2) {
                     if (!same) {
                         // A'^{bd} - D'^d A''^b
                         const double mln = K.m(l, n);
                         cplx<double> z = gz[bj][v];
-                        if (!big) z += mln * (K.V(d, l, n) * K.A(b, n, n));
+                        if (!big) z += mln * (K.Vu(d, l, n) * K.Au(b, n, n));
                         const cplx<double> Y1 = (-dw * mln) * (pv + z);
 #pragma unroll
                         for (int a = 0; a < 3; ++a) {
-                            const cplx<double> va = K.V(a, l, n);
+                            const cplx<double> va = K.Vu(a, l, n);
                             part[bj][a] += va.re * Y1.re + va.im * Y1.im;  // Re conj(V_ln) Y1
                         }
                     } else if (dm ? tc_.s5 : keep_t4<DM, T>() && S.ge[n] - S.gs[n] > SC_T4_LOOP) {
                         // s5 and T4: Re(-i sig (2 E_l + 2 sign E_n) A^a_nl (A' + A^b D'^d)_ln)
-                        const cplx<double> dA = pv + K.Ad(b, d, l, n);
+                        const cplx<double> dA = pv + K.getu(WBMI_ROLE_AD + 3 * (b) + d, l, n);
                         const double w5 = dm ? dw + 2.0 * K.E[l] : dw;
 #pragma unroll
-                        for (int a = 0; a < 3; ++a) part[bj][a] += w5 * (K.A(a, n, l) * dA).im;
+                        for (int a = 0; a < 3; ++a) part[bj][a] += w5 * (K.Au(a, n, l) * dA).im;
                     }
                 } else if constexpr (KIND == 3) {
                     if (same) continue;
                     // B'^{bd} - D'^d B''^b
                     cplx<double> z = gz[bj][v];
-                    if (!big) z -= K.Dp(d, l, n) * K.B(b, n, n);
+                    if (!big) z -= K.Dpu(d, l, n) * K.getu(WBMI_ROLE_B + b, n, n);
                     const cplx<double> YB = pv + z;
 #pragma unroll
-                    for (int a = 0; a < 3; ++a) part[bj][a] -= 2.0 * (K.Dp(a, n, l) * YB).re;  // s6
+                    for (int a = 0; a < 3; ++a) part[bj][a] -= 2.0 * (K.Dpu(a, n, l) * YB).re;  // s6
                 } else if constexpr (KIND == 4) {
                     if (!same) continue;
                     // s5 and T4 with -D'^d A^b in place of dA; Omega block: 2 sign coef Re(DA_ln V^e_nl)
                     if (dm ? tc_.s5 : S.ge[n] - S.gs[n] > SC_T4_LOOP) {
                         const double w5 = dm ? dw + 2.0 * K.E[l] : dw;
 #pragma unroll
-                        for (int a = 0; a < 3; ++a) part[bj][a] -= w5 * (K.A(a, n, l) * pv).im;
+                        for (int a = 0; a < 3; ++a) part[bj][a] -= w5 * (K.Au(a, n, l) * pv).im;
                     }
                     if constexpr (DM)
 #pragma unroll
-                        for (int e = 0; e < 3; ++e) part[bj][3 + e] += (pv * K.V(e, n, l)).re;
+                        for (int e = 0; e < 3; ++e) part[bj][3 + e] += (pv * K.Vu(e, n, l)).re;
                 } else if constexpr (KIND == 5 || KIND == 6) {
                     if (!same) continue;
                     // Omega block term -i P_ln: 2 sign Re(-i P_ln V^e_nl)
 #pragma unroll
-                    for (int w = 0; w < 3; ++w) part[bj][w] += (pv * K.V(w, n, l)).im;
+                    for (int w = 0; w < 3; ++w) part[bj][w] += (pv * K.Vu(w, n, l)).im;
                 } else {
                     if (!same) continue;
                     // s4: Re(-2i A^al_np (V''^d A''^be)_pn)
-                    part[bj][0] += (K.A(c_alpha[s1c], n, l) * pv).im;
+                    part[bj][0] += (K.Au(c_alpha[s1c], n, l) * pv).im;
                 }
             }
         }
@@ -660,6 +661,79 @@ __device__ __attribute__((always_inline)) void formula_task(const Smem& S, const
     }
 }
 
+// DerOmega's per-band terms where V and A are not in LDS, for the partition of the labels:
+//   T5: 0.5 dO.nn = 0.5 [O'^{cd}_nn - (D'^d O^c)_nn + (O^c D'^d)_nn].  O is Hermitian and D' anti-Hermitian, so
+//     (D'^d O^c)_nn = -conj((O^c D'^d)_nn) and only the real part, Re O'_nn + 2 Re sum_l conj(O_ln) D'_ln, is used;
+//   T4 of the groups of one band where it is kept (keep_t4): 2 Im A^a_nn dA_nn^{bd},
+//     dA_nn = A'_nn + sum_l A^b_nl D'^d_ln - D'^d_nl A^b_ln.
+// 8 x 8 bands a wave and all components, as in diag_traces (a thread per (n, c, d) read the columns, and for T4
+// also rows, nine times: DerOmega of 216 k-points at nw = 128 3.66 -> 3.27 ms complex64, 2.72 -> 2.56 complex128;
+// with V in LDS the threads are faster, 4096 at nw = 32 0.73 against 0.79 ms).
+template <typename T, bool LM, bool ST, bool SA, int NW, typename TS>
+__device__ __attribute__((always_inline)) void der_diag(const Smem& S, const KCtx<T, LM, ST, SA, NW, TS>& K) {
+    constexpr bool T4 = keep_t4<false, T>();
+    const int nw = K.n_(), lane = threadIdx.x & 63, nwave = ((int)blockDim.x >> 6) * K.parts;
+    const int n8 = (nw + 7) / 8, split = min(max(nwave / n8, 1), n8);
+    for (int t = ((int)threadIdx.x >> 6) * K.parts + K.part; t < n8 * split; t += nwave) {
+        const int nn = 8 * (t % n8) + (lane >> 3), n = min(nn, nw - 1);
+        const bool on = nn < nw && S.act[n], one = on && S.ge[n] - S.gs[n] == 1;
+        if (!__any(on)) continue;
+        double t5[9];
+        cplx<double> y[T4 ? 9 : 1];
+#pragma unroll
+        for (int q = 0; q < 9; ++q) {
+            t5[q] = 0.0;
+            if constexpr (T4) y[q] = mk(0.0, 0.0);
+        }
+        for (int l0 = 8 * (t / n8); l0 < nw; l0 += 8 * split) {
+            const int ll = l0 + (lane & 7), l = min(ll, nw - 1);
+            const double m = on && ll < nw ? K.m(n, l) : 0.0;
+            cplx<double> D[3], O[3];
+#pragma unroll
+            for (int a = 0; a < 3; ++a) {
+                D[a] = m * K.Vu(a, l, n);  // D'_ln = -m_ln V_ln
+                O[a] = K.getu(WBMI_ROLE_O + a, l, n);
+            }
+#pragma unroll
+            for (int q = 0; q < 9; ++q) t5[q] += 2.0 * (conj(O[q / 3]) * D[q % 3]).re;
+            if constexpr (T4) {
+                cplx<double> Dt[3], A[3], At[3];
+#pragma unroll
+                for (int a = 0; a < 3; ++a) {
+                    Dt[a] = m * K.Vu(a, n, l);
+                    A[a] = K.Au(a, n, l);
+                    At[a] = K.Au(a, l, n);
+                }
+#pragma unroll
+                for (int q = 0; q < 9; ++q) y[q] += A[q / 3] * D[q % 3] + Dt[q % 3] * At[q / 3];
+            }
+        }
+        const bool first = t < n8;  // the elementwise terms once
+#pragma unroll
+        for (int q = 0; q < 9; ++q) {
+            t5[q] = wave_sum(t5[q], 7);
+            if constexpr (T4) {
+                y[q].re = wave_sum(y[q].re, 7);
+                y[q].im = wave_sum(y[q].im, 7);
+            }
+        }
+        if ((lane & 7) || !on) continue;
+#pragma unroll
+        for (int q = 0; q < 9; ++q) {
+            const int b = q / 3, d = q % 3;
+            if (first) t5[q] += K.getu(WBMI_ROLE_OD + q, n, n).re;
+            atomicAdd(&S.acc[n * 9 + q], t5[q]);
+            if constexpr (T4) {
+                if (!one) continue;
+                if (first) y[q] += K.getu(WBMI_ROLE_AD + q, n, n);
+#pragma unroll
+                for (int a = 0; a < 3; ++a)
+                    if (a != b) atomicAdd(&S.acc[n * 9 + third_index(a, b) * 3 + d], 2.0 * pair_sign(a, b) * (K.Au(a, n, n) * y[q]).im);
+            }
+        }
+    }
+}
+
 // DerOmega (formula/covariant.py:212-259) or, dm = true, DerMorb
 // (formula/covariant.py:463-552) per-band values into S.acc[n][c*3+d], for the partition of the
 // labels (cut < 0) or [0, cut) (the labels set likewise).
@@ -669,20 +743,23 @@ __device__ __attribute__((always_inline)) void formula_task(const Smem& S, const
 // matrices times -i: it has no real part and is left out (complex64 channels: keep_t4).
 // DM is compile-time so that the DerOmega kernel carries only the kinds it runs (0 and 2): its
 // register allocation and code size are not those of the DerMorb kinds.
-// The workgroups part = 0, 1, .. of one k share its tasks: each adds up its own (the first also
-// the per-band terms), and the sums over groups are linear in them.
+// The workgroups part = 0, 1, .. of one k share its tasks and per-band terms: each adds up its own,
+// and the sums over groups are linear in them.
 template <bool DM, typename T, bool LM, bool ST, bool SA, int NW, typename TS>
 __device__ __attribute__((always_inline)) void eval_deromega(const Smem& S, const KCtx<T, LM, ST, SA, NW, TS>& K, bool in, bool ex,
                                                             int sign, int cut) {
     constexpr bool dm = DM;
     const int nw = K.n_(), tid = threadIdx.x;
-    const bool lead = K.part == 0;
+    const int t0 = tid + (int)blockDim.x * K.part, tstep = (int)blockDim.x * K.parts;  // per-band terms
     const int l0 = cut >= 0 ? cut : 0;  // D' != 0 from here on
-    // per-band terms, lanes running over (n, c, d)
-    for (int t = tid; t < nw * 9; t += (int)blockDim.x) {
-        const int n = t % nw, c = (t / nw) / 3, d = (t / nw) % 3;
-        double v = 0.0;
-        if (S.act[n] && ex && lead) {
+    constexpr bool diag = !DM && !ST;  // V and A in LDS: a thread per (n, c, d) and group
+    if constexpr (diag) {
+        if (ex) der_diag(S, K);
+    } else {
+        // per-band terms, lanes running over (n, c, d)
+        for (int t = t0; t < nw * 9; t += tstep) {
+            const int n = t % nw, c = (t / nw) / 3, d = (t / nw) % 3;
+            if (!S.act[n] || !ex) continue;
             // T5: 0.5 dO.nn = 0.5 [O'^{cd}_nn - (D'^d O^c)_nn + (O^c D'^d)_nn].  O is Hermitian
             // and D' anti-Hermitian, so (D'^d O^c)_nn = -conj((O^c D'^d)_nn) and only the real part,
             // Re O'_nn + 2 Re sum_l conj(O_ln) D'_ln, is used: column n of O, which consecutive
@@ -690,8 +767,8 @@ __device__ __attribute__((always_inline)) void eval_deromega(const Smem& S, cons
             double t5 = K.Od(c, d, n, n).re;
 #pragma unroll 8
             for (int l = l0; l < nw; ++l) t5 += 2.0 * (conj(K.O(c, l, n)) * K.Dp(d, l, n)).re;
-            v = (dm ? 2.0 * sign * S.E[n] : 2.0) * (0.5 * t5);
-            if (dm) {
+            double v = (dm ? sign * S.E[n] : 1.0) * t5;
+            if constexpr (DM) {
                 // s3: dH.nn = C'^{cd}_nn - (D'^d C^c)_nn + (C^c D'^d)_nn
                 cplx<double> s3 = K.Cd(c, d, n, n);
                 for (int l = l0; l < nw; ++l) s3 += K.C(c, n, l) * K.Dp(d, l, n) - K.Dp(d, n, l) * K.C(c, l, n);
@@ -700,16 +777,16 @@ __device__ __attribute__((always_inline)) void eval_deromega(const Smem& S, cons
                 for (int l = S.gs[n]; l < S.ge[n]; ++l) ov += K.O(c, n, l) * K.V(d, l, n);
                 v += s3.re + sign * ov.re;
             }
+            S.acc[n * 9 + c * 3 + d] = v;
         }
-        S.acc[n * 9 + c * 3 + d] = v;
     }
     int t4 = 0;  // tasks for T4: some group is too large for the loop
     if constexpr (keep_t4<DM, T>()) {
         for (int n = tid; n < nw; n += (int)blockDim.x) t4 |= S.act[n] && S.ge[n] - S.gs[n] > SC_T4_LOOP;
         t4 = __syncthreads_or(t4);
-        for (int t = tid; t < nw * 9 && ex && lead; t += (int)blockDim.x) {
+        for (int t = t0; t < nw * 9 && ex; t += tstep) {
             const int n = t % nw, b = (t / nw) / 3, d = (t / nw) % 3, g0 = S.gs[n], g1 = S.ge[n];
-            if (!S.act[n] || g1 - g0 > SC_T4_LOOP) continue;
+            if (!S.act[n] || (diag && g1 - g0 == 1) || g1 - g0 > SC_T4_LOOP) continue;
             double v[3] = {0.0, 0.0, 0.0};
             for (int m = g0; m < g1; ++m) {
                 cplx<double> y = K.Ad(b, d, m, n);  // dA.nn^{bd}_mn
