@@ -156,7 +156,7 @@ template <typename T, int NB>
 __global__ void __launch_bounds__(64 * NB, NB <= 4 ? 3 : 2) k_rotate_s(int nw, int nch, const cplx<T>* __restrict__ U, cplx<T>* X,
                                                        uint64_t herm_lo, uint64_t herm_hi, uint64_t skip_lo,
                                                        uint64_t skip_hi) {
-    constexpr int NS = 4 * NB, J = 2;
+    constexpr int NS = 4 * NB, J = NB > 4 && sizeof(T) == 4 ? 1 : 2;
     const int c = blockIdx.x;
     if (bit_of(skip_lo, skip_hi, c)) return;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, li = lane & 15, g = lane >> 4;
@@ -225,6 +225,86 @@ __global__ void __launch_bounds__(64 * NB, NB <= 4 ? 3 : 2) k_rotate_s(int nw, i
     };
     for (int bo = 0; bo + 1 < NB; bo += 2) second(bo, std::true_type{});
     if constexpr (NB & 1) second(NB - 1, std::false_type{});
+}
+
+// complex64 in FP64 arithmetic at 32 < nw <= 64 (the mixed form's velocity): one 256-thread workgroup per k, U and a
+// channel in LDS, 4 x 4 register tiles and one FMA chain per element in the order of the summed index.  Slower than
+// the matrix cores (3898 k-points at nw = 48: 356 us a channel against 146), whose order of the same sums moves one element in
+// 1e8 by its complex64 rounding: in the velocity between two close bands the cut sums of DerMorb show it (1e-9 of a
+// whole tensor, one model in forty at nw = 64).
+#define ROTV_THREADS 256
+__device__ inline void rotv_product(int nw, int r0, int c0, cplx<double> (&acc)[4][4], const cplx<double>* sT, const cplx<float>* sU,
+                                    const cplx<float>* sX, bool herm, bool second) {
+    const int ld = nw + 1;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc[i][j] = mk(0.0, 0.0);
+    for (int m = 0; m < nw; ++m) {
+        cplx<double> x[4], y[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int r = min(r0 + i, nw - 1), c = min(c0 + i, nw - 1);
+            const cplx<float> a = second ? sU[m * ld + r] : sX[r * ld + m];
+            x[i] = mk((double)a.re, (double)a.im);
+            if (!second && herm) {
+                const cplx<float> w = sX[m * ld + r];
+                x[i] = mk(0.5 * (x[i].re + (double)w.re), 0.5 * (x[i].im - (double)w.im));
+            }
+            if (second) {
+                y[i] = sT[m * ld + c];
+            } else {
+                const cplx<float> u = sU[m * ld + c];
+                y[i] = mk((double)u.re, (double)u.im);
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                if (second) cfma_cj(acc[i][j], x[i], y[j]);
+                else cfma(acc[i][j], x[i], y[j]);
+            }
+    }
+}
+__global__ void __launch_bounds__(ROTV_THREADS) k_rotate_v(int nw, int nch, const cplx<float>* __restrict__ U, cplx<float>* X,
+                                                          uint64_t herm_lo, uint64_t herm_hi, uint64_t skip_lo, uint64_t skip_hi) {
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    const int ld = nw + 1, nw2 = nw * nw, tid = threadIdx.x;
+    cplx<double>* sT = (cplx<double>*)smem;
+    cplx<float>* sU = (cplx<float>*)(sT + nw * ld);
+    cplx<float>* sX = sU + nw * ld;
+    const int64_t k = blockIdx.x;
+    const cplx<float>* Uk = U + k * nw2;
+    const int r0 = 4 * (tid / 16), c0 = 4 * (tid % 16);
+    const bool active = r0 < nw && c0 < nw;
+    for (int t = tid; t < nw2; t += ROTV_THREADS) sU[(t / nw) * ld + t % nw] = Uk[t];
+    for (int c = 0; c < nch; ++c) {
+        if (bit_of(skip_lo, skip_hi, c)) continue;
+        const bool herm = bit_of(herm_lo, herm_hi, c);
+        cplx<float>* Xc = X + (k * nch + c) * nw2;
+        for (int t = tid; t < nw2; t += ROTV_THREADS) sX[(t / nw) * ld + t % nw] = Xc[t];
+        __syncthreads();
+        cplx<double> acc[4][4];
+        if (active) {
+            rotv_product(nw, r0, c0, acc, sT, sU, sX, herm, false);
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    if (r0 + i < nw && c0 + j < nw) sT[(r0 + i) * ld + c0 + j] = acc[i][j];
+        }
+        __syncthreads();
+        if (active) {
+            rotv_product(nw, r0, c0, acc, sT, sU, sX, herm, true);
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    if (r0 + i < nw && c0 + j < nw) Xc[(r0 + i) * nw + c0 + j] = mk((float)acc[i][j].re, (float)acc[i][j].im);
+        }
+        __syncthreads();
+    }
 }
 
 // Split-half rotation (complex64 storage, nw <= 32): Xbar = U^+ X U with both products
@@ -482,6 +562,14 @@ extern "C" int wbmi_rotate(wbmi_ctx* ctx, int nk, int nw, int nch, const void* U
         if (skip_host && skip_host[c]) s[c / 64] |= 1ull << (c % 64);
     }
     if (prec == WBMI_F64) return launch_rotate<double>(ctx, nk, nw, nch, U_dev, X_dev, h, s);
+    if (prec == WBMI_F32 && nw > 32 && nw <= 64) {
+        const size_t lds = (sizeof(cplx<double>) + 2 * sizeof(cplx<float>)) * nw * (nw + 1);
+        WBMI_HIP_CHECK(ctx, hipFuncSetAttribute((const void*)k_rotate_v, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+        hipLaunchKernelGGL(k_rotate_v, dim3(nk), dim3(ROTV_THREADS), lds, ctx->stream, nw, nch, (const cplx<float>*)U_dev,
+                           (cplx<float>*)X_dev, h[0], h[1], s[0], s[1]);
+        WBMI_LAUNCH_CHECK(ctx);
+        return WBMI_OK;
+    }
     if (prec == WBMI_F32) return launch_rotate<float>(ctx, nk, nw, nch, U_dev, X_dev, h, s);
     if (prec == WBMI_F32_SPLIT) {
         if (nw > 32)  // above one 32 x 32 block per operand: the FP64-arithmetic path

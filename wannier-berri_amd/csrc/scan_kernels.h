@@ -54,7 +54,7 @@
 #define SC_M_NW 64    // dEinv o Off lives in LDS up to this nw (DerOmega / DerMorb: wherever it fits)
 #define SC_LDS_NW 32  // V and A live in LDS up to this nw
 // DerMorb with internal terms only: kernels of their own, for V and W Hermitian to the rounding of FP64
-// sums, and for complex64 channels at nw <= 32, which the rotation forms in FP32 arithmetic
+// sums, and for complex64 channels
 #define SC_DERMORB_IN (WBMI_FORMULA_OMEGAHPLUS + 1000)
 #define SC_DERMORB_IN32 (SC_DERMORB_IN + 1)
 #define SC_DERMORB_EX (SC_DERMORB_IN + 2)  // with external terms, sign = +1, complex128
@@ -424,6 +424,14 @@ __host__ __device__ constexpr int task_nt() {
     return KIND == 0 ? (DM ? 4 : 3) : KIND == 4 ? (DM ? 6 : 3) : KIND == 7 ? 1 : 3;
 }
 
+// V^a_ln of a weight D'^a_nl = m_ln conj(V^a_ln): complex64 channels, whose triangles now and then differ by their
+// rounding at a whole k-point (an element of the transform rounded to either side), read V^a_nl itself
+template <typename T, bool LM, bool ST, bool SA, int NW, typename TS>
+__device__ __attribute__((always_inline)) cplx<double> partner_V(const KCtx<T, LM, ST, SA, NW, TS>& K, int a, int l, int n) {
+    if constexpr (sizeof(T) == 4) return conj(K.Vu(a, n, l));
+    else return K.Vu(a, l, n);
+}
+
 template <int KIND, bool DM, typename T, bool LM, bool ST, bool SA, int NW, typename TS>
 __device__ __attribute__((always_inline)) void formula_task(const Smem& S, const KCtx<T, LM, ST, SA, NW, TS>& K, const TaskCtx& tc_,
                                                            double* acc, int b, int d, int rh, int cb) {
@@ -562,7 +570,7 @@ __device__ __attribute__((always_inline)) void formula_task(const Smem& S, const
 #pragma unroll
                     for (int a = 0; a < 3; ++a) {
                         // -i wD D'_nl, D'_nl = m_ln conj(V_ln)
-                        const cplx<double> va = K.Vu(a, l, n);
+                        const cplx<double> va = partner_V(K, a, l, n);
                         cplx<double> q = (wD * mln) * mk(-va.im, -va.re);
                         if (ex) {
                             q -= dw * conj(K.Au(a, l, n));
@@ -571,7 +579,7 @@ __device__ __attribute__((always_inline)) void formula_task(const Smem& S, const
                         part[bj][a] += q.re * Pm.re - q.im * Pm.im;
                     }
                     if constexpr (DM)
-                        if (in) part[bj][3] += ((mln * conj(K.Vu(c_alpha[s1c], l, n))) * pv).im;  // Re(-i D'^al V^d D'^be)
+                        if (in) part[bj][3] += ((mln * conj(partner_V(K, c_alpha[s1c], l, n))) * pv).im;  // Re(-i D'^al V^d D'^be)
                 } else if constexpr (KIND == 2) {
                     if (!same) {
                         // A'^{bd} - D'^d A''^b
@@ -581,7 +589,7 @@ __device__ __attribute__((always_inline)) void formula_task(const Smem& S, const
                         const cplx<double> Y1 = (-dw * mln) * (pv + z);
 #pragma unroll
                         for (int a = 0; a < 3; ++a) {
-                            const cplx<double> va = K.Vu(a, l, n);
+                            const cplx<double> va = partner_V(K, a, l, n);
                             part[bj][a] += va.re * Y1.re + va.im * Y1.im;  // Re conj(V_ln) Y1
                         }
                     } else if (dm ? tc_.s5 : keep_t4<DM, T>() && S.ge[n] - S.gs[n] > SC_T4_LOOP) {
@@ -959,9 +967,9 @@ struct CutAcc {
 // in both.  U the same with q and n.  So a task, one pair of 16-band blocks and one b, is the products
 //     [P; Q] (n, m) V^b (m, l) over m >= l,   V^b (n, q) [P, Q] (q, l) over q <= n
 // for three d and three a at once: a V and three P elements per 24 MFMAs, which leaves the matrix cores
-// as the bound.  294 k-points at nw = 64, every cut (complex64): 7.5 ms one by one, 0.25 ms together.
-// HERM: V and W are Hermitian to the rounding of the sums.  Otherwise (complex64 from the rotation in FP32
-// arithmetic, whose two triangles differ by their rounding) every term reads the triangle that
+// as the bound.  294 k-points at nw = 64, every cut (complex64): 7.5 ms one by one, 0.4 ms together (0.25 with HERM).
+// HERM: V and W are Hermitian to the rounding of the sums.  Otherwise (complex64: partner_V, and the rotation in
+// FP32 arithmetic, whose two triangles differ by their rounding) every term reads the triangle that
 // formula_task reads, 36 MFMAs: P V with both triangles of V, V P with both of P.
 template <bool HERM, typename T, bool LM, bool ST, bool SA, int NW, typename TS>
 __device__ __attribute__((always_inline)) void eval_dermorb_in(const Smem& S, const KCtx<T, LM, ST, SA, NW, TS>& K, double sign) {
@@ -1003,8 +1011,8 @@ __device__ __attribute__((always_inline)) void eval_dermorb_in(const Smem& S, co
                 cplx<double> P[3], Pu[3];
 #pragma unroll
                 for (int r = 0; r < 3; ++r) {
-                    Pu[r] = FIRST && !HERM ? mk(0.0, 0.0) : (-m) * K.Vu(ax[r], x, y);
-                    P[r] = HERM && !FIRST ? Pu[r] : HERM ? (-m) * K.Vu(ax[r], x, y) : (-m) * conj(K.Vu(ax[r], y, x));
+                    Pu[r] = (-m) * K.Vu(ax[r], x, y);
+                    P[r] = HERM ? Pu[r] : (-m) * conj(K.Vu(ax[r], y, x));
                 }
 #pragma unroll
                 for (int d = 0; d < 3; ++d) {
@@ -1012,7 +1020,7 @@ __device__ __attribute__((always_inline)) void eval_dermorb_in(const Smem& S, co
                     if constexpr (FIRST) f = (HERM ? 0.5 * K.getu(WBMI_ROLE_W + 3 * b + ax[d], x, y) : 0.5 * conj(K.getu(WBMI_ROLE_W + 3 * b + ax[d], y, x))) - f;
 #pragma unroll
                     for (int a = 0; a < 3; ++a) {
-                        const double s = -kap * (P[a] * conj(f)).im - (Z.get(a, v) * conj(P[d])).re;
+                        const double s = -kap * (Pu[a] * conj(f)).im - (Z.get(a, v) * conj(P[d])).re;
                         if (a != 0) {
                             const double e = pair_sign(a, 0) * s;
                             o[(third_index(a, 0) - 1) * 3 + d][v] += ok ? e : 0.0;
@@ -1021,7 +1029,7 @@ __device__ __attribute__((always_inline)) void eval_dermorb_in(const Smem& S, co
                             const bool pos = pair_sign(a, d) > 0.0;
                             const cplx<double> h = G[pos ? 0 : NS - 1].get(d, v);
                             const double hw = FIRST ? -2.0 : -2.0 * sign;
-                            const double e = pair_sign(a, d) * (s + hw * ((!FIRST && pos ? Pu[a] : P[a]) * conj(h)).im);
+                            const double e = pair_sign(a, d) * (s + hw * ((pos ? Pu[a] : P[a]) * conj(h)).im);
                             const int c = third_index(a, d);
                             o[c == 0 ? 6 : (c - 1) * 3][v] += ok ? e : 0.0;
                         }
@@ -1043,10 +1051,10 @@ __device__ __attribute__((always_inline)) void eval_dermorb_in(const Smem& S, co
             const double mm = K.m(n, m), kap = -mm * (2.0 * sign * En + 2.0 * S.E[m]);
 #pragma unroll
             for (int r = 0; r < 3; ++r) {
-                const cplx<double> P = (-mm) * conj(K.Vu(ax[r], m, n));
+                const cplx<double> P = (-mm) * conj(K.Vu(ax[r], m, n)), Pu = HERM ? P : (-mm) * K.Vu(ax[r], n, m);
                 G[0].add(r, P, vu);
-                if constexpr (!HERM) G[1].add(r, P, vl);
-                Z.add(r, mk(-kap * P.im, kap * P.re), vl);
+                if constexpr (!HERM) G[1].add(r, Pu, vl);
+                Z.add(r, mk(-kap * Pu.im, kap * Pu.re), vl);
             }
         }
         add_pairs(std::true_type{});
@@ -1063,7 +1071,7 @@ __device__ __attribute__((always_inline)) void eval_dermorb_in(const Smem& S, co
                 const cplx<double> Pu = (-mm) * K.Vu(ax[r], q, l), P = HERM ? Pu : (-mm) * conj(K.Vu(ax[r], l, q));
                 G[0].add(r, vu, P);
                 if constexpr (!HERM) G[1].add(r, vl, Pu);
-                Z.add(r, vl, mk(-kap * P.im, kap * P.re));
+                Z.add(r, vl, mk(-kap * Pu.im, kap * Pu.re));
             }
         }
         add_pairs(std::false_type{});
@@ -2197,10 +2205,8 @@ static int launch_scan(wbmi_ctx* ctx, int nk, const ScanArgs& a, const double* E
     if constexpr (F == WBMI_FORMULA_MORB_HPM && MODE != 2) {
         return launch_scan_t<T, F, false, false, MODE, 0, 256>(ctx, nk, a, E, X, hist);
     } else if constexpr (SC_IS_DERMORB_CUTS(F)) {
-        // (complex64 channels of the sizes that are staged go to SC_DERMORB_IN32)
-        if constexpr (sizeof(T) == 8 || F == SC_DERMORB_IN32)
-            if (a.stage_va && smem_offsets(a.nw, true, true, a.p.external_terms, MODE == 1, sizeof(cplx<T>)).total <= SC_LDS / 2)
-                return launch_scan_t<T, F, true, true, MODE, 0, 256>(ctx, nk, a, E, X, hist);
+        if (a.stage_va && smem_offsets(a.nw, true, true, a.p.external_terms, MODE == 1, sizeof(cplx<T>)).total <= SC_LDS / 2)
+            return launch_scan_t<T, F, true, true, MODE, 0, 256>(ctx, nk, a, E, X, hist);
         if (smem_offsets(a.nw, true, false, false, MODE == 1, sizeof(cplx<T>)).total <= SC_LDS / 2)
             return launch_scan_t<T, F, true, false, MODE, 0, 256>(ctx, nk, a, E, X, hist);
         return launch_scan_t<T, F, MODE == 0, false, MODE, 0, 512>(ctx, nk, a, E, X, hist);
@@ -2254,9 +2260,7 @@ static int dispatch_scan(wbmi_ctx* ctx, int nk, const ScanArgs& a, const double*
         case WBMI_FORMULA_DERMORB:
             if constexpr (MODE != 2)
                 if (!a.p.external_terms) {
-                    if constexpr (sizeof(T) == 4)
-                        if (a.nw <= 32) return launch_scan<T, SC_DERMORB_IN32, MODE>(ctx, nk, a, E, X, hist);
-                    return launch_scan<T, SC_DERMORB_IN, MODE>(ctx, nk, a, E, X, hist);
+                    return launch_scan<T, sizeof(T) == 4 ? SC_DERMORB_IN32 : SC_DERMORB_IN, MODE>(ctx, nk, a, E, X, hist);
                 }
             if constexpr (MODE != 2 && sizeof(T) == 8)
                 if (a.p.sign == 1) return launch_scan<T, SC_DERMORB_EX, MODE>(ctx, nk, a, E, X, hist);

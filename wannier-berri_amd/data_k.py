@@ -462,7 +462,7 @@ class Data_K:
                     herm[sl:sl + CHANNEL_NCOMP[key]] = 1
             if ("Ham", 0) in slots:
                 skip[slots[("Ham", 0)]] = 1
-            if self.split_rotation and nw <= 32:   # above, both kinds run the FP64-arithmetic kernel: one launch
+            if self.split_rotation:
                 # the velocity in FP64 arithmetic (its elements between close bands enter the
                 # Berry curvature through 1 / (E_n - E_m)^2), the rest on split-fp16 products
                 vel = np.zeros(nch, dtype=np.int32)
