@@ -1215,7 +1215,7 @@ __global__ void __launch_bounds__(OAG_THREADS) k_eigh_refine_g(int n, const cplx
     for (int i = tid; i < n; i += OAG_THREADS) Eout[k * n + rank[i]] = lam[i];
 }
 
-// Scratch of wbmi_eigh_noalloc: the per-k refinement workspace (X, T, S/E, R for
+// Scratch of wbmi_eigh_noalloc: the per-k refinement workspace (X, T, S/E, R;
 // 44 < nw <= 128) in a file-scope device array, so that callers that cannot allocate
 // (graph capture, serving loops) get the refined solver without a workspace.  Each GPU
 // holds its own copy for the life of the process; calls on one GPU share it (their
@@ -1230,7 +1230,7 @@ int wbmi_eigh_scratch_init(void** ptr) {
     return hipGetSymbolAddress(ptr, HIP_SYMBOL(scratch)) == hipSuccess && *ptr ? 0 : 1;
 }
 
-// bytes of global workspace wbmi_eigh needs (refinement for nw > 44)
+// bytes of global workspace wbmi_eigh asks for (refinement for nw > 44; used above 64)
 static size_t eigh_work_bytes(int nk, int nw, int refine) {
     return (refine && nw > 44) ? sizeof(cplx<double>) * 4 * (size_t)nw * nw * nk : 0;
 }
