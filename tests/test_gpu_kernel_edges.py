@@ -197,6 +197,80 @@ def test_scan_diagonal_traces(nw, precision, kramers):
         assert err <= (1e-9 if precision == "fp64" else 2e-5) * scale, name
 
 
+def _given_channels(E, V, W):
+    """The oracle's K-block on given band-basis matrices V [k, n, n, 3], W [k, n, n, 3, 3]."""
+    from oracle import wb_oracle as O
+
+    class Given(O.OracleDataK):
+        E_K = E
+        force_internal_terms_only = False
+
+        def __init__(self):
+            self._cov = {}
+
+        def Xbar(self, name, der=0):
+            return {1: V, 2: W}[der]
+    return Given()
+
+
+@pytest.mark.parametrize("nw", [7, 16, 32, 33, 70])
+def test_scan_velocity_off_its_mirror(ctx, nw):
+    """DerOmega and DerMorb (internal terms; with them the gyrotropic tensor and the Berry-curvature dipole) of
+    complex64 channels whose velocity is Hermitian to storage rounding only: one element of the matrix before
+    its rotation is off its mirror, so every element after it is, the diagonal among them.  Every band a
+    group of its own, two of them 4e-3 apart; against the oracle's formulas on the same stored matrices."""
+    import torch
+    from oracle import wb_oracle as O
+    from wannierberri_amd import _lib
+    rng = np.random.default_rng(nw)
+    nk, dEF = 2, 2e-3
+    step = np.full((nk, nw), 125)
+    step[:, nw // 2] = 2
+    level = np.cumsum(step + (step > 2) * rng.integers(0, 9, (nk, nw)), axis=1)   # the bin of each band
+    E = (level - 0.5) * dEF
+    nbin = int(level.max()) + 2
+    def herm(n):
+        x = rng.standard_normal((nk, n, nw, nw)) + 1j * rng.standard_normal((nk, n, nw, nw))
+        return (0.5 * (x + x.conj().swapaxes(2, 3))).astype(np.complex64).astype(complex)
+    U = np.linalg.qr(rng.standard_normal((nk, nw, nw)) + 1j * rng.standard_normal((nk, nw, nw)))[0]
+    V, W = herm(3), herm(9)
+    W = 0.5 * (W + W[:, [0, 3, 6, 1, 4, 7, 2, 5, 8]])
+    V[:, :, 1, 0] += 6e-8
+    X = np.concatenate([V, W], axis=1)
+    X = (U.conj().swapaxes(1, 2)[:, None] @ X @ U[:, None]).astype(np.complex64)
+    Xd, Ed = torch.from_numpy(X).cuda(), torch.from_numpy(E).cuda()
+    X = np.moveaxis(X.astype(complex), 1, 3)
+    d = _given_channels(E, X[..., :3], X[..., 3:].reshape(nk, nw, nw, 3, 3))
+    for formula, f in ((_lib.FORMULA_DEROMEGA, O.DerOmega(d, external_terms=False)),
+                       (_lib.FORMULA_DERMORB, O.DerMorb(d, sign=1, external_terms=False))):
+        p = _lib.ScanParams()
+        p.formula, p.sign, p.internal_terms, p.external_terms, p.fder = formula, 1, 1, 0, 0
+        p.nEF_extra, p.EFmin, p.EFmax, p.dEF, p.degen_thresh = nbin, 0.0, (nbin - 1) * dEF, dEF, 1e-4
+        for i in range(_lib.NROLES):
+            p.ch[i] = i if i < 12 else -1
+        hist = torch.zeros((nbin, 9), dtype=torch.float64, device="cuda")
+        ctx.static_scan(Ed, Xd, _lib.WBMI_F32, p, 1.0, hist)
+        ref = np.zeros((nbin, 9))
+        for ik in range(nk):
+            bands = np.arange(nw)
+            cuts = np.zeros((nw + 1, 9))
+            for c in range(1, nw + 1):
+                # tr (Omega V + V Omega) / 2, Omega = s + s^+, is formed as 2 Re tr s V (V read as Hermitian here)
+                D, v = d.D_H[ik], d.Xbar("Ham", 1)[ik, :c, :c]
+                s = -1j * np.einsum("mlc,lnc->mnc", D[:c, c:][..., [1, 2, 0]], D[c:, :c][..., [2, 0, 1]])
+                herm = np.einsum("mnc,nmd->cd", s, v) - np.einsum("nmc,nmd->cd", s.conj(), v)
+                cuts[c] = (f.trace(ik, bands[:c], bands[c:]) + herm.real).reshape(9)
+            for n in range(nw):
+                value = cuts[n + 1] - cuts[n] if formula == _lib.FORMULA_DERMORB else \
+                    f.trace(ik, bands[n:n + 1], np.delete(bands, n)).reshape(9)
+                ref[level[ik, n]] += value
+        err = np.abs(hist.cpu().numpy() - ref).max() / np.abs(ref).max()
+        print(f"test_scan_velocity_off_its_mirror nw={nw} formula {formula}: {err:.1e}", flush=True)
+        # about 3 nw roundings of terms of the size of the largest (5e-14 at nw = 70); the energies' differences
+        # are exact.  A real V_nn is off by 1e-9 .. 1e-8: Im V_nn / (V_nn - V_ll)
+        assert err < 1e-12, formula
+
+
 @pytest.mark.parametrize("nw", [1, 2, 15, 16, 17, 31, 32, 33, 48, 49, 64, 65, 80, 81, 97, 112, 113, 128])
 def test_rotate_sizes(ctx, nw):
     """One size at each edge of the rotation's 16-row blocks, flagged (Hermitian part), plain and

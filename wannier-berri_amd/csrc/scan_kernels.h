@@ -561,9 +561,10 @@ __device__ __attribute__((always_inline)) void formula_task(const Smem& S, const
                 if constexpr (KIND == 0) {
                     if (same) continue;
                     // W^{bd}_ln / 2 - (D'^d V''^b)_ln, with D'_xy = -m_xy V_xy and m_nl = -m_ln
+                    // (V_nn is real to its rounding only; its imaginary part enters as V_nn - V_ll does, which may be as small)
                     const double mln = K.m(l, n);
                     cplx<double> z = 0.5 * gz[bj][v];
-                    if (!big) z += (mln * K.Vu(b, n, n).re) * K.Vu(d, l, n);
+                    if (!big) z += mln * (K.Vu(b, n, n) * K.Vu(d, l, n));
                     if constexpr (DM) z += P2.get(bj, v);
                     const cplx<double> Pm = (-mln) * (pv + z);
                     const double wD = in ? (dm ? dw + 2.0 * K.E[l] : dw) : 0.0;
