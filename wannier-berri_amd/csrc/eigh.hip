@@ -15,6 +15,7 @@
 #include <type_traits>
 
 #include "mfma_c64.h"
+#include "round_flag.h"
 #include "wbmi_common.h"
 
 // update items per lane per batch (loads of a batch are issued together)
@@ -299,7 +300,7 @@ __global__ void __launch_bounds__(64 * NWAVE) k_eigh_jacobi_b(int nw, const cplx
     cplx<T>* A = (cplx<T>*)(prm + np);
     cplx<T>* V = A + n * ld;
     int* rank = (int*)(V + n * ld);
-    int* flags = rank + n;  // round flag, double-buffered by round parity (four-wave workgroups)
+    int* flags = rank + n;  // round flag (workgroups of several waves): RoundFlag
     const int tid = threadIdx.x;
     const int64_t k = blockIdx.x;
     const cplx<Tin>* Hk = H + k * Hstride;
@@ -380,6 +381,7 @@ __global__ void __launch_bounds__(64 * NWAVE) k_eigh_jacobi_b(int nw, const cplx
         const int b = tid + NTH * u;
         vij[u] = (b / n) | (b % n) * ld << 16;  // pair, offset of the row
     }
+    RoundFlag flag;
     for (int sweep = 0; sweep < max_sweeps; ++sweep) {
         bool swept = false;
         for (int r = 0; r < n - 1; ++r) {
@@ -396,13 +398,13 @@ __global__ void __launch_bounds__(64 * NWAVE) k_eigh_jacobi_b(int nw, const cplx
                 any = __any(rot);  // the workgroup is one wavefront: uniform over it
                 __syncthreads();
             } else {
-                // the pairs belong to wave 0; the flag's other buffer is read by no one any more
+                // the pairs belong to wave 0
                 if (tid < 64) {
                     const bool w = __any(rot);
-                    if (tid == 0) flags[r & 1] = w;
+                    if (tid == 0) flag.put(flags, w);
                 }
                 __syncthreads();
-                any = flags[r & 1] != 0;
+                any = flag.take(flags) != 0;
             }
             if (!any) continue;
             swept = true;
@@ -528,7 +530,7 @@ __global__ void __launch_bounds__(JREG_THREADS) k_eigh_jacobi_reg(int nw, const 
     float4* prm = (float4*)smem;
     cplx<T>* A = (cplx<T>*)(prm + np);
     int* rank = (int*)(A + n * ld);
-    int* flags = rank + n;  // round flag, double-buffered by round parity
+    int* flags = rank + n;  // RoundFlag
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int64_t k = blockIdx.x;
     const cplx<Tin>* Hk = H + k * Hstride;
@@ -559,6 +561,7 @@ __global__ void __launch_bounds__(JREG_THREADS) k_eigh_jacobi_reg(int nw, const 
         bj[u] = b % np;
     }
     __syncthreads();
+    RoundFlag flag;
     for (int sweep = 0; sweep < max_sweeps; ++sweep) {
         bool swept = false;
         for (int r = 0; r < n - 1; ++r) {
@@ -572,10 +575,10 @@ __global__ void __launch_bounds__(JREG_THREADS) k_eigh_jacobi_reg(int nw, const 
                     prm[tid] = make_float4(c, sc, ss, __int_as_float(p | (q << 16)));
                 }
                 const bool w = __any(rot);
-                if (tid == 0) flags[r & 1] = w;
+                if (tid == 0) flag.put(flags, w);
             }
             __syncthreads();
-            const bool any = flags[r & 1] != 0;
+            const bool any = flag.take(flags) != 0;
             if (any) {
                 swept = true;
 #pragma unroll
