@@ -197,38 +197,17 @@ def test_scan_diagonal_traces(nw, precision, kramers):
         assert err <= (1e-9 if precision == "fp64" else 2e-5) * scale, name
 
 
-def _given_channels(E, V, W):
-    """The oracle's K-block on given band-basis matrices V [k, n, n, 3], W [k, n, n, 3, 3]."""
+def _off_mirror(nw, external):
+    """Complex64 channels of two k-points with V Hermitian to storage rounding only: one element of the
+    matrix before its rotation is off its mirror, so every element after it is, the diagonal among them.  Every
+    band a group of its own in a bin of its own, two bands 4e-3 apart.  Returns the channels (V, W; A, A',
+    rotA, rotA'), E, bin width, bins, and the oracle's K-block on the same stored matrices."""
     from oracle import wb_oracle as O
-
-    class Given(O.OracleDataK):
-        E_K = E
-        force_internal_terms_only = False
-
-        def __init__(self):
-            self._cov = {}
-
-        def Xbar(self, name, der=0):
-            return {1: V, 2: W}[der]
-    return Given()
-
-
-@pytest.mark.parametrize("nw", [7, 16, 32, 33, 70])
-def test_scan_velocity_off_its_mirror(ctx, nw):
-    """DerOmega and DerMorb (internal terms; with them the gyrotropic tensor and the Berry-curvature dipole) of
-    complex64 channels whose velocity is Hermitian to storage rounding only: one element of the matrix before
-    its rotation is off its mirror, so every element after it is, the diagonal among them.  Every band a
-    group of its own, two of them 4e-3 apart; against the oracle's formulas on the same stored matrices."""
-    import torch
-    from oracle import wb_oracle as O
-    from wannierberri_amd import _lib
     rng = np.random.default_rng(nw)
     nk, dEF = 2, 2e-3
     step = np.full((nk, nw), 125)
     step[:, nw // 2] = 2
     level = np.cumsum(step + (step > 2) * rng.integers(0, 9, (nk, nw)), axis=1)   # the bin of each band
-    E = (level - 0.5) * dEF
-    nbin = int(level.max()) + 2
     def herm(n):
         x = rng.standard_normal((nk, n, nw, nw)) + 1j * rng.standard_normal((nk, n, nw, nw))
         return (0.5 * (x + x.conj().swapaxes(2, 3))).astype(np.complex64).astype(complex)
@@ -238,20 +217,53 @@ def test_scan_velocity_off_its_mirror(ctx, nw):
     V[:, :, 1, 0] += 6e-8
     X = np.concatenate([V, W], axis=1)
     X = (U.conj().swapaxes(1, 2)[:, None] @ X @ U[:, None]).astype(np.complex64)
-    Xd, Ed = torch.from_numpy(X).cuda(), torch.from_numpy(E).cuda()
-    X = np.moveaxis(X.astype(complex), 1, 3)
-    d = _given_channels(E, X[..., :3], X[..., 3:].reshape(nk, nw, nw, 3, 3))
+    if external:
+        X = np.concatenate([X, herm(24).astype(np.complex64)], axis=1)
+    E = (level - 0.5) * dEF
+    x = np.moveaxis(X.astype(complex), 1, 3)
+    bar = {("Ham", 1): x[..., :3], ("Ham", 2): x[..., 3:12].reshape(nk, nw, nw, 3, 3)}
+    if external:
+        bar.update({("AA", 0): x[..., 12:15], ("AA", 1): x[..., 15:24].reshape(nk, nw, nw, 3, 3),
+                    ("rotAA", 0): x[..., 24:27], ("rotAA", 1): x[..., 27:].reshape(nk, nw, nw, 3, 3)})
+
+    class Given(O.OracleDataK):
+        E_K = E
+        force_internal_terms_only = False
+
+        def __init__(self):
+            self._cov = {}
+
+        def Xbar(self, name, der=0):
+            return bar[name, der]
+    return X, E, dEF, level, Given()
+
+
+def _scan_bins(ctx, X, E, dEF, level, formula, external):
+    import torch
+    from wannierberri_amd import _lib
+    nbin = int(level.max()) + 2
+    p = _lib.ScanParams()
+    p.formula, p.sign, p.internal_terms, p.external_terms, p.fder = formula, 1, 1, int(external), 0
+    p.nEF_extra, p.EFmin, p.EFmax, p.dEF, p.degen_thresh = nbin, 0.0, (nbin - 1) * dEF, dEF, 1e-4
+    for i in range(_lib.NROLES):
+        p.ch[i] = i if i < X.shape[1] else -1   # V, W, A, A', rotA, rotA' have the first roles in this order
+    hist = torch.zeros((nbin, 9), dtype=torch.float64, device="cuda")
+    ctx.static_scan(torch.from_numpy(E).cuda(), torch.from_numpy(X).cuda(), _lib.WBMI_F32, p, 1.0, hist)
+    return hist.cpu().numpy()
+
+
+@pytest.mark.parametrize("nw", [7, 16, 32, 33, 70])
+def test_scan_velocity_off_its_mirror(ctx, nw):
+    """DerOmega and DerMorb (internal terms; with them the gyrotropic tensor and the Berry-curvature dipole)
+    against the oracle's formulas on the same stored matrices."""
+    from oracle import wb_oracle as O
+    from wannierberri_amd import _lib
+    X, E, dEF, level, d = _off_mirror(nw, False)
     for formula, f in ((_lib.FORMULA_DEROMEGA, O.DerOmega(d, external_terms=False)),
                        (_lib.FORMULA_DERMORB, O.DerMorb(d, sign=1, external_terms=False))):
-        p = _lib.ScanParams()
-        p.formula, p.sign, p.internal_terms, p.external_terms, p.fder = formula, 1, 1, 0, 0
-        p.nEF_extra, p.EFmin, p.EFmax, p.dEF, p.degen_thresh = nbin, 0.0, (nbin - 1) * dEF, dEF, 1e-4
-        for i in range(_lib.NROLES):
-            p.ch[i] = i if i < 12 else -1
-        hist = torch.zeros((nbin, 9), dtype=torch.float64, device="cuda")
-        ctx.static_scan(Ed, Xd, _lib.WBMI_F32, p, 1.0, hist)
-        ref = np.zeros((nbin, 9))
-        for ik in range(nk):
+        hist = _scan_bins(ctx, X, E, dEF, level, formula, False)
+        ref = np.zeros_like(hist)
+        for ik in range(len(E)):
             bands = np.arange(nw)
             cuts = np.zeros((nw + 1, 9))
             for c in range(1, nw + 1):
@@ -264,11 +276,46 @@ def test_scan_velocity_off_its_mirror(ctx, nw):
                 value = cuts[n + 1] - cuts[n] if formula == _lib.FORMULA_DERMORB else \
                     f.trace(ik, bands[n:n + 1], np.delete(bands, n)).reshape(9)
                 ref[level[ik, n]] += value
-        err = np.abs(hist.cpu().numpy() - ref).max() / np.abs(ref).max()
+        err = np.abs(hist - ref).max() / np.abs(ref).max()
         print(f"test_scan_velocity_off_its_mirror nw={nw} formula {formula}: {err:.1e}", flush=True)
         # about 3 nw roundings of terms of the size of the largest (5e-14 at nw = 70); the energies' differences
         # are exact.  A real V_nn is off by 1e-9 .. 1e-8: Im V_nn / (V_nn - V_ll)
         assert err < 1e-12, formula
+
+
+@pytest.mark.parametrize("nw", [7, 16, 32, 33, 70])
+def test_scan_velocity_off_its_mirror_external(ctx, nw):
+    """DerOmega with external terms on such channels.  What the kernel reads as Hermitian is so in the reference:
+    the product V D' of dD.nl = -(dD.ln)^+ (its within-group part has V_nn V_nl as stored), and the real part
+    of dO.nn."""
+    from oracle import wb_oracle as O
+    from wannierberri_amd import _lib
+    X, E, dEF, level, d = _off_mirror(nw, True)
+    f = O.DerOmega(d)
+    V, W, Dh, m = d.Xbar("Ham", 1), d.Xbar("Ham", 2), d.D_H, d.dEig_inv
+
+    class DerD(O.DerDcov):
+        def nl(self, ik, inn, out):   # one band n inside
+            n = inn[0]
+            pv = np.einsum("lpb,pd->lbd", V[ik][out][:, out], Dh[ik][out, n])
+            own = np.einsum("b,ld->lbd", V[ik][n, n], V[ik][n, out]) * m[ik][out, n][:, None, None]
+            s = (W[ik][out, n] + pv + pv.swapaxes(1, 2)).conj() + own + own.swapaxes(1, 2)
+            return (m[ik][out, n][:, None, None] * s)[None]
+
+    class DerO:
+        def nn(self, ik, inn, out):
+            n = inn[0]
+            o, do = d.Xbar("rotAA")[ik], d.Xbar("rotAA", 1)[ik]
+            return (do[n, n] + 2 * np.einsum("lc,ld->cd", o[out, n].conj(), Dh[ik][out, n])).real[None, None]
+    f.dD, f.dO = DerD(d), DerO()
+    hist = _scan_bins(ctx, X, E, dEF, level, _lib.FORMULA_DEROMEGA, True)
+    ref = np.zeros_like(hist)
+    for ik in range(len(E)):
+        for n in range(nw):
+            ref[level[ik, n]] += f.trace(ik, np.array([n]), np.delete(np.arange(nw), n)).reshape(9)
+    err = np.abs(hist - ref).max() / np.abs(ref).max()
+    print(f"test_scan_velocity_off_its_mirror_external nw={nw}: {err:.1e}", flush=True)
+    assert err < 1e-12   # as above
 
 
 @pytest.mark.parametrize("nw", [1, 2, 15, 16, 17, 31, 32, 33, 48, 49, 64, 65, 80, 81, 97, 112, 113, 128])

@@ -567,6 +567,10 @@ __device__ __attribute__((always_inline)) void formula_task(const Smem& S, const
                     if (!big) z += mln * (K.Vu(b, n, n) * K.Vu(d, l, n));
                     if constexpr (DM) z += P2.get(bj, v);
                     const cplx<double> Pm = (-mln) * (pv + z);
+                    // -conj dD.nl: its within-group part from V's other triangle, as stored, in groups of one band
+                    cplx<double> Pn = Pm;
+                    if constexpr (sizeof(T) == 4)
+                        if (ex && !big) Pn = (-mln) * (pv + 0.5 * gz[bj][v] + mln * conj(K.Vu(b, n, n) * K.Vu(d, n, l)));
                     const double wD = in ? (dm ? dw + 2.0 * K.E[l] : dw) : 0.0;
 #pragma unroll
                     for (int a = 0; a < 3; ++a) {
@@ -574,7 +578,8 @@ __device__ __attribute__((always_inline)) void formula_task(const Smem& S, const
                         const cplx<double> va = partner_V(K, a, l, n);
                         cplx<double> q = (wD * mln) * mk(-va.im, -va.re);
                         if (ex) {
-                            q -= dw * conj(K.Au(a, l, n));
+                            const cplx<double> A = K.Au(a, l, n);
+                            part[bj][a] -= dw * (A.re * Pn.re + A.im * Pn.im);
                             if (dm) q -= 2.0 * conj(K.getu(WBMI_ROLE_B + a, l, n));
                         }
                         part[bj][a] += q.re * Pm.re - q.im * Pm.im;
