@@ -343,6 +343,34 @@ def test_rotate_sizes(ctx, nw):
         assert np.abs(got - ref).max() < bound
 
 
+@pytest.mark.parametrize("nw", [2, 15, 16, 17, 29, 32])
+def test_rotate_order_of_sums(ctx, nw):
+    """complex64 channels: at most 32 bands are summed in the order in which more than 64 are (the summed index,
+    four at a time), so that a rounding does not depend on the kernel that a size takes.  The matrices
+    stand alone and in the corner of 70 x 70 ones; sums that cancel to 1e-10 of their terms show the order."""
+    import torch
+    from wannierberri_amd import _lib
+    rng = np.random.default_rng(nw)
+    nk, nch, big = 2, 5, 70
+    def rand(*shape):
+        return (rng.standard_normal(shape) + 1j * rng.standard_normal(shape)).astype(np.complex64)
+    U = rand(nk, nw, nw)
+    X = 1e10 * rand(nk, nch, nw, nw)
+    pick = rng.permutation(nw)   # the terms of pairs (i, j) of the summed index cancel in the products
+    for i, j in zip(pick[0::2], pick[1::2]):
+        U[:, j] = U[:, i]
+        X[:, :, :, j] = -X[:, :, :, i]
+    X[:, :, :, pick[-1]] = rand(nk, nch, nw)
+    Xb, Ub = np.zeros((nk, nch, big, big), np.complex64), np.zeros((nk, big, big), np.complex64)
+    Xb[:, :, :nw, :nw], Ub[:, :nw, :nw] = X, U
+    out = []
+    for x, u in ((X, U), (Xb, Ub)):
+        xd = torch.from_numpy(x.copy()).cuda()
+        ctx.rotate(torch.from_numpy(u).cuda(), xd, None, None, _lib.WBMI_F32)
+        out.append(xd.cpu().numpy()[:, :, :nw, :nw])
+    assert np.array_equal(out[0], out[1])
+
+
 @pytest.mark.parametrize("nk,nw,extra", [(1, 1, 0), (7, 3, 0), (17, 5, 1), (33, 4, 2), (130, 7, 1)])
 def test_klist_pairs(ctx, nk, nw, extra):
     """R -> k with the R-vectors in pairs against the single-vector form and the plain sum: lists with

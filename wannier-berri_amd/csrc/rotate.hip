@@ -67,7 +67,7 @@ __device__ inline void rot_cmac(wbmi_v4d& re, wbmi_v4d& im, cplx<double> a, cplx
 // U (FP64) in LDS, shared by the waves of a workgroup; steps past nw are left out.
 // Bound at nw = 32: the channels' traffic (read and written once) next to the products, which take
 // as long.  Measured against one LDS tile per wave (one workgroup of 8 waves a CU): 4096 k-points of 36
-// channels at nw = 32 1.72 -> 1.50 ms complex128, 1.57 -> 1.41 complex64; 2500 of 9 at nw = 2 67 -> 19 us.
+// channels at nw = 32 1.72 -> 1.50 ms complex128, 1.57 -> 1.40 complex64; 2500 of 9 at nw = 2 67 -> 19 us.
 // (Registers: 8 waves a CU without spills at complex128, 12 at complex64.)
 #define ROTR_WAVES 4
 template <typename T, int NB>
@@ -76,7 +76,9 @@ __global__ void __launch_bounds__(64 * ROTR_WAVES, NB == 1 ? 4 : sizeof(T) == 8 
                                                                              uint64_t herm_hi, uint64_t skip_lo,
                                                                              uint64_t skip_hi) {
     constexpr int NS = 4 * NB, LD = 16 * NB + 1;  // steps of the summed index, LDS row stride
-    constexpr int J = sizeof(T) == 8 ? 2 : 4;
+    // complex64: in the order of the summed index, as above 64 bands, so that one element in 1e8 is not rounded the other
+    // way by the kernel a size takes (J = 4 was no faster: 1.44 ms against 1.40 for 36 channels of 4096 k-points, nw = 32)
+    constexpr int J = sizeof(T) == 8 ? 2 : 1;
     __shared__ cplx<double> sU[16 * NB * LD];
     const int lane = threadIdx.x & 63, li = lane & 15, g = lane >> 4;
     const int nwave = ROTR_WAVES * (int)gridDim.y, wave = (int)(threadIdx.x >> 6) + ROTR_WAVES * (int)blockIdx.y;
