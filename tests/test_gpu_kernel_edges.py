@@ -71,6 +71,28 @@ def test_eigh_refine_blocks(ctx, nw, gap):
     assert np.abs(u.conj().swapaxes(1, 2) @ u - np.eye(nw)).max() < 8 * EPS * nw
 
 
+@pytest.mark.parametrize("nw", [33, 40, 64])
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+def test_eigh_repeats(ctx, nw, prec):
+    """Energies of 33 to 64 bands are the same bits in every call (their norms are summed by three or four
+    waves)."""
+    import torch
+    from wannierberri_amd import _lib
+    p, cd = ((_lib.WBMI_F64, torch.complex128) if prec == "fp64" else (_lib.WBMI_F32, torch.complex64))
+    nk = 6000 if nw < 64 else 4000
+    H = torch.from_numpy(_hermitian(np.random.default_rng(nw), nk, nw)).cuda()
+    first = None
+    for _ in range(25):
+        E = torch.empty((nk, nw), dtype=torch.float64, device="cuda")
+        U = torch.empty((nk, nw, nw), dtype=cd, device="cuda")
+        if prec == "fp64":
+            ctx.eigh(H, nw * nw, E, U, p, nw, refine=16)
+        else:
+            ctx.eigh(None, nw * nw, E, U, p, nw, refine=16, H64=H)
+        first = E if first is None else first
+        assert torch.equal(E, first)
+
+
 @pytest.mark.parametrize("nw", [16, 17, 32, 33, 50, 64])
 @pytest.mark.parametrize("prec", ["fp64", "fp32"])
 def test_eigh_waves_per_k(ctx, nw, prec):

@@ -811,8 +811,8 @@ k_eigh_refine(int nw, const cplx<double>* __restrict__ H64, int64_t Hstride, dou
     cplx<double>* sT = sX + nw * ld;                        // A X, then E
     cplx<double>* sA = sT + nw * ld;                        // A (for the whole solve)
     double* lam = (double*)(ALDS ? sA + nw * ld : sA);
-    double* den = lam + nw;                                 // squared norms of the columns
-    double* red2 = den + nw;                                // two sets, steps in turn:
+    double* den = lam + nw;                                 // squared norms of the columns' parts, [NB][nw]
+    double* red2 = den + NB * nw;                           // two sets, steps in turn:
     // [0] ||S-D||^2, [1] ||R||^2, [2] max|lam|, [3] ||E||^2
     char* cjs = (char*)(red2 + 8);                          // cluster_jacobi scratch
     int* rank = (int*)(cjs + cj_lds(nw));
@@ -911,7 +911,6 @@ k_eigh_refine(int nw, const cplx<double>* __restrict__ H64, int64_t Hstride, dou
             sX[row(v) * ld + c] = mk((double)u.re, (double)u.im);
             if constexpr (ALDS) sA[row(v) * ld + c] = herm(row(v), c);
         }
-    for (int i = tid; i < nw; i += NTH) den[i] = 0.0;
     double scale = 0.0;
     for (int it = 0; it < iters; ++it) {
         double* red = red2 + 4 * (it & 1);
@@ -1004,7 +1003,7 @@ k_eigh_refine(int nw, const cplx<double>* __restrict__ H64, int64_t Hstride, dou
         }
     x2 += __shfl_xor(x2, 16);
     x2 += __shfl_xor(x2, 32);
-    if (lk == 0 && c < nw) atomicAdd(&den[c], x2);
+    if (lk == 0 && c < nw) den[r0 / 16 * nw + c] = x2;  // summed in a fixed order: energies repeat bit for bit
     __syncthreads();
     const double theta = tol, floor_abs = 64.0 * DBL_EPSILON * scale;
     int mixed = 0;
@@ -1024,12 +1023,18 @@ k_eigh_refine(int nw, const cplx<double>* __restrict__ H64, int64_t Hstride, dou
                 d += x.re * x.re + x.im * x.im;
             }
             den[i] = d;
+            for (int q = 1; q < NB; ++q) den[q * nw + i] = 0.0;
             lam[i] = sT[i * ld + i].re;
         }
         __syncthreads();
     }
     // eigenvalues: Rayleigh quotients x_c^+ A x_c / x_c^+ x_c = S_cc / x_c^+ x_c
-    for (int i = tid; i < nw; i += NTH) lam[i] /= den[i];
+    for (int i = tid; i < nw; i += NTH) {
+        double d = den[i];
+#pragma unroll
+        for (int q = 1; q < NB; ++q) d += den[q * nw + i];
+        lam[i] /= d;
+    }
     __syncthreads();
     // ascending order (ties by index)
     for (int i = tid; i < nw; i += NTH) {
@@ -1291,7 +1296,7 @@ static int jacobi_f32_of_f64(wbmi_ctx* ctx, int nk, int nw, const cplx<double>* 
 template <typename TU, int NB>
 static int launch_refine(wbmi_ctx* ctx, int nk, int nw, const cplx<double>* H64, int64_t Hstride, double* E,
                          cplx<TU>* U, int steps, double tol) {
-    const size_t lds = (NB <= 3 ? 3 : 2) * sizeof(cplx<double>) * nw * (nw + 1) + sizeof(double) * (2 * nw + 8) +
+    const size_t lds = (NB <= 3 ? 3 : 2) * sizeof(cplx<double>) * nw * (nw + 1) + sizeof(double) * ((1 + NB) * nw + 8) +
                        cj_lds(nw) + sizeof(int) * nw + 16;
     auto launch = [&](auto split) -> int {
         auto kernel = k_eigh_refine<TU, NB, decltype(split)::value>;
