@@ -427,6 +427,33 @@ def test_klist_pairs(ctx, nk, nw, extra):
                 assert err < bound + (1.2e-7 * np.abs(ref).max() if prec == _lib.WBMI_F32 else 0), (tile, p is None)
 
 
+def test_klist_pairs_on_demand(ctx, monkeypatch):
+    """A grid never forms the pairs (R, -R); the first k-list does, once; while a graph capture is the first,
+    the transform takes every R-vector alone."""
+    import torch
+    import wannierberri_amd as wb
+    from wannierberri_amd import data_k, models
+    formed = []
+    real = data_k.r_pairs
+    monkeypatch.setattr(data_k, "r_pairs", lambda R: formed.append(len(R)) or real(R))
+    Ef = np.linspace(-4, 4, 9)
+    k = np.random.default_rng(1).random((8, 3))
+    calcs = {"ahc": wb.calculators.static.AHC(Efermi=Ef)}
+    s = models.synthetic(num_wann=4, Rmax=1, seed=3)
+    wb.run(s, wb.Grid(system=s, NK=[4, 4, 4], NKFFT=[4, 4, 4]), calcs, save_files=False, verbose=False)
+    assert formed == []
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: True)
+    alone = wb.run_klists(s, [k], calcs).results["ahc"].data
+    assert formed == []
+    monkeypatch.undo()
+    monkeypatch.setattr(data_k, "r_pairs", lambda R: formed.append(len(R)) or real(R))
+    for _ in range(2):
+        pairs = wb.run_klists(s, [k], calcs).results["ahc"].data
+    assert formed == [s.rvec.nRvec]
+    # the phases' rounding (test_klist_pairs) over gaps of order one
+    assert np.abs(alone - pairs).max() < 1e-11 * np.abs(pairs).max()
+
+
 @pytest.mark.parametrize("nw,nef,nom,kbt,smr", [(2, 1, 1, 0.0, "Lorentzian"), (5, 8, 16, 0.05, "Gaussian"), (6, 15, 17, 0.0, "Lorentzian"),
                                                 (9, 7, 129, 0.05, "Lorentzian"), (20, 3, 128, 0.05, "Lorentzian"),
                                                 (34, 2, 3, 0.05, "Lorentzian")])

@@ -85,18 +85,19 @@ def channel_terms(name, der, base_offset):
 def r_pairs(iRvec):
     """The R-vectors as pairs, int32 [npair, 2]: (i, j) with R_j = -R_i, (i, -1) for one without a
     partner (R = 0, a missing -R, repeated vectors beyond the first match)."""
-    R = np.asarray(iRvec).reshape(-1, 3).astype(np.int64)
-    span = 2 * np.abs(R).max(axis=0, initial=0) + 1
-    if len(R) and np.prod(span.astype(float)) < 2.0 ** 62:
-        weight = np.array([span[1] * span[2], span[2], 1])
-        key = R @ weight   # one number per vector, -R's is its negative
-        order = np.argsort(key, kind="stable")
+    R = np.asarray(iRvec).reshape(-1, 3)
+    span = 2 * int(np.abs(R).max(initial=0)) + 1
+    if len(R) and span < 1 << 20:
+        key = R @ np.array([span * span, span, 1], dtype=np.int64)   # one number per vector, -R's is its negative
+        order = key.argsort(kind="stable")
         ks = key[order]
-        if np.all(np.diff(ks) > 0):   # no repeated vector
-            at = np.minimum(np.searchsorted(ks, -key), len(ks) - 1)
-            i, j = np.arange(len(R)), np.where(ks[at] == -key, order[at], -1)
-            keep = (j < 0) | (j >= i)
-            return np.stack([i, np.where(j == i, -1, j)], axis=1)[keep].astype(np.int32)
+        if (ks[1:] > ks[:-1]).all():   # no repeated vector
+            at = ks.searchsorted(-key)
+            at[at == len(ks)] = 0
+            i, j = np.arange(len(R)), order[at]
+            j[(key[j] != -key) | (j == i)] = -1
+            keep = (j < 0) | (j > i)
+            return np.stack([i[keep], j[keep]], axis=1).astype(np.int32)
     partner = {}
     for j, R in enumerate(iRvec.tolist()):
         partner.setdefault(tuple(R), []).append(j)
@@ -138,12 +139,20 @@ class DeviceSystem:
         self.cR = torch.from_numpy(np.ascontiguousarray(system.cRvec_shifted)).to(dev)
         self.iRvec = np.ascontiguousarray(system.rvec.iRvec, dtype=np.int32)
         self.iRvec_dev = torch.from_numpy(self.iRvec).to(dev)
-        self.pairs_dev = torch.from_numpy(r_pairs(self.iRvec)).to(dev)
+        self._pairs = None
         self._stacks = {}
         self._plans = {}
         self._zcache = collections.OrderedDict()   # z-pass outputs, least recently used first
         self._zcache_used = 0
         self.eig_hint = None   # the last grid K-block's eigenvectors (starting basis of the next)
+
+    @property
+    def pairs_dev(self):
+        """r_pairs on the device, formed with the first k-list transform (a grid needs none); None
+        while a graph capture, which takes no copy from the host, is the first (every R alone)."""
+        if self._pairs is None and not self.torch.cuda.is_current_stream_capturing():
+            self._pairs = self.torch.from_numpy(r_pairs(self.iRvec)).to(self.ctx.device)
+        return self._pairs
 
     def has(self, name):
         return name in self.base_offset or (name == "rotAA" and "AA" in self.base_offset)
