@@ -249,12 +249,11 @@ int wbmi_r2k_klist_tile_shape(int tile, int* k_rows, int* elements);
  *   complex128 vectors get a final Newton-Schulz orthonormalisation.
  *   E are the FP64 Rayleigh quotients of the refined vectors.  Separated
  *   spectra take 2-3 steps; a pair closer than the first step's threshold
- *   (~1e-4 |H| at nw = 32) about ten.  For nw > 64 the FP32 Jacobi runs one
- *   workgroup per chunk of eigenvector rows.
+ *   (~1e-4 |H| at nw = 32) about ten.
  *   refine = 0: plain Jacobi in the arithmetic of `prec` (nw <= 64).
  *   work_dev / work_bytes: device workspace of at least
  *   wbmi_eigh_work_bytes(...) bytes (nonzero only for refinement at
- *   nw > 44); may be NULL / 0 otherwise.                                   */
+ *   nw > 64); may be NULL / 0 otherwise.                                   */
 int wbmi_eigh(wbmi_ctx* ctx, int nk, int nw, const void* H_dev, int64_t Hstride,
               double* E_dev, void* U_dev, int prec, int refine, const void* H64_dev,
               void* work_dev, size_t work_bytes);
@@ -266,7 +265,7 @@ size_t wbmi_eigh_work_bytes(int nk, int nw, int prec, int refine);
  * workspace taken from a fixed scratch array in the library, one per GPU, of
  * wbmi_eigh_noalloc_max_bytes() = 64 MiB: sizes whose wbmi_eigh_work_bytes
  * exceed it are refused (at nw = 128 with refinement: 64 k-points per call;
- * nw <= 44 needs none).  Allocates nothing; calls on one GPU share the scratch,
+ * nw <= 64 needs none).  Allocates nothing; calls on one GPU share the scratch,
  * so calls that overlap on one GPU race.                                    */
 int wbmi_eigh_noalloc(wbmi_ctx* ctx, int nk, int nw, const void* H_dev, int64_t Hstride,
                       double* E_dev, void* U_dev, int prec, int refine, const void* H64_dev);

@@ -71,6 +71,24 @@ def test_eigh_refine_blocks(ctx, nw, gap):
     assert np.abs(u.conj().swapaxes(1, 2) @ u - np.eye(nw)).max() < 8 * EPS * nw
 
 
+@pytest.mark.parametrize("nw", [45, 64])
+def test_eigh_needs_no_workspace(ctx, nw):
+    """Refined solves of up to 64 bands without a workspace: more k-points than the no-allocation form's scratch
+    would hold at four matrices each."""
+    import torch
+    from wannierberri_amd import _lib
+    nk = _lib.lib().wbmi_eigh_noalloc_max_bytes() // (4 * 16 * nw * nw) + 3
+    H = torch.from_numpy(_hermitian(np.random.default_rng(nw), 3, nw)).cuda()[torch.arange(nk) % 3].contiguous()
+    E = torch.empty((nk, nw), dtype=torch.float64, device="cuda")
+    U = torch.empty((nk, nw, nw), dtype=torch.complex128, device="cuda")
+    ctx.eigh_noalloc(H, nw * nw, E, U, _lib.WBMI_F64, nw, refine=16)
+    assert torch.equal(E, E[torch.arange(nk) % 3])
+    assert np.abs(E[:3].cpu().numpy() - np.linalg.eigvalsh(H[:3].cpu().numpy())).max() < 8 * EPS * nw * 20
+    L, E1, U1 = _lib.lib(), torch.empty_like(E), torch.empty_like(U)
+    assert L.wbmi_eigh(ctx.h, nk, nw, _lib._ptr(H), nw * nw, _lib._ptr(E1), _lib._ptr(U1), _lib.WBMI_F64, 16, None, None, 0) == 0
+    assert torch.equal(E, E1) and torch.equal(U, U1)
+
+
 @pytest.mark.parametrize("nw", [33, 40, 64])
 @pytest.mark.parametrize("prec", ["fp64", "fp32"])
 def test_eigh_repeats(ctx, nw, prec):

@@ -1224,7 +1224,7 @@ __global__ void __launch_bounds__(OAG_THREADS) k_eigh_refine_g(int n, const cplx
 }
 
 // Scratch of wbmi_eigh_noalloc: the per-k refinement workspace (X, T, S/E, R;
-// 44 < nw <= 128) in a file-scope device array, so that callers that cannot allocate
+// 64 < nw <= 128) in a file-scope device array, so that callers that cannot allocate
 // (graph capture, serving loops) get the refined solver without a workspace.  Each GPU
 // holds its own copy for the life of the process; calls on one GPU share it (their
 // kernels write every element before reading it, so nothing needs clearing, and
@@ -1238,9 +1238,9 @@ int wbmi_eigh_scratch_init(void** ptr) {
     return hipGetSymbolAddress(ptr, HIP_SYMBOL(scratch)) == hipSuccess && *ptr ? 0 : 1;
 }
 
-// bytes of global workspace wbmi_eigh asks for (refinement for nw > 44; used above 64)
+// bytes of global workspace wbmi_eigh needs (refinement for nw > 64: k_eigh_refine_g)
 static size_t eigh_work_bytes(int nk, int nw, int refine) {
-    return (refine && nw > 44) ? sizeof(cplx<double>) * 4 * (size_t)nw * nw * nk : 0;
+    return (refine && nw > 64) ? sizeof(cplx<double>) * 4 * (size_t)nw * nw * nk : 0;
 }
 
 extern "C" size_t wbmi_eigh_work_bytes(int nk, int nw, int prec, int refine) {
@@ -1316,11 +1316,11 @@ template <typename TU>
 static int eigh_refined(wbmi_ctx* ctx, int nk, int nw, const cplx<double>* H64, int64_t Hstride, double* E,
                         cplx<TU>* U, int steps, void* work, size_t work_bytes, const cplx<TU>* U0 = nullptr) {
     const double tol = sizeof(TU) == 4 ? OA_TOL_C64 : OA_TOL_C128;
-    int rc = jacobi_f32_of_f64<TU>(ctx, nk, nw, H64, Hstride, E, U, U0);
-    if (rc) return rc;
-    if (nw > 44 && (!work || work_bytes < eigh_work_bytes(nk, nw, steps)))
+    if (nw > 64 && (!work || work_bytes < eigh_work_bytes(nk, nw, steps)))
         return wbmi_fail(ctx, WBMI_ERR_ARG, "wbmi_eigh: refinement at nw = %d needs %zu bytes of workspace", nw,
                          eigh_work_bytes(nk, nw, steps));
+    int rc = jacobi_f32_of_f64<TU>(ctx, nk, nw, H64, Hstride, E, U, U0);
+    if (rc) return rc;
     if (nw > 64) {
         hipLaunchKernelGGL((k_eigh_refine_g<TU>), dim3(nk), dim3(OAG_THREADS), 0, ctx->stream, nw, H64, Hstride, E, U,
                            steps, tol, (cplx<double>*)work);
