@@ -472,6 +472,34 @@ def test_klist_pairs_on_demand(ctx, monkeypatch):
     assert np.abs(alone - pairs).max() < 1e-11 * np.abs(pairs).max()
 
 
+@pytest.mark.parametrize("nw,limit,nc", [(5, "k", 1), (5, "k", 3), (5, "bytes", 3), (66, "bytes", 3), (66, "bytes", 1)])
+def test_corner_batches(monkeypatch, nw, limit, nc):
+    """Corner energies in batches of one and three of the eight corners (the last batch not full), the batch
+    limited by its k-points or by its memory (Hamiltonians, vectors and, above 64 bands, the eigensolver's
+    workspace): the same energies as all corners together, no call beyond the limit."""
+    import wannierberri_amd as wb
+    from wannierberri_amd import _lib, data_k, models
+    s = models.synthetic(num_wann=nw, Rmax=1, seed=nw)
+    grid = wb.Grid(system=s, NK=[3, 3, 2], NKFFT=[3, 3, 2])
+    Kp = grid.get_K_list(use_symmetry=False)[0]
+    nk = 18
+
+    def corners():
+        return data_k.Data_K(s, dK=Kp.Kp_fullBZ, grid=grid, Kpoint=Kp).corner_energies().cpu().numpy()
+    ref = corners()
+    per_corner = nk * nw * nw * 16 * (2 + (4 if nw > 64 else 0))
+    if limit == "k":
+        monkeypatch.setattr(data_k, "CORNER_BATCH_K", nc * nk + 1)
+    else:
+        monkeypatch.setattr(data_k, "CORNER_BATCH_BYTES", nc * per_corner + 1)
+    calls = []
+    eigh = _lib.Context.eigh
+    monkeypatch.setattr(_lib.Context, "eigh", lambda self, H, st, E, *a, **k: calls.append(len(E)) or eigh(self, H, st, E, *a, **k))
+    got = corners()
+    assert calls[1:] == [nc * nk] * (8 // nc) + ([8 % nc * nk] if 8 % nc else [])   # [0]: the block itself
+    assert np.abs(got - ref).max() < 8 * EPS * nw * np.abs(ref).max()
+
+
 @pytest.mark.parametrize("nw,nef,nom,kbt,smr", [(2, 1, 1, 0.0, "Lorentzian"), (5, 8, 16, 0.05, "Gaussian"), (6, 15, 17, 0.0, "Lorentzian"),
                                                 (9, 7, 129, 0.05, "Lorentzian"), (20, 3, 128, 0.05, "Lorentzian"),
                                                 (34, 2, 3, 0.05, "Lorentzian")])

@@ -285,11 +285,16 @@ class Context:
             self._work = torch.empty(nbytes, dtype=torch.uint8, device=self.device)
         return self._work
 
+    @staticmethod
+    def eigh_work_bytes(nk, nw, prec, refine):
+        """Bytes of device workspace that eigh() takes from the context."""
+        return int(lib().wbmi_eigh_work_bytes(nk, nw, prec, int(refine)))
+
     def eigh(self, H, Hstride, E, U, prec, nw, refine=0, H64=None, U0=None):
         """Batched eigh; refine=n >= 1: FP32 Jacobi + up to n FP64 Ogita-Aishima steps.
         U0: optional starting eigenvectors (same shape and dtype as U; may be U itself)."""
         nk = E.shape[0]
-        wbytes = int(lib().wbmi_eigh_work_bytes(nk, nw, prec, int(refine)))
+        wbytes = self.eigh_work_bytes(nk, nw, prec, refine)
         work = self._workspace(wbytes)
         if U0 is None:
             self.check(self._timed("eigh", (nk, nw), lib().wbmi_eigh, self.h, nk, nw, _ptr(H), Hstride,

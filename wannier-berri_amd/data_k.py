@@ -45,7 +45,8 @@ OA_STEPS = 16
 # transform is shorter than the 45 us of host time that the events and stream changes cost, which a
 # small block waits for (a 2-band layer, 16 blocks of 156 k-points: 2.42 against 3.40 ms)
 PREFETCH_MIN = 1 << 21
-# corner energies: k-points and bytes of a batch of corners diagonalised together
+# corner energies: k-points and bytes (Hamiltonians, eigenvectors and the eigensolver's workspace) of a batch of
+# corners diagonalised together
 CORNER_BATCH_K, CORNER_BATCH_BYTES = 1 << 15, 1 << 30
 _ALPHA = [1, 2, 0]
 _BETA = [2, 0, 1]
@@ -506,7 +507,8 @@ class Data_K:
             Ec = torch.empty((len(shifts), nk, nw), dtype=torch.float64, device=self.ctx.device)
             # several corners per diagonalisation: one K-block alone leaves most of the GPU idle (1728
             # k-points at nw = 12, 8 corners: 1.32 ms for the whole calculation one by one, 1.00 together)
-            nc = max(1, min(len(shifts), CORNER_BATCH_K // nk, CORNER_BATCH_BYTES // (16 * nw * nw * nk)))
+            per_corner = 2 * 16 * nw * nw * nk + self.ctx.eigh_work_bytes(nk, nw, WBMI_F64, OA_STEPS)
+            nc = max(1, min(len(shifts), CORNER_BATCH_K // nk, CORNER_BATCH_BYTES // per_corner))
             H = torch.empty((nc, nk, 1, nw, nw), dtype=torch.complex128, device=self.ctx.device)
             U = torch.empty((nc * nk, nw, nw), dtype=torch.complex128, device=self.ctx.device)
             for c0 in range(0, len(shifts), nc):
