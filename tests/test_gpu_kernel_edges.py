@@ -445,6 +445,24 @@ def test_klist_pairs(ctx, nk, nw, extra):
                 assert err < bound + (1.2e-7 * np.abs(ref).max() if prec == _lib.WBMI_F32 else 0), (tile, p is None)
 
 
+@pytest.mark.parametrize("nk,nelem", [(1, 64 * 65535 + 1), (17, 64 * 65535 + 1), (2, 128 * 65535)])
+def test_klist_many_elements(ctx, nk, nelem):
+    """More elements per k-point than the narrow tiles take: up to 128 x 65535 are accepted for any list."""
+    import torch
+    from wannierberri_amd import _lib
+    iR = torch.tensor([[0, 0, 0], [1, 0, 0]], dtype=torch.int32, device="cuda")
+    X = torch.ones((2, nelem), dtype=torch.complex128, device="cuda")
+    X[1] = torch.linspace(0, 1, nelem, dtype=torch.float64, device="cuda")
+    k = np.random.default_rng(nk).random((nk, 3))
+    out = torch.zeros((nk, nelem), dtype=torch.complex128, device="cuda")
+    ctx.r2k_klist(iR, X, torch.from_numpy(k).cuda(), out, _lib.WBMI_F64, tile=-1)
+    ref = 1 + torch.from_numpy(np.exp(2j * np.pi * k[:, :1])).cuda() * X[1]
+    assert (out - ref).abs().max().item() < 2 * np.pi * 4 * EPS * 2   # the phase's rounding, as in test_klist_pairs
+    with pytest.raises(ValueError, match="elements per k-point"):
+        ctx.r2k_klist(iR, torch.empty((2, 128 * 65535 + 1), dtype=torch.complex128, device="cuda"), torch.from_numpy(k).cuda(),
+                      torch.empty((nk, 128 * 65535 + 1), dtype=torch.complex128, device="cuda"), _lib.WBMI_F64, tile=-1)
+
+
 def test_klist_pairs_on_demand(ctx, monkeypatch):
     """A grid never forms the pairs (R, -R); the first k-list does, once; while a graph capture is the first,
     the transform takes every R-vector alone."""

@@ -673,6 +673,7 @@ int wbmi_r2k_yx(wbmi_ctx* ctx, const wbmi_r2k_plan* p, const void* w1_dev, const
 // ---------------------------------------------------------------------------
 
 #define KLM_RC 32
+#define KLM_YMAX 65535
 
 // Workgroup tiles: 16-row blocks of k-points and 16-column blocks of elements per wave, waves along k,
 // waves along the elements; chosen per nw by the tuning table of the context (wannierberri_amd/autotune.py)
@@ -686,12 +687,14 @@ static const KlmTile klm_tiles[WBMI_KLIST_NTILES] = {{4, 2, 1, 4}, {4, 2, 2, 2},
 // The 32 x 32 wave tile where there are at least two of them for every SIMD (6112 k-points x 5760 elements:
 // 1.91 ms; 64 x 32, with half the waves on a SIMD, 2.00; 32 x 16 2.22), then 32 x 16, else the smallest
 // (a path batch of 50 k-points x 3240 elements: 32 us, against 39 and 52 with the larger ones).
+// The narrow tiles take fewer elements per call (gridDim.y): lists beyond that take the 128 of tile 0.
 static int klm_rule(int nk, int64_t nelem) {
+    auto fits = [&](int t) { return ceil_div(nelem, 16 * klm_tiles[t].et * klm_tiles[t].we) <= KLM_YMAX; };
     for (int t : {4, 5}) {
         const KlmTile& q = klm_tiles[t];
-        if (nk > 8 * q.kt && ceil_div(nk, 16 * q.kt) * ceil_div(nelem, 16 * q.et) >= 2048) return t;
+        if (nk > 8 * q.kt && fits(t) && ceil_div(nk, 16 * q.kt) * ceil_div(nelem, 16 * q.et) >= 2048) return t;
     }
-    return 6;
+    return fits(6) ? 6 : 0;
 }
 
 template <typename Tout, bool PAIRS, int KT, int ET, int WK, int WE>
@@ -794,8 +797,8 @@ template <typename Tout, int KT, int ET, int WK, int WE>
 static int launch_klist(wbmi_ctx* ctx, int nR, int npair, const int32_t* pairs, const int32_t* iR, int64_t nelem,
                         const void* XR, int nk, const double* kl, void* out) {
     constexpr int TK = 16 * KT * WK, TE = 16 * ET * WE;
-    if (ceil_div(nelem, TE) > 65535)
-        return wbmi_fail(ctx, WBMI_ERR_ARG, "wbmi_r2k_klist: more than %d elements per k-point", 65535 * TE);
+    if (ceil_div(nelem, TE) > KLM_YMAX)
+        return wbmi_fail(ctx, WBMI_ERR_ARG, "wbmi_r2k_klist: more than %d elements per k-point", KLM_YMAX * TE);
     dim3 g((unsigned)ceil_div(nk, TK), (unsigned)ceil_div(nelem, TE));
     if (pairs)
         hipLaunchKernelGGL((k_r2k_klist<Tout, true, KT, ET, WK, WE>), g, dim3(64 * WK * WE), 0, ctx->stream, npair,
