@@ -463,6 +463,40 @@ def test_klist_many_elements(ctx, nk, nelem):
                       torch.empty((nk, 128 * 65535 + 1), dtype=torch.complex128, device="cuda"), _lib.WBMI_F64, tile=-1)
 
 
+@pytest.mark.parametrize("ibands", [None, [4, 1, 2]])
+def test_tables_under_way(monkeypatch, ibands):
+    """Tabulated results over several blocks, their host copies at once or behind the queued work: the same
+    numbers, as a result, as its pickle, per block and along a path."""
+    import pickle
+    import wannierberri_amd as wb
+    from wannierberri_amd import models
+    from wannierberri_amd.result import HostCopy
+    tab = wb.calculators.tabulate
+    s = models.synthetic(num_wann=5, Rmax=1, seed=8)
+    path = wb.Path(system=s, k_list=np.linspace([0, 0, 0], [0.5, 0.4, 0.1], 12))
+    grid = wb.Grid(system=s, NK=[4, 4, 2], NKFFT=[2, 2, 2])
+    out = []
+    for limit in (0, 1 << 30):
+        monkeypatch.setattr(HostCopy, "LIMIT", limit)
+        r = []
+        for g, kw in ((path, {"k_batch": 5}), (grid, {"symmetrize": False, "use_irred_kpt": False})):
+            t = tab.TabulatorAll({"Energy": tab.Energy(), "vel": tab.Velocity(), "berry": tab.BerryCurvature()}, ibands=ibands,
+                                 mode="path" if g is path else "grid")
+            res = wb.run(s, g, {"t": t}, save_files=False, verbose=False, **kw).results["t"].results
+            r += [res[k].data for k in ("Energy", "vel", "berry")] + [pickle.loads(pickle.dumps(res["berry"])).data]
+        block = tab.BerryCurvature(ibands=ibands)
+        from wannierberri_amd.data_k import Data_K
+        one = [block(Data_K(s, k_list=[[0.1 * i, 0.2, 0.3], [0.4, 0.1, 0.1 * i]])) for i in range(3)]
+        total = one[0] + one[1] + one[2]
+        r += [total.data] + [x.data for x in one]
+        assert np.array_equal(total.data, np.concatenate([x.data for x in one]))
+        out.append(r)
+    for a, b in zip(*out):
+        assert a.shape == b.shape and a.shape[1] == (5 if ibands is None else 3)
+        # (the traces' partial sums meet in any order)
+        assert np.abs(a - b).max() < 1e-12 * np.abs(a).max()
+
+
 def test_klist_pairs_on_demand(ctx, monkeypatch):
     """A grid never forms the pairs (R, -R); the first k-list does, once; while a graph capture is the first,
     the transform takes every R-vector alone."""

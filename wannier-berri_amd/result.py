@@ -6,6 +6,7 @@ data of a K-block result stays on the GPU (a torch tensor) so the k-sum over
 K-blocks never synchronises; `.data` materialises a NumPy array.
 """
 import os
+import threading
 
 import numpy as np
 
@@ -236,7 +237,8 @@ class HostCopy:
 
     def __init__(self, out, finish, shape):
         self.shape, self.ndim = tuple(shape), len(shape)
-        self._finish, self._array, self._event = finish, None, None
+        self.shared = False   # held by several results
+        self._finish, self._array, self._lock = finish, None, threading.Lock()
         if out.numel() * out.element_size() > self.LIMIT:
             self._array = finish(out.cpu().numpy()).reshape(self.shape)
             return
@@ -246,55 +248,97 @@ class HostCopy:
         self._event.record(torch.cuda.current_stream(out.device))
 
     def array(self):
-        if self._array is None:
-            self._event.synchronize()
-            self._array = self._finish(self._host.numpy()).reshape(self.shape)   # a new array
-            self._host = self._event = None   # the pinned buffer is given back
+        with self._lock:
+            if self._array is None:
+                self._event.synchronize()
+                self._array = self._finish(self._host.numpy()).reshape(self.shape)   # a new array
+                self._host = self._event = None   # the pinned buffer is given back
         return self._array
+
+
+def _array_of(block):
+    return block.array() if isinstance(block, HostCopy) else block
 
 
 class KBandResult(Result):
     """Per-(k, band) data [nk, nband, 3, ...] (result/kbandresult.py): K-blocks concatenate
-    along k; K-point factors do not apply.  The blocks (arrays, the last one also a HostCopy) are
-    joined when the data are read."""
+    along k; K-point factors do not apply.
+
+    `data` is the array given, or (until it is first read) blocks to be joined into one: a HostCopy, or
+    arrays and at most one HostCopy.  Blocks may belong to several results, which never hand them out: what
+    is read is an array of the result's own, and an array that was given or read is copied when it is added."""
 
     def __init__(self, data, transformTR=None, transformInv=None):
-        self._parts = [data if isinstance(data, HostCopy) else np.asarray(data)]
+        self._lock = threading.Lock()
+        self._blocks, self._data = ([data], None) if isinstance(data, HostCopy) else (None, np.asarray(data))
         self.transformTR = transformTR
         self.transformInv = transformInv
 
     @property
     def data(self):
-        if len(self._parts) > 1 or isinstance(self._parts[0], HostCopy):
-            arrays = [p.array() if isinstance(p, HostCopy) else p for p in self._parts]
-            self._parts = [np.concatenate(arrays, axis=0) if len(arrays) > 1 else arrays[0]]
-        return self._parts[0]
+        with self._lock:
+            if self._data is None:
+                arrays = [_array_of(b) for b in self._blocks]
+                alone = len(arrays) == 1 and not self._blocks[0].shared
+                self._data = arrays[0] if alone else np.concatenate(arrays, axis=0)
+                self._blocks = None
+            return self._data
 
     @data.setter
     def data(self, value):
-        self._parts = [value]
+        with self._lock:
+            self._blocks, self._data = None, value
+
+    def _own_blocks(self):
+        """This result's blocks, none of them handed out."""
+        with self._lock:
+            if self._data is not None:
+                return [np.array(self._data)]
+            for b in self._blocks:
+                if isinstance(b, HostCopy):
+                    b.shared = True
+            return list(self._blocks)
 
     def __getstate__(self):
-        return dict(self.__dict__, _parts=[self.data])
+        state = dict(self.__dict__, data=self.data)
+        for name in ("_lock", "_blocks", "_data"):
+            del state[name]
+        return state
+
+    def __setstate__(self, state):
+        self._lock = threading.Lock()
+        self.__dict__.update({k: v for k, v in state.items() if k != "data"})
+        self.data = state["data"]
+
+    @property
+    def _shape(self):
+        with self._lock:
+            if self._data is not None:
+                return np.shape(self._data)
+            return (sum(b.shape[0] for b in self._blocks),) + tuple(self._blocks[0].shape[1:])
 
     @property
     def nk(self):
-        return sum(p.shape[0] for p in self._parts)
+        return self._shape[0]
 
     @property
     def nband(self):
-        return self._parts[0].shape[1]
+        return self._shape[1]
 
     @property
     def rank(self):
-        return self._parts[0].ndim - 2
+        return len(self._shape) - 2
 
     def __add__(self, other):
         if other is None or (isinstance(other, (int, float)) and other == 0):
             return self
-        new = KBandResult(self._parts[0], self.transformTR, self.transformInv)
-        # at most the added block stays a copy under way
-        new._parts = [p.array() if isinstance(p, HostCopy) else p for p in self._parts] + list(other._parts)
+        added = other._own_blocks() if isinstance(other, KBandResult) else [np.array(other.data)]
+        # copies of earlier blocks under way are over: at most the added block's goes on
+        blocks = [_array_of(b) for b in self._own_blocks()] + added
+        if len({tuple(b.shape[1:]) for b in blocks}) > 1 or blocks[0].ndim == 0:
+            raise ValueError(f"K-blocks of shapes {[tuple(b.shape) for b in blocks]} do not concatenate along k")
+        new = KBandResult(blocks[0], self.transformTR, self.transformInv)
+        new._blocks, new._data = blocks, None
         return new
 
     def __mul__(self, other):
