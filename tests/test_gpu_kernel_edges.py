@@ -579,3 +579,26 @@ def test_optical_tiles(ctx, nw, nef, nom, kbt, smr):
         assert np.abs(got.results["opt"].data).max() == 0
     else:
         assert np.abs(got.results["opt"].data - ref).max() < 1e-10 * scale
+
+
+@pytest.mark.parametrize("nw", [4, 34])
+def test_optical_pairs_left_alone(ctx, nw):
+    """A matrix element that is not finite is seen at the Fermi levels that part its two bands only."""
+    import wannierberri_amd as wb
+    from wannierberri_amd import models
+    from wannierberri_amd.data_k import Data_K
+    s = models.synthetic(num_wann=nw, Rmax=1, seed=nw)
+    data = Data_K(s, k_list=[[0.1, 0.2, 0.3]], channels={("Ham", 1), ("AA", 0)})
+    E = data.E_K[0]
+    Ef = [E[0] - 1.0, 0.5 * (E[0] + E[1]), 0.5 * (E[1] + E[2]), 0.5 * (E[2] + E[3]), E[-1] + 1.0]
+    calc = wb.calculators.dynamic.OpticalConductivity(Efermi=Ef, omega=np.linspace(0.0, 2.0, 5), kBT=0.0, smr_fixed_width=0.1)
+    data.ensure(calc.needed_channels(s))
+    for sl in data._slots.values():
+        data.Xk[0, sl:sl + 3, 0, 1] = data.Xk[0, sl:sl + 3, 1, 0] = 0.0
+    ref = calc(data).data
+    sl = data._slots["Ham", 1]
+    data.Xk[0, sl:sl + 3, 0, 1] = float("nan")
+    got = calc(data).data
+    assert np.isnan(got[1]).any()
+    others = [0, 2, 3, 4]
+    assert np.abs(got[others] - ref[others]).max() <= 1e-13 * np.abs(ref).max()

@@ -210,7 +210,9 @@ __global__ void __launch_bounds__(OC_THREADS, 2) k_optcond(int nk, int kchunk, O
                     cplx<double> v = mk(0.0, 0.0);
                     if (p0 + q < np && c < ncol) {
                         const int m = sP[p0 + q] & 0xffff, n = sP[p0 + q] >> 16, e = (c0 + c) / 9 - e0;
-                        v = (sOcc[n * OC_NE + e] - sOcc[m * OC_NE + e]) * sM[q * 9 + (c0 + c) % 9];
+                        // (a pair that this level leaves alone adds nothing, not zero times a value that may not be finite)
+                        const double df = sOcc[n * OC_NE + e] - sOcc[m * OC_NE + e];
+                        if (df != 0.0) v = df * sM[q * 9 + (c0 + c) % 9];
                     }
                     sG[q * (OC_C + 1) + c] = v;
                 }
