@@ -358,10 +358,12 @@ class Data_K:
         else:
             kl = self.k_list_dev
             if kl is None:
-                # behind queued work through pinned memory: a pageable copy would wait for it
+                # a pageable copy waits for the work queued before it, one through pinned memory does not; the
+                # latter is ordered before the transform only on the transform's own stream
                 kl = torch.from_numpy(self.k_list)
-                idle = self.ctx.stream.query()
-                kl = kl.to(self.ctx.device) if idle else kl.pin_memory().to(self.ctx.device, non_blocking=True)
+                own = torch.cuda.current_stream(self.ctx.device) == self.ctx.stream
+                ahead = own and not self.ctx.stream.query()
+                kl = (kl.pin_memory() if ahead else kl).to(self.ctx.device, non_blocking=ahead)
             self.ctx.r2k_klist(self.dev.iRvec_dev, stack, kl, X, prec, pairs=self.dev.pairs_dev)
         return X
 
