@@ -2183,10 +2183,12 @@ static int launch_scan_t(wbmi_ctx* ctx, int nk, const ScanArgs& a, const double*
     const size_t lds = smem_offsets(a.nw, LM, ST, stage_a, MODE == 1, sizeof(cplx<T>)).total;
     if (lds > SC_LDS) return wbmi_fail(ctx, WBMI_ERR_ARG, "wbmi_static_scan: %zu bytes of LDS needed", lds);
     // DerOmega / DerMorb of few k-points: several workgroups share a k-point's tasks, so that there are
-    // about four per CU (above nw = 32, where a k-point's tasks fill them; two below).  Fermi bins only: the
+    // about four per CU (above nw = 32, where a k-point's tasks fill them; two below).  The kernels of all cuts, complex64
+    // internal terms, 294 k-points at nw = 64: 446 us with two per CU, 332 with four, 348 with more; complex128
+    // external terms at nw = 40 529, 416 and 498; 300 at nw = 18 120, 122 and 171.  Fermi bins only: the
     // other modes use a k-point's sums before they are complete.
     constexpr bool tasks = F == WBMI_FORMULA_DEROMEGA || F == WBMI_FORMULA_DERMORB;
-    const int want = SC_IS_DERMORB_CUTS(F) ? (a.nw > 32 ? 4096 : 2048) : a.nw > 32 ? 1024 : 512;
+    const int want = a.nw > 32 ? 1024 : 512;
     const int parts = (tasks || SC_IS_DERMORB_CUTS(F)) && MODE == 0 && nk < want ? std::min(8, want / nk) : 1;
     WBMI_HIP_CHECK(ctx, hipFuncSetAttribute((const void*)k_static_scan<T, F, LM, ST, MODE, NW, NTH>,
                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
