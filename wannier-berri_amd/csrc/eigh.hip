@@ -262,7 +262,9 @@ __device__ inline void rotate_rows(cplx<float>& xp, cplx<float>& xq, float c, fl
 // Bound: VALU issue (about 390 instructions a round and wave at N = 32, 64 LDS operations) and,
 // for few k-points, the latency of a round.
 // One wave per k for N <= 32, four above (LDS holds four such workgroups a CU at N = 48); few k-points: below.
-// The parameters of N = 16, 32 and 64 use the hardware reciprocals.
+// The parameters of N = 16, 32 and 64 use the hardware reciprocals (FAST), those of the sizes between correctly rounded
+// division: either way the rotations are unitary to FP32 rounding and the refinement removes the rest, but where close
+// bands keep a vector from converging further, its complex64 bits depend on it, so each size keeps its formula.
 // Measured against k_eigh_jacobi (sizes at run time, two phases): 9.1 -> 2.6 ms for 3898 k-points
 // at nw = 48, 1.05 -> 0.62 ms for 6112 at nw = 24, 165 -> 67 us for 1728 at nw = 12.
 // ---------------------------------------------------------------------------
@@ -796,9 +798,10 @@ __device__ void cluster_jacobi(int n, FS S, FX X, char* scratch, double theta, d
 // nw = 32, 4096 k-points: complex128 657 -> 406 us (0.18 ms of matrix instructions), complex64 382 -> 192;
 // nw = 12, 1728: 42.5 -> 26.2; nw = 2, 625: 32.9 -> 15.2; through global memory before, nw = 48, 3898
 // k-points, complex64: 1509 -> 725; nw = 64, 294: 314 -> 182.
-// SPLIT: re re, im im, re im and im re summed apart, the order of every complex64 result up to nw = 44 (above,
-// and for complex128, together: half the accumulators).  A last-bit difference in the FP64 vectors moves a
-// complex64 element by its rounding now and then, which close bands magnify.
+// SPLIT: re re, im im, re im and im re summed apart (complex64 up to nw = 44; above, and for complex128, together: half
+// the accumulators).  Neither order is the more accurate; but a last-bit difference in the FP64 vectors
+// moves a complex64 element by its rounding now and then, and close bands magnify that (summed together at nw = 32, a
+// mixed-form dipole moved by 5e-9), so each size keeps one order.
 template <typename TU, int NB, bool SPLIT>
 __global__ void __launch_bounds__(64 * NB * NB, NB == 3 ? 5 : NB == 4 ? 4 : 3)
 k_eigh_refine(int nw, const cplx<double>* __restrict__ H64, int64_t Hstride, double* __restrict__ Eout,
@@ -1305,10 +1308,12 @@ static int launch_refine(wbmi_ctx* ctx, int nk, int nw, const cplx<double>* H64,
         WBMI_LAUNCH_CHECK(ctx);
         return WBMI_OK;
     };
-    if constexpr (sizeof(TU) == 4 && NB <= 3)
-        if (NB < 3 || nw <= 44) return launch(std::true_type{});
-    if constexpr (sizeof(TU) == 8 || NB >= 3) return launch(std::false_type{});
-    return WBMI_OK;
+    if constexpr (sizeof(TU) == 4 && NB < 3)
+        return launch(std::true_type{});
+    else if constexpr (sizeof(TU) == 4 && NB == 3)
+        return nw <= 44 ? launch(std::true_type{}) : launch(std::false_type{});
+    else
+        return launch(std::false_type{});
 }
 
 // FP32 Jacobi of the FP64 Hamiltonian, then FP64 Ogita-Aishima steps; eigenvectors stored as TU

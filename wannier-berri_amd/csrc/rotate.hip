@@ -1,7 +1,10 @@
 // Gauge rotation Xbar = U^+ X U of libwbmi (data_K/data_K.py:130-132).
 //
-// FP64 matrix cores (v_mfma_f64_16x16x4f64, operand layout in mfma_c64.h) whatever the storage
-// type.  No LDS: with the summed index enumerated as 4 s + lane / 16 for step s,
+// k_rotate_r (nw <= 32) and k_rotate_s (above) run on the FP64 matrix cores (v_mfma_f64_16x16x4f64, operand
+// layout in mfma_c64.h) whatever the storage type, k_rotate_v (complex64 velocity, 32 < nw <= 64) on FP64 FMAs,
+// k_rotate_h (complex64, nw <= 32, every channel but the velocity) on the fp16 matrix cores.  In the first two neither
+// X nor the product between passes through LDS (k_rotate_r keeps U there): with the summed index
+// enumerated as 4 s + lane / 16 for step s,
 //   * lane l's U element of step s and column block b, U[4 s + l / 16][16 b + l % 16], is the B
 //     operand of T = X U and, conjugated, the A operand of U^+ T for row block b;
 //   * register v of T's row block i, T[16 i + l / 16 + 4 v][l % 16], is the B operand of step
@@ -229,11 +232,13 @@ __global__ void __launch_bounds__(64 * NB, NB <= 4 ? 3 : 2) k_rotate_s(int nw, i
     if constexpr (NB & 1) second(NB - 1, std::false_type{});
 }
 
-// complex64 in FP64 arithmetic at 32 < nw <= 64 (the mixed form's velocity): one 256-thread workgroup per k, U and a
-// channel in LDS, 4 x 4 register tiles and one FMA chain per element in the order of the summed index.  Slower than
-// the matrix cores (3898 k-points at nw = 48: 356 us a channel against 146), whose order of the same sums moves one element in
-// 1e8 by its complex64 rounding: in the velocity between two close bands the cut sums of DerMorb show it (1e-9 of a
-// whole tensor, one model in forty at nw = 64).
+// complex64 in FP64 arithmetic at 32 < nw <= 64 (the mixed form's velocity): one 256-thread workgroup per k, U, X and T
+// = X U in LDS, 4 x 4 register tiles and one FMA chain per element in the order of the summed index.  Slower than
+// the matrix cores (3898 k-points at nw = 48: 356 us a channel against 146) and no more accurate; but the order of the
+// sums decides the complex64 rounding of one element in 1e8, and in the velocity between two close bands
+// the cut sums of DerMorb show it: with k_rotate_s here the gyrotropic tensor moves by up to 1.7e-9 of itself (more than
+// 1e-10 in 6 of 150 models at nw = 64, without it 1).  So these sizes keep the order of this kernel, and those
+// above 64 and below 33 that of the matrix cores; the channels that enter with one energy denominator less take k_rotate_s.
 #define ROTV_THREADS 256
 __device__ inline void rotv_product(int nw, int r0, int c0, cplx<double> (&acc)[4][4], const cplx<double>* sT, const cplx<float>* sU,
                                     const cplx<float>* sX, bool herm, bool second) {

@@ -1,9 +1,10 @@
 // Covariant formula traces + Fermi-level scan of libwbmi.
 //
 // Replaces the per-(k, band group) loop of StaticCalculator.__call__
-// (calculators/static.py:60-136).  One workgroup per k-point (512 threads;
-// DerOmega / DerMorb: scan_threads); the formula is a template parameter, so
-// every calculator gets its own kernel.
+// (calculators/static.py:60-136).  One workgroup per k-point, several where few
+// k-points leave the GPU idle (launch_scan_t), of a size per formula and nw
+// (launch_scan); the formula is a template parameter, so every calculator gets
+// its own kernel.
 //
 // Band partition.  The reference evaluates, for every band group G, the
 // formula with inn = G and out = all other bands.  Every sum in the formulas
@@ -83,7 +84,7 @@ struct ScanArgs {
 
 // dynamic shared-memory layout
 struct Smem {
-    char* V;            // [3][nw][ld] staged V (element type scan_stage)
+    char* V;            // [3][nw][ld] staged V (elements as stored)
     char* A;            // [3][nw][ld] staged A (external terms)
     double* acc;        // [nw][9] per-band values of the partition
     double* M;          // [nw][ld] dEinv o Off
@@ -187,7 +188,7 @@ __device__ __attribute__((always_inline)) inline Smem make_smem(char* base, int 
 // channels; SA: the same for A (staged together with V, and only with external terms, the only
 // case that reads it).
 // Both are compile-time so that every access is a plain LDS or global load.
-template <typename T, bool LM, bool ST, bool SA, int NW = 0, typename TS = T>
+template <typename T, bool LM, bool ST, bool SA, int NW = 0>
 struct KCtx {
     const cplx<T>* X;  // channels of this k: [nch][nw][nw]
     int nw, ld;  // run-time size (NW = 0); NW > 0 fixes both at compile time
@@ -205,8 +206,8 @@ struct KCtx {
     const int* lab;
     const int* gs;
     const int* ge;
-    const cplx<TS>* sV;  // LDS copies of V and A (ST), element type TS
-    const cplx<TS>* sA;
+    const cplx<T>* sV;  // LDS copies of V and A (ST)
+    const cplx<T>* sA;
     const double* bv;    // WBMI_FORMULA_BANDVALUES: this k's caller values [nw][nbv]
     int nbv;
     int part, parts;  // this workgroup's share of the k-point's tasks
@@ -230,7 +231,7 @@ struct KCtx {
     }
     __device__ inline cplx<double> V(int a, int x, int y) const {
         if constexpr (ST) {
-            const cplx<TS> v = sV[(a * n_() + x) * ld_() + y];
+            const cplx<T> v = sV[(a * n_() + x) * ld_() + y];
             return mk((double)v.re, (double)v.im);
         } else {
             return get(WBMI_ROLE_V + a, x, y);
@@ -238,7 +239,7 @@ struct KCtx {
     }
     __device__ inline cplx<double> A(int a, int x, int y) const {
         if constexpr (SA) {
-            const cplx<TS> v = sA[(a * n_() + x) * ld_() + y];
+            const cplx<T> v = sA[(a * n_() + x) * ld_() + y];
             return mk((double)v.re, (double)v.im);
         } else {
             return get(WBMI_ROLE_A + a, x, y);
@@ -273,8 +274,8 @@ struct KCtx {
 
 // pre-Hermitian Omega summand s^c_xy for x, y in the same group
 // (formula/covariant.py:175-200): Omega.nn = s + s^+
-template <typename T, bool LM, bool ST, bool SA, int NW, typename TS>
-__device__ __attribute__((always_inline)) cplx<double> omega_s(const KCtx<T, LM, ST, SA, NW, TS>& K, int c, int x, int y, bool internal, bool external) {
+template <typename T, bool LM, bool ST, bool SA, int NW>
+__device__ __attribute__((always_inline)) cplx<double> omega_s(const KCtx<T, LM, ST, SA, NW>& K, int c, int x, int y, bool internal, bool external) {
     const int al = c_alpha[c], be = c_beta[c];
     cplx<double> s = mk(0.0, 0.0);
     for (int l = 0; l < K.n_(); ++l) {
@@ -292,8 +293,8 @@ __device__ __attribute__((always_inline)) cplx<double> omega_s(const KCtx<T, LM,
 
 // pre-Hermitian Morb_H summand h^c_xy for x, y in the same group
 // (formula/covariant.py:390-414)
-template <typename T, bool LM, bool ST, bool SA, int NW, typename TS>
-__device__ __attribute__((always_inline)) cplx<double> morbh_s(const KCtx<T, LM, ST, SA, NW, TS>& K, int c, int x, int y, bool internal, bool external) {
+template <typename T, bool LM, bool ST, bool SA, int NW>
+__device__ __attribute__((always_inline)) cplx<double> morbh_s(const KCtx<T, LM, ST, SA, NW>& K, int c, int x, int y, bool internal, bool external) {
     const int al = c_alpha[c], be = c_beta[c];
     cplx<double> s = mk(0.0, 0.0);
     for (int l = 0; l < K.n_(); ++l) {
@@ -313,8 +314,8 @@ __device__ __attribute__((always_inline)) cplx<double> morbh_s(const KCtx<T, LM,
 // formula/formula.py:95-107 with A = V, dA = W): for x, y in one band group,
 //   M^{bd}_xy = W^{bd}_xy - sum_{l off} D^d_xl V^b_ly + sum_{l off} V^b_xl D^d_ly
 // (D' carries the off-group mask, so the sums run over every l).
-template <typename T, bool LM, bool ST, bool SA, int NW, typename TS>
-__device__ __attribute__((always_inline)) cplx<double> mass_xy(const KCtx<T, LM, ST, SA, NW, TS>& K, int b, int d, int x,
+template <typename T, bool LM, bool ST, bool SA, int NW>
+__device__ __attribute__((always_inline)) cplx<double> mass_xy(const KCtx<T, LM, ST, SA, NW>& K, int b, int d, int x,
                                                                int y) {
     cplx<double> v = K.W(b, d, x, y);
     for (int l = 0; l < K.n_(); ++l) {
@@ -426,14 +427,14 @@ __host__ __device__ constexpr int task_nt() {
 
 // V^a_ln of a weight D'^a_nl = m_ln conj(V^a_ln): complex64 channels, whose triangles now and then differ by their
 // rounding at a whole k-point (an element of the transform rounded to either side), read V^a_nl itself
-template <typename T, bool LM, bool ST, bool SA, int NW, typename TS>
-__device__ __attribute__((always_inline)) cplx<double> partner_V(const KCtx<T, LM, ST, SA, NW, TS>& K, int a, int l, int n) {
+template <typename T, bool LM, bool ST, bool SA, int NW>
+__device__ __attribute__((always_inline)) cplx<double> partner_V(const KCtx<T, LM, ST, SA, NW>& K, int a, int l, int n) {
     if constexpr (sizeof(T) == 4) return conj(K.Vu(a, n, l));
     else return K.Vu(a, l, n);
 }
 
-template <int KIND, bool DM, typename T, bool LM, bool ST, bool SA, int NW, typename TS>
-__device__ __attribute__((always_inline)) void formula_task(const Smem& S, const KCtx<T, LM, ST, SA, NW, TS>& K, const TaskCtx& tc_,
+template <int KIND, bool DM, typename T, bool LM, bool ST, bool SA, int NW>
+__device__ __attribute__((always_inline)) void formula_task(const Smem& S, const KCtx<T, LM, ST, SA, NW>& K, const TaskCtx& tc_,
                                                            double* acc, int b, int d, int rh, int cb) {
     constexpr bool dm = DM;
     const int nw = K.n_(), lane = threadIdx.x & 63;
@@ -683,8 +684,8 @@ __device__ __attribute__((always_inline)) void formula_task(const Smem& S, const
 // 8 x 8 bands a wave and all components, as in diag_traces (a thread per (n, c, d) read the columns, and for T4
 // also rows, nine times: DerOmega of 216 k-points at nw = 128 3.66 -> 3.27 ms complex64, 2.72 -> 2.56 complex128;
 // with V in LDS the threads are faster, 4096 at nw = 32 0.73 against 0.79 ms).
-template <typename T, bool LM, bool ST, bool SA, int NW, typename TS>
-__device__ __attribute__((always_inline)) void der_diag(const Smem& S, const KCtx<T, LM, ST, SA, NW, TS>& K) {
+template <typename T, bool LM, bool ST, bool SA, int NW>
+__device__ __attribute__((always_inline)) void der_diag(const Smem& S, const KCtx<T, LM, ST, SA, NW>& K) {
     constexpr bool T4 = keep_t4<false, T>();
     const int nw = K.n_(), lane = threadIdx.x & 63, nwave = ((int)blockDim.x >> 6) * K.parts;
     const int n8 = (nw + 7) / 8, split = min(max(nwave / n8, 1), n8);
@@ -759,8 +760,8 @@ __device__ __attribute__((always_inline)) void der_diag(const Smem& S, const KCt
 // register allocation and code size are not those of the DerMorb kinds.
 // The workgroups part = 0, 1, .. of one k share its tasks and per-band terms: each adds up its own,
 // and the sums over groups are linear in them.
-template <bool DM, typename T, bool LM, bool ST, bool SA, int NW, typename TS>
-__device__ __attribute__((always_inline)) void eval_deromega(const Smem& S, const KCtx<T, LM, ST, SA, NW, TS>& K, bool in, bool ex,
+template <bool DM, typename T, bool LM, bool ST, bool SA, int NW>
+__device__ __attribute__((always_inline)) void eval_deromega(const Smem& S, const KCtx<T, LM, ST, SA, NW>& K, bool in, bool ex,
                                                             int sign, int cut) {
     constexpr bool dm = DM;
     const int nw = K.n_(), tid = threadIdx.x;
@@ -977,8 +978,8 @@ struct CutAcc {
 // HERM: V and W are Hermitian to the rounding of the sums.  Otherwise (complex64: partner_V, and the rotation in
 // FP32 arithmetic, whose two triangles differ by their rounding) every term reads the triangle that
 // formula_task reads, 36 MFMAs: P V with both triangles of V, V P with both of P.
-template <bool HERM, typename T, bool LM, bool ST, bool SA, int NW, typename TS>
-__device__ __attribute__((always_inline)) void eval_dermorb_in(const Smem& S, const KCtx<T, LM, ST, SA, NW, TS>& K, double sign) {
+template <bool HERM, typename T, bool LM, bool ST, bool SA, int NW>
+__device__ __attribute__((always_inline)) void eval_dermorb_in(const Smem& S, const KCtx<T, LM, ST, SA, NW>& K, double sign) {
     constexpr int NS = HERM ? 1 : 2;
     const int nw = K.n_(), lane = threadIdx.x & 63, lk = lane >> 4, li = lane & 15;
     const int nblk = (nw + 15) / 16, ntask = 3 * (nblk * (nblk + 1) / 2);
@@ -1098,8 +1099,8 @@ __device__ __attribute__((always_inline)) void eval_dermorb_in(const Smem& S, co
 // A task is a pair of 16-band blocks and one b, in two passes (V, then A and B), or the per-band terms of one c.
 // 1287 k-points at nw = 18, a narrow window: 0.94 ms one by one, 0.50 together, 0.39 with V and A in LDS
 // and the per-band terms as tasks.
-template <typename T, bool LM, bool ST, bool SA, int NW, typename TS>
-__device__ __attribute__((always_inline)) void eval_dermorb_ex(const Smem& S, const KCtx<T, LM, ST, SA, NW, TS>& K, bool in) {
+template <typename T, bool LM, bool ST, bool SA, int NW>
+__device__ __attribute__((always_inline)) void eval_dermorb_ex(const Smem& S, const KCtx<T, LM, ST, SA, NW>& K, bool in) {
     const int nw = K.n_(), tid = threadIdx.x, lane = tid & 63, lk = lane >> 4, li = lane & 15;
     const int nblk = (nw + 15) / 16, ntask = 6 * (nblk * (nblk + 1) / 2);
     const double win = in ? 1.0 : 0.0;
@@ -1321,8 +1322,8 @@ __device__ __attribute__((always_inline)) void eval_dermorb_ex(const Smem& S, co
 // Morb_Hpm (formula/covariant.py:390-414), every needed cut into S.cut: the sums over l outside are
 // pair values, those over m inside are r(max(n, m)).  One wave per pair of 16-band blocks.
 // 294 k-points at nw = 64, every cut: 1.72 ms with a loop over l per cut and band, 0.028 ms.
-template <typename T, bool LM, bool ST, bool SA, int NW, typename TS>
-__device__ __attribute__((always_inline)) void eval_morb_cuts(const Smem& S, const KCtx<T, LM, ST, SA, NW, TS>& K, bool in, bool ex,
+template <typename T, bool LM, bool ST, bool SA, int NW>
+__device__ __attribute__((always_inline)) void eval_morb_cuts(const Smem& S, const KCtx<T, LM, ST, SA, NW>& K, bool in, bool ex,
                                                              double sign) {
     const int nw = K.n_(), tid = threadIdx.x, lane = tid & 63, lk = lane >> 4, li = lane & 15;
     const int nblk = (nw + 15) / 16;
@@ -1387,8 +1388,8 @@ __device__ __attribute__((always_inline)) void eval_morb_cuts(const Smem& S, con
 // 255 -> 105 us complex128, 127 -> 100 complex64; 5832 at nw = 24 172 -> 90 and 95 -> 78; 3375 at nw = 48
 // 540 -> 201 and 490 -> 193.  Velocity products (one thread per (n, a, b), each Omega or Morb_Hpm element formed
 // for every a and both orders) of 1331 k-points at nw = 18: 105 -> 28 (Omega), 186 -> 41 us (Morb_Hpm).
-template <bool MORB, typename T, bool LM, bool ST, bool SA, int NW, typename TS>
-__device__ __attribute__((always_inline)) void diag_traces(const Smem& S, const KCtx<T, LM, ST, SA, NW, TS>& K, bool in, bool ex, double sign,
+template <bool MORB, typename T, bool LM, bool ST, bool SA, int NW>
+__device__ __attribute__((always_inline)) void diag_traces(const Smem& S, const KCtx<T, LM, ST, SA, NW>& K, bool in, bool ex, double sign,
                                                           bool single) {
     const int nw = K.n_(), lane = threadIdx.x & 63, nwave = (int)blockDim.x >> 6;
     const int n8 = (nw + 7) / 8, split = min(max(nwave / n8, 1), n8);  // waves that share 8 rows
@@ -1454,8 +1455,8 @@ __device__ __attribute__((always_inline)) void diag_traces(const Smem& S, const 
 
 // Products with the velocity, acc[n][a][b] = Re sum_{m in G} V^a_nm H^b_mn: groups of one band from their
 // diagonal elements H^b_nn in acc[n][b], larger ones from H(b, m, n)
-template <typename T, bool LM, bool ST, bool SA, int NW, typename TS, class FH>
-__device__ __attribute__((always_inline)) void vel_times(const Smem& S, const KCtx<T, LM, ST, SA, NW, TS>& K, FH H) {
+template <typename T, bool LM, bool ST, bool SA, int NW, class FH>
+__device__ __attribute__((always_inline)) void vel_times(const Smem& S, const KCtx<T, LM, ST, SA, NW>& K, FH H) {
     const int nw = K.n_(), tid = threadIdx.x;
     __syncthreads();
     for (int n = tid; n < nw; n += (int)blockDim.x) {
@@ -1484,8 +1485,8 @@ __device__ __attribute__((always_inline)) void vel_times(const Smem& S, const KC
 
 // Per-band values for the current partition (the labels'; cut >= 0: they are those of [0, cut), and M
 // holds the unmasked dEinv) into S.acc[n][comp].
-template <int F, typename T, bool LM, bool ST, bool SA, int NW, typename TS>
-__device__ __attribute__((always_inline)) void eval_partition(const Smem& S, const KCtx<T, LM, ST, SA, NW, TS>& K, const wbmi_scan_params& p, int cut = -1) {
+template <int F, typename T, bool LM, bool ST, bool SA, int NW>
+__device__ __attribute__((always_inline)) void eval_partition(const Smem& S, const KCtx<T, LM, ST, SA, NW>& K, const wbmi_scan_params& p, int cut = -1) {
     const int nw = K.n_();
     const int tid = threadIdx.x;
     const bool in = p.internal_terms, ex = p.external_terms;
@@ -1848,13 +1849,12 @@ k_static_scan(ScanArgs args, const double* __restrict__ Eall, const cplx<T>* __r
     if (MODE != 2) hist += k * args.hist_stride;
     constexpr bool tasks = F == WBMI_FORMULA_DEROMEGA || F == WBMI_FORMULA_DERMORB;
     static_assert(tasks || SC_IS_DERMORB_CUTS(F) || !ST, "V and A are staged for DerOmega and DerMorb");
-    using TS = T;
     constexpr bool SA = ST;
     constexpr bool stage_v = ST;
     const bool stage_a = SA && p.external_terms;
     constexpr bool tetra = MODE == 1;  // compile-time: the Fermi-bin kernels carry no tetrahedron code
     constexpr bool tab = MODE == 2;
-    const Smem S = make_smem(smem_raw, nw, LM, stage_v, stage_a, tetra, sizeof(cplx<TS>));
+    const Smem S = make_smem(smem_raw, nw, LM, stage_v, stage_a, tetra, sizeof(cplx<T>));
     for (int n = tid; n < nw; n += (int)blockDim.x) S.E[n] = Eall[k * nw + n];
     for (int r = tid; r < WBMI_NROLES; r += (int)blockDim.x) S.ch[r] = p.ch[r];
     if (tetra)
@@ -2021,7 +2021,7 @@ k_static_scan(ScanArgs args, const double* __restrict__ Eall, const cplx<T>* __r
     const int ng = S.misc[0];
     const int sea_lo = S.misc[1], sea_hi = S.misc[2];
 
-    KCtx<T, LM, ST, SA, NW, TS> K;
+    KCtx<T, LM, ST, SA, NW> K;
     K.X = Xk;
     K.nw = nw;
     K.ld = ld;
@@ -2031,8 +2031,8 @@ k_static_scan(ScanArgs args, const double* __restrict__ Eall, const cplx<T>* __r
     K.lab = S.lab;
     K.gs = S.gs;
     K.ge = S.ge;
-    K.sV = (const cplx<TS>*)S.V;
-    K.sA = (const cplx<TS>*)S.A;
+    K.sV = (const cplx<T>*)S.V;
+    K.sA = (const cplx<T>*)S.A;
     K.bv = (const double*)(const void*)Xall + k * (int64_t)nw * args.nch;
     K.nbv = args.nch;
     K.parts = parts;
