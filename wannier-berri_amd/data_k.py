@@ -87,6 +87,13 @@ def r_pairs(iRvec):
     """The R-vectors as pairs, int32 [npair, 2]: (i, j) with R_j = -R_i, (i, -1) for one without a
     partner (R = 0, a missing -R, repeated vectors beyond the first match)."""
     R = np.asarray(iRvec).reshape(-1, 3)
+    n = len(R)
+    if np.array_equal(R, -R[::-1]):   # in the usual order -R stands where R does from the end
+        i = np.arange((n + 1) // 2, dtype=np.int32)
+        pairs = np.stack([i, n - 1 - i], axis=1)
+        if n % 2:
+            pairs[-1, 1] = -1   # R = 0
+        return pairs
     span = 2 * int(np.abs(R).max(initial=0)) + 1
     if len(R) and span < 1 << 20:
         key = R @ np.array([span * span, span, 1], dtype=np.int64)   # one number per vector, -R's is its negative
@@ -331,12 +338,25 @@ class Data_K:
             self._requested |= set(self._slots)
         self._evaluate(sorted(self._requested, key=CHANNEL_ORDER.index))
 
+    def _klist_on_device(self):
+        if self.k_list_dev is not None:
+            return self.k_list_dev
+        # a pageable copy waits for the work queued before it, one through pinned memory does not (but costs more
+        # where nothing is queued); the latter is ordered before the transform only on the transform's own stream
+        kl = self.torch.from_numpy(self.k_list)
+        ahead = self.torch.cuda.current_stream(self.ctx.device) == self.ctx.stream and not self.ctx.stream.query()
+        return (kl.pin_memory() if ahead else kl).to(self.ctx.device, non_blocking=ahead)
+
     def _transform(self, keys, dtype, prec, shift=None, keep=None, out=None):
         """R -> k of the channel keys into `out` or a new [nk, nch, nw, nw] tensor (grid blocks:
         at the points j/NKFFT + dK, or + shift in place of dK).  `keep`: a list that takes the
         work buffer instead of freeing it (work launched on another stream)."""
         torch = self.torch
         nw, nk = self.num_wann, self.nk
+        kl = pairs = None
+        if self.k_list is not None:
+            # before the stack is built, which a copy would wait for
+            kl, pairs = self._klist_on_device(), self.dev.pairs_dev
         stack = self.dev.stack(keys)
         X = out
         if X is None:
@@ -356,15 +376,7 @@ class Data_K:
                 keep.extend([work, box])
             del work
         else:
-            kl = self.k_list_dev
-            if kl is None:
-                # a pageable copy waits for the work queued before it, one through pinned memory does not; the
-                # latter is ordered before the transform only on the transform's own stream
-                kl = torch.from_numpy(self.k_list)
-                own = torch.cuda.current_stream(self.ctx.device) == self.ctx.stream
-                ahead = own and not self.ctx.stream.query()
-                kl = (kl.pin_memory() if ahead else kl).to(self.ctx.device, non_blocking=ahead)
-            self.ctx.r2k_klist(self.dev.iRvec_dev, stack, kl, X, prec, pairs=self.dev.pairs_dev)
+            self.ctx.r2k_klist(self.dev.iRvec_dev, stack, kl, X, prec, pairs=pairs)
         return X
 
     def _channel_keys(self):
