@@ -237,17 +237,19 @@ def test_scan_diagonal_traces(nw, precision, kramers):
         assert err <= (1e-9 if precision == "fp64" else 2e-5) * scale, name
 
 
-def _off_mirror(nw, external):
+def _off_mirror(nw, external, group=1):
     """Complex64 channels of two k-points with V Hermitian to storage rounding only: one element of the
     matrix before its rotation is off its mirror, so every element after it is, the diagonal among them.  Every
-    band a group of its own in a bin of its own, two bands 4e-3 apart.  Returns the channels (V, W; A, A',
-    rotA, rotA'), E, bin width, bins, and the oracle's K-block on the same stored matrices."""
+    `group` bands (5e-5 apart) a group in a bin of its own, two groups 4e-3 apart.  Returns the channels (V, W;
+    A, A', rotA, rotA'), E, bin width, the bin of each band, and the oracle's K-block on the same stored matrices."""
     from oracle import wb_oracle as O
     rng = np.random.default_rng(nw)
     nk, dEF = 2, 2e-3
-    step = np.full((nk, nw), 125)
-    step[:, nw // 2] = 2
-    level = np.cumsum(step + (step > 2) * rng.integers(0, 9, (nk, nw)), axis=1)   # the bin of each band
+    ng = -(-nw // group)
+    step = np.full((nk, ng), 125)
+    step[:, ng // 2] = 2
+    level = np.cumsum(step + (step > 2) * rng.integers(0, 9, (nk, ng)), axis=1)   # the bin of each group
+    level = np.repeat(level, group, axis=1)[:, :nw]
     def herm(n):
         x = rng.standard_normal((nk, n, nw, nw)) + 1j * rng.standard_normal((nk, n, nw, nw))
         return (0.5 * (x + x.conj().swapaxes(2, 3))).astype(np.complex64).astype(complex)
@@ -259,7 +261,7 @@ def _off_mirror(nw, external):
     X = (U.conj().swapaxes(1, 2)[:, None] @ X @ U[:, None]).astype(np.complex64)
     if external:
         X = np.concatenate([X, herm(24).astype(np.complex64)], axis=1)
-    E = (level - 0.5) * dEF
+    E = (level - 0.5) * dEF + 5e-5 * (np.arange(nw) % group)
     x = np.moveaxis(X.astype(complex), 1, 3)
     bar = {("Ham", 1): x[..., :3], ("Ham", 2): x[..., 3:12].reshape(nk, nw, nw, 3, 3)}
     if external:
@@ -323,38 +325,40 @@ def test_scan_velocity_off_its_mirror(ctx, nw):
         assert err < 1e-12, formula
 
 
-@pytest.mark.parametrize("nw", [7, 16, 32, 33, 70])
-def test_scan_velocity_off_its_mirror_external(ctx, nw):
-    """DerOmega with external terms on such channels.  What the kernel reads as Hermitian is so in the reference:
-    the product V D' of dD.nl = -(dD.ln)^+ (its within-group part has V_nn V_nl as stored), and the real part
-    of dO.nn."""
+@pytest.mark.parametrize("nw,group", [(7, 1), (16, 1), (32, 1), (33, 1), (70, 1), (7, 2), (18, 2), (32, 4), (33, 2), (70, 3)])
+def test_scan_velocity_off_its_mirror_external(ctx, nw, group):
+    """DerOmega with external terms on such channels, in groups of one band and of a few.  What the kernel reads
+    as Hermitian is so in the reference: the product V D' of dD.nl = -(dD.ln)^+ (its within-group part has
+    V''_nq D'_ql as stored), and the real part of dO.nn."""
     from oracle import wb_oracle as O
     from wannierberri_amd import _lib
-    X, E, dEF, level, d = _off_mirror(nw, True)
+    X, E, dEF, level, d = _off_mirror(nw, True, group)
     f = O.DerOmega(d)
     V, W, Dh, m = d.Xbar("Ham", 1), d.Xbar("Ham", 2), d.D_H, d.dEig_inv
 
     class DerD(O.DerDcov):
-        def nl(self, ik, inn, out):   # one band n inside
-            n = inn[0]
-            pv = np.einsum("lpb,pd->lbd", V[ik][out][:, out], Dh[ik][out, n])
-            own = np.einsum("b,ld->lbd", V[ik][n, n], V[ik][n, out]) * m[ik][out, n][:, None, None]
-            s = (W[ik][out, n] + pv + pv.swapaxes(1, 2)).conj() + own + own.swapaxes(1, 2)
-            return (m[ik][out, n][:, None, None] * s)[None]
+        def nl(self, ik, inn, out):
+            pv = np.einsum("lpb,pnd->lnbd", V[ik][out][:, out], Dh[ik][out][:, inn])
+            own = np.einsum("nqb,qld->lnbd", V[ik][inn][:, inn], Dh[ik][inn][:, out])
+            s = (W[ik][out][:, inn] + pv + pv.swapaxes(2, 3)).conj() + own + own.swapaxes(2, 3)
+            return (m[ik][out][:, inn][:, :, None, None] * s).swapaxes(0, 1)
 
-    class DerO:
+    class DerO:   # the diagonal, which a trace reads
         def nn(self, ik, inn, out):
-            n = inn[0]
             o, do = d.Xbar("rotAA")[ik], d.Xbar("rotAA", 1)[ik]
-            return (do[n, n] + 2 * np.einsum("lc,ld->cd", o[out, n].conj(), Dh[ik][out, n])).real[None, None]
+            diag = (do[inn, inn] + 2 * np.einsum("lnc,lnd->ncd", o[out][:, inn].conj(), Dh[ik][out][:, inn])).real
+            return np.eye(len(inn))[:, :, None, None] * diag[:, None]
     f.dD, f.dO = DerD(d), DerO()
     hist = _scan_bins(ctx, X, E, dEF, level, _lib.FORMULA_DEROMEGA, True)
     ref = np.zeros_like(hist)
+    bands = np.arange(nw)
     for ik in range(len(E)):
-        for n in range(nw):
-            ref[level[ik, n]] += f.trace(ik, np.array([n]), np.delete(np.arange(nw), n)).reshape(9)
+        for g in np.unique(bands // group):
+            inn = bands[bands // group == g]
+            e = E[ik, inn].mean()
+            ref[int(np.ceil(e / dEF))] += f.trace(ik, inn, np.delete(bands, inn)).reshape(9)
     err = np.abs(hist - ref).max() / np.abs(ref).max()
-    print(f"test_scan_velocity_off_its_mirror_external nw={nw}: {err:.1e}", flush=True)
+    print(f"test_scan_velocity_off_its_mirror_external nw={nw} group={group}: {err:.1e}", flush=True)
     assert err < 1e-12   # as above
 
 

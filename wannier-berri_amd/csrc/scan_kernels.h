@@ -568,10 +568,20 @@ __device__ __attribute__((always_inline)) void formula_task(const Smem& S, const
                     if (!big) z += mln * (K.Vu(b, n, n) * K.Vu(d, l, n));
                     if constexpr (DM) z += P2.get(bj, v);
                     const cplx<double> Pm = (-mln) * (pv + z);
-                    // -conj dD.nl: its within-group part from V's other triangle, as stored, in groups of one band
+                    // -conj dD.nl: its within-group part from V's other triangle, as stored, in groups of up to SC_T4_LOOP bands
                     cplx<double> Pn = Pm;
                     if constexpr (sizeof(T) == 4)
-                        if (ex && !big) Pn = (-mln) * (pv + 0.5 * gz[bj][v] + mln * conj(K.Vu(b, n, n) * K.Vu(d, n, l)));
+                        if (ex) {
+                            if (!big) {
+                                Pn = (-mln) * (pv + 0.5 * gz[bj][v] + mln * conj(K.Vu(b, n, n) * K.Vu(d, n, l)));
+                            } else if (S.ge[n] - S.gs[n] <= SC_T4_LOOP) {
+                                cplx<double> c = mk(0.0, 0.0);
+#pragma unroll 1
+                                for (int q = S.gs[n]; q < S.ge[n]; ++q)
+                                    c += K.m(l, q) * (conj(K.Vu(b, n, q) * K.Vu(d, q, l)) - K.Vu(d, l, q) * K.Vu(b, q, n));
+                                Pn = Pm - mln * c;
+                            }
+                        }
                     const double wD = in ? (dm ? dw + 2.0 * K.E[l] : dw) : 0.0;
 #pragma unroll
                     for (int a = 0; a < 3; ++a) {
