@@ -101,7 +101,7 @@ __global__ void __launch_bounds__(64 * ROTR_WAVES, NB == 1 ? 4 : sizeof(T) == 8 
 #pragma unroll
         for (int bi = 0; bi < NB; ++bi) {
             // 16 rows of X as the A operand (its Hermitian part when flagged): step s of lane group g is
-            // k = 4 J (s / J) + J g + s % J, J consecutive elements a lane (128 bytes of a row per load group)
+            // k = 4 J (s / J) + J g + s % J, J consecutive elements a lane (complex128: 128 bytes of a row per load group)
             cplx<T> x[NS], w[NS];
             const int r = 16 * bi + li;
 #pragma unroll
